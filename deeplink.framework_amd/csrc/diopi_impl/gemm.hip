@@ -94,6 +94,9 @@ struct MfmaArgs {
   int colScaleDtype = 0;
   const void* colBias = nullptr;
   int colBiasDtype = 0;
+  // 4-wave kernel, K-split tail: the first wholeTiles tiles of the order are multiplied whole, each of the others in
+  // kSlices slices of K whose accumulators go to partial (see gemmMfma4WaveKernel)
+  int wholeTiles = 0, kSlices = 1;
 };
 
 constexpr int kBK = 64;  // K elements per LDS tile (128-byte rows)
@@ -317,6 +320,7 @@ struct MfmaOp16<half_t> {
 // kEpiAddendLds (4-wave kernel only) is kEpiLinear with an addend whose pieces for an output tile's first two fragment
 // rows wait in LDS when the epilogue starts (see addendToLds).
 enum PipeEpilogue { kEpiLinear = 0, kEpiSiluMul = 1, kEpiPartial = 2, kEpiRotary = 3, kEpiRotaryUniform = 4, kEpiRotaryLds = 5, kEpiAddendLds = 6, kEpiColScale = 7 };
+constexpr int kTailSlotFloats = 256 * 256;  // accumulators of one K slice of a tile
 constexpr int kAddendLdsBytes = 32768;  // behind the two K-tile stages of the 4-wave kernel: 4 waves x 32 rows x 128 columns x 2 bytes
 constexpr int kRotaryLdsBytes = 32768;  // behind the two K-tile stages of the 4-wave kernel: 128 rows x (64 cos | 64 sin) x 2 bytes
 
@@ -1115,20 +1119,37 @@ __device__ __forceinline__ void accRegisters16(f32x4 (&f)[4]) {
     for (int r = 0; r < 4; ++r) f[q][r] = v[4 * q + r];
 }
 
-template <typename T, int EPI>
+// SPLIT: the last, partly filled round of tiles is cut along K. With R tiles left for C workgroups a plain last round takes
+// nearly as long as a full one while C - R compute units idle, which is up to half of a launch of a few rounds. Here the
+// first g.wholeTiles tiles (whole rounds, or none) are multiplied as before and each of the R others in g.kSlices slices of
+// consecutive K-tile pairs, dealt over all workgroups (4525 x 4096 x 14336: 533 -> 369 us; see tailSplit). A slice's accumulators leave in the layout they
+// have in the registers, 1 KiB of consecutive bytes per store instruction, to a slot of 256 x 256 fp32 of its own, and
+// tailReduceKernel adds the slices of a tile and applies the epilogue. (A reduction by the workgroup that finishes last
+// would run on R compute units, each at the rate one of them can read.) The slices are dealt out slice by slice, so the
+// workgroups of one XCD read the same stretch of K of neighbouring tiles.
+template <typename T, int EPI, bool SPLIT = false>
 __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
   constexpr int BM = 256, BN = 256, WM = 128, WN = 128, TM = 8, TN = 8;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
-  const int total = g.tilesM * g.tilesN;
+  const int whole = SPLIT ? g.wholeTiles : g.tilesM * g.tilesN;
+  const int rest = SPLIT ? g.tilesM * g.tilesN - whole : 0;
+  const int total = SPLIT ? whole + rest * g.kSlices : whole;  // items of work: whole tiles, then slices
   // Persistent: the workgroup takes output tiles blockIdx.x, blockIdx.x + gridDim.x, ... (the grid is a multiple of
   // 8 or covers every tile, so a workgroup's tiles all belong to the XCD it runs on, as in the one-tile-per-workgroup
   // order). XCD x works on a contiguous band of tiles, walked in groups of 8 tile rows.
-  auto tileOf = [&](int pid, int& tm, int& tn) {
-    const int xcd = pid & 7, idx = pid >> 3;
-    const int q = total >> 3, r = total & 7;
-    const int logical = xcd * q + min(xcd, r) + idx;
+  auto tileOf = [&](int pid, int& tm, int& tn, int& slice) {
+    const bool tail = SPLIT && pid >= whole;
+    const int item = tail ? pid - whole : pid, items = tail ? total - whole : whole;
+    const int xcd = item & 7, idx = item >> 3;
+    const int q = items >> 3, r = items & 7;
+    int logical = xcd * q + min(xcd, r) + idx;
+    slice = -1;
+    if (tail) {
+      slice = logical / rest;
+      logical += whole - slice * rest;
+    }
     constexpr int GROUP = 8;
     const int width = GROUP * g.tilesN;
     const int group = logical / width;
@@ -1137,6 +1158,7 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
     const int in = logical - group * width;
     tm = first + in % gsize;
     tn = in / gsize;
+    if (tail) slice += (logical - whole) * g.kSlices;  // slot of this slice: the slices of a tile lie side by side
   };
   const int batch = blockIdx.z;
   const T* A = reinterpret_cast<const T*>(g.A) + (int64_t)batch * g.sAb;
@@ -1160,7 +1182,14 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
     return l;
   };
   unsigned voA[8], voB[8];
-  auto laneOffsets = [&](int tm, int tn) {
+  const int pairs = g.K / (2 * kBK);
+  // K-tile pairs of a slice: the first pairs % kSlices slices have one more than the others
+  auto slicePairs = [&](int slot, int* firstPair) {
+    const int s = slot % g.kSlices, per = pairs / g.kSlices, more = pairs - per * g.kSlices;
+    *firstPair = s * per + min(s, more);
+    return per + (s < more ? 1 : 0);
+  };
+  auto laneOffsets = [&](int tm, int tn, int k0) {
     // recomputed on every call from the lane number the hardware hands out: the eight row numbers and the chunk
     // offset (or the thread index they come from) would otherwise be kept live across the K loop, whose text owns
     // v120-v247, and spilled; a reload between two pieces of that text waits for every tile load in flight (loads
@@ -1171,8 +1200,8 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int ra = tm * BM + srow + 32 * i, rb = tn * BN + srow + 32 * i;
-      voA[i] = ra < g.M ? (unsigned)(((int64_t)ra * g.lda + c8) * 2) : kFar;
-      voB[i] = rb < g.N ? (unsigned)(((int64_t)rb * g.ldb + c8) * 2) : kFar;
+      voA[i] = ra < g.M ? (unsigned)(((int64_t)ra * g.lda + c8 + k0) * 2) : kFar;
+      voB[i] = rb < g.N ? (unsigned)(((int64_t)rb * g.ldb + c8 + k0) * 2) : kFar;
     }
   };
   const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem;
@@ -1182,7 +1211,6 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
   const unsigned adA1 = base + ((wm * WM + frow) * kBK + (((4 + kq) ^ swz) << 3)) * 2;
   const unsigned adB0 = base + 65536 + ((wn * WN + frow) * kBK + ((kq ^ swz) << 3)) * 2;
   const unsigned adB1 = base + 65536 + ((wn * WN + frow) * kBK + (((4 + kq) ^ swz) << 3)) * 2;
-  const int pairs = g.K / (2 * kBK);
   unsigned kcur = 0, m0s = 0;
   T* out = reinterpret_cast<T*>(g.out) + (int64_t)batch * g.sOb;
   const T* cin = g.Cin ? reinterpret_cast<const T*>(g.Cin) + (int64_t)batch * g.sCb : nullptr;
@@ -1202,33 +1230,59 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
     else                                                                         \
       asm volatile(GEMM4W_##NAME##_F16 GEMM4W_OPERANDS);                         \
   } while (0)
-  int pid = blockIdx.x, tm, tn;
-  tileOf(pid, tm, tn);
-  laneOffsets(tm, tn);
+  int pid = blockIdx.x, tm, tn, slot = -1, itemPairs = pairs, k0 = 0;
+  tileOf(pid, tm, tn, slot);
+  if constexpr (SPLIT) {
+    if (slot >= 0) itemPairs = slicePairs(slot, &k0);
+  }
+  laneOffsets(tm, tn, k0 * 2 * kBK);
   bool first = true;
   while (true) {
     if (first)
       GEMM4W_RUN(PROLOGUE);
     else
       GEMM4W_RUN(PROLOGUE_LOADED);
-    for (int p = 1; p < pairs; ++p) GEMM4W_RUN(BODY);
+    for (int p = 1; p < itemPairs; ++p) GEMM4W_RUN(BODY);
     // (rotary tables through LDS: this output tile's entries are copied now, behind every tile load of its K loop; tiles
     // of v heads need none; the decision is the same for the whole workgroup)
     if constexpr (EPI == kEpiRotaryLds) {
-      if (tn * BN < g.rotCols) rotaryTablesToLds<T>(g, tm * BM, waveS, laneNow(), base + 131072u);
+      if (tn * BN < g.rotCols && slot < 0) rotaryTablesToLds<T>(g, tm * BM, waveS, laneNow(), base + 131072u);
     }
     // (addend through LDS: every wave copies the addend of its own first two fragment rows, likewise behind the tile loads)
     if constexpr (EPI == kEpiAddendLds)
-      addendToLds<T>(g, cin, tm * BM + (waveS >> 1) * WM, tn * BN + (waveS & 1) * WN, laneNow(), base + 131072u + (unsigned)waveS * 8192u);
+      if (slot < 0) addendToLds<T>(g, cin, tm * BM + (waveS >> 1) * WM, tn * BN + (waveS & 1) * WN, laneNow(), base + 131072u + (unsigned)waveS * 8192u);
     const int next = pid + (int)gridDim.x;
-    int ntm = 0, ntn = 0;
+    int ntm = 0, ntn = 0, nslot = -1, npairs = pairs;
     if (next < total) {
       // the last K tile also issues the first loads of the next output tile: they land while the epilogue runs
-      tileOf(next, ntm, ntn);
-      laneOffsets(ntm, ntn);
+      tileOf(next, ntm, ntn, nslot);
+      int nk0 = 0;
+      if constexpr (SPLIT) {
+        if (nslot >= 0) npairs = slicePairs(nslot, &nk0);
+      }
+      laneOffsets(ntm, ntn, nk0 * 2 * kBK);
       GEMM4W_RUN(TAIL_NEXT);
     } else {
       GEMM4W_RUN(TAIL);
+    }
+    if constexpr (SPLIT) {
+      if (slot >= 0) {
+        const __amdgpu_buffer_rsrc_t rsP =
+            __builtin_amdgcn_make_buffer_rsrc(g.partial + (int64_t)slot * kTailSlotFloats + waveS * (kTailSlotFloats / 4), 0, kTailSlotFloats / 4 * 4, 0x00020000);
+        const int voff = laneNow() * 16;
+        staticFor<TM>([&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+          f32x4 lo[4], hi[4];
+          accRegisters16<32 * i>(lo);
+          accRegisters16<32 * i + 16>(hi);
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, j < 4 ? lo[j & 3] : hi[j & 3]), rsP, voff, (i * TN + j) * 1024, 0);
+        });
+        if (next >= total) break;
+        pid = next, tm = ntm, tn = ntn, slot = nslot, itemPairs = npairs, first = false;
+        continue;
+      }
     }
     if constexpr (EPI == kEpiRotaryLds) {
       if (tn * BN < g.rotCols) {
@@ -1259,9 +1313,48 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
     }, base + 131072u + (EPI == kEpiAddendLds ? (unsigned)waveS * 8192u : 0u));
     if (next >= total) break;
     pid = next, tm = ntm, tn = ntn, first = false;
+    if constexpr (SPLIT) slot = nslot, itemPairs = npairs;
   }
 #undef GEMM4W_RUN
 #undef GEMM4W_OPERANDS
+}
+
+// Second launch of the K-split tail: adds the slices of every tail tile in their order and applies the epilogue. A wave
+// takes 4 x 4 of the 64 fragments of one wave's quadrant, so a tile is 16 waves and each load instruction fetches the 1 KiB
+// that one store instruction of gemmMfma4WaveKernel wrote; the lanes hold what they would have held there, and the
+// epilogue is the same function.
+template <typename T, int EPI>
+__global__ __launch_bounds__(256) void tailReduceKernel(MfmaArgs g) {
+  const int lane = threadIdx.x & 63, unit = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  const int tile = unit >> 4, quadrant = (unit >> 2) & 3, ih = (unit >> 1) & 1, jh = unit & 1;
+  const float* src = g.partial + (int64_t)tile * g.kSlices * kTailSlotFloats + quadrant * (kTailSlotFloats / 4) + (ih * 4 * 8 + jh * 4) * 256 + lane * 4;
+  f32x4 acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = *reinterpret_cast<const f32x4*>(src + (i * 8 + j) * 256);
+  for (int s = 1; s < g.kSlices; ++s) {
+    src += kTailSlotFloats;
+    f32x4 v[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[i][j] = *reinterpret_cast<const f32x4*>(src + (i * 8 + j) * 256);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] += v[i][j];
+  }
+  constexpr int GROUP = 8;
+  const int logical = g.wholeTiles + tile, width = GROUP * g.tilesN, group = logical / width, firstRow = group * GROUP;
+  const int gsize = min(g.tilesM - firstRow, GROUP), in = logical - group * width;
+  const int tm = firstRow + in % gsize, tn = in / gsize;
+  vectorEpilogue<T, EPI, 4, 4>(g, reinterpret_cast<T*>(g.out), reinterpret_cast<const T*>(g.Cin), reinterpret_cast<const T*>(g.bias),
+                               tm * 256 + (quadrant >> 1) * 128 + ih * 64, tn * 256 + (quadrant & 1) * 128 + jh * 64, lane & 15, lane >> 4,
+                               [&](auto ic, f32x4(&row)[4]) {
+#pragma unroll
+                                 for (int j = 0; j < 4; ++j) row[j] = acc[decltype(ic)::value][j];
+                               });
 }
 
 // ------------------------------------------------------------ skinny M (decode) ---
@@ -2248,9 +2341,54 @@ struct RotaryEpilogue {
   float sinSign;
 };
 
+// How the tiles of a 4-wave launch are worked off: whole tiles first, the rest in K slices (slices == 1: no split), and
+// what the rest then costs in us.
+struct TailSplit {
+  int whole, slices;
+  float us;
+};
+
+// The number of slices with the least estimated time. Fitted to launches of 16 to 432 tiles at K = 4096 ... 14336: a pair
+// of K tiles takes 2.0 us with few CUs at work and 2.5 - 2.8 with all (the power limit), a slice's 256 KiB of accumulators
+// cost 0.07 - 0.1 us of the chip's time to write and read back, the second launch and the start of the slices about 12 us.
+// A plain last round is replaced only where that saves a twentieth of it. Measured, plain -> split (us):
+//   4525 x 4096 x 14336 (288 tiles, 32 left, 8 slices) 533 -> 369      4525 x 4096 x 4096 (4 slices) 151 -> 122
+//   1554 x 11008 x 4096 (301 tiles, 45 left, 4 slices) 145 -> 127      1554 x 12288 x 4096 rotary (80 left) 158 -> 143
+//   6001 x 4096 x 14336 (384 tiles, 128 left, 2 slices) 568 -> 490     6001 x 4096 x 4096 (128 left) 166 -> 170: stays plain
+//   5000 x 5120 x 13824 (400 tiles, 144 left, 3 slices in two rounds) 551 -> 525
+static TailSplit tailSplit(int64_t tiles, int64_t pairs, int resident) {
+  const int rest = (int)(tiles % resident), most = (int)std::min<int64_t>(rest ? 2 * resident / rest : 0, pairs / 2);
+  const float share = (float)rest / resident;
+  TailSplit best = {(int)tiles, 1, rest ? pairs * (2.f + 0.8f * share) * 0.95f : 0.f};
+  for (int s = 2; s <= most; ++s) {
+    const float us = 12.f + ceilDiv(rest * s, resident) * ceilDiv(pairs, (int64_t)s) * (1.95f + 0.5f * std::min(1.f, share * s)) + 0.08f * rest * s;
+    if (us < best.us) best = {(int)tiles - rest, s, us};
+  }
+  return best;
+}
+
+template <typename T, int EPI>
+static diopiError_t launchTailSplit(diopiContextHandle_t ctx, hipStream_t stream, MfmaArgs g, const TailSplit& tail, int resident) {
+  const int rest = g.tilesM * g.tilesN - tail.whole, items = rest * tail.slices;
+  void* ws = nullptr;
+  AMD_TRY(requireWorkspace(ctx, (int64_t)items * kTailSlotFloats * 4, &ws));
+  g.partial = static_cast<float*>(ws), g.wholeTiles = tail.whole, g.kSlices = tail.slices;
+  // a launch with whole tiles has one workgroup per CU (whole is a multiple of that); one of slices alone has one per slice
+  const dim3 grid((unsigned)(tail.whole ? resident : std::min(items, resident)));
+  constexpr size_t lds = 2 * (size_t)(256 + 256) * kBK * sizeof(T) +
+                         (EPI == kEpiRotaryLds ? kRotaryLdsBytes : EPI == kEpiAddendLds ? kAddendLdsBytes : 0);
+  AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(&gemmMfma4WaveKernel<T, EPI, true>), (int)lds));
+  hipLaunchKernelGGL((gemmMfma4WaveKernel<T, EPI, true>), grid, dim3(256), lds, stream, g);
+  AMD_LAUNCH_CHECK();
+  constexpr int kReduceEpi = EPI == kEpiRotaryLds ? (int)kEpiRotaryUniform : EPI == kEpiAddendLds ? (int)kEpiLinear : EPI;
+  hipLaunchKernelGGL((tailReduceKernel<T, kReduceEpi>), dim3((unsigned)(rest * 4)), dim3(256), 0, stream, g);
+  AMD_LAUNCH_CHECK();
+  return diopiSuccess;
+}
+
 // bT: the second operand is [K, N] with N contiguous and is used in place (p.sBk is then its row stride).
 template <typename T, int EPI = kEpiLinear>
-static diopiError_t launchMfmaPipelined(hipStream_t stream, const GemmProblem& p, float* partial = nullptr, int splits = 1,
+static diopiError_t launchMfmaPipelined(diopiContextHandle_t ctx, hipStream_t stream, const GemmProblem& p, float* partial = nullptr, int splits = 1,
                                         int kTilesPerSplit = 0, const RotaryEpilogue* rot = nullptr, bool bT = false) {
   MfmaArgs g;
   g.A = p.A, g.B = p.B, g.out = p.out, g.Cin = p.Cin, g.bias = p.bias;
@@ -2295,6 +2433,15 @@ static diopiError_t launchMfmaPipelined(hipStream_t stream, const GemmProblem& p
     if (g.vecEpilogue && p.K % (2 * kBK) == 0 && p.M * p.sAm * 2 < (int64_t(1) << 31) && p.N * p.sBn * 2 < (int64_t(1) << 31)) {
       // one workgroup per CU (its LDS ring takes most of a CU's), each walking its share of the tiles
       const int resident = computeUnits() / 8 * 8;
+      if (p.batch == 1 && resident >= 8) {
+        const TailSplit tail = tailSplit((int64_t)g.tilesM * g.tilesN, p.K / (2 * kBK), resident);
+        if (tail.slices > 1) {
+          if constexpr (EPI == kEpiLinear) {
+            if (p.Cin) return launchTailSplit<T, kEpiAddendLds>(ctx, stream, g, tail, resident);
+          }
+          return launchTailSplit<T, EPI>(ctx, stream, g, tail, resident);
+        }
+      }
       if (resident >= 8 && (int)grid.x > resident) grid.x = (unsigned)resident;
       if constexpr (EPI == kEpiLinear) {
         if (p.Cin) {
@@ -2585,13 +2732,39 @@ diopiError_t transposeCopy(hipStream_t stream, void* dst, const void* src, int i
   return launchTranspose<uint32_t>(stream, dst, src, batch, rows, cols, sRow, sCol, sBatch);
 }
 
+// Whether a product with too few 256 x 256 tiles for a round of the chip runs faster as K slices of such tiles than on the
+// 128 x 128 kernel (itself split over K when its tiles are few): a long K, or a round's worth of slices that leaves each
+// of them a dozen K-tile pairs. The 128 x 128 kernel takes 0.75 us per K tile with one workgroup on a CU and 1.19 with
+// two, and its slices are written and read back as fp32 too. Measured, 128 x 128 -> slices of 256 x 256 (us):
+// 882 x 5120 x 13824 185 -> 116 (3 slices), 512 x 4096 x 11008 70 -> 56 (8), 512 x 12288 x 4096 73 -> 63 (2),
+// 203 x 12288 x 4096 48 -> 42 (5); not taken: 882 x 4096 x 4096 38 against 42, 300 x 4096 x 11008 48 against 52.
+static bool tailSplitPays(const GemmProblem& p) {
+  const int resident = computeUnits() / 8 * 8;
+  const int64_t tiles = ceilDiv(p.M, 256) * ceilDiv(p.N, 256), kTiles = p.K / kBK;
+  const bool vec = p.N % 8 == 0 && mult8(p.sOm) && ptr16(p.out) && ((p.M - 1) * p.sOm + p.N) * 2 < (int64_t(1) << 31) &&
+                   (!p.Cin || (p.sCn == 1 && mult8(p.sCm) && ptr16(p.Cin) && ((p.M - 1) * p.sCm + p.N) * 2 < (int64_t(1) << 31))) &&
+                   (!p.bias || ptr16(p.bias));
+  if (p.batch != 1 || p.K % (2 * kBK) != 0 || !vec || tiles >= resident || p.M * p.sAm * 2 >= (int64_t(1) << 31) ||
+      p.N * p.sBn * 2 >= (int64_t(1) << 31))
+    return false;
+  const TailSplit split = tailSplit(tiles, p.K / (2 * kBK), resident);
+  if (split.slices == 1) return false;
+  int per = (int)kTiles;
+  const int64_t tiles128 = ceilDiv(p.M, 128) * ceilDiv(p.N, 128);
+  const int ways = p.M * p.N * 4 < (int64_t(1) << 31) ? splitKWays(tiles128, kTiles, &per) : 1;
+  const float wgs = (float)(tiles128 * ways) / resident;  // workgroups per CU
+  const float us128 = (wgs <= 1.f ? 0.75f : wgs <= 2.f ? 0.75f + 0.44f * (wgs - 1.f) : 0.6f * wgs) * per +
+                      (ways > 1 ? 6.f + (float)(p.M * p.N) * ways * 1.6e-6f : 2.f);
+  return split.us < 0.95f * us128;
+}
+
 bool gemmAppliesColumnScale(const GemmProblem& p) {
   // the conditions under which runGemm below reaches the 4-wave kernel without touching the operands
   const bool half = p.dtype == diopi_dtype_bfloat16 || p.dtype == diopi_dtype_float16;
   if (!half || p.batch != 1 || p.Cin || p.bias || p.K <= 0 || p.M >= (int64_t(1) << 31) || p.N >= (int64_t(1) << 31)) return false;
   if (p.sAk != 1 || !mult8(p.sAm) || !ptr16(p.A) || p.sBk != 1 || !mult8(p.sBn) || !ptr16(p.B)) return false;
   if (p.M <= kSkinnyMaxM) return false;
-  const bool big = ceilDiv(p.M, 256) * ceilDiv(p.N, 256) >= 144 && p.N > 128 && p.K > 2 * kBK;
+  const bool big = (ceilDiv(p.M, 256) * ceilDiv(p.N, 256) >= 144 || tailSplitPays(p)) && p.N > 128 && p.K > 2 * kBK;
   const bool fits2g = ((p.M - 1) * p.sAm + p.K) * 2 < (int64_t(1) << 31) && ((p.N - 1) * p.sBn + p.K) * 2 < (int64_t(1) << 31);
   if (!big || p.K % (2 * kBK) != 0 || !fits2g) return false;
   const bool vec = p.N % 8 == 0 && p.sOm % 8 == 0 && ptr16(p.out) && ((p.M - 1) * p.sOm + p.N) * 2 < (int64_t(1) << 31);
@@ -2640,14 +2813,14 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
     // (a matrix at most 128 columns wide would leave half of every 256-wide tile empty: it takes the 128 x 128 form)
     // and so does a product of only two K tiles, which is all tile turnover: two workgroups per CU overlap one tile's
     // stores with the other's loads (bmm [128, 2048, 128] x [128, 128, 2048]: 421 -> 368 us)
-    const bool big = ceilDiv(p.M, 256) * ceilDiv(p.N, 256) * p.batch >= 144 && p.N > 128 && p.K > 2 * kBK;
+    const bool big = (ceilDiv(p.M, 256) * ceilDiv(p.N, 256) * p.batch >= 144 || (!bT && tailSplitPays(p))) && p.N > 128 && p.K > 2 * kBK;
     const bool fits2g = bT || (((p.M - 1) * p.sAm + p.K) * 2 < (int64_t(1) << 31) && ((p.N - 1) * p.sBn + p.K) * 2 < (int64_t(1) << 31));
     if (big && p.K % kBK == 0 && p.K >= 2 * kBK && fits2g) {
       if (p.colScale)
-        return p.dtype == diopi_dtype_bfloat16 ? launchMfmaPipelined<bf16_t, kEpiColScale>(stream, p)
-                                               : launchMfmaPipelined<half_t, kEpiColScale>(stream, p);
-      return p.dtype == diopi_dtype_bfloat16 ? launchMfmaPipelined<bf16_t>(stream, p, nullptr, 1, 0, nullptr, bT)
-                                             : launchMfmaPipelined<half_t>(stream, p, nullptr, 1, 0, nullptr, bT);
+        return p.dtype == diopi_dtype_bfloat16 ? launchMfmaPipelined<bf16_t, kEpiColScale>(ctx, stream, p)
+                                               : launchMfmaPipelined<half_t, kEpiColScale>(ctx, stream, p);
+      return p.dtype == diopi_dtype_bfloat16 ? launchMfmaPipelined<bf16_t>(ctx, stream, p, nullptr, 1, 0, nullptr, bT)
+                                             : launchMfmaPipelined<half_t>(ctx, stream, p, nullptr, 1, 0, nullptr, bT);
     }
     AMD_CHECK(!p.colScale, "gemm: a column scale was set on a problem gemmAppliesColumnScale does not accept");
     // In between (too few 256 x 256 tiles for the chip, too many rows for the weight-streaming kernel): the same
@@ -2755,8 +2928,8 @@ static diopiError_t runGatedSiluGemm(diopiContextHandle_t ctx, hipStream_t strea
                       ((p.M - 1) * p.sAm + p.K) * 2 < (int64_t(1) << 31) && ((p.N - 1) * p.sBn + p.K) * 2 < (int64_t(1) << 31) &&
                       mult8(p.sOm) && ptr16(p.out) && p.M < (int64_t(1) << 31) && p.N < (int64_t(1) << 31);
   if (direct) {
-    return p.dtype == diopi_dtype_bfloat16 ? launchMfmaPipelined<bf16_t, kEpiSiluMul>(stream, p)
-                                           : launchMfmaPipelined<half_t, kEpiSiluMul>(stream, p);
+    return p.dtype == diopi_dtype_bfloat16 ? launchMfmaPipelined<bf16_t, kEpiSiluMul>(ctx, stream, p)
+                                           : launchMfmaPipelined<half_t, kEpiSiluMul>(ctx, stream, p);
   }
   // decode-sized: the weight-streaming kernel that stages both operands through LDS applies the gate to its sums
   if (half && p.batch == 1 && p.M <= kSkinnyMaxM && p.K % kSkinnyLdsBK == 0 && p.N % 64 == 0 && p.N >= 4096 && p.sAk == 1 &&
@@ -3178,14 +3351,14 @@ GEMM_EXPORT diopiError_t diopiLinearRotary(diopiContextHandle_t ctx, diopiTensor
     const bool fourWave = k % (2 * kBK) == 0 && n % 8 == 0 && ptr16(p.out) && p.M * k * 2 < (int64_t(1) << 31) && n * k * 2 < (int64_t(1) << 31) &&
                           (p.M - 1) * n * 2 + n * 2 < (int64_t(1) << 31);
     if (!p.bias && r.cols % 32 == 0 && !r.tableF32 && r.headDim == 128 && fourWave)
-      AMD_TRY(p.dtype == diopi_dtype_bfloat16 ? (launchMfmaPipelined<bf16_t, kEpiRotaryLds>(stream, p, nullptr, 1, 0, &r))
-                                              : (launchMfmaPipelined<half_t, kEpiRotaryLds>(stream, p, nullptr, 1, 0, &r)));
+      AMD_TRY(p.dtype == diopi_dtype_bfloat16 ? (launchMfmaPipelined<bf16_t, kEpiRotaryLds>(ctx, stream, p, nullptr, 1, 0, &r))
+                                              : (launchMfmaPipelined<half_t, kEpiRotaryLds>(ctx, stream, p, nullptr, 1, 0, &r)));
     else if (!p.bias && r.cols % 32 == 0)
-      AMD_TRY(p.dtype == diopi_dtype_bfloat16 ? (launchMfmaPipelined<bf16_t, kEpiRotaryUniform>(stream, p, nullptr, 1, 0, &r))
-                                              : (launchMfmaPipelined<half_t, kEpiRotaryUniform>(stream, p, nullptr, 1, 0, &r)));
+      AMD_TRY(p.dtype == diopi_dtype_bfloat16 ? (launchMfmaPipelined<bf16_t, kEpiRotaryUniform>(ctx, stream, p, nullptr, 1, 0, &r))
+                                              : (launchMfmaPipelined<half_t, kEpiRotaryUniform>(ctx, stream, p, nullptr, 1, 0, &r)));
     else
-      AMD_TRY(p.dtype == diopi_dtype_bfloat16 ? (launchMfmaPipelined<bf16_t, kEpiRotary>(stream, p, nullptr, 1, 0, &r))
-                                              : (launchMfmaPipelined<half_t, kEpiRotary>(stream, p, nullptr, 1, 0, &r)));
+      AMD_TRY(p.dtype == diopi_dtype_bfloat16 ? (launchMfmaPipelined<bf16_t, kEpiRotary>(ctx, stream, p, nullptr, 1, 0, &r))
+                                              : (launchMfmaPipelined<half_t, kEpiRotary>(ctx, stream, p, nullptr, 1, 0, &r)));
   } else {
     // decode-sized: the weight-streaming kernel that stages both operands through LDS rotates its sums
     bool fused = false;

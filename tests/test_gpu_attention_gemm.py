@@ -268,6 +268,52 @@ def test_four_wave_gemm_every_instantiation_exact(ops, dev, dtype, epilogue):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("epilogue,m,n,k", [
+    ("linear", 1554, 11000, 4096),            # 301 tiles: a whole round, then 45 tiles in slices; ragged rows and columns
+    ("bias", 1554, 11008, 4096 + 128),        # 33 K-tile pairs: slices of unequal length
+    ("addend", 300, 8192, 8192),              # 64 tiles: slices only
+    ("addend", 5000, 5120, 13824),            # 400 tiles, 144 left: more slices than workgroups
+    ("rotary", 1554, 12288, 4096), ("silu_mul", 1554, 22016, 4096), ("column_scale", 882, 5120, 13824)])
+def test_four_wave_gemm_last_round_split_along_k_exact(ops, dev, dtype, epilogue, m, n, k):
+    """The tiles of a partly filled last round in slices of K (the 4-wave kernel's accumulators as fp32 partial sums, added
+    and given the epilogue by a second launch). One-hot activations over the whole of K: every product is one weight
+    element, found by exactly one slice, and the expected result is exact."""
+    g0 = g(78)
+    cols = torch.randint(0, k, (m,), generator=g0)
+    cols[:4] = torch.tensor([0, k - 1, 127, 128])
+    x = torch.zeros(m, k, dtype=dtype)
+    x[torch.arange(m), cols] = 1
+    if epilogue == "column_scale":
+        w = torch.randint(-127, 128, (n, k), generator=g0, dtype=torch.int8)
+        scale = (0.001 + 0.019 * torch.rand(n, generator=g0)).to(torch.float16)
+        assert_exact(ops.weight_only_int8_linear(x.to(dev), w.to(dev), scale.to(dev)),
+                     (w[:, cols].float() * scale.float()[:, None]).t().to(dtype))
+        return
+    w = torch.randn(n, k, generator=g0).to(dtype)
+    sel = w[:, cols].float().t()
+    if epilogue == "linear":
+        assert_exact(ops.linear(x.to(dev), w.to(dev)), sel.to(dtype))
+    elif epilogue == "bias":
+        b = torch.randn(n, generator=g0).to(dtype)
+        assert_exact(ops.linear(x.to(dev), w.to(dev), b.to(dev)), (sel + b.float()).to(dtype))
+    elif epilogue == "addend":
+        c = torch.randn(m, n, generator=g0).to(dtype)
+        assert_exact(ops.addmm(c.to(dev), x.to(dev), w.to(dev).t(), beta=0.5, alpha=2), (0.5 * c.float() + 2 * sel).to(dtype))
+    elif epilogue == "silu_mul":
+        y = sel.reshape(m, n // 64, 2, 32)
+        assert_half(ops.linear_silu_mul(x.to(dev), w.to(dev)), (torch.nn.functional.silu(y[:, :, 0]) * y[:, :, 1]).reshape(m, n // 2))
+    else:
+        hd, rot = 128, n - 256
+        e = torch.randint(-3, 1, (m, hd // 2), generator=g0).float()
+        cos, sin = 2.0 ** e, 2.0 ** (e - 1)             # powers of two: a sum of two exactly scaled terms, rounded once
+        v = sel.clone().reshape(m, n // hd, hd // 2, 2)
+        out = torch.stack([v[..., 0] * cos[:, None] - v[..., 1] * sin[:, None], v[..., 0] * sin[:, None] + v[..., 1] * cos[:, None]], dim=-1)
+        out[:, rot // hd:] = v[:, rot // hd:]
+        got = ops.linear_rotary(x.to(dev), w.to(dev), cos.to(dtype).to(dev), sin.to(dtype).to(dev), rot, hd, interleaved=True)
+        assert_exact(got, out.reshape(m, n).to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k", [(1024, 4096, 4096), (300, 520, 1024), (65, 4096, 4096 + 64), (2047, 2048, 576),
                                    (512, 768, 4096)])
 def test_split_k_gemm(ops, dev, dtype, m, n, k):
