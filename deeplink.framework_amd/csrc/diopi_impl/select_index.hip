@@ -91,6 +91,44 @@ __global__ __launch_bounds__(kSelThreads) void selectVecKernel(E* __restrict__ o
   reinterpret_cast<E8*>(out)[i] = r;
 }
 
+// The same for a condition whose period over the trailing dims is no multiple of 8 elements, or that is not 8-byte aligned
+// (the [s, s] mask of an odd sequence length): the 8 condition bytes of a piece start anywhere and may wrap around the end
+// of the period; a last piece of fewer than 8 elements goes element by element. Bound by memory: masked_fill of
+// [64, 777, 777] bf16 scores 158 -> 27 us.
+template <typename E>
+__global__ __launch_bounds__(kSelThreads) void selectVecRaggedKernel(E* __restrict__ out, const uint8_t* __restrict__ cond,
+                                                                     const E* __restrict__ a, const E* __restrict__ b, unsigned n,
+                                                                     unsigned period, E aBits) {
+  typedef E E8 __attribute__((ext_vector_type(8)));
+  typedef uint8_t C8 __attribute__((ext_vector_type(8), aligned(1)));
+  const unsigned i = (blockIdx.x * kSelThreads + threadIdx.x) * 8u;
+  if (i >= n) return;
+  const unsigned at = i % period;
+  if (i + 8 <= n) {
+    C8 c;
+    if (at + 8 <= period) {
+      c = *reinterpret_cast<const C8*>(cond + at);
+    } else {
+#pragma unroll
+      for (unsigned j = 0; j < 8; ++j) c[j] = cond[(at + j) % period];
+    }
+    const E8 vb = *reinterpret_cast<const E8*>(b + i);
+    E8 va;
+    if (a != nullptr) {
+      va = *reinterpret_cast<const E8*>(a + i);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) va[j] = aBits;
+    }
+    E8 r;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) r[j] = c[j] != 0 ? va[j] : vb[j];
+    *reinterpret_cast<E8*>(out + i) = r;
+  } else {
+    for (unsigned j = 0; i + j < n; ++j) out[i + j] = cond[(at + j) % period] != 0 ? (a != nullptr ? a[i + j] : aBits) : b[i + j];
+  }
+}
+
 // out = cond ? a : b. `a` is the scalar `sa` when aScalar (masked_fill with a Scalar value).
 template <typename C>
 __global__ __launch_bounds__(kSelThreads) void selectKernel(void* out, const void* cond, const void* a, const void* b,
@@ -341,7 +379,7 @@ static diopiError_t runSelect(diopiContextHandle_t ctx, diopiTensorHandle_t outH
     };
     // the condition: dense like the output, or dense over the trailing dims and broadcast over all the leading ones
     auto trailing = [&](const TensorView& t) {
-      if (!t.isContiguous() || t.ndim > out.ndim || t.numel % 8 != 0 || t.numel == 0) return false;
+      if (!t.isContiguous() || t.ndim > out.ndim || t.numel == 0) return false;
       int64_t covered = 1;
       bool lead = false;  // once a dim is broadcast, every dim before it must be too
       for (int d = out.ndim - 1; d >= 0; --d) {
@@ -360,8 +398,8 @@ static diopiError_t runSelect(diopiContextHandle_t ctx, diopiTensorHandle_t outH
       return covered == t.numel;
     };
     const bool floatScalarIntoInt = aScalar && scalarIsFloat(aScalar) && !isFloatDtype(out.dtype);
-    if ((out.itemsize == 2 || out.itemsize == 4) && out.numel % 8 == 0 && out.isContiguous() && out.aligned16() &&
-        (dense(cond) || trailing(cond)) && cond.itemsize == 1 && (reinterpret_cast<uintptr_t>(cond.data) & 7) == 0 && dense(b) && b.dtype == out.dtype && b.aligned16() &&
+    if ((out.itemsize == 2 || out.itemsize == 4) && out.isContiguous() && out.aligned16() &&
+        (dense(cond) || trailing(cond)) && cond.itemsize == 1 && dense(b) && b.dtype == out.dtype && b.aligned16() &&
         (aScalar ? !floatScalarIntoInt : (dense(a) && a.dtype == out.dtype && a.aligned16()))) {
       // the scalar in the output dtype's bits, through the same conversion the one-element path applies
       uint32_t bits = 0;
@@ -378,7 +416,21 @@ static diopiError_t runSelect(diopiContextHandle_t ctx, diopiTensorHandle_t outH
           bits = (uint32_t)scalarToInt(aScalar, 0);
         }
       }
-      const int64_t nvec = out.numel / 8, blocks = ceilDiv(nvec, kSelThreads), condVecs = cond.numel / 8;
+      const int64_t nvec = ceilDiv(out.numel, (int64_t)8), blocks = ceilDiv(nvec, kSelThreads), condVecs = cond.numel / 8;
+      const bool whole8 = out.numel % 8 == 0 && cond.numel % 8 == 0 && (reinterpret_cast<uintptr_t>(cond.data) & 7) == 0;
+      if (!whole8 && out.numel < ((int64_t)1 << 31)) {  // (32-bit indices)
+        if (out.itemsize == 2)
+          hipLaunchKernelGGL((selectVecRaggedKernel<uint16_t>), dim3((unsigned)blocks), dim3(kSelThreads), 0, stream, out.ptr<uint16_t>(),
+                             cond.ptr<uint8_t>(), aScalar ? nullptr : a.ptr<uint16_t>(), b.ptr<uint16_t>(), (unsigned)out.numel,
+                             (unsigned)cond.numel, (uint16_t)bits);
+        else
+          hipLaunchKernelGGL((selectVecRaggedKernel<uint32_t>), dim3((unsigned)blocks), dim3(kSelThreads), 0, stream, out.ptr<uint32_t>(),
+                             cond.ptr<uint8_t>(), aScalar ? nullptr : a.ptr<uint32_t>(), b.ptr<uint32_t>(), (unsigned)out.numel,
+                             (unsigned)cond.numel, bits);
+        AMD_LAUNCH_CHECK();
+        return diopiSuccess;
+      }
+      if (whole8) {
       AMD_CHECK(blocks <= 0x7fffffff, "%s: %ld elements exceed the grid limit", name, (long)out.numel);
       if (out.itemsize == 2)
         hipLaunchKernelGGL((selectVecKernel<uint16_t>), dim3((unsigned)blocks), dim3(kSelThreads), 0, stream, out.ptr<uint16_t>(),
@@ -389,6 +441,7 @@ static diopiError_t runSelect(diopiContextHandle_t ctx, diopiTensorHandle_t outH
                            cond.ptr<uint8_t>(), aScalar ? nullptr : a.ptr<uint32_t>(), b.ptr<uint32_t>(), nvec, condVecs, bits);
       AMD_LAUNCH_CHECK();
       return diopiSuccess;
+      }
     }
   }
   if (isFloatDtype(out.dtype)) {

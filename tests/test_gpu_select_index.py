@@ -218,3 +218,18 @@ def test_masked_fill_with_a_mask_over_the_trailing_dims(ops, dev):
         m = torch.rand(mshape, generator=g(71)) > 0.5
         assert_exact(ops.masked_fill(sc.to(dev), m.to(dev), float("-inf")), sc.masked_fill(m, float("-inf")))
         assert_exact(ops.where(m.to(dev), sc.to(dev), sc.neg().to(dev)), torch.where(m, sc, sc.neg()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape,mask_shape", [((3, 77, 77), (77, 77)), ((5, 7), (7,)), ((4, 3), (3,)), ((2, 2049), (2, 2049)), ((7, 9), (1, 1)),
+                                              ((64, 65, 8), (65, 8))])
+def test_masked_fill_and_where_with_masks_of_any_period(ops, dev, dtype, shape, mask_shape):
+    """Pieces of 8 elements whose mask bytes start anywhere, wrap around the end of a mask shorter than a piece or not, a
+    last piece of fewer than 8 elements, and a mask that is not 8-byte aligned."""
+    x, y = torch.randn(*shape, generator=g(21)).to(dtype), torch.randn(*shape, generator=g(22)).to(dtype)
+    m = torch.rand(*mask_shape, generator=g(23)) > 0.5
+    assert_exact(ops.masked_fill(x.to(dev), m.to(dev), float("-inf")), x.masked_fill(m, float("-inf")))
+    assert_exact(ops.where(m.to(dev), x.to(dev), y.to(dev)), torch.where(m, x, y))
+    held = torch.zeros(m.numel() + 1, dtype=torch.bool, device=dev)
+    held[1:] = m.to(dev).reshape(-1)
+    assert_exact(ops.masked_fill(x.to(dev), held[1:].view(mask_shape), 2.5), x.masked_fill(m, 2.5))
