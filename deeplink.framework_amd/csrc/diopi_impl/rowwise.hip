@@ -174,6 +174,83 @@ __global__ __launch_bounds__(256) void rowWaveKernel(T* __restrict__ out, const 
   }  // persistent row loop
 }
 
+// ------------------------------------------------------ softmax, unaligned rows ---
+// Softmax over rows whose length is no multiple of a 16-byte vector (attention scores of an odd sequence length): a wave
+// per row as in rowWaveKernel, the row's pieces of 16 bytes read and written at element alignment, which global memory
+// accesses allow. The last piece of a row may end inside the next row: its surplus is masked off after the load, except
+// at the end of the tensor (`total` elements from `in`), where the piece is read element by element; it is stored element
+// by element. Bound by memory: [64 x 777, 777] bf16 84 -> 34 us (a workgroup per row, one element per load).
+template <typename T, int NV>
+__global__ __launch_bounds__(256) void softmaxRaggedKernel(T* __restrict__ out, const T* __restrict__ in, int64_t rows, int cols,
+                                                           int64_t total) {
+  constexpr int N = Vec16<T>::N;
+  typedef T VU __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
+  const int lane = threadIdx.x & 63;
+  const int64_t nWaves = (int64_t)gridDim.x * 4;
+  int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  VU pre[NV];
+  auto fetch = [&](int64_t r) {
+    const T* src = in + r * cols;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (lane + 64 * i) * N;
+      if (c >= cols) continue;
+      if (r * cols + c + N <= total) {
+        pre[i] = *reinterpret_cast<const VU*>(src + c);
+      } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j) pre[i][j] = c + j < cols ? src[c + j] : T(0);
+      }
+    }
+  };
+  fetch(row);
+  for (; row < rows; row += nWaves) {
+    float f[NV][N];
+    float m = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (lane + 64 * i) * N;
+      if (c >= cols) continue;
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        f[i][j] = c + j < cols ? static_cast<float>(pre[i][j]) : -INFINITY;
+        m = fmaxf(m, f[i][j]);
+      }
+    }
+    if (row + nWaves < rows) fetch(row + nWaves);
+    m = waveMax(m);
+    const float mScaled = (m == -INFINITY) ? 0.f : m * kLog2e;  // all -inf row -> nan like the CPU kernel
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      if ((lane + 64 * i) * N >= cols) continue;
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        f[i][j] = __builtin_amdgcn_exp2f(fmaf(f[i][j], kLog2e, -mScaled));
+        s += f[i][j];
+      }
+    }
+    s = waveSum(s);
+    const float inv = 1.f / s;
+    T* dst = out + row * cols;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (lane + 64 * i) * N;
+      if (c + N <= cols) {
+        VU v;
+#pragma unroll
+        for (int j = 0; j < N; ++j) v[j] = static_cast<T>(f[i][j] * inv);
+        *reinterpret_cast<VU*>(dst + c) = v;
+      } else if (c < cols) {
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+          if (c + j < cols) dst[c + j] = static_cast<T>(f[i][j] * inv);
+      }
+    }
+  }
+}
+
 // ------------------------------------------------- several short rows per wave ---
 // Rows of at most 32 vectors (256 elements of a 16-bit type): a wave-per-row kernel would leave most lanes without a
 // vector. Here LPR lanes share a row, a wave takes 64 / LPR rows at a time, one vector per lane, and the reductions are
@@ -886,6 +963,17 @@ static diopiError_t launchRows(hipStream_t stream, T* out, const T* in, const WT
     else
       hipLaunchKernelGGL((rowStreamKernel<T, OP, WT, false>), grid, block, 0, stream, out, in, weight, bias, invRms, rows, cols,
                          inStride, outStride, eps);
+  } else if (OP == kRowSoftmax && cols > 32 && cols <= 64 * 8 * N && inStride == cols && outStride == cols) {
+    // (up to 8 vectors per lane; longer unaligned rows keep the workgroup-per-row kernel below)
+    const int nv = (int)ceilDiv(ceilDiv(cols, (int64_t)N), (int64_t)64);
+    const int64_t rowsPerWave = ceilDiv(rows, (int64_t)computeUnits() * 16);
+    dim3 grid((unsigned)ceilDiv(ceilDiv(rows, rowsPerWave), (int64_t)4)), block(256);
+#define RAGGED_LAUNCH(NV) hipLaunchKernelGGL((softmaxRaggedKernel<T, NV>), grid, block, 0, stream, out, in, rows, (int)cols, rows * cols)
+    if (nv <= 1) RAGGED_LAUNCH(1);
+    else if (nv <= 2) RAGGED_LAUNCH(2);
+    else if (nv <= 4) RAGGED_LAUNCH(4);
+    else RAGGED_LAUNCH(8);
+#undef RAGGED_LAUNCH
   } else {
     int stage = (int)cols;  // at most 48 KiB of fp32 staging
     size_t lds = (8 + (size_t)stage) * sizeof(float);

@@ -290,6 +290,20 @@ def test_copy_from_a_transposed_view(ops, dev):
         assert_exact(dst, view.contiguous())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,cols", [(1, 33), (5, 777), (4099, 515), (70, 2047), (33, 4095), (3, 4097), (20000, 65)])
+def test_softmax_unaligned_rows(ops, dev, dtype, rows, cols):
+    """Rows that are no multiple of a 16-byte vector: the last piece of a row overlaps the next row, the tensor's last one
+    its end; -inf entries, a row of nothing else, and rows that several rounds of the persistent waves reach."""
+    x = torch.randn(rows, cols, generator=g(31)).to(dtype)
+    x[torch.rand(rows, cols, generator=g(32)) > 0.9] = float("-inf")
+    if rows > 1:
+        x[1] = float("-inf")
+    got, want = ops.softmax(x.to(dev), -1).cpu(), oracle.softmax(x.float(), -1)
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert_close(got.nan_to_num(7.0), want.nan_to_num(7.0) if dtype == torch.float32 else want.nan_to_num(7.0).to(dtype))
+
+
 def test_softmax_rows_sum_to_one_at_full_size(ops, dev):
     x = torch.randn(8192, 4096, generator=g(20)).bfloat16().to(dev)
     y = ops.softmax(x, -1)
