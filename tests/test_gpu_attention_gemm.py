@@ -314,6 +314,27 @@ def test_four_wave_gemm_last_round_split_along_k_exact(ops, dev, dtype, epilogue
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("batch,m,n,k", [(3, 777, 128, 777), (2, 129, 131, 65), (1, 1, 1, 1), (5, 128, 127, 7), (1, 300, 500, 4097)])
+def test_products_over_a_k_that_is_no_multiple_of_eight(ops, dev, dtype, batch, m, n, k):
+    """Rows that start at any element: K ends inside a 16-byte piece, inside a 64-wide K tile and one element into one;
+    the [K, N] and the transposed second operand, a K-strided first one, and a linear with a bias. The fp32 product, and
+    exactly on one-hot rows. The operands end where their allocations do: nothing may be read past them."""
+    a, b = torch.randn(batch, m, k, generator=g(91)).to(dtype), torch.randn(batch, k, n, generator=g(92)).to(dtype)
+    want = a.float() @ b.float()
+    da, db = a.to(dev), b.to(dev)
+    assert_half(ops.bmm(da, db), want)
+    assert_half(ops.bmm(da, db.transpose(1, 2).contiguous().transpose(1, 2)), want)
+    assert_half(ops.bmm(da.transpose(1, 2).contiguous().transpose(1, 2), db), want)
+    bias = torch.randn(n, generator=g(93)).to(dtype)
+    assert_half(ops.linear(da, db[0].t().contiguous(), bias.to(dev)), a.float() @ b[0].float() + bias.float())
+    onehot = torch.zeros(batch, m, k, dtype=dtype)
+    cols = torch.randint(0, k, (batch, m), generator=g(94))
+    cols[:, -1] = k - 1
+    onehot.scatter_(2, cols[:, :, None], 1)
+    assert_exact(ops.bmm(onehot.to(dev), db), torch.gather(b, 1, cols[:, :, None].expand(batch, m, n)))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k", [(1024, 4096, 4096), (300, 520, 1024), (65, 4096, 4096 + 64), (2047, 2048, 576),
                                    (512, 768, 4096)])
 def test_split_k_gemm(ops, dev, dtype, m, n, k):
