@@ -7,8 +7,11 @@ LIB_DIR = os.path.join(HERE, "lib")
 RT_PATH = os.path.join(LIB_DIR, "libdipu_amd_rt.so")
 IMPL_PATH = os.path.join(LIB_DIR, "libdiopi_impl.so")
 
+HOST_PATH = os.path.join(LIB_DIR, "dipu_amd_host.so")
+
 _rt = None
 _impl = None
+_host = None
 
 
 class NativeLibraryMissing(RuntimeError):
@@ -43,3 +46,20 @@ def impl():
         _require(IMPL_PATH)
         _impl = ctypes.CDLL(IMPL_PATH, mode=ctypes.RTLD_GLOBAL)
     return _impl
+
+
+def host():
+    """dipu_amd_host.so, the native half of the op adapter (csrc/host/host_module.cpp)."""
+    global _host
+    if _host is None:
+        impl()
+        _require(HOST_PATH)
+        import importlib.machinery
+        import importlib.util
+        from . import diopi
+        loader = importlib.machinery.ExtensionFileLoader("dipu_amd_host", HOST_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("dipu_amd_host", loader))
+        loader.exec_module(mod)
+        mod.setup(diopi.DiopiError, diopi.raise_failure)
+        _host = mod
+    return _host

@@ -1,12 +1,14 @@
-"""Builds the two shared libraries of the MI355X backend with hipcc (gfx950 only).
+"""Builds the shared libraries of the MI355X backend: two with hipcc (gfx950 only) and the Python host module.
 
   lib/libdiopi_impl.so   DIOPI operator entry points + hand-written HIP kernels.
                          Leaves the diopirt callbacks undefined: DIPU (or lib/libdipu_amd_rt.so)
                          provides them at load time.
   lib/libdipu_amd_rt.so  dipu::devapis over HIP, stream/event pools, caching allocators,
                          diopirt callbacks and the C facade declared in include/dipu_amd/runtime.h.
+  lib/dipu_amd_host.so   CPython extension over torch's C++ interface: the native half of the op adapter
+                         (host code only, so the host compiler builds it).
 
-Usage: python build.py [-j N] [--only impl|rt]
+Usage: python build.py [-j N] [--only impl|rt|host]
 """
 import argparse
 import concurrent.futures
@@ -98,11 +100,29 @@ def compile_one(src, obj):
     return src, rc, err
 
 
+HOST_SOURCE = os.path.join(HERE, "csrc", "host", "host_module.cpp")
+HOST_OUT = os.path.join(LIB_DIR, "dipu_amd_host.so")
+
+
+def build_host():
+    import sysconfig
+
+    from torch.utils import cpp_extension as ext
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-fPIC", "-shared", "-std=c++20", "-fvisibility=hidden", "-Wall",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", f"-I{INCLUDE}", f"-I{sysconfig.get_paths()['include']}",
+           f"-I{os.path.join(os.environ.get('ROCM_PATH', '/opt/rocm'), 'include')}"]
+    cmd += [f"-isystem{p}" for p in ext.include_paths()] + [HOST_SOURCE, "-o", HOST_OUT]
+    cmd += [f"-L{p}" for p in ext.library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    return HOST_SOURCE, r.returncode, r.stderr
+
+
 def build(only=None, jobs=None):
     os.makedirs(LIB_DIR, exist_ok=True)
     os.makedirs(OBJ_DIR, exist_ok=True)
     jobs = jobs or min(8, os.cpu_count() or 1)
-    names = [only] if only else list(TARGETS)
+    names = [n for n in ([only] if only else TARGETS) if n != "host"]
+    host = only in (None, "host")
     work = []
     for name in names:
         t = TARGETS[name]
@@ -111,7 +131,7 @@ def build(only=None, jobs=None):
             work.append((name, src, obj))
     failed = False
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as ex:
-        futs = [ex.submit(compile_one, src, obj) for _, src, obj in work]
+        futs = [ex.submit(compile_one, src, obj) for _, src, obj in work] + ([ex.submit(build_host)] if host else [])
         for f in concurrent.futures.as_completed(futs):
             src, rc, err = f.result()
             if err.strip():
@@ -120,7 +140,7 @@ def build(only=None, jobs=None):
                 sys.stderr.write(f"FAILED: {src}\n")
                 failed = True
     if failed:
-        raise RuntimeError("hipcc compilation failed")
+        raise RuntimeError("compilation failed")
     for name in names:
         t = TARGETS[name]
         objs = [obj for n, _, obj in work if n == name]
@@ -129,13 +149,13 @@ def build(only=None, jobs=None):
         if r.returncode != 0:
             sys.stderr.write(r.stderr)
             raise RuntimeError(f"link failed: {t['out']}")
-    return [TARGETS[n]["out"] for n in names]
+    return [TARGETS[n]["out"] for n in names] + ([HOST_OUT] if host else [])
 
 
 if __name__ == "__main__":
     ap = argparse.ArgumentParser()
     ap.add_argument("-j", type=int, default=None)
-    ap.add_argument("--only", choices=list(TARGETS), default=None)
+    ap.add_argument("--only", choices=list(TARGETS) + ["host"], default=None)
     a = ap.parse_args()
     for out in build(a.only, a.j):
         print("built", out)

@@ -316,7 +316,14 @@ def call(name, ctx, *args):
     else:
         ret = fn(name)(ctx.ptr, *args)
     if ret != DIOPI_SUCCESS:
-        msg = last_error()
-        if "runtime holds the cause" in msg:  # a workspace request failed: the runtime library knows why
-            msg += f" [{rt_error()}]"
-        raise DiopiError(f"{name} failed, ret = {ret}: {msg}")
+        raise_failure(name, ret)
+
+
+def raise_failure(name, ret):
+    """Raises for entry point `name` with the text the library (or, for a context, the runtime) left behind."""
+    if name == "dipuAmdContextCreate":
+        raise DiopiError(rt_error())
+    msg = last_error()
+    if "runtime holds the cause" in msg:  # a workspace request failed: the runtime library knows why
+        msg += f" [{rt_error()}]"
+    raise DiopiError(f"{name} failed, ret = {ret}: {msg}")

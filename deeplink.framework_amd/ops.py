@@ -8,17 +8,15 @@ DIPU (dipu/scripts/autogen_diopi_wrapper/diopi_wrapper_template.py:100-141):
   3. marshal tensors / scalars / sizes and call the diopi* entry point,
   4. raise on any return code other than diopiSuccess.
 
-Nothing here computes: a missing libdiopi_impl.so raises, there is no torch fallback.
+Steps 2 to 4, and output inference where it is more than a shape, are native (csrc/host/host_module.cpp). Nothing here
+computes: a missing library raises, there is no torch fallback.
 Names follow the aten op (or, for the ext ops, the lightllm op names the reference's
 dicp/dicp/vendor/AscendGraph/ext_ops.py registers).
 """
-import ctypes
-from ctypes import byref, c_void_p
-
 import torch
 
-from . import diopi
-from .diopi import Context, call, handle, scalar
+from . import _native, diopi
+from .diopi import Context
 
 
 def _is_number(x):
@@ -33,14 +31,22 @@ def _peel_cpu_scalar(x):
 
 
 def _binary_out(a, b, out):
-    if out is not None:
-        return out
-    shape = torch.broadcast_shapes(a.shape, b.shape) if isinstance(b, torch.Tensor) else a.shape
-    dtype = torch.result_type(a, b)
-    return torch.empty(shape, dtype=dtype, device=a.device)
+    return _host.broadcast_of(a, b, False) if out is None else out
 
 
-_scope = None
+class _HostModule:
+    """Stands in for the native host module until the first op asks it for an entry point, then takes itself out."""
+
+    def __getattr__(self, name):
+        global _host
+        _host = _native.host()
+        return getattr(_host, name)
+
+
+_host = _HostModule()
+# The context every op runs in: 0 lets the call open one on the current stream and close it when it returns, a scope puts
+# its own here (see WorkspaceScope).
+_ctx = 0
 
 
 class WorkspaceScope:
@@ -55,24 +61,16 @@ class WorkspaceScope:
         self.ctx = Context(stream)
 
     def __enter__(self):
-        global _scope
-        self._outer, _scope = _scope, self
+        global _ctx
+        self._outer, _ctx = _ctx, self.ctx.ptr.value
         return self
 
     def __exit__(self, *exc):
-        global _scope
-        _scope = self._outer
+        global _ctx
+        _ctx = self._outer
 
     def close(self):
         self.ctx.close()
-
-
-def _call(name, *args, stream=None):
-    if _scope is not None and stream is None:
-        call(name, _scope.ctx, *args)
-        return
-    with Context(stream) as ctx:
-        call(name, ctx, *args)
 
 
 # ------------------------------------------------------------------ arithmetic
@@ -80,43 +78,29 @@ def add(self, other, *, alpha=1, out=None):
     """aten::add.Tensor / add.Scalar -> diopiAdd / diopiAddScalar (diopi_functions.yaml:31-63)."""
     other = _peel_cpu_scalar(other)
     out = _binary_out(self, other, out)
-    ho, po = handle(out)
-    hs, ps = handle(self)
-    al = scalar(alpha)
     if _is_number(other):
-        sc = scalar(other)
-        _call("diopiAddScalar", po, ps, byref(sc), byref(al))
+        _host.diopiAddScalar(_ctx, out, self, other, alpha)
     else:
-        hb, pb = handle(other)
-        _call("diopiAdd", po, ps, pb, byref(al))
+        _host.diopiAdd(_ctx, out, self, other, alpha)
     return out
 
 
 def add_(self, other, *, alpha=1):
     other = _peel_cpu_scalar(other)
-    hs, ps = handle(self)
-    al = scalar(alpha)
     if _is_number(other):
-        sc = scalar(other)
-        _call("diopiAddInpScalar", ps, byref(sc), byref(al))
+        _host.diopiAddInpScalar(_ctx, self, other, alpha)
     else:
-        hb, pb = handle(other)
-        _call("diopiAddInp", ps, pb, byref(al))
+        _host.diopiAddInp(_ctx, self, other, alpha)
     return self
 
 
 def sub(self, other, *, alpha=1, out=None):
     other = _peel_cpu_scalar(other)
     out = _binary_out(self, other, out)
-    ho, po = handle(out)
-    hs, ps = handle(self)
-    al = scalar(alpha)
     if _is_number(other):
-        sc = scalar(other)
-        _call("diopiSubScalar", po, ps, byref(sc), byref(al))
+        _host.diopiSubScalar(_ctx, out, self, other, alpha)
     else:
-        hb, pb = handle(other)
-        _call("diopiSub", po, ps, pb, byref(al))
+        _host.diopiSub(_ctx, out, self, other, alpha)
     return out
 
 
@@ -124,55 +108,40 @@ def mul(self, other, *, out=None):
     """aten::mul.Tensor / mul.Scalar -> diopiMul / diopiMulScalar (diopi_functions.yaml:159-196)."""
     other = _peel_cpu_scalar(other)
     out = _binary_out(self, other, out)
-    ho, po = handle(out)
-    hs, ps = handle(self)
     if _is_number(other):
-        sc = scalar(other)
-        _call("diopiMulScalar", po, ps, byref(sc))
+        _host.diopiMulScalar(_ctx, out, self, other)
     else:
-        hb, pb = handle(other)
-        _call("diopiMul", po, ps, pb)
+        _host.diopiMul(_ctx, out, self, other)
     return out
 
 
 def mul_(self, other):
     other = _peel_cpu_scalar(other)
-    hs, ps = handle(self)
     if _is_number(other):
-        sc = scalar(other)
-        _call("diopiMulInpScalar", ps, byref(sc))
+        _host.diopiMulInpScalar(_ctx, self, other)
     else:
-        hb, pb = handle(other)
-        _call("diopiMulInp", ps, pb)
+        _host.diopiMulInp(_ctx, self, other)
     return self
 
 
 def div(self, other, *, rounding_mode=None, out=None):
     other = _peel_cpu_scalar(other)
     if out is None:
-        shape = torch.broadcast_shapes(self.shape, other.shape) if isinstance(other, torch.Tensor) else self.shape
-        dtype = torch.result_type(self, other)
-        if rounding_mode is None and not dtype.is_floating_point:
-            dtype = torch.get_default_dtype()
-        out = torch.empty(shape, dtype=dtype, device=self.device)
-    ho, po = handle(out)
-    hs, ps = handle(self)
+        out = _host.broadcast_of(self, other, False)
+        if rounding_mode is None and not out.dtype.is_floating_point:
+            out = torch.empty(out.shape, dtype=torch.get_default_dtype(), device=out.device)
     mode = diopi.ROUND_MODE[rounding_mode]
     if _is_number(other):
-        sc = scalar(other)
-        _call("diopiDivScalar", po, ps, byref(sc), mode)
+        _host.diopiDivScalar(_ctx, out, self, other, mode)
     else:
-        hb, pb = handle(other)
-        _call("diopiDiv", po, ps, pb, mode)
+        _host.diopiDiv(_ctx, out, self, other, mode)
     return out
 
 
 def _unary(name, self, out):
     if out is None:
-        out = torch.empty_like(self, memory_format=torch.contiguous_format)
-    ho, po = handle(out)
-    hs, ps = handle(self)
-    _call(name, po, ps)
+        out = _host.like(self)
+    getattr(_host, name)(_ctx, out, self)
     return out
 
 
@@ -182,8 +151,7 @@ def silu(self, *, out=None):
 
 
 def silu_(self):
-    hs, ps = handle(self)
-    _call("diopiSiluInp", ps)
+    _host.diopiSiluInp(_ctx, self)
     return self
 
 
@@ -214,30 +182,21 @@ def exp(self, *, out=None):
 def pow(self, exponent, *, out=None):
     """aten::pow.Tensor_Scalar -> diopiPow (diopi_functions.yaml:1306-1318)."""
     if out is None:
-        dtype = torch.result_type(self, exponent)
-        out = torch.empty(self.shape, dtype=dtype, device=self.device)
-    ho, po = handle(out)
-    hs, ps = handle(self)
-    sc = scalar(exponent)
-    _call("diopiPow", po, ps, byref(sc))
+        out = _host.broadcast_of(self, exponent, False)
+    _host.diopiPow(_ctx, out, self, exponent)
     return out
 
 
 def fill_(self, value):
-    hs, ps = handle(self)
-    sc = scalar(value)
-    _call("diopiFill", ps, byref(sc))
+    _host.diopiFill(_ctx, self, value)
     return self
 
 
 def silu_mul(gate, up, *, out=None):
     """silu(gate) * up in one pass (backend extension; see functions_ext.h)."""
     if out is None:
-        out = torch.empty_like(gate, memory_format=torch.contiguous_format)
-    ho, po = handle(out)
-    hg, pg = handle(gate)
-    hu, pu = handle(up)
-    _call("diopiSiluMul", po, pg, pu)
+        out = _host.like(gate)
+    _host.diopiSiluMul(_ctx, out, gate, up)
     return out
 
 
@@ -254,11 +213,8 @@ def linear_silu_mul(input, weight_gate_up, *, out=None):
     weight_gate_up = interleave_gate_up(w_gate, w_up)."""
     f = weight_gate_up.shape[0] // 2
     if out is None:
-        out = torch.empty(*input.shape[:-1], f, dtype=input.dtype, device=input.device)
-    ho, po = handle(out)
-    hi, pi = handle(input)
-    hw, pw = handle(weight_gate_up)
-    _call("diopiLinearSiluMul", po, pi, pw)
+        out = _host.rows_of(input, f)
+    _host.diopiLinearSiluMul(_ctx, out, input, weight_gate_up)
     return out
 
 
@@ -275,14 +231,8 @@ def linear_rotary(input, weight, cos, sin, rotary_cols, head_dim, bias=None, *, 
     """input @ weight^T (+ bias) with the rotary embedding applied to the first rotary_cols output columns
     (backend extension; see functions_ext.h). cos / sin: [rows, head_dim / 2]."""
     if out is None:
-        out = torch.empty(*input.shape[:-1], weight.shape[0], dtype=input.dtype, device=input.device)
-    ho, po = handle(out)
-    hi, pi = handle(input)
-    hw, pw = handle(weight)
-    hb, pb = handle(bias)
-    hc, pc = handle(cos)
-    hs, ps = handle(sin)
-    _call("diopiLinearRotary", po, pi, pw, pb, pc, ps, int(rotary_cols), int(head_dim), bool(conj), bool(interleaved))
+        out = _host.rows_of(input, weight.shape[0])
+    _host.diopiLinearRotary(_ctx, out, input, weight, bias, cos, sin, int(rotary_cols), int(head_dim), bool(conj), bool(interleaved))
     return out
 
 
@@ -290,10 +240,8 @@ def linear_rotary(input, weight, cos, sin, rotary_cols, head_dim, bias=None, *, 
 def softmax(self, dim, *, out=None):
     """aten::_softmax.out -> diopiSoftmax (diopi_functions.yaml:1290-1292)."""
     if out is None:
-        out = torch.empty_like(self, memory_format=torch.contiguous_format)
-    ho, po = handle(out)
-    hs, ps = handle(self)
-    _call("diopiSoftmax", po, ps, int(dim))
+        out = _host.like(self)
+    _host.diopiSoftmax(_ctx, out, self, int(dim))
     return out
 
 
@@ -304,19 +252,14 @@ def mean(self, dim, keepdim=False, *, out=None):
     if out is None:
         shape = [(1 if i in dims else n) for i, n in enumerate(self.shape) if keepdim or i not in dims]
         out = torch.empty(shape, dtype=self.dtype, device=self.device)
-    ho, po = handle(out)
-    hs, ps = handle(self)
-    sz = diopi.size(dims)
-    _call("diopiMean", po, ps, sz)
+    _host.diopiMean(_ctx, out, self, dims)
     return out
 
 
 # ------------------------------------------------------------------ movement
 def copy_(self, src):
     """aten::copy_ on-device part -> diopiCopyInp(ctx, src, dest) (diopi_functions.yaml:2969-2973)."""
-    hs, ps = handle(src)
-    hd, pd = handle(self)
-    _call("diopiCopyInp", ps, pd)
+    _host.diopiCopyInp(_ctx, src, self)
     return self
 
 
@@ -331,20 +274,14 @@ def cat(tensors, dim=0, *, out=None):
         for t in tensors:
             dtype = torch.promote_types(dtype, t.dtype)
         out = torch.empty(shape, dtype=dtype, device=ref.device)
-    hs = [handle(t) for t in tensors]
-    arr = (c_void_p * len(hs))(*[p for _, p in hs])
-    ho, po = handle(out)
-    _call("diopiCat", po, arr, len(hs), int(dim))
+    _host.diopiCat(_ctx, out, tensors, len(tensors), int(dim))
     return out
 
 
 def index_put_(self, indices, values, accumulate=False):
     """aten::_index_put_impl_ -> diopiIndexPutInp (diopi_functions.yaml:2370-2382)."""
-    hs = [handle(t) for t in indices]
-    arr = (c_void_p * len(hs))(*[p for _, p in hs])
-    hd, pd = handle(self)
-    hv, pv = handle(values)
-    _call("diopiIndexPutInp", pd, pv, arr, len(hs), bool(accumulate))
+    indices = list(indices)
+    _host.diopiIndexPutInp(_ctx, self, values, indices, len(indices), bool(accumulate))
     return self
 
 
@@ -363,11 +300,7 @@ def where(condition, self, other, *, out=None):
     if out is None:
         shape = torch.broadcast_shapes(condition.shape, self.shape, other.shape)
         out = torch.empty(shape, dtype=torch.result_type(self, other), device=dev)
-    hc, pc = handle(condition)
-    ha, pa = handle(self)
-    hb, pb = handle(other)
-    ho, po = handle(out)
-    _call("diopiWhere", po, pc, pa, pb)
+    _host.diopiWhere(_ctx, out, condition, self, other)
     return out
 
 
@@ -376,51 +309,37 @@ def masked_fill(self, mask, value, *, out=None):
     (diopi_functions.yaml:1432-1453); a CPU value tensor is moved to the device first (:1436)."""
     if out is None:
         out = torch.empty(torch.broadcast_shapes(self.shape, mask.shape), dtype=self.dtype, device=self.device)
-    ho, po = handle(out)
-    hs, ps = handle(self)
-    hm, pm = handle(mask)
     if _is_number(value):
-        sc = scalar(value)
-        _call("diopiMaskedFillScalar", po, ps, pm, byref(sc))
+        _host.diopiMaskedFillScalar(_ctx, out, self, mask, value)
     else:
-        hv, pv = handle(value.to(self.device))
-        _call("diopiMaskedFill", po, ps, pm, pv)
+        _host.diopiMaskedFill(_ctx, out, self, mask, value.to(self.device))
     return out
 
 
 def masked_fill_(self, mask, value):
-    hs, ps = handle(self)
-    hm, pm = handle(mask)
     if _is_number(value):
-        sc = scalar(value)
-        _call("diopiMaskedFillInpScalar", ps, pm, byref(sc))
+        _host.diopiMaskedFillInpScalar(_ctx, self, mask, value)
     else:
-        hv, pv = handle(value.to(self.device))
-        _call("diopiMaskedFillInp", ps, pm, pv)
+        _host.diopiMaskedFillInp(_ctx, self, mask, value.to(self.device))
     return self
 
 
 def tril(self, diagonal=0, *, out=None):
     """aten::tril -> diopiTril (diopi_functions.yaml:1191-1197)."""
     out = torch.empty_like(self) if out is None else out
-    ho, po = handle(out)
-    hs, ps = handle(self)
-    _call("diopiTril", po, ps, int(diagonal))
+    _host.diopiTril(_ctx, out, self, int(diagonal))
     return out
 
 
 def triu(self, diagonal=0, *, out=None):
     """aten::triu -> diopiTriu (diopi_functions.yaml:2505-2516)."""
     out = torch.empty_like(self) if out is None else out
-    ho, po = handle(out)
-    hs, ps = handle(self)
-    _call("diopiTriu", po, ps, int(diagonal))
+    _host.diopiTriu(_ctx, out, self, int(diagonal))
     return out
 
 
 def triu_(self, diagonal=0):
-    hs, ps = handle(self)
-    _call("diopiTriuInp", ps, int(diagonal))
+    _host.diopiTriuInp(_ctx, self, int(diagonal))
     return self
 
 
@@ -434,9 +353,7 @@ def arange(start, end=None, step=1, *, dtype=None, device=None, out=None):
         if dtype is None:
             dtype = torch.get_default_dtype() if any(isinstance(v, float) for v in (start, end, step)) else torch.int64
         out = torch.empty(int(math.ceil((end - start) / step)), dtype=dtype, device=device)
-    ho, po = handle(out)
-    s0, s1, s2 = scalar(start), scalar(end), scalar(step)
-    _call("diopiArange", po, byref(s0), byref(s1), byref(s2))
+    _host.diopiArange(_ctx, out, start, end, step)
     return out
 
 
@@ -446,10 +363,7 @@ def index_select(self, dim, index, *, out=None):
         shape = list(self.shape)
         shape[dim % self.dim()] = index.numel()
         out = torch.empty(shape, dtype=self.dtype, device=self.device)
-    ho, po = handle(out)
-    hs, ps = handle(self)
-    hi, pi = handle(index)
-    _call("diopiIndexSelect", po, ps, int(dim), pi)
+    _host.diopiIndexSelect(_ctx, out, self, int(dim), index)
     return out
 
 
@@ -457,26 +371,18 @@ def gather(self, dim, index, *, out=None):
     """aten::gather.out -> diopiGather (diopi_functions.yaml:1923-1924)."""
     if out is None:
         out = torch.empty(index.shape, dtype=self.dtype, device=self.device)
-    ho, po = handle(out)
-    hs, ps = handle(self)
-    hi, pi = handle(index)
-    _call("diopiGather", po, ps, int(dim), pi)
+    _host.diopiGather(_ctx, out, self, int(dim), index)
     return out
 
 
 def _compare(name, self, other, out):
     other = _peel_cpu_scalar(other)
     if out is None:
-        shape = torch.broadcast_shapes(self.shape, other.shape) if isinstance(other, torch.Tensor) else self.shape
-        out = torch.empty(shape, dtype=torch.bool, device=self.device)
-    ho, po = handle(out)
-    hs, ps = handle(self)
+        out = _host.broadcast_of(self, other, True)
     if _is_number(other):
-        sc = scalar(other)
-        _call(f"diopi{name}Scalar", po, ps, byref(sc))
+        getattr(_host, f"diopi{name}Scalar")(_ctx, out, self, other)
     else:
-        hb, pb = handle(other)
-        _call(f"diopi{name}", po, ps, pb)
+        getattr(_host, f"diopi{name}")(_ctx, out, self, other)
     return out
 
 
@@ -510,10 +416,7 @@ def mm(self, mat2, *, out=None):
     """aten::mm -> diopiMm (diopi_functions.yaml:1829-1837)."""
     if out is None:
         out = torch.empty((self.shape[0], mat2.shape[1]), dtype=self.dtype, device=self.device)
-    ho, po = handle(out)
-    ha, pa = handle(self)
-    hb, pb = handle(mat2)
-    _call("diopiMm", po, pa, pb)
+    _host.diopiMm(_ctx, out, self, mat2)
     return out
 
 
@@ -521,10 +424,7 @@ def bmm(self, mat2, *, out=None):
     """aten::bmm -> diopiBmm (diopi_functions.yaml:1755-1765)."""
     if out is None:
         out = torch.empty((self.shape[0], self.shape[1], mat2.shape[2]), dtype=self.dtype, device=self.device)
-    ho, po = handle(out)
-    ha, pa = handle(self)
-    hb, pb = handle(mat2)
-    _call("diopiBmm", po, pa, pb)
+    _host.diopiBmm(_ctx, out, self, mat2)
     return out
 
 
@@ -543,10 +443,7 @@ def matmul(self, other, *, out=None):
     """aten::matmul -> diopiMatmul (diopi_functions.yaml:1852-1893)."""
     if out is None:
         out = torch.empty(_matmul_shape(self, other), dtype=self.dtype, device=self.device)
-    ho, po = handle(out)
-    ha, pa = handle(self)
-    hb, pb = handle(other)
-    _call("diopiMatmul", po, pa, pb)
+    _host.diopiMatmul(_ctx, out, self, other)
     return out
 
 
@@ -554,12 +451,7 @@ def addmm(self, mat1, mat2, *, beta=1, alpha=1, out=None):
     """aten::addmm -> diopiAddmm (diopi_functions.yaml:594-597)."""
     if out is None:
         out = torch.empty((mat1.shape[0], mat2.shape[1]), dtype=mat1.dtype, device=mat1.device)
-    ho, po = handle(out)
-    hi, pi = handle(self)
-    ha, pa = handle(mat1)
-    hb, pb = handle(mat2)
-    sb, sa = scalar(beta), scalar(alpha)
-    _call("diopiAddmm", po, pi, pa, pb, byref(sb), byref(sa))
+    _host.diopiAddmm(_ctx, out, self, mat1, mat2, beta, alpha)
     return out
 
 
@@ -568,23 +460,15 @@ def baddbmm(self, batch1, batch2, *, beta=1, alpha=1, out=None):
     if out is None:
         out = torch.empty((batch1.shape[0], batch1.shape[1], batch2.shape[2]), dtype=batch1.dtype,
                           device=batch1.device)
-    ho, po = handle(out)
-    hi, pi = handle(self)
-    ha, pa = handle(batch1)
-    hb, pb = handle(batch2)
-    _call("diopiBaddbmm", po, pi, pa, pb, float(beta), float(alpha))
+    _host.diopiBaddbmm(_ctx, out, self, batch1, batch2, float(beta), float(alpha))
     return out
 
 
 def linear(input, weight, bias=None, *, out=None):
     """aten::linear -> diopiLinear, weight [N, K] (diopi_functions.yaml:902-909)."""
     if out is None:
-        out = torch.empty(tuple(input.shape[:-1]) + (weight.shape[0],), dtype=input.dtype, device=input.device)
-    ho, po = handle(out)
-    hi, pi = handle(input)
-    hw, pw = handle(weight)
-    hb, pb = handle(bias)
-    _call("diopiLinear", po, pi, pw, pb)
+        out = _host.rows_of(input, weight.shape[0])
+    _host.diopiLinear(_ctx, out, input, weight, bias)
     return out
 
 
@@ -592,68 +476,38 @@ def linear(input, weight, bias=None, *, out=None):
 def rms_norm(x, weight, eps, *, bias=None, out=None, inv_rms=None):
     """lightllm::rms_norm (ext_ops.py:36-49) -> diopiRMSNorm over the last dim."""
     if out is None:
-        out = torch.empty_like(x, memory_format=torch.contiguous_format)
-    ho, po = handle(out)
-    hr, pr = handle(inv_rms)
-    hx, px = handle(x)
-    hw, pw = handle(weight)
-    hb, pb = handle(bias)
-    sz = diopi.size([x.shape[-1]])
-    _call("diopiRMSNorm", po, pr, px, sz, pw, pb, float(eps))
+        out = _host.like(x)
+    _host.diopiRMSNorm(_ctx, out, inv_rms, x, [x.shape[-1]], weight, bias, float(eps))
     return out
 
 
 def rotary_emb(x, cos, sin, *, conj=False, interleaved=False, out=None):
     """lightllm::rotary_emb (ext_ops.py:13-33; interleaved form model.py:58-69) -> diopiRotaryEmbedding."""
     if out is None:
-        out = torch.empty_like(x, memory_format=torch.contiguous_format)
-    ho, po = handle(out)
-    hx, px = handle(x)
-    hc, pc = handle(cos)
-    hs, ps = handle(sin)
-    _call("diopiRotaryEmbedding", po, px, pc, ps, bool(conj), bool(interleaved))
+        out = _host.like(x)
+    _host.diopiRotaryEmbedding(_ctx, out, x, cos, sin, bool(conj), bool(interleaved))
     return out
 
 
 def dest_index_copy_kv(k, dest_loc, out):
     """out[dest_loc[i]] = k[i] -> diopiDestIndexCopyKV (bit-exact scatter into the KV pool)."""
-    ho, po = handle(out)
-    hk, pk = handle(k)
-    hl, pl = handle(dest_loc)
-    _call("diopiDestIndexCopyKV", po, pk, pl)
+    _host.diopiDestIndexCopyKV(_ctx, out, k, dest_loc)
     return out
 
 
 def dest_index_copy_kv_pair(k, v, dest_loc, out_k, out_v):
     """out_k[dest_loc[i]] = k[i] and out_v[dest_loc[i]] = v[i] in one launch (backend extension, functions_ext.h)."""
-    hok, pok = handle(out_k)
-    hk, pk = handle(k)
-    hov, pov = handle(out_v)
-    hv, pv = handle(v)
-    hl, pl = handle(dest_loc)
-    _call("diopiDestIndexCopyKVPair", pok, pk, pov, pv, pl)
+    _host.diopiDestIndexCopyKVPair(_ctx, out_k, k, out_v, v, dest_loc)
     return out_k, out_v
 
 
 def token_attention(q, k, attention_out, b_loc, b_start_loc, b_seq_len, max_input_len):
-    ho, po = handle(attention_out)
-    hq, pq = handle(q)
-    hk, pk = handle(k)
-    h1, p1 = handle(b_loc)
-    h2, p2 = handle(b_start_loc)
-    h3, p3 = handle(b_seq_len)
-    _call("diopiTokenAttentionInference", po, pq, pk, p1, p2, p3, int(max_input_len))
+    _host.diopiTokenAttentionInference(_ctx, attention_out, q, k, b_loc, b_start_loc, b_seq_len, int(max_input_len))
     return attention_out
 
 
 def token_softmax_reducev(logics, v, out, b_loc, b_start_loc, b_seq_len, max_input_len, other_kv_index=0):
-    ho, po = handle(out)
-    hl, pl = handle(logics)
-    hv, pv = handle(v)
-    h1, p1 = handle(b_loc)
-    h2, p2 = handle(b_start_loc)
-    h3, p3 = handle(b_seq_len)
-    _call("diopiTokenSoftmaxReduceVInference", po, pl, pv, p1, p2, p3, int(max_input_len), int(other_kv_index))
+    _host.diopiTokenSoftmaxReduceVInference(_ctx, out, logics, v, b_loc, b_start_loc, b_seq_len, int(max_input_len), int(other_kv_index))
     return out
 
 
@@ -662,15 +516,8 @@ def token_decode_attention(q, k, v, b_loc, b_start_loc, b_seq_len, max_input_len
     point whose partial results live in the library's own device array (the caller then passes `out`)."""
     if out is None:
         out = torch.empty_like(q)
-    ho, po = handle(out)
-    hq, pq = handle(q)
-    hk, pk = handle(k)
-    hv, pv = handle(v)
-    h1, p1 = handle(b_loc)
-    h2, p2 = handle(b_start_loc)
-    h3, p3 = handle(b_seq_len)
-    _call("diopiTokenDecodeAttentionInferenceNoAlloc" if no_alloc else "diopiTokenDecodeAttentionInference",
-          po, pq, pk, pv, p1, p2, p3, int(max_input_len))
+    decode = _host.diopiTokenDecodeAttentionInferenceNoAlloc if no_alloc else _host.diopiTokenDecodeAttentionInference
+    decode(_ctx, out, q, k, v, b_loc, b_start_loc, b_seq_len, int(max_input_len))
     return out
 
 
@@ -678,23 +525,12 @@ def context_attention(q, k, v, b_start_loc, b_seq_len, max_input_len, *, out=Non
     """lightllm::prompt_attention_inference (ext_ops.py:52-87) over packed sequences."""
     if out is None:
         out = torch.empty_like(q)
-    ho, po = handle(out)
-    hq, pq = handle(q)
-    hk, pk = handle(k)
-    hv, pv = handle(v)
-    h2, p2 = handle(b_start_loc)
-    h3, p3 = handle(b_seq_len)
-    _call("diopiContextAttentionInference", po, pq, pk, pv, p2, p3, int(max_input_len))
+    _host.diopiContextAttentionInference(_ctx, out, q, k, v, b_start_loc, b_seq_len, int(max_input_len))
     return out
 
 
 def weight_only_int8_linear(input, weight, scale, bias=None, *, out=None):
     if out is None:
-        out = torch.empty(tuple(input.shape[:-1]) + (weight.shape[0],), dtype=input.dtype, device=input.device)
-    ho, po = handle(out)
-    hi, pi = handle(input)
-    hw, pw = handle(weight)
-    hs, ps = handle(scale)
-    hb, pb = handle(bias)
-    _call("diopiWeightOnlyInt8Linear", po, pi, pw, ps, pb)
+        out = _host.rows_of(input, weight.shape[0])
+    _host.diopiWeightOnlyInt8Linear(_ctx, out, input, weight, scale, bias)
     return out

@@ -183,3 +183,31 @@ def test_generated_gemm_loop_is_current(tmp_path):
     out = tmp_path / "loop.inc"
     subprocess.run([sys.executable, os.path.join(d, "gen_gemm_loop_4wave.py"), str(out)], check=True)
     assert out.read_text() == open(os.path.join(d, "gemm_loop_4wave.inc")).read()
+
+
+def test_host_module_covers_the_signature_table_and_infers_like_torch(pkg):
+    """The native half of the op adapter: a callable for every entry point the ctypes view knows, marshalling errors of the
+    same class as that view's, and output inference equal to torch's own."""
+    import torch
+    h = pkg._native.host()
+    assert all(hasattr(h, n) for n in pkg.diopi.SIGNATURES)
+    for a, b in [((3, 1), (4,)), ((), (2, 3)), ((2, 0), (1, 1)), ((5,), (5,))]:
+        for da in (torch.bfloat16, torch.float32, torch.int64, torch.bool):
+            for db in (torch.float16, torch.float32, torch.uint8):
+                x, y = torch.zeros(a, dtype=da), torch.zeros(b, dtype=db)
+                o = h.broadcast_of(x, y, False)
+                assert o.shape == torch.broadcast_shapes(a, b) and o.dtype == torch.result_type(x, y) and o.is_contiguous()
+                assert h.broadcast_of(x, y, True).dtype == torch.bool
+    for da in (torch.bfloat16, torch.int32, torch.bool):
+        for v in (True, 2, 2.5):
+            assert h.broadcast_of(torch.zeros(3, dtype=da), v, False).dtype == torch.result_type(torch.zeros(3, dtype=da), v)
+    t = torch.zeros(2, 3, 4).transpose(0, 2)
+    assert h.like(t).shape == t.shape and h.like(t).is_contiguous() and h.rows_of(t, 7).shape == (4, 3, 7)
+    with pytest.raises(pkg.diopi.DiopiError, match="rank 9"):
+        h.diopiSilu(1, torch.zeros([1] * 9), None)
+    with pytest.raises(pkg.diopi.DiopiError, match="complex64"):
+        h.diopiSilu(1, torch.zeros(1, dtype=torch.complex64), None)
+    with pytest.raises(TypeError):
+        h.diopiSilu(1, torch.zeros(1))
+    with pytest.raises(RuntimeError, match="must match"):
+        h.broadcast_of(torch.zeros(3), torch.zeros(4), False)
