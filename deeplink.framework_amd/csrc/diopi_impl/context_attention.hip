@@ -448,6 +448,122 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void contextAttnSingleBlockKe
   contextAttnBlock<T, D, PART>(a, numQBlocks - 1 - rank, h, b);
 }
 
+// fp32 with head sizes 64 and 128 on the fp32 matrix instructions (true fp32 products and sums). A workgroup takes 16
+// queries of a head and its four waves every fourth tile of 16 keys, each with a softmax state of its own; the states meet
+// in LDS at the end, so a short sequence is four times as many waves and a chain of loads a quarter as long. What bounds
+// the short sequences of the fp32 configuration is exactly that chain of latencies (2 x 128 tokens, 8 heads of 64: 55 us
+// with a workgroup per query and scores in LDS, 6 now; 4 x 2048 tokens, 8 heads of 128: 622 us, 0.4 of the fp32 matrix peak).
+// v_mfma_f32_16x16x4_f32: lane (c = l & 15, g = l >> 4) feeds row c, k = g of both operands and receives D[4 g + r][c].
+//   S^T = K Q^T: the contraction order is free as long as both operands agree, so group g takes the D / 4 consecutive
+//   elements from g D / 4 on: 16-byte loads straight into operand registers. The lane ends up with keys 4 g .. 4 g + 3 of
+//   query c, which is P^T's operand layout when step r takes key 4 g + r from group g: no data moves between lanes.
+//   O^T = V^T P^T: row i of output tile t stands for element i (D / 16) + t, so a lane's D / 16 operands of a key are
+//   consecutive in memory, and its results are D / 4 consecutive elements of query c.
+template <int D>
+__global__ __launch_bounds__(256) void contextAttnF32Kernel(CaArgs a) {
+  constexpr int S = D / 4, T = D / 16, PITCH = D + 4;
+  __shared__ __attribute__((aligned(16))) float so[4][16][PITCH];
+  __shared__ float sm[4][16], sl[4][16];
+  const int h = blockIdx.y, b = blockIdx.z, qb = (int)(gridDim.x - 1 - blockIdx.x);  // the longest rows first
+  const int64_t start = ldIdxCA(a.bStart, b, a.start64);
+  const int len = (int)ldIdxCA(a.bLen, b, a.len64), q0 = qb * 16;
+  if (q0 >= len) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+  const int kvh = h / (a.heads / a.kvHeads), tiles = qb + 1;
+  const float* kg = reinterpret_cast<const float*>(a.k) + start * a.kTok + (int64_t)kvh * a.kHead + g * S;
+  const float* vg = reinterpret_cast<const float*>(a.v) + start * a.vTok + (int64_t)kvh * a.vHead + c * T;
+  f32x4 qf[S / 4], kf[2][S / 4], vf[2][4][T / 4], o[T];
+  {
+    const float* q = reinterpret_cast<const float*>(a.q) + (start + min(q0 + c, len - 1)) * a.qTok + (int64_t)h * a.qHead + g * S;
+#pragma unroll
+    for (int s = 0; s < S / 4; ++s) qf[s] = *reinterpret_cast<const f32x4*>(q + 4 * s);
+  }
+  auto fetch = [&](int t, auto buf) {  // keys past the sequence are clamped: they are past the diagonal too
+    constexpr int B = decltype(buf)::value;
+    const float* kr = kg + (int64_t)min(t * 16 + c, len - 1) * a.kTok;
+#pragma unroll
+    for (int s = 0; s < S / 4; ++s) kf[B][s] = *reinterpret_cast<const f32x4*>(kr + 4 * s);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float* vr = vg + (int64_t)min(t * 16 + 4 * g + r, len - 1) * a.vTok;
+#pragma unroll
+      for (int i = 0; i < T / 4; ++i) vf[B][r][i] = *reinterpret_cast<const f32x4*>(vr + 4 * i);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < T; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  auto tile = [&](int t, auto buf) {
+    constexpr int B = decltype(buf)::value;
+    f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};  // two chains: half the dependent latency
+#pragma unroll
+    for (int s = 0; s < S; ++s) acc[s & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[B][s >> 2][s & 3], qf[s >> 2][s & 3], acc[s & 1], 0, 0, 0);
+    float p[4], mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      p[r] = t * 16 + 4 * g + r <= q0 + c ? (acc[0][r] + acc[1][r]) * a.scale : -INFINITY;
+      mx = fmaxf(mx, p[r]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float mNew = fmaxf(m, mx), keep = expf(m - mNew);  // (key 16 t is at or before every query of the block)
+    m = mNew;
+    l *= keep;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      p[r] = expf(p[r] - mNew);
+      l += p[r];
+    }
+#pragma unroll
+    for (int i = 0; i < T; ++i) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[i][r] *= keep;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < T; ++i) o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[B][r][i >> 2][i & 3], p[r], o[i], 0, 0, 0);
+  };
+  using B0 = std::integral_constant<int, 0>;
+  using B1 = std::integral_constant<int, 1>;
+  if (wave < tiles) fetch(wave, B0{});
+  for (int t = wave; t < tiles; t += 8) {
+    if (t + 4 < tiles) fetch(t + 4, B1{});
+    tile(t, B0{});
+    if (t + 4 < tiles) {
+      if (t + 8 < tiles) fetch(t + 8, B0{});
+      tile(t + 4, B1{});
+    }
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (g == 0) sm[wave][c] = m, sl[wave][c] = l;
+  __syncthreads();
+  const float mAll = fmaxf(fmaxf(sm[0][c], sm[1][c]), fmaxf(sm[2][c], sm[3][c]));
+  const float f = expf(m - mAll);  // 0 for a wave without a tile
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int i = 0; i < T / 4; ++i)
+      *reinterpret_cast<f32x4*>(&so[wave][c][(4 * g + r) * T + 4 * i]) = f32x4{o[4 * i][r] * f, o[4 * i + 1][r] * f, o[4 * i + 2][r] * f, o[4 * i + 3][r] * f};
+  __syncthreads();
+  const int row = threadIdx.x >> 4, e0 = (threadIdx.x & 15) * T;
+  if (q0 + row >= len) return;
+  const float mRow = fmaxf(fmaxf(sm[0][row], sm[1][row]), fmaxf(sm[2][row], sm[3][row]));
+  float sum = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) sum += sl[w][row] * expf(sm[w][row] - mRow);
+  const float inv = 1.f / sum;
+  float* out = reinterpret_cast<float*>(a.out) + (start + q0 + row) * a.oTok + (int64_t)h * a.oHead + e0;
+#pragma unroll
+  for (int i = 0; i < T / 4; ++i) {
+    f32x4 v = *reinterpret_cast<const f32x4*>(&so[0][row][e0 + 4 * i]);
+#pragma unroll
+    for (int w = 1; w < 4; ++w) v += *reinterpret_cast<const f32x4*>(&so[w][row][e0 + 4 * i]);
+    *reinterpret_cast<f32x4*>(out + 4 * i) = v * inv;
+  }
+}
+
 // One workgroup per (query token, head): scores to LDS, softmax, then P.V with lanes over d.
 template <typename T>
 __global__ __launch_bounds__(256) void contextAttnScalarKernel(CaArgs a, int maxLen) {
@@ -594,6 +710,12 @@ extern "C" __attribute__((visibility("default"))) diopiError_t diopiContextAtten
       err = a.d <= 64    ? launchCaMfma<half_t, 64>(stream, a, maxInputLen, batch)
             : a.d <= 128 ? launchCaMfma<half_t, 128>(stream, a, maxInputLen, batch)
                          : launchCaMfma<half_t, 256>(stream, a, maxInputLen, batch);
+  } else if (q.dtype == diopi_dtype_float32 && (a.d == 64 || a.d == 128) && al(cq) && al(ck) && al(cv) && al(co)) {
+    const dim3 grid((unsigned)ceilDiv(maxInputLen, 16), (unsigned)a.heads, (unsigned)batch);
+    if (a.d == 64) hipLaunchKernelGGL(contextAttnF32Kernel<64>, grid, dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL(contextAttnF32Kernel<128>, grid, dim3(256), 0, stream, a);
+    err = hipGetLastError() == hipSuccess ? diopiSuccess : diopiErrorOccurred;
+    if (err != diopiSuccess) setLastError("context attention: fp32 kernel launch failed");
   } else {
     AMD_CHECK(maxInputLen <= 12000, "context attention: the scalar path supports sequences up to 12000 tokens, got %d", maxInputLen);
     AMD_CHECK(maxInputLen <= 65535, "context attention: grid limits exceeded");

@@ -114,6 +114,24 @@ def test_fp32_gemm_on_the_matrix_cores(ops, dev, m, n, k, form):
         assert_exact(ops.linear(onehot.to(dev), w.to(dev)), w.t()[torch.arange(m) % k])
 
 
+@pytest.mark.parametrize("batch,m,n,k", [(1, 256, 512, 1376), (1, 1, 33, 4), (1, 31, 100, 516), (3, 65, 64, 1024 + 28), (1, 700, 512, 96)])
+def test_fp32_gemm_with_few_tiles(ops, dev, batch, m, n, k):
+    """32 x 32 tiles with K dealt over the waves: fewer stretches of 32 than waves, none at all, a K that ends inside one,
+    ragged rows and columns, a batch, bias and addend; and exactly on one-hot rows."""
+    x, w = torch.randn(batch, m, k, generator=g(95)), torch.randn(n, k, generator=g(96))
+    bias, c = torch.randn(n, generator=g(97)), torch.randn(batch, m, n, generator=g(98))
+    want = x.double() @ w.double().t()
+    dx, dw = x.to(dev), w.to(dev)
+    assert_fp32(ops.linear(dx, dw, bias.to(dev)), want + bias.double())
+    wb = dw.t().unsqueeze(0).expand(batch, k, n)
+    assert_fp32(ops.baddbmm(c.to(dev), dx, wb, beta=0.5, alpha=2), 0.5 * c.double() + 2 * want)
+    onehot = torch.zeros(m, k)
+    cols = torch.randint(0, k, (m,), generator=g(99))
+    cols[-1] = k - 1
+    onehot[torch.arange(m), cols] = 1
+    assert_exact(ops.linear(onehot.to(dev), dw), w[:, cols].t().contiguous())
+
+
 def test_gemm_linearity_at_7b_shapes(ops, dev):
     # size-independent property at the full prefill shape: f(x1 + x2) = f(x1) + f(x2), and a
     # one-hot row selects a weight column exactly
@@ -519,6 +537,28 @@ def test_context_attention_gqa_and_strided_inputs(ops, dev):
     got = ops.context_attention(dq[0].reshape(total, heads, d), dq[1].reshape(total, kvh, d), dq[2].reshape(total, kvh, d),
                                 st.to(dev), ln.to(dev), 157)
     assert_half(got, want)
+
+
+@pytest.mark.parametrize("heads,kvh,d,lens", [(8, 8, 64, [128, 128]), (8, 2, 128, [1, 15, 16, 17, 33]), (4, 4, 64, [64, 65, 200]), (2, 1, 128, [130])])
+def test_context_attention_fp32_on_the_matrix_cores(ops, dev, heads, kvh, d, lens):
+    """16 queries per workgroup, key tiles dealt over its four waves: fewer key tiles than waves, one and several rounds of
+    them, lengths around a tile's edge, shared K/V heads, and q, k, v as slices of one projection."""
+    total = sum(lens)
+    qkv = torch.randn(total, heads + 2 * kvh, d, generator=g(43))
+    starts = torch.tensor([sum(lens[:i]) for i in range(len(lens))], dtype=torch.int32)
+    ln = torch.tensor(lens, dtype=torch.int32)
+    dq = qkv.to(dev)
+    q, k, v = qkv[:, :heads], qkv[:, heads:heads + kvh], qkv[:, heads + kvh:]
+    got = ops.context_attention(dq[:, :heads], dq[:, heads:heads + kvh], dq[:, heads + kvh:], starts.to(dev), ln.to(dev), max(lens),
+                                out=torch.empty(total, heads, d, device=dev))
+    want = torch.empty(total, heads, d, dtype=torch.float64)
+    for s, n in zip(starts.tolist(), lens):
+        kk = k[s:s + n].double().repeat_interleave(heads // kvh, 1)
+        vv = v[s:s + n].double().repeat_interleave(heads // kvh, 1)
+        sc = torch.einsum("qhd,khd->hqk", q[s:s + n].double(), kk) / d ** 0.5
+        sc = sc.masked_fill(torch.ones(n, n, dtype=torch.bool).triu(1), float("-inf"))
+        want[s:s + n] = torch.einsum("hqk,khd->qhd", torch.softmax(sc, -1), vv)
+    assert_fp32(got, want)
 
 
 def test_context_attention_uniform_keys_give_running_mean_at_length_2048(ops, dev):
