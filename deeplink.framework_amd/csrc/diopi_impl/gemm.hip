@@ -2194,6 +2194,116 @@ __global__ __launch_bounds__(256) void gemmMfmaF32DirectKernel(GemmProblem p) {
   gemmF32StoreTile<WT>(p, acc, m0, n0, batch, wm, wn, l32, half);
 }
 
+// fp32 products with few tiles (the fp32 configuration's 256 rows): 32 x 32 output tiles, the K range dealt over the
+// workgroup's waves in stretches of 32 and the partial sums added in LDS, so that a 256 x 512 output is 128 workgroups of
+// 8 waves instead of 32 of 4 and a wave walks K / 256 stretches instead of K / 32. What bounds these products is the chain
+// of load latencies along K. Every wave has a two-stage LDS ring of its own (a stretch is 32 rows of 128 bytes of either
+// operand, copied straight into LDS, 8 rows to an instruction, and swizzled as in the kernel above), so there is no barrier
+// before the reduction. (Loading the operands straight into MFMA registers, 32 row pieces of 32 bytes to an instruction, is
+// bound by the vector cache: 12 us where this form takes 8.)
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void gemmF32SmallKernel(GemmProblem p) {
+  extern __shared__ __attribute__((aligned(1024))) float ring[];  // [WAVES][2 stages][A | B][32 rows][32]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l32 = lane & 31, half = lane >> 5;
+  int tm, tn;
+  xcdBandTile(blockIdx.x, (int)((p.M + 31) / 32), (int)((p.N + 31) / 32), &tm, &tn);
+  const int64_t m0 = (int64_t)tm * 32, n0 = (int64_t)tn * 32, batch = blockIdx.z;
+  // rows past the end are clamped (their products land in rows or columns that are never stored)
+  const float* A = reinterpret_cast<const float*>(p.A) + batch * p.sAb;
+  const float* B = reinterpret_cast<const float*>(p.B) + batch * p.sBb;
+  const int whole = (int)(p.K / 32), count = (whole - wave + WAVES - 1) / WAVES;  // this wave's stretches: wave, wave + WAVES, ...
+  const float* pa[4];
+  const float* pb[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = i * 8 + (lane >> 3), chunk = (lane & 7) ^ f32Swz(row);
+    pa[i] = A + min(m0 + row, p.M - 1) * p.sAm + wave * 32 + chunk * 4;
+    pb[i] = B + min(n0 + row, p.N - 1) * p.sBn + wave * 32 + chunk * 4;
+  }
+  typedef __attribute__((address_space(3))) void* LdsPtr;
+  float* mine = ring + wave * 4096;
+  const unsigned mineLds = (unsigned)(uintptr_t)(LdsPtr)mine;
+  auto fetch = [&](int stage) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the fragment reads of this stage are back
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      globalLoadToLds16(pa[i], mineLds + stage * 8192u + i * 1024u);
+      globalLoadToLds16(pb[i], mineLds + stage * 8192u + 4096u + i * 1024u);
+      pa[i] += WAVES * 32;
+      pb[i] += WAVES * 32;
+    }
+  };
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  f32x4 fa[4], fb[4];
+  auto multiply = [&]() {  // lane half h takes k = 8 q + 4 h + j at step (q, j)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[q][j], fa[q][j], acc, 0, 0, 0);
+  };
+  if (count > 0) fetch(0);
+  for (int i = 0; i < count; ++i) {
+    if (i + 1 < count) {
+      fetch((i + 1) & 1);
+      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    const float* s = mine + (i & 1) * 2048 + l32 * 32;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int at = ((2 * q + half) ^ f32Swz(l32)) << 2;
+      fa[q] = *reinterpret_cast<const f32x4*>(s + at);
+      fb[q] = *reinterpret_cast<const f32x4*>(s + 1024 + at);
+    }
+    multiply();
+  }
+  if (wave == WAVES - 1 && (p.K & 31) != 0) {  // what is left of K behind the whole stretches
+    const float* a = A + min(m0 + l32, p.M - 1) * p.sAm;
+    const float* b = B + min(n0 + l32, p.N - 1) * p.sBn;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int64_t k = (int64_t)whole * 32 + 8 * q + 4 * half;
+      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+      fa[q] = k < p.K ? *reinterpret_cast<const f32x4*>(a + k) : zero;  // K is a multiple of 4: a piece is entirely in or out
+      fb[q] = k < p.K ? *reinterpret_cast<const f32x4*>(b + k) : zero;
+    }
+    multiply();
+  }
+  // (over this wave's own ring, whose reads are all back: they fed the products)
+  f32x4* red = reinterpret_cast<f32x4*>(ring);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) red[wave * 1024 + g * 64 + lane] = f32x4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+  __syncthreads();
+  if (threadIdx.x >= 256) return;
+  // thread (g = wave, lane): row l32, columns 8 g + 4 half .. + 3 of the tile
+  f32x4 s = red[wave * 64 + lane];
+#pragma unroll
+  for (int w = 1; w < WAVES; ++w) s += red[w * 1024 + wave * 64 + lane];
+  const int64_t row = m0 + l32, col = n0 + 8 * wave + 4 * half;
+  if (row >= p.M || col >= p.N) return;
+  float* out = reinterpret_cast<float*>(p.out) + batch * p.sOb;
+  const float* cin = p.Cin ? reinterpret_cast<const float*>(p.Cin) + batch * p.sCb : nullptr;
+  const float* bias = reinterpret_cast<const float*>(p.bias);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    s[r] *= p.alpha;
+    if (col + r < p.N) {
+      if (bias) s[r] += bias[col + r];
+      if (cin) s[r] += p.beta * cin[row * p.sCm + (col + r) * p.sCn];
+    }
+  }
+  if ((p.N & 3) == 0 && (p.sOm & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
+    *reinterpret_cast<f32x4*>(out + row * p.sOm + col) = s;
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (col + r < p.N) out[row * p.sOm + col + r] = s[r];
+  }
+}
+
 // Whether gemmMfmaF32Kernel can take the problem: each operand contiguous along K or along its rows, 16-byte pieces
 // whole and aligned.
 constexpr int kF32BKBig = 32;  // stage depth of the 128 x 128 tile
@@ -2902,6 +3012,23 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
     dim3 grid((unsigned)ceilDiv(p.N, 256), (unsigned)p.M, (unsigned)p.batch);
     AMD_CHECK(p.M <= 65535, "gemm(float64): M exceeds the grid limit");
     hipLaunchKernelGGL(gemmFmaKernelF64, grid, dim3(256), 0, stream, p);
+    AMD_LAUNCH_CHECK();
+    return diopiSuccess;
+  }
+  if (p.dtype == diopi_dtype_float32 && p.sAk == 1 && p.sBk == 1 && f32MfmaEligible(p) &&
+      ceilDiv(p.M, 64) * ceilDiv(p.N, 64) * p.batch * 4 < (int64_t)computeUnits() * 3) {
+    // Tiles of 64 x 64 for less than three quarters of the compute units (any number of rows): 32 x 32 tiles with K dealt
+    // over the waves. us, 64 x 64 tiles -> this form: 256 x 1536 x 512 (96 tiles) 13.2 -> 8.7, 256 x 512 x 1376 (32) 29.5 ->
+    // 10.5, 1024 x 512 x 1376 (128) 29.7 -> 19.5, 16 x 512 x 1376 108 -> 9.9 (the FMA engine took fewer than 32 rows); from a
+    // tile per unit on the larger tile wins (1024 x 1024 x 2816, 256 tiles: 57 against 67).
+    dim3 grid((unsigned)(ceilDiv(p.N, 32) * ceilDiv(p.M, 32)), 1, (unsigned)p.batch);
+    if (p.K >= 1024) {
+      AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(&gemmF32SmallKernel<8>), 8 * 16384));
+      hipLaunchKernelGGL(gemmF32SmallKernel<8>, grid, dim3(512), 8 * 16384, stream, p);
+    } else {
+      AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(&gemmF32SmallKernel<4>), 4 * 16384));
+      hipLaunchKernelGGL(gemmF32SmallKernel<4>, grid, dim3(256), 4 * 16384, stream, p);
+    }
     AMD_LAUNCH_CHECK();
     return diopiSuccess;
   }
