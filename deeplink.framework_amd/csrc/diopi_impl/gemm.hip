@@ -2480,6 +2480,20 @@ struct RotaryEpilogue {
   float sinSign;
 };
 
+// Workspace for a form that is only faster than one without: null where the runtime has none to give, and null while the
+// stream is recorded into a graph. A recorded buffer has to outlive the recording, which only callers of the functions
+// that cannot do without one see to.
+static bool recording(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();  // (the null stream beside a global capture)
+  return true;
+}
+static void* spareWorkspace(diopiContextHandle_t ctx, hipStream_t stream, int64_t nbytes) {
+  void* ws = nullptr;
+  return !recording(stream) && requireWorkspace(ctx, nbytes, &ws) == diopiSuccess ? ws : nullptr;
+}
+
 // How the tiles of a 4-wave launch are worked off: whole tiles first, the rest in K slices (slices == 1: no split), and
 // what the rest then costs in us.
 struct TailSplit {
@@ -2507,10 +2521,8 @@ static TailSplit tailSplit(int64_t tiles, int64_t pairs, int resident) {
 }
 
 template <typename T, int EPI>
-static diopiError_t launchTailSplit(diopiContextHandle_t ctx, hipStream_t stream, MfmaArgs g, const TailSplit& tail, int resident) {
+static diopiError_t launchTailSplit(hipStream_t stream, MfmaArgs g, const TailSplit& tail, int resident, void* ws) {
   const int rest = g.tilesM * g.tilesN - tail.whole, items = rest * tail.slices;
-  void* ws = nullptr;
-  AMD_TRY(requireWorkspace(ctx, (int64_t)items * kTailSlotFloats * 4, &ws));
   g.partial = static_cast<float*>(ws), g.wholeTiles = tail.whole, g.kSlices = tail.slices;
   // a launch with whole tiles has one workgroup per CU (whole is a multiple of that); one of slices alone has one per slice
   const dim3 grid((unsigned)(tail.whole ? resident : std::min(items, resident)));
@@ -2574,11 +2586,12 @@ static diopiError_t launchMfmaPipelined(diopiContextHandle_t ctx, hipStream_t st
       const int resident = computeUnits() / 8 * 8;
       if (p.batch == 1 && resident >= 8) {
         const TailSplit tail = tailSplit((int64_t)g.tilesM * g.tilesN, p.K / (2 * kBK), resident);
-        if (tail.slices > 1) {
+        const int64_t slots = ((int64_t)g.tilesM * g.tilesN - tail.whole) * tail.slices;
+        if (void* ws = tail.slices > 1 ? spareWorkspace(ctx, stream, slots * kTailSlotFloats * 4) : nullptr) {
           if constexpr (EPI == kEpiLinear) {
-            if (p.Cin) return launchTailSplit<T, kEpiAddendLds>(ctx, stream, g, tail, resident);
+            if (p.Cin) return launchTailSplit<T, kEpiAddendLds>(stream, g, tail, resident, ws);
           }
-          return launchTailSplit<T, EPI>(ctx, stream, g, tail, resident);
+          return launchTailSplit<T, EPI>(stream, g, tail, resident, ws);
         }
       }
       if (resident >= 8 && (int)grid.x > resident) grid.x = (unsigned)resident;
@@ -2952,7 +2965,9 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
     // (a matrix at most 128 columns wide would leave half of every 256-wide tile empty: it takes the 128 x 128 form)
     // and so does a product of only two K tiles, which is all tile turnover: two workgroups per CU overlap one tile's
     // stores with the other's loads (bmm [128, 2048, 128] x [128, 128, 2048]: 421 -> 368 us)
-    const bool big = (ceilDiv(p.M, 256) * ceilDiv(p.N, 256) * p.batch >= 144 || (!bT && tailSplitPays(p))) && p.N > 128 && p.K > 2 * kBK;
+    // (a column scale: the caller has asked gemmAppliesColumnScale)
+    const bool big = (ceilDiv(p.M, 256) * ceilDiv(p.N, 256) * p.batch >= 144 || p.colScale || (!bT && !recording(stream) && tailSplitPays(p))) &&
+                     p.N > 128 && p.K > 2 * kBK;
     const bool fits2g = bT || (((p.M - 1) * p.sAm + p.K) * 2 < (int64_t(1) << 31) && ((p.N - 1) * p.sBn + p.K) * 2 < (int64_t(1) << 31));
     if (big && p.K % kBK == 0 && p.K >= 2 * kBK && fits2g) {
       if (p.colScale)
@@ -2990,22 +3005,27 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
     }
     return big ? launchMfma<half_t, 256, 256>(stream, p) : launchMfma<half_t, 128, 128>(stream, p);
   }
-  if (half && p.K > 0 && p.M < (int64_t(1) << 31) && p.N < (int64_t(1) << 31) && p.K <= 65535 * 64) {  // (the transposing copies' grid limit)
-    // K is no multiple of 8: the 128 x 128 kernel that reads rows at element alignment; an operand whose K is not
-    // contiguous is transposed into workspace first
-    if (p.sAk != 1) {
-      void* ws = nullptr;
-      AMD_TRY(requireWorkspace(ctx, p.batch * p.M * p.K * 2, &ws));
+  // K is no multiple of 8: the 128 x 128 kernel that reads rows at element alignment; an operand whose K is not contiguous
+  // is transposed into workspace first, and where there is none to spare the FMA engine below takes the product
+  bool ragged = half && p.K > 0 && p.M < (int64_t(1) << 31) && p.N < (int64_t(1) << 31) && p.K <= 65535 * 64;  // (the transposing copies' grid limit)
+  if (ragged) {
+    const int64_t nb = p.sBb == 0 ? 1 : p.batch;  // a shared (broadcast) weight is transposed once
+    const int64_t aBytes = p.sAk != 1 ? p.batch * p.M * p.K * 2 : 0, bBytes = p.sBk != 1 ? nb * p.N * p.K * 2 : 0;
+    char* ws = nullptr;
+    if (aBytes + bBytes > 0) {
+      ws = static_cast<char*>(spareWorkspace(ctx, stream, aBytes + bBytes));
+      ragged = ws != nullptr;
+    }
+    if (ragged && aBytes) {
       AMD_TRY(launchTranspose<uint16_t>(stream, ws, p.A, p.batch, p.K, p.M, p.sAk, p.sAm, p.sAb));
       p.A = ws, p.sAk = 1, p.sAm = p.K, p.sAb = p.M * p.K;
     }
-    if (p.sBk != 1) {
-      const int64_t nb = p.sBb == 0 ? 1 : p.batch;  // a shared (broadcast) weight is transposed once
-      void* ws = nullptr;
-      AMD_TRY(requireWorkspace(ctx, nb * p.N * p.K * 2, &ws));
-      AMD_TRY(launchTranspose<uint16_t>(stream, ws, p.B, nb, p.K, p.N, p.sBk, p.sBn, p.sBb));
-      p.B = ws, p.sBk = 1, p.sBn = p.K, p.sBb = p.sBb == 0 ? 0 : p.N * p.K;
+    if (ragged && bBytes) {
+      AMD_TRY(launchTranspose<uint16_t>(stream, ws + aBytes, p.B, nb, p.K, p.N, p.sBk, p.sBn, p.sBb));
+      p.B = ws + aBytes, p.sBk = 1, p.sBn = p.K, p.sBb = p.sBb == 0 ? 0 : p.N * p.K;
     }
+  }
+  if (ragged) {
     return p.dtype == diopi_dtype_bfloat16 ? launchMfma<bf16_t, 128, 128, true>(stream, p) : launchMfma<half_t, 128, 128, true>(stream, p);
   }
   if (p.dtype == diopi_dtype_float64) {

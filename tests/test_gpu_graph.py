@@ -133,3 +133,26 @@ def test_workspace_request_during_capture_is_served_from_the_cache_or_refused(op
     assert torch.allclose(out.cpu(), torch.softmax(x.cpu(), 1), atol=1e-6)
     del graph
     scope.close()
+
+
+def test_products_that_can_do_without_workspace_record_without_it(pkg, ops, dev):
+    """Products whose fast form takes workspace and whose plain form needs none: recorded with nothing held for them they take
+    the plain form. Each replay is checked with eager work, which uses the cached workspace, in between."""
+    rnd = lambda *shape: torch.randint(-2, 3, shape, generator=gen).to(torch.bfloat16).to(dev)     # (exact sums)
+    gen = torch.Generator().manual_seed(7)
+    x, w = rnd(1554, 4096), rnd(11008, 4096)
+    a, b = rnd(2, 77, 65), rnd(2, 65, 40)
+    calls = [lambda: ops.linear(x, w), lambda: ops.bmm(a, b)]
+    want = [f() for f in calls]
+    torch.cuda.synchronize()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=side):
+        got = [f() for f in calls]
+    for _ in range(4):
+        for t in got:
+            t.zero_()
+        graph.replay()
+        again = [f() for f in calls]
+        torch.cuda.synchronize()
+        for t, u, v in zip(got, want, again):
+            assert torch.equal(t, u) and torch.equal(u, v)
