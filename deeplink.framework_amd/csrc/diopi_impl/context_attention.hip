@@ -506,18 +506,43 @@ __global__ __launch_bounds__(256) void contextAttnF32Kernel(CaArgs a) {
     }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float mNew = fmaxf(m, mx), keep = expf(m - mNew);  // (key 16 t is at or before every query of the block)
+    const float mNew = fmaxf(m, mx), from = mNew == -INFINITY ? 0.f : mNew;  // (-inf: scores that overflowed, so far nothing else)
+    const float keep = expf(m - from);
     m = mNew;
     l *= keep;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      p[r] = expf(p[r] - mNew);
+      p[r] = expf(p[r] - from);
       l += p[r];
     }
 #pragma unroll
     for (int i = 0; i < T; ++i) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[i][r] *= keep;
+    }
+    if (t == qb) {
+      // the diagonal tile: a weight of 0 does not keep a later key's infinity or NaN out of an earlier query's sum, so with
+      // such a value in the tile every query takes products of its own keys only
+      float odd = 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < T; ++i) odd += vf[B][r][i >> 2][i & 3] * 0.f;
+      if (__ballot(odd != 0.f) != 0) {
+        for (int own = 0; own < 16; ++own)
+#pragma unroll
+          for (int i = 0; i < T; ++i) {
+            f32x4 one = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float v = 4 * g + r <= own ? vf[B][r][i >> 2][i & 3] : 0.f;
+              one = __builtin_amdgcn_mfma_f32_16x16x4f32(v, p[r], one, 0, 0, 0);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[i][r] += c == own ? one[r] : 0.f;
+          }
+        return;
+      }
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r)

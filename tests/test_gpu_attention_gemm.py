@@ -561,6 +561,29 @@ def test_context_attention_fp32_on_the_matrix_cores(ops, dev, heads, kvh, d, len
     assert_fp32(got, want)
 
 
+@pytest.mark.parametrize("d,n", [(64, 44), (128, 100)])
+def test_context_attention_fp32_keeps_later_keys_and_overflowed_scores_out(ops, dev, d, n):
+    """A V row that is infinite or NaN reaches the queries from its own position on and no earlier one, and a key whose score
+    is -inf has weight 0 even if it is the first that a wave meets."""
+    q, k, v = (torch.randn(n, 2, d, generator=g(44)) for _ in range(3))
+    at = n - 9
+    v[at, 0, 3], v[at, 1, 5] = float("inf"), float("nan")
+    q[:, :, 0] = q[:, :, 0].abs() + 1
+    k[17:32, :, 0] = float("-inf")
+    k[16, :, 0] = float("-inf")
+    starts, ln = torch.zeros(1, dtype=torch.int32, device=dev), torch.full((1,), n, dtype=torch.int32, device=dev)
+    got = ops.context_attention(q.to(dev), k.to(dev), v.to(dev), starts, ln, n, out=torch.empty(n, 2, d, device=dev)).cpu()
+    clean = v.clone()
+    clean[at] = 0
+    sc = torch.einsum("qhd,khd->hqk", q.double(), k.double()) / d ** 0.5
+    sc = sc.masked_fill(torch.ones(n, n, dtype=torch.bool).triu(1), float("-inf"))
+    p = torch.softmax(sc, -1)
+    want = torch.einsum("hqk,khd->qhd", p, clean.double()) + torch.einsum("hq,hd->qhd", p[:, :, at], v[at].double().nan_to_num(0, 0))
+    assert_fp32(torch.where(got.isfinite(), got, want.float()), want)
+    assert got[:at].isfinite().all() and (got[at:, 0, 3] == float("inf")).all() and got[at:, 1, 5].isnan().all()
+    assert (~got.isfinite()).sum() == 2 * (n - at)
+
+
 def test_context_attention_uniform_keys_give_running_mean_at_length_2048(ops, dev):
     # property that holds at the full sequence length: identical keys -> uniform weights
     n, heads, d = 2048, 2, 128
