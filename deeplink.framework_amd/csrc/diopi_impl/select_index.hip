@@ -431,16 +431,16 @@ static diopiError_t runSelect(diopiContextHandle_t ctx, diopiTensorHandle_t outH
         return diopiSuccess;
       }
       if (whole8) {
-      AMD_CHECK(blocks <= 0x7fffffff, "%s: %ld elements exceed the grid limit", name, (long)out.numel);
-      if (out.itemsize == 2)
-        hipLaunchKernelGGL((selectVecKernel<uint16_t>), dim3((unsigned)blocks), dim3(kSelThreads), 0, stream, out.ptr<uint16_t>(),
-                           cond.ptr<uint8_t>(), aScalar ? nullptr : a.ptr<uint16_t>(), b.ptr<uint16_t>(), nvec, condVecs,
-                           (uint16_t)bits);
-      else
-        hipLaunchKernelGGL((selectVecKernel<uint32_t>), dim3((unsigned)blocks), dim3(kSelThreads), 0, stream, out.ptr<uint32_t>(),
-                           cond.ptr<uint8_t>(), aScalar ? nullptr : a.ptr<uint32_t>(), b.ptr<uint32_t>(), nvec, condVecs, bits);
-      AMD_LAUNCH_CHECK();
-      return diopiSuccess;
+        AMD_CHECK(blocks <= 0x7fffffff, "%s: %ld elements exceed the grid limit", name, (long)out.numel);
+        if (out.itemsize == 2)
+          hipLaunchKernelGGL((selectVecKernel<uint16_t>), dim3((unsigned)blocks), dim3(kSelThreads), 0, stream, out.ptr<uint16_t>(),
+                             cond.ptr<uint8_t>(), aScalar ? nullptr : a.ptr<uint16_t>(), b.ptr<uint16_t>(), nvec, condVecs,
+                             (uint16_t)bits);
+        else
+          hipLaunchKernelGGL((selectVecKernel<uint32_t>), dim3((unsigned)blocks), dim3(kSelThreads), 0, stream, out.ptr<uint32_t>(),
+                             cond.ptr<uint8_t>(), aScalar ? nullptr : a.ptr<uint32_t>(), b.ptr<uint32_t>(), nvec, condVecs, bits);
+        AMD_LAUNCH_CHECK();
+        return diopiSuccess;
       }
     }
   }
