@@ -304,6 +304,7 @@ __device__ __forceinline__ void ldsBarrier() {
 
 // 8 waves (2 x 4, wave tile 128 x 64): two waves per SIMD, so one wave's LDS / VMEM issue
 // overlaps the other's MFMAs; measured faster than 4 waves of 128 x 128 and 16 of 64 x 64.
+constexpr int kDeepStages = 4;  // K tiles in the LDS ring of the 128 x 128 form with one workgroup per CU
 constexpr int kPipeWavesM = 2, kPipeWavesN = 4, kPipeThreads = kPipeWavesM * kPipeWavesN * 64;
 
 // v_mfma_f32_16x16x32: lane l feeds row (l & 15), K elements [8 * (l >> 4), +8) of both operands and
@@ -810,8 +811,14 @@ __device__ __forceinline__ void vectorEpilogue(const MfmaArgs& g, T* out, const 
 // values of column i). The 32-byte pieces of row k are XOR-swizzled with (k & 3) | 4 (k >> 3 & 1), which puts the 8
 // row pieces one half-wave touches (k .. k + 3 and k + 8 .. k + 11) on 8 different bank groups. g.ldb is then the
 // stride between k rows.
-template <typename T, int EPI, int TILE = 256, bool BT = false>
-__global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 ? 1 : 2) void gemmMfmaPipelinedKernel(MfmaArgs g) {
+//
+// STAGES: how many K tiles the LDS ring holds. With two, a tile is requested one tile's worth of products ahead; the 128 x
+// 128 form then takes 0.75 us per K tile, which is the latency of memory under load and not its 0.21 us of products or 0.3 us
+// of LDS traffic, and 1.19 us with two workgroups on the CU. With four (128 KiB, one workgroup per CU, three tiles under way)
+// it takes 0.5 us. From a second workgroup per CU on, two stages and two at once win (882 x 5120 x 5120, 280 tiles: 73
+// against 81 us).
+template <typename T, int EPI, int TILE = 256, bool BT = false, int STAGES = 2>
+__global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 || STAGES > 2 ? 1 : 2) void gemmMfmaPipelinedKernel(MfmaArgs g) {
   using Frag = typename MfmaOp<T>::Frag;
   constexpr int kWavesN = TILE == 256 ? kPipeWavesN : 2, kThreads = TILE == 256 ? kPipeThreads : 256;
   constexpr int BM = TILE, BN = TILE, WM = BM / kPipeWavesM, WN = BN / kWavesN, TM = WM / 16, TN = WN / 16;
@@ -820,8 +827,8 @@ __global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 ? 1 :
   constexpr int RS = kThreads / 8;           // rows covered by one pass of the workgroup
   static_assert((HM == 4 || HM == 2) && TN == 4 && CH == 4, "the phase schedule below is written for 4 (or 2) x 4 fragments");
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  T* sA = reinterpret_cast<T*>(smem);  // [2][BM][64]
-  T* sB = sA + 2 * BM * kBK;           // [2][BN][64]
+  T* sA = reinterpret_cast<T*>(smem);  // [STAGES][BM][64]
+  T* sB = sA + STAGES * BM * kBK;      // [STAGES][BN][64]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / kWavesN, wn = wave % kWavesN;
   int tm, tn;
@@ -876,7 +883,7 @@ __global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 ? 1 :
       bOffG[i] = (int)(((int64_t)min(tn * BN + srow + RS * i, g.N - 1) * g.ldb + c8) * 2);
     }
   }
-  // LDS byte address of this wave's 1 KiB block in stage 0 of A; stage 1 is kStageBytes further, B 2 * kStageBytes
+  // LDS byte address of this wave's 1 KiB block in stage 0 of A; stage 1 is kStageBytes further, B STAGES * kStageBytes
   constexpr unsigned kStageBytes = BM * kBK * sizeof(T), kPassBytes = RS * kBK * sizeof(T);
   const unsigned ldsWave = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem +
                            __builtin_amdgcn_readfirstlane(wave) * 1024u;
@@ -903,7 +910,7 @@ __global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 ? 1 :
   };
   const int bTileStep = BT ? kBK * (int)g.ldb * (int)sizeof(T) : kBK * (int)sizeof(T);  // bytes from one K tile to the next
   auto dmaB = [&](int stage, int kt, int i) {
-    loadToLds16(rsB, bOffG[i], kt * bTileStep, ldsWave + (2 + stage) * kStageBytes + i * kPassBytes);
+    loadToLds16(rsB, bOffG[i], kt * bTileStep, ldsWave + (STAGES + stage) * kStageBytes + i * kPassBytes);
   };
   auto loadA = [&](int stage, int ks, int half, int buf, int i) {
     fa[buf][i] = *reinterpret_cast<const Frag*>(sA + stage * BM * kBK + aBase + kx[ks] + (half * HM + i) * 16 * kBK);
@@ -921,7 +928,7 @@ __global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 ? 1 :
     if constexpr (BT) {
       typedef typename MfmaOp<T>::Half HalfFrag;
       typedef __attribute__((address_space(3))) s16x4* LdsTr;
-      const unsigned at = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem + (2 + stage) * kStageBytes +
+      const unsigned at = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem + (STAGES + stage) * kStageBytes +
                           (unsigned)((ks * 32 + btRow) * BN * (int)sizeof(T) + btCol[j]);
       const HalfFrag lo = __builtin_bit_cast(HalfFrag, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsTr)(uintptr_t)at));
       const HalfFrag hi = __builtin_bit_cast(HalfFrag, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsTr)(uintptr_t)(at + 4 * BN * (unsigned)sizeof(T))));
@@ -947,32 +954,40 @@ __global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 ? 1 :
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // Publishes a stage: this wave's loads into it have landed (vmcnt) and its fragment reads of the
-  // stage about to be refilled are done (lgkmcnt), then all waves meet.
-  auto publish = [&]() {
-    __builtin_amdgcn_s_waitcnt(0x0070);
+  // Publishes a stage: this wave's loads into it have landed (vmcnt: loads arrive in order, and behind them only those of
+  // `behind` later tiles, eight each, may still be under way) and its fragment reads of the stage about to be refilled are
+  // done (lgkmcnt), then all waves meet.
+  auto publish = [&](auto behind) {
+    constexpr int loads = decltype(behind)::value * 2 * CH;
+    __builtin_amdgcn_s_waitcnt(0x0070 | (loads & 15) | (loads >> 4) << 14);
     __builtin_amdgcn_s_barrier();
   };
+  using std::integral_constant;
 
 #pragma unroll
-  for (int i = 0; i < CH; ++i) dmaA(0, 0, i);
+  for (int t = 0; t < STAGES - 1; ++t) {
 #pragma unroll
-  for (int i = 0; i < CH; ++i) dmaB(0, 0, i);
-  publish();
+    for (int i = 0; i < CH; ++i) dmaA(t, t, i);
 #pragma unroll
-  for (int i = 0; i < CH; ++i) dmaA(1, 1, i);  // the B half of tile 1 goes out in phase 0 below
+    for (int i = 0; i < CH; ++i) dmaB(t, t, i);
+  }
+  publish(integral_constant<int, STAGES - 2>{});
+#pragma unroll
+  for (int i = 0; i < CH; ++i) dmaA(STAGES - 1, STAGES - 1, i);  // the B half of this tile goes out in phase 0 below
 #pragma unroll
   for (int j = 0; j < TN; ++j) loadB(0, 0, j);
 #pragma unroll
   for (int i = 0; i < HM; ++i) loadA(0, 0, 0, 0, i);
 
-  // Iteration kt multiplies tile kt out of stage kt & 1 while tile kt + 1 lands in the other stage. Once
+  // Iteration kt multiplies tile kt out of stage kt % STAGES while the tiles after it land in the other stages. Once
   // every wave has passed the barrier before phase 3 nobody reads this stage any more, so the A half of
-  // tile kt + 2 is loaded into it right there and the B half in phase 0 of the next iteration: one load
+  // tile kt + STAGES is loaded into it right there and the B half in phase 0 of the next iteration: one load
   // per group of four MFMAs (all eight in one phase measured 1-4 % slower, all in phases 0-1 up to 7 %).
-  auto iter = [&](auto hasNext, auto hasNext2, int kt) {
-    constexpr bool kNext = decltype(hasNext)::value, kNext2 = decltype(hasNext2)::value;
-    const int cur = kt & 1;
+  // ahead: how many tiles follow this one, STAGES for that many or more.
+  auto iter = [&](auto ahead, int kt) {
+    constexpr int kAhead = decltype(ahead)::value;
+    constexpr bool kNext = kAhead >= 1;
+    const int cur = kt & (STAGES - 1), nxt = (kt + 1) & (STAGES - 1);
     __builtin_amdgcn_sched_barrier(0);
     // ---- phase 0: k-step 0, rows 0-63 | A fragments of phase 1 | B half of the next tile
     phase(0, 0,
@@ -983,7 +998,7 @@ __global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 ? 1 :
             }
           },
           [&](int j) {
-            if constexpr (kNext) dmaB(cur ^ 1, kt + 1, j);
+            if constexpr (kAhead >= STAGES - 1) dmaB((kt + STAGES - 1) & (STAGES - 1), kt + STAGES - 1, j);
           });
     // ---- phase 1: k-step 0, rows 64-127 | A of phase 2, B of k-step 1
     phase(1, 1,
@@ -1003,28 +1018,25 @@ __global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 ? 1 :
             }
           },
           [&](int) {});
-    if constexpr (kNext) publish();
+    if constexpr (kNext) publish(integral_constant<int, (kAhead >= STAGES ? STAGES - 1 : kAhead) - 1>{});
     __builtin_amdgcn_sched_barrier(0);
     // ---- phase 3: k-step 1, rows 64-127 | A and B of phase 0 of the next tile | A half of tile kt + 2
     phase(1, 1,
           [&](int j) {
-            if constexpr (kNext2) dmaA(cur, kt + 2, j);
+            if constexpr (kAhead >= STAGES) dmaA(cur, kt + STAGES, j);
             if constexpr (kNext) {
               if (j < HM / 2) {
-                loadA(cur ^ 1, 0, 0, 0, 2 * j);
-                loadA(cur ^ 1, 0, 0, 0, 2 * j + 1);
+                loadA(nxt, 0, 0, 0, 2 * j);
+                loadA(nxt, 0, 0, 0, 2 * j + 1);
               }
             }
           },
           [&](int j) {
-            if constexpr (kNext) loadB(cur ^ 1, 0, j);
+            if constexpr (kNext) loadB(nxt, 0, j);
           });
   };
-  using std::false_type;
-  using std::true_type;
-  for (int kt = 0; kt < nK - 2; ++kt) iter(true_type{}, true_type{}, kt);
-  iter(true_type{}, false_type{}, nK - 2);
-  iter(false_type{}, false_type{}, nK - 1);
+  for (int kt = 0; kt < nK - STAGES; ++kt) iter(integral_constant<int, STAGES>{}, kt);  // (nK >= STAGES)
+  staticFor<STAGES>([&](auto i) { iter(integral_constant<int, STAGES - 1 - decltype(i)::value>{}, nK - STAGES + decltype(i)::value); });
 
   // ---- epilogue
   if constexpr (EPI == kEpiPartial) {
@@ -2459,15 +2471,17 @@ static void launchSplitKReduce(hipStream_t stream, const MfmaArgs& g, int splits
   hipLaunchKernelGGL(splitKReduceKernel<T>, dim3((unsigned)ceilDiv(items, (int64_t)threads)), dim3(threads), 0, stream, g, splits);
 }
 
-// How many ways to split K so that a problem with few 128 x 128 tiles still fills the chip (two workgroups per CU):
-// tiles * splits close to twice the CU count, at least four K tiles per split, at most 16 splits. 1 = do not split.
-// *perSplit receives the K tiles per split; the last split has the remainder, never fewer than two (the kernel's
-// pipeline needs two).
+// How many ways to split K so that a problem with few 128 x 128 tiles still fills the chip with the four-stage kernel (one
+// workgroup per CU): tiles * splits up to the CU count, at least four K tiles per split, at most 16 splits. 1 = do not
+// split. *perSplit receives the K tiles per split; the last split has the remainder, never fewer than four unless K itself
+// is shorter. (Two stages and two workgroups per CU, the split of twice as many ways that this replaces, against it, us:
+// 128 x 4096 x 4096 21.5 -> 17.5, 203 x 12288 x 4096 47.3 -> 36.9, 203 x 4096 x 11008 40.8 -> 36.5, 400 x 5632 x 1024 23.1 -> 11.4,
+// 512 x 4096 x 11008 70 -> 63, 300 x 10240 x 8192 82 -> 64; 300 x 4096 x 11008, where 192 workgroups come out, 49.6 -> 51.2.)
 static int splitKWays(int64_t tiles, int64_t kTiles, int* perSplit) {
-  const int64_t byChip = 2 * computeUnits() / std::max<int64_t>(tiles, 1), byK = kTiles / 4;
+  const int64_t byChip = computeUnits() / std::max<int64_t>(tiles, 1), byK = kTiles / kDeepStages;
   int64_t splits = std::max<int64_t>(1, std::min<int64_t>(16, std::min(byChip, byK)));
   int64_t per = ceilDiv(kTiles, splits);
-  while (per < kTiles && kTiles % per == 1) ++per;
+  while (per < kTiles && kTiles % per != 0 && kTiles % per < kDeepStages) ++per;  // (the last slice too fills the ring)
   *perSplit = (int)per;
   return (int)ceilDiv(kTiles, per);
 }
@@ -2652,16 +2666,18 @@ static diopiError_t launchMfmaPipelined128(hipStream_t stream, const GemmProblem
   g.partial = partial;
   g.kTilesPerSplit = kTilesPerSplit;
   if (EPI == kEpiPartial) AMD_CHECK(g.vecEpilogue && p.batch == 1 && partial, "split-K: needs the vector epilogue and one batch");
-  constexpr size_t lds = 2 * (size_t)(128 + 128) * kBK * sizeof(T);
   dim3 grid((unsigned)(g.tilesM * g.tilesN), (unsigned)splits, (unsigned)p.batch);
-  if (bT) {
-    AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(&gemmMfmaPipelinedKernel<T, EPI, 128, true>), (int)lds));
-    hipLaunchKernelGGL((gemmMfmaPipelinedKernel<T, EPI, 128, true>), grid, dim3(256), lds, stream, g);
-  } else {
-    AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(&gemmMfmaPipelinedKernel<T, EPI, 128>), (int)lds));
-    hipLaunchKernelGGL((gemmMfmaPipelinedKernel<T, EPI, 128>), grid, dim3(256), lds, stream, g);
-  }
-  AMD_LAUNCH_CHECK();
+  auto launch = [&](auto stages) -> diopiError_t {
+    constexpr int STAGES = decltype(stages)::value;
+    constexpr size_t lds = STAGES * (size_t)(128 + 128) * kBK * sizeof(T);
+    auto* kernel = bT ? &gemmMfmaPipelinedKernel<T, EPI, 128, true, STAGES> : &gemmMfmaPipelinedKernel<T, EPI, 128, false, STAGES>;
+    AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(kernel), (int)lds));
+    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, stream, g);
+    AMD_LAUNCH_CHECK();
+    return diopiSuccess;
+  };
+  const int64_t kTiles = p.K / kBK, fewest = EPI == kEpiPartial ? kTiles - (int64_t)(splits - 1) * kTilesPerSplit : kTiles;
+  AMD_TRY(fewest >= kDeepStages && (int64_t)grid.x * grid.y * grid.z <= computeUnits() ? launch(std::integral_constant<int, kDeepStages>{}) : launch(std::integral_constant<int, 2>{}));
   if (EPI == kEpiPartial) {
     const int64_t items = p.M * (p.N / 8);
     launchSplitKReduce<T>(stream, g, splits, items);
@@ -2886,10 +2902,11 @@ diopiError_t transposeCopy(hipStream_t stream, void* dst, const void* src, int i
 
 // Whether a product with too few 256 x 256 tiles for a round of the chip runs faster as K slices of such tiles than on the
 // 128 x 128 kernel (itself split over K when its tiles are few): a long K, or a round's worth of slices that leaves each
-// of them a dozen K-tile pairs. The 128 x 128 kernel takes 0.75 us per K tile with one workgroup on a CU and 1.19 with
-// two, and its slices are written and read back as fp32 too. Measured, 128 x 128 -> slices of 256 x 256 (us):
-// 882 x 5120 x 13824 185 -> 116 (3 slices), 512 x 4096 x 11008 70 -> 56 (8), 512 x 12288 x 4096 73 -> 63 (2),
-// 203 x 12288 x 4096 48 -> 42 (5); not taken: 882 x 4096 x 4096 38 against 42, 300 x 4096 x 11008 48 against 52.
+// of them a dozen K-tile pairs. The 128 x 128 kernel takes about 0.5 us per K tile while its workgroups are no
+// more than the CUs and up to 1.19 with two on a CU, and its slices are written and read back as fp32 too. Measured,
+// 128 x 128 -> slices of 256 x 256 (us): 882 x 5120 x 13824 183 -> 111 (3 slices), 882 x 5120 x 5120 73 -> 58 (3), 512 x 12288 x
+// 4096 75 -> 58 (2), 203 x 22016 x 4096 71 -> 63 (2); not taken: 203 x 12288 x 4096 37 against 42, 300 x 10240 x 8192 64 against
+// 74, 300 x 4096 x 11008 51 against 52, 512 x 4096 x 11008 63 against 58.
 static bool tailSplitPays(const GemmProblem& p) {
   const int resident = computeUnits() / 8 * 8;
   const int64_t tiles = ceilDiv(p.M, 256) * ceilDiv(p.N, 256), kTiles = p.K / kBK;
@@ -2905,8 +2922,8 @@ static bool tailSplitPays(const GemmProblem& p) {
   const int64_t tiles128 = ceilDiv(p.M, 128) * ceilDiv(p.N, 128);
   const int ways = p.M * p.N * 4 < (int64_t(1) << 31) ? splitKWays(tiles128, kTiles, &per) : 1;
   const float wgs = (float)(tiles128 * ways) / resident;  // workgroups per CU
-  const float us128 = (wgs <= 1.f ? 0.75f : wgs <= 2.f ? 0.75f + 0.44f * (wgs - 1.f) : 0.6f * wgs) * per +
-                      (ways > 1 ? 6.f + (float)(p.M * p.N) * ways * 1.6e-6f : 2.f);
+  const float us128 = (wgs <= 1.f ? 0.42f + 0.13f * wgs : wgs <= 2.f ? std::min(1.17f, 0.9f + 0.55f * (wgs - 1.f)) : 0.6f * wgs) * per +
+                      (ways > 1 ? 8.f + (float)(p.M * p.N) * ways * 1.6e-6f : 3.f);
   return split.us < 0.95f * us128;
 }
 

@@ -331,6 +331,21 @@ def test_four_wave_gemm_last_round_split_along_k_exact(ops, dev, dtype, epilogue
         assert_exact(got, out.reshape(m, n).to(dtype))
 
 
+@pytest.mark.parametrize("m,n,k", [(70, 136, 192), (70, 136, 256), (129, 264, 320), (129, 264, 384), (65, 136, 448), (130, 264, 2752), (100, 4096, 11008)])
+def test_products_with_few_tiles_four_stage_ring_exact(ops, dev, m, n, k):
+    """K shorter than the four-stage ring, as long, and one to three K tiles longer; K slices of unequal length; the [K, N]
+    operand in place and the K-contiguous one. One-hot rows over the whole of K: exact."""
+    g0 = g(79)
+    cols = torch.randint(0, k, (m,), generator=g0)
+    cols[:3] = torch.tensor([0, k - 1, k - 64])
+    x = torch.zeros(m, k, dtype=torch.bfloat16)
+    x[torch.arange(m), cols] = 1
+    w = torch.randn(n, k, generator=g0).to(torch.bfloat16)
+    want = w[:, cols].t().contiguous()
+    assert_exact(ops.linear(x.to(dev), w.to(dev)), want)
+    assert_exact(ops.mm(x.to(dev), w.t().contiguous().to(dev)), want)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("batch,m,n,k", [(3, 777, 128, 777), (2, 129, 131, 65), (1, 1, 1, 1), (5, 128, 127, 7), (1, 300, 500, 4097)])
 def test_products_over_a_k_that_is_no_multiple_of_eight(ops, dev, dtype, batch, m, n, k):
