@@ -347,6 +347,40 @@ def test_products_with_few_tiles_four_stage_ring_exact(ops, dev, m, n, k):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k,bias", [
+    (203, 12288, 256, False),          # 192 tiles of 128: one round of the 128 x 128 kernel
+    (65, 17408 + 64, 192, True),       # K shorter than its ring, a last tile of half the columns, the general rotary form
+    (300, 13312, 320, False),          # 312 tiles: two workgroups per CU
+    (203, 22016, 4096, False),         # 86 tiles of 256 in two K slices each
+    (130, 1024, 1024, False)])         # a product split over K: the separate pass
+def test_gate_and_rotation_in_the_epilogue_at_a_few_hundred_rows(ops, dev, dtype, m, n, k, bias):
+    """One-hot activations: every product is one weight element, so the rotation by powers of two is exact."""
+    g0 = g(81)
+    cols = torch.randint(0, k, (m,), generator=g0)
+    cols[:2] = torch.tensor([0, k - 1])
+    x = torch.zeros(m, k, dtype=dtype)
+    x[torch.arange(m), cols] = 1
+    w = torch.randn(n, k, generator=g0).to(dtype)
+    sel = w[:, cols].float().t()
+    y = sel.reshape(m, n // 64, 2, 32)
+    assert_half(ops.linear_silu_mul(x.to(dev), w.to(dev)), (torch.nn.functional.silu(y[:, :, 0]) * y[:, :, 1]).reshape(m, n // 2))
+    hd = 64
+    rot = n - 256
+    b = torch.zeros(n, dtype=dtype)
+    if bias:
+        b[rot:] = 1
+    e = torch.randint(-3, 1, (m, hd // 2), generator=g0).float()
+    cos, sin = 2.0 ** e, 2.0 ** (e - 1)
+    v = sel.clone().reshape(m, n // hd, hd // 2, 2)
+    out = torch.stack([v[..., 0] * cos[:, None] - v[..., 1] * sin[:, None], v[..., 0] * sin[:, None] + v[..., 1] * cos[:, None]], dim=-1)
+    out[:, rot // hd:] = v[:, rot // hd:]
+    want = out.reshape(m, n) + b.float()
+    got = ops.linear_rotary(x.to(dev), w.to(dev), cos.to(dtype).to(dev), sin.to(dtype).to(dev), rot, hd, b.to(dev) if bias else None,
+                            interleaved=True)
+    assert_exact(got, want.to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("batch,m,n,k", [(3, 777, 128, 777), (2, 129, 131, 65), (1, 1, 1, 1), (5, 128, 127, 7), (1, 300, 500, 4097)])
 def test_products_over_a_k_that_is_no_multiple_of_eight(ops, dev, dtype, batch, m, n, k):
     """Rows that start at any element: K ends inside a 16-byte piece, inside a 64-wide K tile and one element into one;
