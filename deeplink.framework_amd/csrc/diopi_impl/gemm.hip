@@ -801,7 +801,7 @@ __device__ __forceinline__ void vectorEpilogue(const MfmaArgs& g, T* out, const 
 
 
 // TILE is the edge of the square macro tile: 256 (8 waves, 2 x 4, wave tile 128 x 64) or 128 (4 waves, 2 x 2, wave
-// tile 64 x 64, 64 KiB of LDS, two workgroups per CU) for problems with too few 256 x 256 tiles to fill the chip:
+// tile 64 x 64, 32 KiB of LDS per stage, one or two workgroups per CU) for problems with too few 256 x 256 tiles to fill the chip:
 // the same pipeline with half as many A fragments per phase.
 //
 // BT: the second operand lies in memory as [K, N] with N contiguous (the right-hand side of mm / bmm / matmul as the
@@ -3020,11 +3020,9 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
                                              : launchMfmaPipelined<half_t>(ctx, stream, p, nullptr, 1, 0, nullptr, bT);
     }
     AMD_CHECK(!p.colScale, "gemm: a column scale was set on a problem gemmAppliesColumnScale does not accept");
-    // In between (too few 256 x 256 tiles for the chip, too many rows for the weight-streaming kernel): the same
-    // large-tile kernel with K split over grid.y, fp32 partial products in workspace and a reduction pass.
     // In between (too few 256 x 256 tiles for the chip, too many rows for the weight-streaming kernels): the 128 x 128
-    // form of the pipelined kernel, two workgroups per CU, and when even its tiles are fewer than the 2 x CUs the chip
-    // holds, K split over grid.y with fp32 partial products in workspace and a reduction pass. Measured against
+    // form of the pipelined kernel, and when its tiles are at most half the CUs, K split over grid.y with fp32 partial
+    // products in workspace and a reduction pass (see splitKWays). Measured against
     // the 256 x 256 tiles split over K that this replaces (rows x 4096 x 4096, us): 128 rows 23.6 -> 21.5, 256 33.5 -> 22.3,
     // 512 37.4 -> 27.9, 1024 48.0 -> 41.7, 2048 71.3 -> 58.0; x 22016 x 4096: 128 rows 51.0 -> 38.8; K = 11008: 256 rows 45.0 -> 35.9.
     if (!big && p.K % kBK == 0 && p.K >= 2 * kBK && fits2g) {
