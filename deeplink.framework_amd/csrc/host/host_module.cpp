@@ -62,6 +62,17 @@ int dtypeOf(at::ScalarType t) {
   }
 }
 
+// The address in the `ptr` of an object of the ctypes view (a Handle, a Context): a c_void_p, or None for a closed one.
+bool addressOf(PyObject* o, void** p) {
+  PyObject* ptr = PyObject_GetAttrString(o, "ptr");
+  PyObject* value = ptr && ptr != Py_None ? PyObject_GetAttrString(ptr, "value") : ptr;
+  if (value != ptr) Py_XDECREF(ptr);
+  if (!value) return false;
+  *p = value == Py_None ? nullptr : PyLong_AsVoidPtr(value);
+  Py_DECREF(value);
+  return !PyErr_Occurred();
+}
+
 // A tensor's descriptor lives here for the length of the call; None is the null handle, and an object with a `ptr` (a
 // Handle made by the ctypes view) passes that.
 struct TensorArg {
@@ -70,16 +81,9 @@ struct TensorArg {
   bool load(PyObject* o) {
     if (o == Py_None) return true;
     if (!THPVariable_Check(o)) {
-      PyObject* ptr = PyObject_GetAttrString(o, "ptr");
-      PyObject* value = ptr ? PyObject_GetAttrString(ptr, "value") : nullptr;
-      Py_XDECREF(ptr);
-      if (!value) {
-        PyErr_Format(PyExc_TypeError, "expected a tensor, got %s", Py_TYPE(o)->tp_name);
-        return false;
-      }
-      if (value != Py_None) p = PyLong_AsVoidPtr(value);
-      Py_DECREF(value);
-      return !PyErr_Occurred();
+      if (addressOf(o, &p)) return true;
+      PyErr_Format(PyExc_TypeError, "expected a tensor, got %s", Py_TYPE(o)->tp_name);
+      return false;
     }
     const at::Tensor& t = THPVariable_Unpack(o);
     const int64_t nd = t.dim();
@@ -220,17 +224,21 @@ PyObject* translated(F&& f) {
   END_HANDLE_TH_ERRORS
 }
 
-// args[0]: the context's address, or 0 to open one on the current stream for this call.
+// args[0]: 0 to open a context on the current stream for this call, a Context to run in that (its address is read on every
+// call: one that has been closed since is a null context, which the entry point refuses), or an address.
 template <class... A, size_t... I>
 PyObject* invoke(diopiError_t (*fn)(diopiContextHandle_t, A...), const char* name, PyObject* const* args, Py_ssize_t n, std::index_sequence<I...>) {
   if (n != (Py_ssize_t)sizeof...(A) + 1) return PyErr_Format(PyExc_TypeError, "%s takes %d arguments, got %d", name, (int)sizeof...(A) + 1, (int)n);
   return translated([&]() -> PyObject* {
-    void* ctx = PyLong_AsVoidPtr(args[0]);
-    if (!ctx && PyErr_Occurred()) return nullptr;
+    void* ctx = nullptr;
+    const bool number = PyLong_Check(args[0]);
+    if (number) ctx = PyLong_AsVoidPtr(args[0]);
+    else if (!addressOf(args[0], &ctx)) return nullptr;
+    if (number && !ctx && PyErr_Occurred()) return nullptr;
     std::tuple<Arg<A>...> held;
     if (!(std::get<I>(held).load(args[I + 1]) && ...)) return nullptr;
     void* own = nullptr;
-    if (!ctx) {
+    if (number && !ctx) {
       if (g_contextCreate(c10::hip::getCurrentHIPStream().stream(), &own) != 0) return PyObject_CallFunction(g_onFailure, "si", "dipuAmdContextCreate", 1);
       ctx = own;
     }

@@ -45,7 +45,8 @@ class _HostModule:
 
 _host = _HostModule()
 # The context every op runs in: 0 lets the call open one on the current stream and close it when it returns, a scope puts
-# its own here (see WorkspaceScope).
+# its Context here (see WorkspaceScope): the object and not its address, so that it lives while ops run in it and refuses
+# them once it is closed.
 _ctx = 0
 
 
@@ -62,7 +63,7 @@ class WorkspaceScope:
 
     def __enter__(self):
         global _ctx
-        self._outer, _ctx = _ctx, self.ctx.ptr.value
+        self._outer, _ctx = _ctx, self.ctx
         return self
 
     def __exit__(self, *exc):

@@ -211,3 +211,33 @@ def test_host_module_covers_the_signature_table_and_infers_like_torch(pkg):
         h.diopiSilu(1, torch.zeros(1))
     with pytest.raises(RuntimeError, match="must match"):
         h.broadcast_of(torch.zeros(3), torch.zeros(4), False)
+
+
+def test_ops_refuse_a_scope_that_was_closed(pkg):
+    """An op inside `with scope:` after close(), of this scope or of the one around it, is an error and runs in no freed
+    context; a scope nobody else holds lives as long as ops run in it."""
+    import gc
+    import torch
+    ops, x = pkg.ops, torch.zeros(4)
+    refused = lambda: pytest.raises(pkg.diopi.DiopiError, match="null diopiContext")
+    outer, inner = ops.WorkspaceScope(stream=0), ops.WorkspaceScope(stream=0)
+    with outer:
+        with inner:
+            outer.close()
+            with pytest.raises(pkg.diopi.DiopiError, match="lives on the host"):     # the open scope's context got this far
+                ops.silu(x)
+            inner.close()
+            with refused():
+                ops.silu(x)
+        with refused():
+            ops.silu(x)
+        with inner, refused():                                                        # entered after its close()
+            ops.silu(x)
+    ops.WorkspaceScope(stream=0).__enter__()
+    gc.collect()
+    with pytest.raises(pkg.diopi.DiopiError, match="lives on the host"):
+        ops.silu(x)
+    ops._ctx.close()
+    with refused():
+        ops.silu(x)
+    ops._ctx = 0
