@@ -125,20 +125,22 @@ struct Arg<diopiConstTensorHandle_t> : TensorArg {
   diopiConstTensorHandle_t get() { return static_cast<diopiConstTensorHandle_t>(p); }
 };
 struct TensorListArg {
+  PyObject* items = nullptr;  // a tuple of the tensors for the length of the call: a sequence may make them as it is read, a list may change
   std::vector<TensorArg> held;
   std::vector<diopiConstTensorHandle_t> handles;
+  TensorListArg() = default;
+  TensorListArg(const TensorListArg&) = delete;
+  ~TensorListArg() { Py_XDECREF(items); }
   bool load(PyObject* o) {
-    PyObject* seq = PySequence_Fast(o, "expected a list of tensors");
-    if (!seq) return false;
-    const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
+    items = PySequence_Tuple(o);
+    if (!items) return false;
+    const Py_ssize_t n = PyTuple_GET_SIZE(items);
     held.resize(n), handles.resize(n);
-    bool ok = true;
-    for (Py_ssize_t i = 0; i < n && ok; ++i) {
-      ok = held[i].load(PySequence_Fast_GET_ITEM(seq, i));
+    for (Py_ssize_t i = 0; i < n; ++i) {
+      if (!held[i].load(PyTuple_GET_ITEM(items, i))) return false;
       handles[i] = static_cast<diopiConstTensorHandle_t>(held[i].p);
     }
-    Py_DECREF(seq);  // (the caller's list keeps the tensors)
-    return ok;
+    return true;
   }
 };
 template <>
@@ -224,6 +226,12 @@ PyObject* translated(F&& f) {
   END_HANDLE_TH_ERRORS
 }
 
+// The interpreter lock is released for the life of this object, and taken again also where an exception passes.
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
 // args[0]: 0 to open a context on the current stream for this call, a Context to run in that (its address is read on every
 // call: one that has been closed since is a null context, which the entry point refuses), or an address.
 template <class... A, size_t... I>
@@ -243,13 +251,14 @@ PyObject* invoke(diopiError_t (*fn)(diopiContextHandle_t, A...), const char* nam
       ctx = own;
     }
     diopiError_t rc;
-    Py_BEGIN_ALLOW_THREADS
-    void* record = nullptr;
-    g_recordStart(name, &record);
-    rc = fn(static_cast<diopiContextHandle_t>(ctx), std::get<I>(held).get()...);
-    g_recordEnd(&record);
-    if (own && rc == diopiSuccess) g_contextDestroy(own);
-    Py_END_ALLOW_THREADS
+    {
+      Unlocked unlocked;
+      void* record = nullptr;
+      g_recordStart(name, &record);
+      rc = fn(static_cast<diopiContextHandle_t>(ctx), std::get<I>(held).get()...);
+      g_recordEnd(&record);
+      if (own && rc == diopiSuccess) g_contextDestroy(own);
+    }
     if (rc != diopiSuccess) {
       PyObject* r = PyObject_CallFunction(g_onFailure, "si", name, (int)rc);  // (reads the error text before the context goes)
       if (own) g_contextDestroy(own);

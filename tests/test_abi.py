@@ -241,3 +241,36 @@ def test_ops_refuse_a_scope_that_was_closed(pkg):
     with refused():
         ops.silu(x)
     ops._ctx = 0
+
+
+def test_tensors_of_a_list_argument_live_for_the_call(pkg):
+    """A sequence that makes its tensors as it is read: they are alive while the entry point runs (here: while its failure,
+    a closed context, is reported)."""
+    import weakref
+    import torch
+    h, made, alive = pkg._native.host(), [], []
+
+    class Made:
+        def __len__(self):
+            return 2
+
+        def __getitem__(self, i):
+            if i > 1:
+                raise IndexError
+            t = torch.zeros(3)
+            made.append(weakref.ref(t))
+            return t
+
+    def failure(name, ret):
+        alive.extend(r() is not None for r in made)
+        pkg.diopi.raise_failure(name, ret)
+
+    ctx = pkg.diopi.Context(0)
+    ctx.close()
+    h.setup(pkg.diopi.DiopiError, failure)
+    try:
+        with pytest.raises(pkg.diopi.DiopiError, match="null diopiContext"):
+            h.diopiCat(ctx, torch.zeros(6), Made(), 2, 0)
+    finally:
+        h.setup(pkg.diopi.DiopiError, pkg.diopi.raise_failure)
+    assert alive == [True, True]
