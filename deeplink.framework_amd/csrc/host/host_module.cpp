@@ -114,6 +114,9 @@ struct TensorArg {
   }
 };
 
+// Python integers are reduced modulo 2^64, as the fields of the ctypes view reduce them: a mask like 2^64 - 1 is -1.
+int64_t integerOf(PyObject* o) { return static_cast<int64_t>(PyLong_AsUnsignedLongLongMask(o)); }
+
 template <class T>
 struct Arg;
 template <>
@@ -157,7 +160,7 @@ struct Arg<const diopiScalar_t*> {  // dipu/torch_dipu/csrc_dipu/diopirt/diopi_h
   bool load(PyObject* o) {
     if (PyLong_Check(o)) {  // (a bool is one too)
       s.stype = diopi_dtype_int64;
-      s.ival = PyLong_AsLongLong(o);
+      s.ival = integerOf(o);
       return !PyErr_Occurred();
     }
     if (PyFloat_Check(o)) {
@@ -176,7 +179,7 @@ struct Arg<diopiSize_t> {
   bool load(PyObject* o) {
     PyObject* seq = PySequence_Fast(o, "expected a list of integers");
     if (!seq) return false;
-    for (Py_ssize_t i = 0; i < PySequence_Fast_GET_SIZE(seq); ++i) v.push_back(PyLong_AsLongLong(PySequence_Fast_GET_ITEM(seq, i)));
+    for (Py_ssize_t i = 0; i < PySequence_Fast_GET_SIZE(seq); ++i) v.push_back(integerOf(PySequence_Fast_GET_ITEM(seq, i)));
     Py_DECREF(seq);
     return !PyErr_Occurred();
   }
@@ -186,7 +189,7 @@ template <class I>
 struct IntegerArg {
   I v;
   bool load(PyObject* o) {
-    v = static_cast<I>(PyLong_AsLongLong(o));
+    v = static_cast<I>(integerOf(o));
     return !PyErr_Occurred();
   }
   I get() { return v; }
@@ -344,7 +347,13 @@ PyObject* broadcastOf(PyObject*, PyObject* const* args, Py_ssize_t n) {
     at::ScalarType dt = at::kBool;
     if (!toBool) {
       if (PyBool_Check(o)) dt = at::result_type(*a, at::Scalar(o == Py_True));
-      else if (PyLong_Check(o)) dt = at::result_type(*a, at::Scalar((int64_t)0));  // the kind of the number counts, not its value
+      else if (PyLong_Check(o)) {
+        int beyond = 0;
+        (void)PyLong_AsLongLongAndOverflow(o, &beyond);
+        if (beyond) (void)PyLong_AsUnsignedLongLong(o);  // (torch promotes with whatever 64 bits hold, and refuses the rest)
+        if (PyErr_Occurred()) return nullptr;
+        dt = at::result_type(*a, at::Scalar((int64_t)0));  // the kind of the number counts, not its value
+      }
       else if (PyFloat_Check(o)) dt = at::result_type(*a, at::Scalar(0.0));
       else return PyErr_Format(PyExc_TypeError, "invalid scalar type %R", (PyObject*)Py_TYPE(o));
     }

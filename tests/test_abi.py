@@ -274,3 +274,21 @@ def test_tensors_of_a_list_argument_live_for_the_call(pkg):
     finally:
         h.setup(pkg.diopi.DiopiError, pkg.diopi.raise_failure)
     assert alive == [True, True]
+
+
+def test_integers_of_more_than_63_bits_marshal_as_the_ctypes_view_does(pkg):
+    """A number that an int64 field reduces modulo 2^64 is taken (the call gets as far as the host tensor); output
+    inference refuses what torch's promotion does."""
+    import torch
+    ops, d, x = pkg.ops, pkg.diopi, torch.zeros(3, dtype=torch.int64)
+    assert d.scalar(2 ** 64 - 1).ival == -1
+    with ops.WorkspaceScope(stream=0):
+        for call in (lambda: ops.fill_(x, 2 ** 64 - 1), lambda: ops.masked_fill_(x, x == 0, 2 ** 70), lambda: ops.eq(x, 2 ** 64 - 1),
+                     lambda: ops.add(x, 2 ** 63), lambda: ops.tril(x.view(1, 3), 2 ** 63)):
+            with pytest.raises(d.DiopiError, match="lives on the host"):
+                call()
+        for v in (2 ** 64, -2 ** 63 - 1):
+            with pytest.raises(OverflowError):
+                torch.result_type(x, v)
+            with pytest.raises(OverflowError):
+                ops.add(x, v)
