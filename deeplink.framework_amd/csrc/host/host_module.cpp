@@ -108,7 +108,7 @@ struct TensorArg {
     d.reserved = 0;
     d.storage_offset = t.storage_offset();
     d.storage_nbytes = t.storage().nbytes();
-    d.storage_ptr = d.storage_nbytes ? static_cast<char*>(d.data) - d.storage_offset * t.element_size() : nullptr;
+    d.storage_ptr = d.storage_nbytes ? const_cast<void*>(t.storage().data()) : nullptr;
     p = &d;
     return true;
   }

@@ -292,3 +292,36 @@ def test_integers_of_more_than_63_bits_marshal_as_the_ctypes_view_does(pkg):
                 torch.result_type(x, v)
             with pytest.raises(OverflowError):
                 ops.add(x, v)
+
+
+def test_native_descriptors_equal_the_ctypes_view_field_by_field(pkg, tmp_path):
+    """What an entry point receives for a tensor: a stand-in for one, loaded before the library, keeps its descriptor."""
+    import subprocess
+    import sys
+    (tmp_path / "probe.cpp").write_text('''
+#include <dipu_amd/runtime.h>
+extern "C" { dipuAmdTensor kept; int diopiSiluInp(void*, dipuAmdTensor* t) { kept = *t; return 0; } }
+''')
+    subprocess.run(["g++", "-shared", "-fPIC", f"-I{INC}", str(tmp_path / "probe.cpp"), "-o", str(tmp_path / "probe.so")], check=True)
+    code = '''
+import ctypes, sys
+import torch
+sys.path.insert(0, sys.argv[1])
+from __graft_entry__ import load_package
+pkg = load_package()
+probe = ctypes.CDLL(sys.argv[2], mode=ctypes.RTLD_GLOBAL)
+h, d = pkg._native.host(), pkg.diopi
+kept = d.dipuAmdTensor.in_dll(probe, "kept")
+base = torch.arange(48, dtype=torch.float32).view(2, 4, 6)
+for t in [base, base[1:, 2], base[:, :, 3:3], base[2:], base.transpose(0, 2), torch.empty(0), torch.empty(3, 0, 2, dtype=torch.int64),
+          torch.tensor(5, dtype=torch.uint8), base[1, 1, 1], base.to(torch.bfloat16)[1:], base[:, :1].expand(2, 4, 6)]:
+    h.diopiSiluInp(1, t)
+    want = d.Handle(t).desc
+    for name, _ in d.dipuAmdTensor._fields_:
+        a, b = getattr(kept, name), getattr(want, name)
+        if hasattr(a, "__len__"):
+            a, b = list(a)[:t.dim()], list(b)[:t.dim()]
+        assert name == "reserved" or a == b, (tuple(t.shape), name, a, b)
+'''
+    r = subprocess.run([sys.executable, "-c", code, ROOT, str(tmp_path / "probe.so")], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
