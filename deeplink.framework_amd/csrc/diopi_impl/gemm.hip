@@ -2605,7 +2605,7 @@ static diopiError_t launchMfmaPipelined(diopiContextHandle_t ctx, hipStream_t st
       if (p.batch == 1 && resident >= 8) {
         const TailSplit tail = tailSplit((int64_t)g.tilesM * g.tilesN, p.K / (2 * kBK), resident);
         const int64_t slots = ((int64_t)g.tilesM * g.tilesN - tail.whole) * tail.slices;
-        if (void* ws = tail.slices > 1 ? spareWorkspace(ctx, stream, slots * kTailSlotFloats * 4) : nullptr) {
+        if (void* ws = tail.slices <= 1 ? nullptr : p.tailSlots ? p.tailSlots : spareWorkspace(ctx, stream, slots * kTailSlotFloats * 4)) {
           if constexpr (EPI == kEpiLinear) {
             if (p.Cin) return launchTailSplit<T, kEpiAddendLds>(stream, g, tail, resident, ws);
           }
@@ -2942,28 +2942,39 @@ static bool tailSplitPays(const GemmProblem& p) {
   return split.us < 0.95f * us128;
 }
 
+// Settles whether a product with too few 256 x 256 tiles goes to K slices of them, and reserves the workspace without which
+// that form loses: unsplit, 40 tiles (400 x 5120 x 13824) take 257 us on 40 compute units and the 128 x 128 form 146.
+static bool reserveTail(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem* p) {
+  if (!tailSplitPays(*p)) return false;
+  const int64_t tiles = ceilDiv(p->M, 256) * ceilDiv(p->N, 256);
+  p->tailSlots = spareWorkspace(ctx, stream, tiles * tailSplit(tiles, p->K / (2 * kBK), computeUnits() / 8 * 8).slices * kTailSlotFloats * 4);
+  return p->tailSlots != nullptr;
+}
+
 // Which kernel applies the gate or the rotation to its fp32 sums: the 256 x 256 one, or the 128 x 128 one where the plain
 // product would take that without a K split (whose slices meet in the reduction pass of the plain product). The pass over
 // the result that this saves took 4.5 us (rotary) and 6.4 us (gate) at 203 rows.
 enum FusedTile { kFusedNone = 0, kFused256, kFused128 };
-static FusedTile fusedTile(const GemmProblem& p, hipStream_t stream) {
-  if (ceilDiv(p.M, 256) * ceilDiv(p.N, 256) >= 144 || (p.M > kSkinnyMaxM && !recording(stream) && tailSplitPays(p))) return kFused256;
+static FusedTile fusedTile(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem* problem) {
+  if (ceilDiv(problem->M, 256) * ceilDiv(problem->N, 256) >= 144 || (problem->M > kSkinnyMaxM && reserveTail(ctx, stream, problem))) return kFused256;
+  const GemmProblem& p = *problem;
   int per = 0;
   const bool one = p.M > kSkinnyMaxM && splitKWays(ceilDiv(p.M, 128) * ceilDiv(p.N, 128), p.K / kBK, &per) == 1;
   return one && p.N % 8 == 0 && ((p.M - 1) * p.sOm + p.N) * 2 < (int64_t(1) << 31) ? kFused128 : kFusedNone;
 }
 
-bool gemmAppliesColumnScale(const GemmProblem& p) {
+bool gemmAppliesColumnScale(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem* problem) {
+  const GemmProblem& p = *problem;
   // the conditions under which runGemm below reaches the 4-wave kernel without touching the operands
   const bool half = p.dtype == diopi_dtype_bfloat16 || p.dtype == diopi_dtype_float16;
   if (!half || p.batch != 1 || p.Cin || p.bias || p.K <= 0 || p.M >= (int64_t(1) << 31) || p.N >= (int64_t(1) << 31)) return false;
   if (p.sAk != 1 || !mult8(p.sAm) || !ptr16(p.A) || p.sBk != 1 || !mult8(p.sBn) || !ptr16(p.B)) return false;
   if (p.M <= kSkinnyMaxM) return false;
-  const bool big = (ceilDiv(p.M, 256) * ceilDiv(p.N, 256) >= 144 || tailSplitPays(p)) && p.N > 128 && p.K > 2 * kBK;
   const bool fits2g = ((p.M - 1) * p.sAm + p.K) * 2 < (int64_t(1) << 31) && ((p.N - 1) * p.sBn + p.K) * 2 < (int64_t(1) << 31);
-  if (!big || p.K % (2 * kBK) != 0 || !fits2g) return false;
+  if (p.N <= 128 || p.K <= 2 * kBK || p.K % (2 * kBK) != 0 || !fits2g) return false;
   const bool vec = p.N % 8 == 0 && p.sOm % 8 == 0 && ptr16(p.out) && ((p.M - 1) * p.sOm + p.N) * 2 < (int64_t(1) << 31);
-  return vec && p.M * p.sAm * 2 < (int64_t(1) << 31) && p.N * p.sBn * 2 < (int64_t(1) << 31);
+  if (!vec || p.M * p.sAm * 2 >= (int64_t(1) << 31) || p.N * p.sBn * 2 >= (int64_t(1) << 31)) return false;
+  return ceilDiv(p.M, 256) * ceilDiv(p.N, 256) >= 144 || reserveTail(ctx, stream, problem);
 }
 
 diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p) {
@@ -3009,8 +3020,7 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
     // and so does a product of only two K tiles, which is all tile turnover: two workgroups per CU overlap one tile's
     // stores with the other's loads (bmm [128, 2048, 128] x [128, 128, 2048]: 421 -> 368 us)
     // (a column scale: the caller has asked gemmAppliesColumnScale)
-    const bool big = (ceilDiv(p.M, 256) * ceilDiv(p.N, 256) * p.batch >= 144 || p.colScale || (!bT && !recording(stream) && tailSplitPays(p))) &&
-                     p.N > 128 && p.K > 2 * kBK;
+    const bool big = p.N > 128 && p.K > 2 * kBK && (ceilDiv(p.M, 256) * ceilDiv(p.N, 256) * p.batch >= 144 || p.colScale || (!bT && reserveTail(ctx, stream, &p)));
     const bool fits2g = bT || (((p.M - 1) * p.sAm + p.K) * 2 < (int64_t(1) << 31) && ((p.N - 1) * p.sBn + p.K) * 2 < (int64_t(1) << 31));
     if (big && p.K % kBK == 0 && p.K >= 2 * kBK && fits2g) {
       if (p.colScale)
@@ -3163,7 +3173,7 @@ static diopiError_t runGatedSiluGemm(diopiContextHandle_t ctx, hipStream_t strea
                       p.K % kBK == 0 && p.K >= 2 * kBK &&
                       ((p.M - 1) * p.sAm + p.K) * 2 < (int64_t(1) << 31) && ((p.N - 1) * p.sBn + p.K) * 2 < (int64_t(1) << 31) &&
                       mult8(p.sOm) && ptr16(p.out) && p.M < (int64_t(1) << 31) && p.N < (int64_t(1) << 31);
-  const FusedTile fused = direct ? fusedTile(p, stream) : kFusedNone;
+  const FusedTile fused = direct ? fusedTile(ctx, stream, &p) : kFusedNone;
   if (fused == kFused256)
     return p.dtype == diopi_dtype_bfloat16 ? launchMfmaPipelined<bf16_t, kEpiSiluMul>(ctx, stream, p)
                                            : launchMfmaPipelined<half_t, kEpiSiluMul>(ctx, stream, p);
@@ -3582,7 +3592,7 @@ GEMM_EXPORT diopiError_t diopiLinearRotary(diopiContextHandle_t ctx, diopiTensor
                       k % kBK == 0 && k >= 2 * kBK && n % 8 == 0 && ptr16(p.out) &&
                       (!p.bias || ptr16(p.bias)) && p.M * k * 2 < (int64_t(1) << 31) && n * k * 2 < (int64_t(1) << 31) &&
                       p.M * n * 2 < (int64_t(1) << 31);
-  const FusedTile tile = direct ? fusedTile(p, stream) : kFusedNone;
+  const FusedTile tile = direct ? fusedTile(ctx, stream, &p) : kFusedNone;
   if (tile != kFusedNone) {
     RotaryEpilogue r;
     r.cosT = cc.data, r.sinT = cs.data, r.cols = (int)rotaryCols, r.headDim = (int)headDim, r.tableRows = (int)tableRows;

@@ -29,13 +29,17 @@ struct GemmProblem {
   diopiDtype_t colScaleDtype = diopi_dtype_float32;
   const void* colBias = nullptr;
   diopiDtype_t colBiasDtype = diopi_dtype_float32;
+  // Workspace for K slices of 256 x 256 tiles, held once it is settled that the product takes that form (reserveTail in
+  // gemm.hip). Not for callers to set.
+  void* tailSlots = nullptr;
 };
 
 diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p);
 
 // Whether runGemm would send p to the kernel whose epilogue can multiply every column by a scale of its own (the
 // 4-wave large-tile kernel): the caller sets colScale only then, and applies the scale in a pass of its own otherwise.
-bool gemmAppliesColumnScale(const GemmProblem& p);
+// What it settles and reserves for that stays in *p, which then goes to runGemm.
+bool gemmAppliesColumnScale(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem* p);
 
 // diopiRotaryEmbedding on views (rotary_kv.hip): out and x of shape [..., heads, head_dim], strided views allowed.
 diopiError_t runRotary(diopiContextHandle_t ctx, hipStream_t stream, const TensorView& out, const TensorView& x,

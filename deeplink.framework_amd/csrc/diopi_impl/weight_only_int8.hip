@@ -617,7 +617,7 @@ extern "C" __attribute__((visibility("default"))) diopiError_t diopiWeightOnlyIn
   // meet the fp32 sum there: 8192 x 11008 x 4096 594 -> 544 us, 2048 rows 204 -> 183 us (the same products with 16-bit
   // weights: 499 and 151 us; what remains above them is the expansion)
   const bool manyRows = M >= kW8ExpandFromRows && K % 16 == 0 && cw.aligned16() && (N == 1 || cw.stride[0] % 16 == 0);
-  const bool scaleInEpilogue = manyRows && gemmAppliesColumnScale(p);
+  const bool scaleInEpilogue = manyRows && gemmAppliesColumnScale(ctx, stream, &p);
   if (manyRows && (scaleInEpilogue || !bias.defined())) {
     void* expanded = nullptr;
     AMD_TRY(requireWorkspace(ctx, N * K * in.itemsize, &expanded));

@@ -156,3 +156,42 @@ def test_products_that_can_do_without_workspace_record_without_it(pkg, ops, dev)
         torch.cuda.synchronize()
         for t, u, v in zip(got, want, again):
             assert torch.equal(t, u) and torch.equal(u, v)
+
+
+def test_recorded_int8_products_of_a_few_hundred_rows_keep_a_form_that_fills_the_chip(pkg, ops, dev):
+    """An int8 linear whose eager form multiplies K slices of 256 x 256 tiles, with the channel scale on the fp32 sums, has no
+    workspace for them while it is recorded: it runs the 128 x 128 form and the scale in a pass over the 16-bit result, not
+    40 unsplit tiles. Rows of ones at 64 places: sums that 16 bits round, so that the two forms differ."""
+    m, n, k = 400, 5120, 13824
+    gen = torch.Generator().manual_seed(8)
+    x = torch.zeros(m, k, dtype=torch.bfloat16)
+    x.scatter_(1, torch.stack([torch.randperm(k, generator=gen)[:64] for _ in range(m)]), 1)
+    w = torch.randint(-127, 128, (n, k), generator=gen, dtype=torch.int8)
+    scale = (0.001 + 0.019 * torch.rand(n, generator=gen)).to(torch.float16)
+    dx, dw, ds = x.to(dev), w.to(dev), scale.to(dev)
+    sums = (dx.float() @ dw.float().t()).round()                              # (whole numbers: exact)
+    once = (sums * ds.float()).to(torch.bfloat16)
+    twice = (sums.to(torch.bfloat16).float() * ds.float()).to(torch.bfloat16)
+    assert not torch.equal(once, twice)
+    assert torch.equal(ops.weight_only_int8_linear(dx, dw, ds), once)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        warm = ops.WorkspaceScope()
+        with warm:
+            ops.weight_only_int8_linear(dx, dw, ds)
+        side.synchronize()
+        warm.close()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        scope = ops.WorkspaceScope()
+        with scope:
+            out = ops.weight_only_int8_linear(dx, dw, ds)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        assert torch.equal(ops.weight_only_int8_linear(dx, dw, ds), once)
+        torch.cuda.synchronize()
+        assert torch.equal(out, twice)
+    del graph
+    scope.close()
