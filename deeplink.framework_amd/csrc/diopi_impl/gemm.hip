@@ -48,6 +48,10 @@
 
 #include "gemm.hpp"
 
+// Of the runtime library in this repository (include/dipu_amd/runtime.h); absent where DIPU provides the callbacks, whose
+// contexts live for one call.
+extern "C" __attribute__((weak)) int dipuAmdContextIsSparing(void* ctx);
+
 namespace amd {
 
 // ------------------------------------------------------------- MFMA engine ---
@@ -2499,9 +2503,10 @@ static void setRotary(MfmaArgs* g, const RotaryEpilogue& rot) {
   g->rotTableF32 = rot.tableF32, g->rotSinSign = rot.sinSign;
 }
 
-// Workspace for a form that is only faster than one without: null where the runtime has none to give, and null while the
-// stream is recorded into a graph. A recorded buffer has to outlive the recording, which only callers of the functions
-// that cannot do without one see to.
+// Workspace for a form that is only faster than one without: null where the runtime has none to give, null while the
+// stream is recorded into a graph, and null in a context that holds the workspace of many calls. A recorded buffer has to
+// outlive the recording, which only callers of the functions that cannot do without one see to; and the passes before a
+// recording, held in such a context, are to ask for what the recording will, and not for 128 MiB more a product.
 static bool recording(hipStream_t stream) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
@@ -2510,7 +2515,8 @@ static bool recording(hipStream_t stream) {
 }
 static void* spareWorkspace(diopiContextHandle_t ctx, hipStream_t stream, int64_t nbytes) {
   void* ws = nullptr;
-  return !recording(stream) && requireWorkspace(ctx, nbytes, &ws) == diopiSuccess ? ws : nullptr;
+  const bool sparing = dipuAmdContextIsSparing != nullptr && dipuAmdContextIsSparing(ctx) != 0;
+  return !sparing && !recording(stream) && requireWorkspace(ctx, nbytes, &ws) == diopiSuccess ? ws : nullptr;
 }
 
 // How the tiles of a 4-wave launch are worked off: whole tiles first, the rest in K slices (slices == 1: no split), and

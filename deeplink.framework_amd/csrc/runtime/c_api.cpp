@@ -18,6 +18,8 @@ namespace amdrt {
 void* contextCreate(deviceStream_t s);
 void contextDestroy(void* c);
 void contextReset(void* c);
+void contextSetSparing(void* c, bool sparing);
+bool contextIsSparing(void* c);
 void contextWorkspace(void* c, uint64_t* tensors, uint64_t* bytes);
 void noteError(const char* what);
 }  // namespace amdrt
@@ -447,6 +449,8 @@ uint64_t dipuAmdSegmentSize(uint64_t rounded, const char* conf) {
 int dipuAmdContextCreate(void* stream, void** ctx) { return guarded([&] { *ctx = contextCreate(S(stream)); }); }
 int dipuAmdContextDestroy(void* ctx) { return guarded([&] { contextDestroy(ctx); }); }
 int dipuAmdContextReset(void* ctx) { return guarded([&] { contextReset(ctx); }); }
+int dipuAmdContextSetSparing(void* ctx, int sparing) { return guarded([&] { contextSetSparing(ctx, sparing != 0); }); }
+int dipuAmdContextIsSparing(void* ctx) { return contextIsSparing(ctx) ? 1 : 0; }
 int dipuAmdContextWorkspace(void* ctx, uint64_t* tensors, uint64_t* bytes) {
   return guarded([&] { contextWorkspace(ctx, tensors, bytes); });
 }

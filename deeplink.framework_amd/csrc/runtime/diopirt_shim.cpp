@@ -41,6 +41,7 @@ struct WorkspaceTensor {
 struct diopiContext {
   dipu::deviceStream_t stream;
   std::list<WorkspaceTensor> arrays;
+  bool sparing = false;  // operators are to take no workspace that they can do without
   explicit diopiContext(dipu::deviceStream_t s) : stream(s) {}
   void release() {
     for (auto& w : arrays) {
@@ -280,6 +281,8 @@ namespace dipu {
 namespace amdrt {
 void* contextCreate(deviceStream_t s) { return new diopiContext(s); }
 void contextDestroy(void* c) { delete static_cast<diopiContext*>(c); }
+void contextSetSparing(void* c, bool sparing) { static_cast<diopiContext*>(c)->sparing = sparing; }
+bool contextIsSparing(void* c) { return static_cast<diopiContext*>(c)->sparing; }
 void contextReset(void* c) { static_cast<diopiContext*>(c)->release(); }
 void contextWorkspace(void* c, uint64_t* tensors, uint64_t* bytes) {
   auto* ctx = static_cast<diopiContext*>(c);

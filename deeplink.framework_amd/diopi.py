@@ -165,9 +165,10 @@ class Generator:
 
 class Context:
     """diopiContext bound to a stream (diopirt_impl.h:19-26). Workspace the impl library
-    requests lives until the context is closed; DIPU closes it when the wrapper returns."""
+    requests lives until the context is closed; DIPU closes it when the wrapper returns. In a sparing one operators
+    take no workspace that they can do without."""
 
-    def __init__(self, stream=None):
+    def __init__(self, stream=None, sparing=False):
         rt = _native.runtime()
         if stream is None:
             stream = torch.cuda.current_stream().cuda_stream
@@ -176,6 +177,8 @@ class Context:
         if rt.dipuAmdContextCreate(c_void_p(stream), byref(p)) != 0:
             raise DiopiError(rt_error())
         self.ptr = p
+        if sparing:
+            rt.dipuAmdContextSetSparing(p, c_int(1))
 
     def workspace(self):
         n, b = c_uint64(), c_uint64()

@@ -56,10 +56,12 @@ class WorkspaceScope:
     recorded into a HIP graph: the graph's kernels keep the workspace addresses they were recorded with, so the scope
     is created on the capturing stream and closed only after the last replay. Recording may not allocate device
     memory: run the same calls under a scope on that stream beforehand, and again until a pass leaves the
-    allocator's num_device_malloc unchanged; the recording then finds every block in the cache."""
+    allocator's num_device_malloc unchanged; the recording then finds every block in the cache. For that, ops in a
+    scope run the forms that a recording runs: those that take no workspace where there is a choice (outside a scope
+    a product may be faster, with its sums in another order)."""
 
     def __init__(self, stream=None):
-        self.ctx = Context(stream)
+        self.ctx = Context(stream, sparing=True)
 
     def __enter__(self):
         global _ctx

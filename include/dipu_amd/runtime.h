@@ -187,6 +187,11 @@ DIPU_AMD_API int dipuAmdContextCreate(void* stream, void** ctx);
 DIPU_AMD_API int dipuAmdContextDestroy(void* ctx);
 DIPU_AMD_API int dipuAmdContextReset(void* ctx);  /* release workspace, keep the context */
 DIPU_AMD_API int dipuAmdContextWorkspace(void* ctx, uint64_t* tensors, uint64_t* bytes);
+/* In a sparing context operators take no workspace that they can do without: they run the form that needs none, as they do
+ * while a stream is recorded into a graph. For contexts that hold the workspace of many calls, such as the passes before
+ * a recording. Off when a context is created; dipuAmdContextIsSparing returns 0 or 1. */
+DIPU_AMD_API int dipuAmdContextSetSparing(void* ctx, int sparing);
+DIPU_AMD_API int dipuAmdContextIsSparing(void* ctx);
 
 /* ---- profiler hooks: dipu/torch_dipu/csrc_dipu/runtime/device/profilerapis.h:12-14 (enableProfiler /
  * disableProfiler) and the diopiRecordStart / diopiRecordEnd pair, diopirt/diopirt_impl.cpp:224-237.

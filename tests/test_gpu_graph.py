@@ -195,3 +195,45 @@ def test_recorded_int8_products_of_a_few_hundred_rows_keep_a_form_that_fills_the
         assert torch.equal(out, twice)
     del graph
     scope.close()
+
+
+def test_a_scope_takes_no_workspace_that_its_recording_does_not(pkg, ops, dev):
+    """Products whose fast form takes workspace (K slices, a ragged K with a strided operand, a column scale) run the plain form
+    in a scope, as they do while recorded: the passes before a recording hold nothing for them, and their results are the
+    recording's bit for bit."""
+    gen = torch.Generator().manual_seed(9)
+    rnd = lambda *shape: torch.randn(*shape, generator=gen).to(torch.bfloat16).to(dev)
+    x, w, a, b = rnd(1554, 4096), rnd(11008, 4096), rnd(2, 77, 65), rnd(2, 65, 40)
+    y, w8 = rnd(400, 5120), torch.randint(-127, 128, (5120, 5120), generator=gen, dtype=torch.int8).to(dev)
+    scale = (0.001 + 0.019 * torch.rand(5120, generator=gen)).to(torch.float16).to(dev)
+    expanded = w8.numel() * 2                                       # the int8 weight in 16 bits, which no form goes without
+    step = lambda: [ops.linear(x, w), ops.linear(x, w), ops.bmm(a, b), ops.weight_only_int8_linear(y, w8, scale)]
+    with pkg.diopi.Context() as ctx:                                # outside a scope the K slices of 45 tiles take theirs
+        handles = [pkg.diopi.handle(t) for t in (torch.empty(1554, 11008, dtype=x.dtype, device=dev), x, w, None)]
+        pkg.diopi.call("diopiLinear", ctx, *[p for _, p in handles])
+        assert ctx.workspace() == (1, 45 * 4 * 256 * 1024)
+        torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        warm = ops.WorkspaceScope()
+        with warm:
+            want = step()
+        side.synchronize()
+        assert warm.ctx.workspace() == (1, expanded)
+        warm.close()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        scope = ops.WorkspaceScope()
+        with scope:
+            got = step()
+    assert scope.ctx.workspace() == (1, expanded)
+    for _ in range(3):
+        for t in got:
+            t.zero_()
+        graph.replay()
+        step()
+        torch.cuda.synchronize()
+        assert all(torch.equal(t, u) for t, u in zip(got, want))
+    del graph
+    scope.close()
