@@ -304,6 +304,27 @@ def test_softmax_unaligned_rows(ops, dev, dtype, rows, cols):
     assert_close(got.nan_to_num(7.0), want.nan_to_num(7.0) if dtype == torch.float32 else want.nan_to_num(7.0).to(dtype))
 
 
+def test_softmax_unaligned_rows_in_32_bits(ops, dev):
+    """Against 64 bits. A row of 33 is added in 6 + 2 steps, so its error is that of the exponential and of the rounded
+    result; a row of 2047 is added in pairs, 3 steps more per lane, which measured 1.07 times as much (entry by entry, 32
+    steps down a lane: 1.30). No result below 2^-126 is flushed."""
+    err = {}
+    for cols in (33, 777, 2047):
+        x = torch.randn(8192, cols, generator=g(33)) * 3
+        got, want = ops.softmax(x.to(dev), -1).cpu().double(), torch.softmax(x.double(), -1)
+        err[cols] = float((got - want).norm() / want.norm())
+    assert err[777] < 1.18 * err[33] and err[2047] < 1.18 * err[33], err
+    for dtype in (torch.float32, torch.bfloat16):
+        step = 2.0 ** (-149 if dtype == torch.float32 else -133)             # denormal numbers are this far apart
+        for cols in (33, 777, 2047):
+            x = torch.full((7, cols), -200.0)
+            x[:, 0], x[:, cols // 2], x[:, cols - 1] = 0.0, -88.0, -90.0
+            got, want = ops.softmax(x.to(dtype).to(dev), -1).cpu().double(), torch.softmax(x.double(), -1)
+            # (the exponential's argument, here down to -130, is rounded to 2^-17 at worst: 5.3e-6 of the result)
+            assert bool(((got - want)[:, 1:].abs() <= step + 6e-6 * want[:, 1:]).all()), (dtype, cols)
+            assert float(got[:, cols - 1].min()) > 0, (dtype, cols)
+
+
 def test_softmax_rows_sum_to_one_at_full_size(ops, dev):
     x = torch.randn(8192, 4096, generator=g(20)).bfloat16().to(dev)
     y = ops.softmax(x, -1)
