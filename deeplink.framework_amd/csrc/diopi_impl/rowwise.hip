@@ -27,6 +27,15 @@ namespace amd {
 
 constexpr float kLog2e = 1.4426950408889634f;
 
+// The exponentials of a row with the maximum m are exp2(x * scale - mScaled). For |m| from 2.3e38 on, where m * log2 e leaves
+// the fp32 range (rows of nothing but the lowest number, which fully masked rows hold), a scale of 1 / 4 gives the same
+// numbers: entries then equal m or lie 2^104 and more below it. A row of nothing but -inf gives NaN like the CPU kernel.
+__device__ __forceinline__ float softmaxScale(float m, float* mScaled) {
+  const float scale = fabsf(m) < 2.3e38f ? kLog2e : 0.25f;
+  *mScaled = m == -INFINITY ? 0.f : m * scale;
+  return scale;
+}
+
 // ------------------------------------------------------------ wave-per-row ---
 enum RowOp { kRowSoftmax = 0, kRowRmsNorm = 1 };
 
@@ -98,14 +107,15 @@ __global__ __launch_bounds__(256) void rowWaveKernel(T* __restrict__ out, const 
         if (lane + 64 * i < nvec) pre[i] = src[lane + 64 * i];
     }
     m = waveMax(m);
-    const float mScaled = (m == -INFINITY) ? 0.f : m * kLog2e;  // all -inf row -> nan like the CPU kernel
+    float mScaled;
+    const float scale = softmaxScale(m, &mScaled);
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i)
       if (lane + 64 * i < nvec) {
 #pragma unroll
         for (int j = 0; j < N; ++j) {
-          f[i][j] = __builtin_amdgcn_exp2f(fmaf(f[i][j], kLog2e, -mScaled));
+          f[i][j] = __builtin_amdgcn_exp2f(fmaf(f[i][j], scale, -mScaled));
           s += f[i][j];
         }
       }
@@ -237,14 +247,15 @@ __global__ __launch_bounds__(256) void softmaxRaggedKernel(T* __restrict__ out, 
     }
     if (row + nWaves < rows) fetch(row + nWaves);
     m = waveMax(m);
-    const float mScaled = (m == -INFINITY) ? 0.f : m * kLog2e;  // all -inf row -> nan like the CPU kernel
+    float mScaled;
+    const float scale = softmaxScale(m, &mScaled);
     float part[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       part[i] = 0.f;
       if ((lane + 64 * i) * N >= cols) continue;
 #pragma unroll
-      for (int j = 0; j < N; ++j) f[i][j] = expOf(fmaf(f[i][j], kLog2e, -mScaled));
+      for (int j = 0; j < N; ++j) f[i][j] = expOf(fmaf(f[i][j], scale, -mScaled));
       part[i] = pairSum(f[i]);
     }
     float s = pairSum(part);
@@ -336,11 +347,12 @@ __global__ __launch_bounds__(256) void rowSubWaveKernel(T* __restrict__ out, con
           m = fmaxf(m, f[j]);
         }
         m = groupReduce<LPR>(m, true);
-        const float mScaled = (m == -INFINITY) ? 0.f : m * kLog2e;  // all -inf row -> nan like the CPU kernel
+        float mScaled;
+        const float scale = softmaxScale(m, &mScaled);
         float sum = 0.f;
 #pragma unroll
         for (int j = 0; j < N; ++j) {
-          f[j] = ok[u] ? __builtin_amdgcn_exp2f(fmaf(f[j], kLog2e, -mScaled)) : 0.f;
+          f[j] = ok[u] ? __builtin_amdgcn_exp2f(fmaf(f[j], scale, -mScaled)) : 0.f;
           sum += f[j];
         }
         sum = groupReduce<LPR>(sum, false);
@@ -404,18 +416,19 @@ __global__ __launch_bounds__(256) void rowBlockKernel(T* out, const T* in, const
       m = fmaxf(m, v);
     }
     m = blockReduce(m, true, red);
-    const float mScaled = (m == -INFINITY) ? 0.f : m * kLog2e;
+    float mScaled;
+    const float scale = softmaxScale(m, &mScaled);
     float s = 0.f;
     for (int64_t c = threadIdx.x; c < cols; c += blockDim.x) {
       float v = staged ? rowBuf[c] : static_cast<float>(src[c]);
-      v = exp2f(v * kLog2e - mScaled);
+      v = exp2f(v * scale - mScaled);
       if (staged) rowBuf[c] = v;
       s += v;
     }
     s = blockReduce(s, false, red);
     const float inv = 1.f / s;
     for (int64_t c = threadIdx.x; c < cols; c += blockDim.x) {
-      float v = staged ? rowBuf[c] : exp2f(static_cast<float>(src[c]) * kLog2e - mScaled);
+      float v = staged ? rowBuf[c] : exp2f(static_cast<float>(src[c]) * scale - mScaled);
       dst[c] = static_cast<T>(v * inv);
     }
   } else {
@@ -480,13 +493,14 @@ __global__ __launch_bounds__(256) void rowBlockVecKernel(T* __restrict__ out, co
           for (int j = 0; j < N; ++j) m = fmaxf(m, static_cast<float>(x[i][j]));
         }
       m = blockReduce(m, true, red);
-      const float mScaled = (m == -INFINITY) ? 0.f : m * kLog2e;
+      float mScaled;
+      const float scale = softmaxScale(m, &mScaled);
       float sum = 0.f;
 #pragma unroll
       for (int i = 0; i < NVT; ++i)
         if (tid + 256 * i < nvec) {
 #pragma unroll
-          for (int j = 0; j < N; ++j) sum += __builtin_amdgcn_exp2f(fmaf(static_cast<float>(x[i][j]), kLog2e, -mScaled));
+          for (int j = 0; j < N; ++j) sum += __builtin_amdgcn_exp2f(fmaf(static_cast<float>(x[i][j]), scale, -mScaled));
         }
       sum = blockReduce(sum, false, red);
       const float inv = 1.f / sum;
@@ -496,7 +510,7 @@ __global__ __launch_bounds__(256) void rowBlockVecKernel(T* __restrict__ out, co
           V v;
 #pragma unroll
           for (int j = 0; j < N; ++j)
-            v[j] = static_cast<T>(__builtin_amdgcn_exp2f(fmaf(static_cast<float>(x[i][j]), kLog2e, -mScaled)) * inv);
+            v[j] = static_cast<T>(__builtin_amdgcn_exp2f(fmaf(static_cast<float>(x[i][j]), scale, -mScaled)) * inv);
           __builtin_nontemporal_store(v, dst + tid + 256 * i);
         }
     } else {
@@ -585,33 +599,33 @@ __global__ __launch_bounds__(1024) void rowStreamKernel(T* __restrict__ out, con
     const T* src = in + row * inRowStride;
     T* dst = out + row * outRowStride;
     if constexpr (OP == kRowSoftmax) {
-      float m = -INFINITY, sum = 0.f;  // in units of log2
+      // (differences are taken before the scaling by log2 e, whose product with the lowest number is out of range)
+      float m = -INFINITY, sum = 0.f;
       for (int64_t i = threadIdx.x; i < pieces; i += 1024) {
         float f[N];
         load(src, i, f);
         float pm = f[0];
 #pragma unroll
         for (int j = 1; j < N; ++j) pm = fmaxf(pm, f[j]);
-        pm *= kLog2e;
         if (pm > m) {
-          sum *= __builtin_amdgcn_exp2f(m - pm);  // (m = -inf: sum is still 0, and exp2(-inf) = 0)
+          sum *= __builtin_amdgcn_exp2f((m - pm) * kLog2e);  // (m = -inf: sum is still 0, and exp2(-inf) = 0)
           m = pm;
         }
         if (m != -INFINITY) {
 #pragma unroll
-          for (int j = 0; j < N; ++j) sum += __builtin_amdgcn_exp2f(fmaf(f[j], kLog2e, -m));
+          for (int j = 0; j < N; ++j) sum += __builtin_amdgcn_exp2f((f[j] - m) * kLog2e);
         }
       }
       const float rowMax = blockReduce(m, true, red);
-      const float mScaled = (rowMax == -INFINITY) ? 0.f : rowMax;  // all -inf row: the sum is 0 and every output 0 * inf = nan, like the CPU kernel
-      sum = (m == -INFINITY) ? 0.f : sum * __builtin_amdgcn_exp2f(m - mScaled);
+      const float from = (rowMax == -INFINITY) ? 0.f : rowMax;  // all -inf row: the sum is 0 and every output 0 * inf = nan, like the CPU kernel
+      sum = (m == -INFINITY) ? 0.f : sum * __builtin_amdgcn_exp2f((m - from) * kLog2e);
       const float total = blockReduce(sum, false, red);
       const float inv = 1.f / total;
       for (int64_t i = threadIdx.x; i < pieces; i += 1024) {
         float f[N];
         load(src, i, f);
 #pragma unroll
-        for (int j = 0; j < N; ++j) f[j] = __builtin_amdgcn_exp2f(fmaf(f[j], kLog2e, -mScaled)) * inv;
+        for (int j = 0; j < N; ++j) f[j] = __builtin_amdgcn_exp2f((f[j] - from) * kLog2e) * inv;
         store(dst, i, f);
       }
     } else {
@@ -653,12 +667,13 @@ __global__ __launch_bounds__(256) void softmaxStridedKernel(T* out, const T* in,
   T* dst = out + o * dim * inner + i;
   float m = -INFINITY;
   for (int64_t d = 0; d < dim; ++d) m = fmaxf(m, static_cast<float>(src[d * inner]));
-  const float mScaled = (m == -INFINITY) ? 0.f : m * kLog2e;
+  float mScaled;
+  const float scale = softmaxScale(m, &mScaled);
   float s = 0.f;
-  for (int64_t d = 0; d < dim; ++d) s += exp2f(static_cast<float>(src[d * inner]) * kLog2e - mScaled);
+  for (int64_t d = 0; d < dim; ++d) s += exp2f(static_cast<float>(src[d * inner]) * scale - mScaled);
   const float inv = 1.f / s;
   for (int64_t d = 0; d < dim; ++d)
-    dst[d * inner] = static_cast<T>(exp2f(static_cast<float>(src[d * inner]) * kLog2e - mScaled) * inv);
+    dst[d * inner] = static_cast<T>(exp2f(static_cast<float>(src[d * inner]) * scale - mScaled) * inv);
 }
 
 // The same softmax for long columns: a workgroup of 1024 takes 32 adjacent `inner` positions of one outer index, its 32

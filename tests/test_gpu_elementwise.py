@@ -325,6 +325,23 @@ def test_softmax_unaligned_rows_in_32_bits(ops, dev):
             assert float(got[:, cols - 1].min()) > 0, (dtype, cols)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_softmax_of_masks_at_the_lowest_number(ops, dev, dtype):
+    """Masks of the type's lowest value, as model code writes them: a fully masked row is uniform, not NaN, in every form
+    (rows sharing a wave, a wave or a workgroup per row, unaligned, streamed, along another dim); so is a row of the largest
+    value, and an infinity among finite entries or nothing else still gives NaN."""
+    low, high = torch.finfo(dtype).min, torch.finfo(dtype).max
+    for shape, dim in [((33, 64), 1), ((9, 4096), 1), ((500, 4096), 1), ((9, 777), 1), ((9, 31), 1), ((9, 5001), 1), ((9, 12000), 1),
+                       ((9, 70000), 1), ((9, 70001), 1), ((64, 9), 0), ((300, 40), 0)]:
+        x = torch.randn(shape, generator=g(34)).to(dtype)
+        rows = x.movedim(dim, -1)
+        rows[0], rows[1], rows[2], rows[3], rows[4] = low, high, low, float("-inf"), 1.0
+        rows[2, 3:5], rows[4, 1], rows[5, ::2], rows[6, 1] = 0.25, float("inf"), low, high
+        got, want = ops.softmax(x.to(dev), dim).cpu(), torch.softmax(x.double(), dim).to(dtype)
+        assert torch.equal(got.isnan(), want.isnan()), (shape, dim)
+        assert_close(got.nan_to_num(7.0), want.nan_to_num(7.0))
+
+
 def test_softmax_rows_sum_to_one_at_full_size(ops, dev):
     x = torch.randn(8192, 4096, generator=g(20)).bfloat16().to(dev)
     y = ops.softmax(x, -1)
