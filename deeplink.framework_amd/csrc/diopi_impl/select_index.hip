@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kSelThreads) void selectVecRaggedKernel(E* __restri
   typedef uint8_t C8 __attribute__((ext_vector_type(8), aligned(1)));
   const unsigned i = (blockIdx.x * kSelThreads + threadIdx.x) * 8u;
   if (i >= n) return;
-  const unsigned at = i % period;
+  unsigned at = i % period;
   if (i + 8 <= n) {
     C8 c;
     if (at + 8 <= period) {
@@ -125,7 +125,21 @@ __global__ __launch_bounds__(kSelThreads) void selectVecRaggedKernel(E* __restri
     for (int j = 0; j < 8; ++j) r[j] = c[j] != 0 ? va[j] : vb[j];
     *reinterpret_cast<E8*>(out + i) = r;
   } else {
-    for (unsigned j = 0; i + j < n; ++j) out[i + j] = cond[(at + j) % period] != 0 ? (a != nullptr ? a[i + j] : aBits) : b[i + j];
+    // all loads first, the surplus ones at the last element: one after the other they are as many latencies, which is what
+    // a tensor of a few elements consists of
+    uint8_t c[8];
+    E va[8], vb[8];
+#pragma unroll
+    for (unsigned j = 0; j < 8; ++j) {
+      const unsigned k = min(i + j, n - 1);
+      c[j] = cond[at];
+      va[j] = a != nullptr ? a[k] : aBits;
+      vb[j] = b[k];
+      at = at + 1 == period ? 0 : at + 1;
+    }
+#pragma unroll
+    for (unsigned j = 0; j < 8; ++j)
+      if (i + j < n) out[i + j] = c[j] != 0 ? va[j] : vb[j];
   }
 }
 

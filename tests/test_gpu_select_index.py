@@ -233,3 +233,13 @@ def test_masked_fill_and_where_with_masks_of_any_period(ops, dev, dtype, shape, 
     held = torch.zeros(m.numel() + 1, dtype=torch.bool, device=dev)
     held[1:] = m.to(dev).reshape(-1)
     assert_exact(ops.masked_fill(x.to(dev), held[1:].view(mask_shape), 2.5), x.masked_fill(m, 2.5))
+
+
+@pytest.mark.parametrize("n,period", [(7, 7), (13, 13), (15, 5), (6, 2), (333, 333)])
+def test_masked_fill_in_place_over_a_last_piece(ops, dev, n, period):
+    """The surplus loads of a last piece read the last element again, which the same lane overwrites in place."""
+    x = torch.randn(n // period, period, generator=g(24))
+    m = torch.rand(period, generator=g(25)) > 0.4
+    got = x.to(dev)
+    ops.masked_fill_(got, m.to(dev), 3.5)
+    assert_exact(got, x.masked_fill(m, 3.5))
