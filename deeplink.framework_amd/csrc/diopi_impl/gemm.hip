@@ -2983,6 +2983,26 @@ bool gemmAppliesColumnScale(diopiContextHandle_t ctx, hipStream_t stream, GemmPr
   return ceilDiv(p.M, 256) * ceilDiv(p.N, 256) >= 144 || reserveTail(ctx, stream, problem);
 }
 
+// Whether a product over a K that is no multiple of 8 runs faster on the matrix cores, its operands transposed where their K
+// is not contiguous, than on the FMA engine, in us fitted to 890 products of K = 1 ... 11007 in all four layouts. The FMA
+// engine takes 0.077 us per K while its 64 x 64 tiles are few and 0.04 per K and tile on a CU from two on (a batch of tiny
+// matrices less: most of a tile is empty); the matrix kernel 3.4 us a round of 128 x 128 tiles, two on a CU, 0.8 to 1.8 per 64
+// of K and 0.5 per element that K ends in; a transposing copy 4 us and 3.6 ns per 64 x 64 piece. FMA -> matrix cores (us):
+//   B contiguous along K: 2048 x 2048 x 33 12.3 -> 9.0, x 7 8.0 -> 11.2; 1000 of 1 x 64 x 129 19.4 -> 18.8, x 65 12.4 -> 15.2
+//   B as [K, N]: 64 of 64 x 64 x 129 16.7 -> 15.2, x 65 10.4 -> 13.9; 500 of 100 x 100 x 65 33.9 -> 24.3; 2000 of 30 x 30 x 33 17 -> 30
+static bool raggedPays(const GemmProblem& p) {
+  const float cus = (float)computeUnits();
+  auto tiles = [&](int64_t edge) { return (float)(p.batch * ceilDiv(p.M, edge) * ceilDiv(p.N, edge)); };
+  const float perTile = p.M <= 32 && p.N <= 32 ? 0.03f : 0.04f;
+  const float fma = 3.2f + (float)p.K * std::max(0.077f, perTile * tiles(64) / cus);
+  const float onCu = tiles(128) / cus, kTiles = (float)ceilDiv(p.K, (int64_t)kBK);
+  const float perK = 0.8f + std::min(1.f, std::max(0.f, onCu - 1.f));
+  float us = 0.9f + std::max(1.f, onCu / 2) * (3.4f + perK * kTiles + 0.5f * (float)(p.K % 8));
+  if (p.sAk != 1) us += 3.9f + 0.0036f * (float)(p.batch * ceilDiv(p.M, (int64_t)64)) * kTiles;
+  if (p.sBk != 1) us += 3.9f + 0.0036f * (float)((p.sBb == 0 ? 1 : p.batch) * ceilDiv(p.N, (int64_t)64)) * kTiles;
+  return us < 0.93f * fma;
+}
+
 diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p) {
   if (p.batch == 0 || p.M == 0 || p.N == 0) return diopiSuccess;
   AMD_CHECK(p.batch <= 65535, "gemm: batch %ld exceeds the grid limit", (long)p.batch);
@@ -3064,7 +3084,8 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
   }
   // K is no multiple of 8: the 128 x 128 kernel that reads rows at element alignment; an operand whose K is not contiguous
   // is transposed into workspace first, and where there is none to spare the FMA engine below takes the product
-  bool ragged = half && p.K > 0 && p.M < (int64_t(1) << 31) && p.N < (int64_t(1) << 31) && p.K <= 65535 * 64;  // (the transposing copies' grid limit)
+  bool ragged = half && p.K > 0 && p.M < (int64_t(1) << 31) && p.N < (int64_t(1) << 31) && p.K <= 65535 * 64 &&  // (the transposing copies' grid limit)
+                raggedPays(p);
   if (ragged) {
     const int64_t nb = p.sBb == 0 ? 1 : p.batch;  // a shared (broadcast) weight is transposed once
     const int64_t aBytes = p.sAk != 1 ? p.batch * p.M * p.K * 2 : 0, bBytes = p.sBk != 1 ? nb * p.N * p.K * 2 : 0;
@@ -3145,7 +3166,8 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
   dim3 grid((unsigned)ceilDiv(p.N, 64), (unsigned)ceilDiv(p.M, 64), (unsigned)p.batch);
   switch (p.dtype) {
     case diopi_dtype_float32: hipLaunchKernelGGL(gemmFmaKernel<float>, grid, dim3(256), 0, stream, p); break;
-    // (16-bit types: only K = 0 and extents beyond the grids of the kernels above arrive here)
+    // (16-bit types: K that is no multiple of 8 where that is small (raggedPays) or an operand wants a transposed copy and no
+    // workspace is to be spared, as for every recorded one; K = 0; and extents beyond the grids of the kernels above)
     case diopi_dtype_bfloat16: hipLaunchKernelGGL(gemmFmaKernel<bf16_t>, grid, dim3(256), 0, stream, p); break;
     case diopi_dtype_float16: hipLaunchKernelGGL(gemmFmaKernel<half_t>, grid, dim3(256), 0, stream, p); break;
     default: setLastError("gemm: unsupported dtype %s", dtypeName(p.dtype)); return diopiErrorOccurred;

@@ -381,9 +381,11 @@ def test_gate_and_rotation_in_the_epilogue_at_a_few_hundred_rows(ops, dev, dtype
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("batch,m,n,k", [(3, 777, 128, 777), (2, 129, 131, 65), (1, 1, 1, 1), (5, 128, 127, 7), (1, 300, 500, 4097)])
+@pytest.mark.parametrize("batch,m,n,k", [(3, 777, 128, 777), (2, 129, 131, 65), (1, 1, 1, 1), (5, 128, 127, 7), (1, 300, 500, 4097),
+                                           (1, 130, 257, 1031), (2, 127, 129, 390), (1, 2048, 2048, 33)])
 def test_products_over_a_k_that_is_no_multiple_of_eight(ops, dev, dtype, batch, m, n, k):
-    """Rows that start at any element: K ends inside a 16-byte piece, inside a 64-wide K tile and one element into one;
+    """Rows that start at any element: K ends inside a 16-byte piece, inside a 64-wide K tile and one element into one, and
+    lies inside the first; a K of which the matrix kernel has too little (65 and below) on the FMA engine;
     the [K, N] and the transposed second operand, a K-strided first one, and a linear with a bias. The fp32 product, and
     exactly on one-hot rows. The operands end where their allocations do: nothing may be read past them."""
     a, b = torch.randn(batch, m, k, generator=g(91)).to(dtype), torch.randn(batch, k, n, generator=g(92)).to(dtype)

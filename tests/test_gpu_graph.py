@@ -141,7 +141,7 @@ def test_products_that_can_do_without_workspace_record_without_it(pkg, ops, dev)
     rnd = lambda *shape: torch.randint(-2, 3, shape, generator=gen).to(torch.bfloat16).to(dev)     # (exact sums)
     gen = torch.Generator().manual_seed(7)
     x, w = rnd(1554, 4096), rnd(11008, 4096)
-    a, b = rnd(2, 77, 65), rnd(2, 65, 40)
+    a, b = rnd(2, 77, 385), rnd(2, 385, 40)
     calls = [lambda: ops.linear(x, w), lambda: ops.bmm(a, b)]
     want = [f() for f in calls]
     torch.cuda.synchronize()
@@ -203,7 +203,7 @@ def test_a_scope_takes_no_workspace_that_its_recording_does_not(pkg, ops, dev):
     recording's bit for bit."""
     gen = torch.Generator().manual_seed(9)
     rnd = lambda *shape: torch.randn(*shape, generator=gen).to(torch.bfloat16).to(dev)
-    x, w, a, b = rnd(1554, 4096), rnd(11008, 4096), rnd(2, 77, 65), rnd(2, 65, 40)
+    x, w, a, b = rnd(1554, 4096), rnd(11008, 4096), rnd(2, 77, 385), rnd(2, 385, 40)
     y, w8 = rnd(400, 5120), torch.randint(-127, 128, (5120, 5120), generator=gen, dtype=torch.int8).to(dev)
     scale = (0.001 + 0.019 * torch.rand(5120, generator=gen)).to(torch.float16).to(dev)
     expanded = w8.numel() * 2                                       # the int8 weight in 16 bits, which no form goes without
