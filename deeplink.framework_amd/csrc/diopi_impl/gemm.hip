@@ -3113,12 +3113,17 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
     AMD_LAUNCH_CHECK();
     return diopiSuccess;
   }
+  const bool f32Rounds = ceilDiv(p.M, 32) * ceilDiv(p.N, 32) * p.batch > (int64_t)computeUnits() * 2;  // of 32 x 32 tiles, two on a unit
   if (p.dtype == diopi_dtype_float32 && p.sAk == 1 && p.sBk == 1 && f32MfmaEligible(p) &&
-      ceilDiv(p.M, 64) * ceilDiv(p.N, 64) * p.batch * 4 < (int64_t)computeUnits() * 3) {
+      ceilDiv(p.M, 64) * ceilDiv(p.N, 64) * p.batch * 4 < (int64_t)computeUnits() * 3 &&
+      !(f32Rounds && p.M >= 32 && p.N >= 32 && (p.K <= 64 || (p.K < 256 && p.K % 32 == 0)))) {
     // Tiles of 64 x 64 for less than three quarters of the compute units (any number of rows): 32 x 32 tiles with K dealt
     // over the waves. us, 64 x 64 tiles -> this form: 256 x 1536 x 512 (96 tiles) 13.2 -> 8.7, 256 x 512 x 1376 (32) 29.5 ->
     // 10.5, 1024 x 512 x 1376 (128) 29.7 -> 19.5, 16 x 512 x 1376 108 -> 9.9 (the FMA engine took fewer than 32 rows); from a
-    // tile per unit on the larger tile wins (1024 x 1024 x 2816, 256 tiles: 57 against 67).
+    // tile per unit on the larger tile wins (1024 x 1024 x 2816, 256 tiles: 57 against 67). In more rounds than one a short K,
+    // which leaves waves without a stretch, goes to the larger tile too (64 x 11000, 172 tiles of 64 x 64 and 688 of 32 x 32:
+    // K = 64 5.2 against 6.1, 192 7.8 against 8.1, 256 9.0 against 8.4, and 100, which that kernel does not copy straight into
+    // LDS, 7.6 against 6.5).
     dim3 grid((unsigned)(ceilDiv(p.N, 32) * ceilDiv(p.M, 32)), 1, (unsigned)p.batch);
     if (p.K >= 1024) {
       AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(&gemmF32SmallKernel<8>), 8 * 16384));

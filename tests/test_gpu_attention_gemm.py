@@ -76,16 +76,21 @@ def test_mm_bmm_matmul_addmm_baddbmm(ops, dev, dtype):
 @pytest.mark.parametrize("m,n,k,form", [
     (2048, 2048, 64, "linear"),      # 256 tiles of 128 x 128, operands straight into LDS
     (2048, 2048, 64, "mm"),          # the same with a row-major [K, N] second operand
-    (200, 328, 96, "linear"),        # 64 x 64 tiles, ragged rows and columns
+    (1000, 1030, 96, "linear"),      # 64 x 64 tiles, ragged rows and columns
+    (200, 328, 96, "linear"),        # the same in 32 x 32 tiles: fewer than 192 of 64 x 64
     (200, 328, 96, "mm"),
     (1100, 2100, 32, "addmm"),       # one stage; alpha, beta and a matrix addend in the epilogue
-    (130, 200, 72, "linear"),        # K no multiple of 32: tiles staged through registers
+    (1000, 1030, 72, "linear"),      # K no multiple of 32: tiles staged through registers
+    (130, 200, 72, "linear"),        # 32 x 32 tiles, a K that ends inside a stretch
     (130, 200, 72, "mm"),
     (136, 200, 36, "mm_at"),         # transposed first operand (row-contiguous along M)
     (2304, 2048, 40, "mm"),          # staged, 128 x 128 tiles, ragged last stage
     (64, 64, 4100, "bmm"),           # long K, batch 3
     (33, 40, 8, "linear"),           # one partial tile
-    (31, 64, 64, "linear"),          # fewer than 32 rows: the FMA engine
+    (31, 64, 64, "linear"),          # fewer than 32 rows
+    (31, 12300, 64, "linear"),       # the same over 193 tiles: the FMA engine
+    (64, 8200, 64, "linear"),        # 514 tiles of 32 x 32, more than two on a compute unit: 64 x 64 at a short K ...
+    (64, 8200, 256, "linear"),       # ... and 32 x 32 at a longer one
 ])
 def test_fp32_gemm_on_the_matrix_cores(ops, dev, m, n, k, form):
     """fp32 operands through the fp32 MFMA kernels (both tile sizes, operands straight into LDS or staged through
