@@ -2475,19 +2475,36 @@ static void launchSplitKReduce(hipStream_t stream, const MfmaArgs& g, int splits
   hipLaunchKernelGGL(splitKReduceKernel<T>, dim3((unsigned)ceilDiv(items, (int64_t)threads)), dim3(threads), 0, stream, g, splits);
 }
 
-// How many ways to split K so that a problem with few 128 x 128 tiles still fills the chip with the four-stage kernel (one
-// workgroup per CU): tiles * splits up to the CU count, at least four K tiles per split, at most 16 splits. 1 = do not
-// split. *perSplit receives the K tiles per split; the last split has the remainder, never fewer than four unless K itself
-// is shorter. (Two stages and two workgroups per CU, the split of twice as many ways that this replaces, against it, us:
-// 128 x 4096 x 4096 21.5 -> 17.5, 203 x 12288 x 4096 47.3 -> 36.9, 203 x 4096 x 11008 40.8 -> 36.5, 400 x 5632 x 1024 23.1 -> 11.4,
-// 512 x 4096 x 11008 70 -> 63, 300 x 10240 x 8192 82 -> 64; 300 x 4096 x 11008, where 192 workgroups come out, 49.6 -> 51.2.)
-static int splitKWays(int64_t tiles, int64_t kTiles, int* perSplit) {
-  const int64_t byChip = computeUnits() / std::max<int64_t>(tiles, 1), byK = kTiles / kDeepStages;
-  int64_t splits = std::max<int64_t>(1, std::min<int64_t>(16, std::min(byChip, byK)));
-  int64_t per = ceilDiv(kTiles, splits);
-  while (per < kTiles && kTiles % per != 0 && kTiles % per < kDeepStages) ++per;  // (the last slice too fills the ring)
-  *perSplit = (int)per;
-  return (int)ceilDiv(kTiles, per);
+// K in slices of per K tiles, so that few 128 x 128 tiles become up to `workgroups` workgroups: at least four K tiles a slice,
+// at most 16 slices; the last slice has the remainder, never fewer than four unless K itself is shorter (it too fills the
+// ring of the four-stage kernel).
+struct KSplit {
+  int ways, per;
+};
+static KSplit splitK(int64_t workgroups, int64_t tiles, int64_t kTiles) {
+  const int64_t byChip = workgroups / std::max<int64_t>(tiles, 1), byK = kTiles / kDeepStages;
+  const int64_t ways = std::max<int64_t>(1, std::min<int64_t>(16, std::min(byChip, byK)));
+  int64_t per = ceilDiv(kTiles, ways);
+  while (per < kTiles && kTiles % per != 0 && kTiles % per < kDeepStages) ++per;
+  return {(int)ceilDiv(kTiles, per), (int)per};
+}
+
+// Whether K is sliced for one workgroup on a CU (the four-stage kernel) or for two (two stages): 1 way = not at all. us, fitted
+// to 680 products of 65 to 6001 rows with weights out of memory: a K tile takes 0.41 to 0.57 in the one, 0.81 to 1.07 with two
+// on a CU, the slices' sums and their launch 6 and 1.8 ns for each 1000 elements. Two on a CU -> one:
+//   128 x 4096 x 4096 21.4 -> 17.3, 203 x 12288 x 4096 47.9 -> 37.6, 400 x 5632 x 1024 21.9 -> 10.9, 512 x 4096 x 11008 69.8 -> 64.1;
+// and left at two, for tiles that fill half to all of the CUs with a long K or too few slices of one:
+//   600 x 4096 x 11008 75.4 against 98.4, 512 x 5120 x 13824 102.9 against 130.8, 300 x 4096 x 11008 50.5 against 53.1.
+static int splitKWays(int64_t m, int64_t n, int64_t tiles, int64_t kTiles, int* perSplit) {
+  auto us = [&](const KSplit& s) {
+    const float onCu = (float)(tiles * s.ways) / (float)computeUnits();
+    const float perTile = onCu <= 1.f ? 0.41f + 0.16f * onCu : onCu <= 2.f ? 0.81f + 0.255f * (onCu - 1.f) : 0.63f * onCu;
+    return perTile * (float)s.per + (s.ways > 1 ? 6.f + 1.8e-6f * (float)(m * n) * (float)s.ways : 3.f);
+  };
+  const KSplit one = splitK(computeUnits(), tiles, kTiles), two = splitK(2 * computeUnits(), tiles, kTiles);
+  const KSplit best = us(two) < us(one) ? two : one;
+  *perSplit = best.per;
+  return best.ways;
 }
 
 struct RotaryEpilogue {
@@ -2939,12 +2956,11 @@ static bool tailSplitPays(const GemmProblem& p) {
     return false;
   const TailSplit split = tailSplit(tiles, p.K / (2 * kBK), resident);
   if (split.slices == 1) return false;
-  int per = (int)kTiles;
   const int64_t tiles128 = ceilDiv(p.M, 128) * ceilDiv(p.N, 128);
-  const int ways = p.M * p.N * 4 < (int64_t(1) << 31) ? splitKWays(tiles128, kTiles, &per) : 1;
-  const float wgs = (float)(tiles128 * ways) / resident;  // workgroups per CU
-  const float us128 = (wgs <= 1.f ? 0.42f + 0.13f * wgs : wgs <= 2.f ? std::min(1.17f, 0.9f + 0.55f * (wgs - 1.f)) : 0.6f * wgs) * per +
-                      (ways > 1 ? 8.f + (float)(p.M * p.N) * ways * 1.6e-6f : 3.f);
+  const KSplit one = p.M * p.N * 4 < (int64_t(1) << 31) ? splitK(computeUnits(), tiles128, kTiles) : KSplit{1, (int)kTiles};
+  const float wgs = (float)(tiles128 * one.ways) / resident;  // workgroups per CU
+  const float us128 = (wgs <= 1.f ? 0.42f + 0.13f * wgs : wgs <= 2.f ? std::min(1.17f, 0.9f + 0.55f * (wgs - 1.f)) : 0.6f * wgs) * one.per +
+                      (one.ways > 1 ? 8.f + (float)(p.M * p.N) * one.ways * 1.6e-6f : 3.f);
   return split.us < 0.95f * us128;
 }
 
@@ -2965,7 +2981,7 @@ static FusedTile fusedTile(diopiContextHandle_t ctx, hipStream_t stream, GemmPro
   if (ceilDiv(problem->M, 256) * ceilDiv(problem->N, 256) >= 144 || (problem->M > kSkinnyMaxM && reserveTail(ctx, stream, problem))) return kFused256;
   const GemmProblem& p = *problem;
   int per = 0;
-  const bool one = p.M > kSkinnyMaxM && splitKWays(ceilDiv(p.M, 128) * ceilDiv(p.N, 128), p.K / kBK, &per) == 1;
+  const bool one = p.M > kSkinnyMaxM && splitKWays(p.M, p.N, ceilDiv(p.M, 128) * ceilDiv(p.N, 128), p.K / kBK, &per) == 1;
   return one && p.N % 8 == 0 && ((p.M - 1) * p.sOm + p.N) * 2 < (int64_t(1) << 31) ? kFused128 : kFusedNone;
 }
 
@@ -3057,7 +3073,7 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
     }
     AMD_CHECK(!p.colScale, "gemm: a column scale was set on a problem gemmAppliesColumnScale does not accept");
     // In between (too few 256 x 256 tiles for the chip, too many rows for the weight-streaming kernels): the 128 x 128
-    // form of the pipelined kernel, and when its tiles are at most half the CUs, K split over grid.y with fp32 partial
+    // form of the pipelined kernel, and when its tiles are too few for the chip, K split over grid.y with fp32 partial
     // products in workspace and a reduction pass (see splitKWays). Measured against
     // the 256 x 256 tiles split over K that this replaces (rows x 4096 x 4096, us): 128 rows 23.6 -> 21.5, 256 33.5 -> 22.3,
     // 512 37.4 -> 27.9, 1024 48.0 -> 41.7, 2048 71.3 -> 58.0; x 22016 x 4096: 128 rows 51.0 -> 38.8; K = 11008: 256 rows 45.0 -> 35.9.
@@ -3066,7 +3082,7 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
       const bool vecOk = p.N % 8 == 0 && p.sOm % 8 == 0 && ptr16(p.out) && (!p.Cin || (p.sCn == 1 && p.sCm % 8 == 0 && ptr16(p.Cin))) &&
                          (!p.bias || ptr16(p.bias)) && p.M * p.N * 4 < (int64_t(1) << 31);
       int per = 0;
-      const int splits = p.batch == 1 && vecOk ? splitKWays(tiles128, p.K / kBK, &per) : 1;
+      const int splits = p.batch == 1 && vecOk ? splitKWays(p.M, p.N, tiles128, p.K / kBK, &per) : 1;
       if (splits >= 2) {
         void* ws = nullptr;
         AMD_TRY(requireWorkspace(ctx, (int64_t)splits * p.M * p.N * 4, &ws));

@@ -431,6 +431,23 @@ def test_split_k_gemm(ops, dev, dtype, m, n, k):
     assert_exact(ops.linear(onehot, dw), dw[:, cols].t().contiguous().cpu())
 
 
+@pytest.mark.parametrize("m,n,k,ways", [(600, 4096, 11008, 3), (300, 4096, 11008, 5), (512, 4096, 11008, 2), (203, 4096, 4096, 4),
+                                        (1024, 4096, 4096, 1), (1300, 2048, 512, 1)])
+def test_slices_of_k_for_one_or_two_workgroups_on_a_compute_unit(ops, dev, pkg, m, n, k, ways):
+    """Tiles of 128 x 128 against a [K, N] operand: K in slices for two workgroups on a CU where a long K would leave too few
+    of one (the first two), for one, and not at all, which the workspace of the partial sums tells. Sums of small whole
+    numbers, exact in fp32."""
+    gen = torch.Generator().manual_seed(65)
+    x, w = (torch.randint(-2, 3, s, generator=gen).to(torch.bfloat16).to(dev) for s in ((m, k), (k, n)))
+    out = torch.empty(m, n, dtype=torch.bfloat16, device=dev)
+    with pkg.diopi.Context() as ctx:
+        handles = [pkg.diopi.handle(t) for t in (out, x, w)]
+        pkg.diopi.call("diopiMm", ctx, *[p for _, p in handles])
+        assert ctx.workspace() == ((1, ways * m * n * 4) if ways > 1 else (0, 0))
+        torch.cuda.synchronize()
+    assert torch.equal(out, (x.float() @ w.float()).to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k", [(1, 4096, 4096), (5, 100, 8192 + 128), (16, 11008, 4096), (17, 4096, 11008),
                                    (40, 16 * 7 + 3, 384), (64, 16000, 128), (1, 16, 128), (64, 4096, 4096),
