@@ -1024,7 +1024,7 @@ __global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 || ST
           [&](int) {});
     if constexpr (kNext) publish(integral_constant<int, (kAhead >= STAGES ? STAGES - 1 : kAhead) - 1>{});
     __builtin_amdgcn_sched_barrier(0);
-    // ---- phase 3: k-step 1, rows 64-127 | A and B of phase 0 of the next tile | A half of tile kt + 2
+    // ---- phase 3: k-step 1, rows 64-127 | A and B of phase 0 of the next tile | A half of tile kt + STAGES
     phase(1, 1,
           [&](int j) {
             if constexpr (kAhead >= STAGES) dmaA(cur, kt + STAGES, j);
@@ -2715,7 +2715,10 @@ static diopiError_t launchMfmaPipelined128(hipStream_t stream, const GemmProblem
     return diopiSuccess;
   };
   const int64_t kTiles = p.K / kBK, fewest = EPI == kEpiPartial ? kTiles - (int64_t)(splits - 1) * kTilesPerSplit : kTiles;
-  AMD_TRY(fewest >= kDeepStages && (int64_t)grid.x * grid.y * grid.z <= computeUnits() ? launch(std::integral_constant<int, kDeepStages>{}) : launch(std::integral_constant<int, 2>{}));
+  // (of four K tiles and no more, all of which the ring would wait for: 65 x 1536 x 256 4.7 us in two stages, 5.0 in four; six,
+  // 65 x 4096 x 384: 6.5 against 5.8)
+  const bool deep = (EPI == kEpiPartial ? fewest >= kDeepStages : fewest > kDeepStages) && (int64_t)grid.x * grid.y * grid.z <= computeUnits();
+  AMD_TRY(deep ? launch(std::integral_constant<int, kDeepStages>{}) : launch(std::integral_constant<int, 2>{}));
   if (EPI == kEpiPartial) {
     const int64_t items = p.M * (p.N / 8);
     launchSplitKReduce<T>(stream, g, splits, items);
