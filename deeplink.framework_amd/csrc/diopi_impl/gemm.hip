@@ -833,6 +833,9 @@ __global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 || ST
   extern __shared__ __attribute__((aligned(16))) char smem[];
   T* sA = reinterpret_cast<T*>(smem);  // [STAGES][BM][64]
   T* sB = sA + STAGES * BM * kBK;      // [STAGES][BN][64]
+  // What the first loads need of the arguments, requested at once: left to where it is used it is three scalar loads that wait
+  // for each other, a quarter of a microsecond (65 x 1536 x 256: 4.70 -> 4.40 us).
+  asm volatile("" ::"s"(g.A), "s"(g.B), "s"(g.sAb), "s"(g.lda), "s"(g.sBb), "s"(g.ldb), "s"(g.M), "s"(g.N), "s"(g.K), "s"(g.tilesM), "s"(g.tilesN));
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / kWavesN, wn = wave % kWavesN;
   int tm, tn;
