@@ -834,7 +834,7 @@ __global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 || ST
   T* sA = reinterpret_cast<T*>(smem);  // [STAGES][BM][64]
   T* sB = sA + STAGES * BM * kBK;      // [STAGES][BN][64]
   // What the first loads need of the arguments, requested at once: left to where it is used it is three scalar loads that wait
-  // for each other, a quarter of a microsecond (65 x 1536 x 256: 4.70 -> 4.40 us).
+  // for each other, a quarter of a microsecond (65 x 1536 x 256: 4.70 -> 4.48 us).
   asm volatile("" ::"s"(g.A), "s"(g.B), "s"(g.sAb), "s"(g.lda), "s"(g.sBb), "s"(g.ldb), "s"(g.M), "s"(g.N), "s"(g.K), "s"(g.tilesM), "s"(g.tilesN));
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / kWavesN, wn = wave % kWavesN;
@@ -2718,7 +2718,7 @@ static diopiError_t launchMfmaPipelined128(hipStream_t stream, const GemmProblem
     return diopiSuccess;
   };
   const int64_t kTiles = p.K / kBK, fewest = EPI == kEpiPartial ? kTiles - (int64_t)(splits - 1) * kTilesPerSplit : kTiles;
-  // (of four K tiles and no more, all of which the ring would wait for: 65 x 1536 x 256 4.7 us in two stages, 5.0 in four; six,
+  // (of four K tiles and no more, all of which the ring would wait for: 65 x 1536 x 256 4.5 us in two stages, 4.8 in four; six,
   // 65 x 4096 x 384: 6.5 against 5.8)
   const bool deep = (EPI == kEpiPartial ? fewest >= kDeepStages : fewest > kDeepStages) && (int64_t)grid.x * grid.y * grid.z <= computeUnits();
   AMD_TRY(deep ? launch(std::integral_constant<int, kDeepStages>{}) : launch(std::integral_constant<int, 2>{}));
@@ -2967,7 +2967,9 @@ static bool tailSplitPays(const GemmProblem& p) {
   const float wgs = (float)(tiles128 * one.ways) / resident;  // workgroups per CU
   const float us128 = (wgs <= 1.f ? 0.42f + 0.13f * wgs : wgs <= 2.f ? std::min(1.17f, 0.9f + 0.55f * (wgs - 1.f)) : 0.6f * wgs) * one.per +
                       (one.ways > 1 ? 8.f + (float)(p.M * p.N) * one.ways * 1.6e-6f : 3.f);
-  return split.us < 0.95f * us128;
+  // (a small weight stays in the caches between its rows of tiles, of which the smaller tile has twice as many: 6001 x 1024 x
+  // 4096 51 us against 56 in slices, 4000 x 2048 x 4096 63 against 68, where 400 x 12288 x 4096 has 64 against 57)
+  return split.us < (0.95f - 0.07f * std::min(2.f, (float)(16 << 20) / (float)(p.N * p.K * 2))) * us128;
 }
 
 // Settles whether a product with too few 256 x 256 tiles goes to K slices of them, and reserves the workspace without which
