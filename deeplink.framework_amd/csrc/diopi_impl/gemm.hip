@@ -421,6 +421,28 @@ __device__ __forceinline__ void addendToLds(const MfmaArgs& g, const T* cin, int
   }
 }
 
+// Eight column values in one load at element alignment, of types other than the usual three one by one (which is as many
+// latencies: the reduction of K slices at 400 x 5120 14.6 us against 12.3, int8 linears of 2048 x 12288 x 4096 196 against 182).
+__device__ __forceinline__ void columnPiece(const void* p, int dtype, int col, float (&f)[8]) {
+  auto piece = [&](auto zero) {
+    using S = decltype(zero);
+    typedef S S8 __attribute__((ext_vector_type(8), aligned(sizeof(S))));
+    const S8 v = *reinterpret_cast<const S8*>(static_cast<const S*>(p) + col);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = static_cast<float>(v[e]);
+  };
+  if (dtype == diopi_dtype_bfloat16) {
+    piece(bf16_t(0.f));
+  } else if (dtype == diopi_dtype_float16) {
+    piece(half_t(0.f));
+  } else if (dtype == diopi_dtype_float32) {
+    piece(0.f);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = loadAs<float>(p, col + e, dtype);
+  }
+}
+
 template <typename T, int EPI, int TM, int TN, typename AccRow>
 __device__ __forceinline__ void vectorEpilogue(const MfmaArgs& g, T* out, const T* cin, const T* bias, int row0, int colBase,
                                                int frow, int kq, AccRow&& accRow, unsigned ldsTab = 0) {
@@ -680,10 +702,12 @@ __device__ __forceinline__ void vectorEpilogue(const MfmaArgs& g, T* out, const 
 #pragma unroll
     for (int jp = 0; jp < TN / 2; ++jp) {
       const int col = min(col0 + jp * 32, g.N - 8);  // N % 8 == 0 here; a clamped piece is never stored
+      columnPiece(g.colScale, g.colScaleDtype, col, sv[jp]);
+      if (g.colBias) columnPiece(g.colBias, g.colBiasDtype, col, bv[jp]);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        sv[jp][e] = loadAs<float>(g.colScale, col + e, g.colScaleDtype) * g.alpha;
-        bv[jp][e] = g.colBias ? loadAs<float>(g.colBias, col + e, g.colBiasDtype) : 0.f;
+        sv[jp][e] *= g.alpha;
+        if (!g.colBias) bv[jp][e] = 0.f;
       }
     }
     staticFor<TM>([&](auto ic) {
