@@ -291,16 +291,34 @@ def test_four_wave_gemm_every_instantiation_exact(ops, dev, dtype, epilogue):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("epilogue,m,n,k", [
-    ("linear", 1554, 11000, 4096),            # 301 tiles: a whole round, then 45 tiles in slices; ragged rows and columns
-    ("bias", 1554, 11008, 4096 + 128),        # 33 K-tile pairs: slices of unequal length
-    ("addend", 300, 8192, 8192),              # 64 tiles: slices only
-    ("addend", 5000, 5120, 13824),            # 400 tiles, 144 left: more slices than workgroups
-    ("rotary", 1554, 12288, 4096), ("silu_mul", 1554, 22016, 4096), ("column_scale", 882, 5120, 13824)])
-def test_four_wave_gemm_last_round_split_along_k_exact(ops, dev, dtype, epilogue, m, n, k):
+@pytest.mark.parametrize("epilogue,m,n,k,left,slices,other", [
+    ("linear", 1554, 11000, 4096, 45, 4, 0),          # 301 tiles: a whole round, then 45 tiles in slices; ragged rows and columns
+    ("bias", 1554, 11008, 4096 + 128, 45, 5, 0),      # 33 K-tile pairs: slices of unequal length
+    ("linear", 4525, 4096, 4096, 32, 4, 0), ("linear", 4525, 4096, 14336, 32, 8, 0), ("linear", 6001, 4096, 4096, 128, 2, 0),
+    ("linear", 882, 5120, 5120, 80, 3, 0),            # 80 tiles: slices only
+    ("addend", 882, 5120, 13824, 80, 3, 0),
+    ("addend", 300, 8192, 8192, 0, 0, 0),             # 64 tiles: 128 x 128 ones instead
+    ("linear", 512, 4096, 11008, 0, 0, 2 * 512 * 4096 * 4),                      # the same, split over K
+    ("addend", 5000, 5120, 13824, 144, 3, 0),         # 400 tiles, 144 left: more slices than workgroups
+    ("rotary", 1554, 12288, 4096, 80, 3, 0), ("rotary", 203, 22016, 4096, 86, 2, 0),
+    ("silu_mul", 1554, 22016, 4096, 90, 2, 0), ("silu_mul", 400, 12288, 4096, 96, 2, 0),
+    ("column_scale", 882, 5120, 13824, 80, 3, 5120 * 13824 * 2)])                # and the weight in 16 bits
+def test_four_wave_gemm_last_round_split_along_k_exact(ops, dev, pkg, dtype, epilogue, m, n, k, left, slices, other):
     """The tiles of a partly filled last round in slices of K (the 4-wave kernel's accumulators as fp32 partial sums, added
-    and given the epilogue by a second launch). One-hot activations over the whole of K: every product is one weight
-    element, found by exactly one slice, and the expected result is exact."""
+    and given the epilogue by a second launch): as many as the workspace tells, with whole rounds before them and without.
+    One-hot activations over the whole of K: every product is one weight element, found by exactly one slice, and the
+    expected result is exact."""
+    ops._ctx = ctx = pkg.diopi.Context()             # outside a scope, whose products take no such workspace
+    try:
+        check_last_round(ops, dev, dtype, epilogue, m, n, k)
+        assert ctx.workspace()[1] == left * slices * 256 * 1024 + other
+        torch.cuda.synchronize()
+    finally:
+        ops._ctx = 0
+        ctx.close()
+
+
+def check_last_round(ops, dev, dtype, epilogue, m, n, k):
     g0 = g(78)
     cols = torch.randint(0, k, (m,), generator=g0)
     cols[:4] = torch.tensor([0, k - 1, 127, 128])
@@ -336,9 +354,9 @@ def test_four_wave_gemm_last_round_split_along_k_exact(ops, dev, dtype, epilogue
         assert_exact(got, out.reshape(m, n).to(dtype))
 
 
-@pytest.mark.parametrize("m,n,k", [(70, 136, 192), (70, 136, 256), (129, 264, 320), (129, 264, 384), (65, 136, 448), (130, 264, 2752), (100, 4096, 11008)])
+@pytest.mark.parametrize("m,n,k", [(70, 136, 192), (70, 136, 256), (129, 264, 320), (129, 264, 384), (65, 136, 448), (100, 136, 512), (130, 264, 2752), (100, 4096, 11008)])
 def test_products_with_few_tiles_four_stage_ring_exact(ops, dev, m, n, k):
-    """K shorter than the four-stage ring, as long, and one to three K tiles longer; K slices of unequal length; the [K, N]
+    """K no longer than the four-stage ring (two stages), two slices as long as it, and one to three K tiles longer; K slices of unequal length; the [K, N]
     operand in place and the K-contiguous one. One-hot rows over the whole of K: exact."""
     g0 = g(79)
     cols = torch.randint(0, k, (m,), generator=g0)
