@@ -452,7 +452,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void contextAttnSingleBlockKe
 // queries of a head and its four waves every fourth tile of 16 keys, each with a softmax state of its own; the states meet
 // in LDS at the end, so a short sequence is four times as many waves and a chain of loads a quarter as long. What bounds
 // the short sequences of the fp32 configuration is exactly that chain of latencies (2 x 128 tokens, 8 heads of 64: 55 us
-// with a workgroup per query and scores in LDS, 6 now; 4 x 2048 tokens, 8 heads of 128: 622 us, 0.4 of the fp32 matrix peak).
+// with a workgroup per query and scores in LDS, 6 now; 4 x 2048 tokens, 8 heads of 128: 622 us, 0.35 of the fp32 matrix peak).
 // v_mfma_f32_16x16x4_f32: lane (c = l & 15, g = l >> 4) feeds row c, k = g of both operands and receives D[4 g + r][c].
 //   S^T = K Q^T: the contraction order is free as long as both operands agree, so group g takes the D / 4 consecutive
 //   elements from g D / 4 on: 16-byte loads straight into operand registers. The lane ends up with keys 4 g .. 4 g + 3 of

@@ -2576,7 +2576,7 @@ struct TailSplit {
 // A plain last round is replaced only where that saves a twentieth of it. Measured, plain -> split (us):
 //   4525 x 4096 x 14336 (288 tiles, 32 left, 8 slices) 533 -> 369      4525 x 4096 x 4096 (4 slices) 151 -> 122
 //   1554 x 11008 x 4096 (301 tiles, 45 left, 4 slices) 145 -> 127      1554 x 12288 x 4096 rotary (80 left) 158 -> 143
-//   6001 x 4096 x 14336 (384 tiles, 128 left, 2 slices) 568 -> 490     6001 x 4096 x 4096 (128 left) 166 -> 170: stays plain
+//   6001 x 4096 x 14336 (384 tiles, 128 left, 2 slices) 568 -> 490     6001 x 4096 x 4096 (2 slices) 162 -> 157, rotary 170 -> 160
 //   5000 x 5120 x 13824 (400 tiles, 144 left, 3 slices in two rounds) 551 -> 525
 static TailSplit tailSplit(int64_t tiles, int64_t pairs, int resident) {
   const int rest = (int)(tiles % resident), most = (int)std::min<int64_t>(rest ? 2 * resident / rest : 0, pairs / 2);
@@ -2974,7 +2974,7 @@ diopiError_t transposeCopy(hipStream_t stream, void* dst, const void* src, int i
 // more than the CUs and up to 1.19 with two on a CU, and its slices are written and read back as fp32 too. Measured,
 // 128 x 128 -> slices of 256 x 256 (us): 882 x 5120 x 13824 183 -> 111 (3 slices), 882 x 5120 x 5120 73 -> 58 (3), 512 x 12288 x
 // 4096 75 -> 58 (2), 203 x 22016 x 4096 71 -> 63 (2); not taken: 203 x 12288 x 4096 37 against 42, 300 x 10240 x 8192 64 against
-// 74, 300 x 4096 x 11008 51 against 52, 512 x 4096 x 11008 63 against 58.
+// 74, 300 x 4096 x 11008 51 against 52, and 512 x 4096 x 11008 63 against 58, which the estimates miss by 2 %.
 static bool tailSplitPays(const GemmProblem& p) {
   const int resident = computeUnits() / 8 * 8;
   const int64_t tiles = ceilDiv(p.M, 256) * ceilDiv(p.N, 256), kTiles = p.K / kBK;

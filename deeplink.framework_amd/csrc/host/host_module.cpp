@@ -5,7 +5,7 @@
 // success raises. Output shapes and dtypes are inferred here too (like, rows_of, broadcast_of).
 //
 // Why native: with the marshalling in Python (ctypes structures filled field by field) a call cost 25 us of host time, of
-// which the launch itself is three, and every layer of small kernels was bound by it (14 calls of the fp32 block of
+// which the launch itself is three, and every layer of small kernels was bound by it (16 calls of the fp32 block of
 // 2 x 128 tokens: 357 us for 175 us of kernels).
 //
 // The diopi* and runtime symbols are looked up in the process when the module is imported (both libraries are loaded with

@@ -361,7 +361,7 @@ class SimAllocator:
 
 
 # ---- profiler hooks (runtime/device/profilerapis.h:12-14; diopirt_impl.cpp:224-237) ----
-profiler_on = False   # read by diopi.call on every op: a plain attribute, no C call while the profiler is off
+profiler_on = False   # read by diopi.call: a plain attribute, no C call while the profiler is off (ops.py: ranges open in the native module)
 
 
 def enableProfiler(dump_path=""):
