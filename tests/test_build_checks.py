@@ -1,6 +1,9 @@
 """The build script's own guard: kernels whose K loop is hand-placed register text may not use scratch memory."""
 import importlib.util
 import os
+import subprocess
+
+import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -28,3 +31,24 @@ def test_scratch_guard_reads_the_resource_usage_remarks():
     other = spilled.replace("gemmMfma4WaveKernel", "gemmFmaKernel")
     assert b.scratch_users(other, ("gemmMfma4WaveKernel",)) == []
     assert "gemm.hip" in b.NO_SCRATCH_KERNELS
+
+
+def test_libraries_are_linked_where_the_host_module_does_not_build(monkeypatch):
+    b = _build_module()
+    linked = []
+
+    def run(cmd, **_):
+        linked.append(cmd[cmd.index("-o") + 1])
+        return subprocess.CompletedProcess(cmd, 0, "", "")
+
+    monkeypatch.setattr(b, "compile_one", lambda src, obj: (src, 0, ""))
+    monkeypatch.setattr(b, "build_host", lambda: (b.HOST_SOURCE, 1, "no torch headers"))
+    monkeypatch.setattr(b.subprocess, "run", run)
+    with pytest.raises(RuntimeError, match="host module"):
+        b.build()
+    assert linked == [b.TARGETS["impl"]["out"], b.TARGETS["rt"]["out"]]
+    linked.clear()
+    monkeypatch.setattr(b, "compile_one", lambda src, obj: (src, int(src.endswith("gemm.hip")), ""))
+    with pytest.raises(RuntimeError, match="compilation failed"):
+        b.build()
+    assert linked == []
