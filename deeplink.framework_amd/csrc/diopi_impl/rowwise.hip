@@ -599,33 +599,44 @@ __global__ __launch_bounds__(1024) void rowStreamKernel(T* __restrict__ out, con
     const T* src = in + row * inRowStride;
     T* dst = out + row * outRowStride;
     if constexpr (OP == kRowSoftmax) {
-      // (differences are taken before the scaling by log2 e, whose product with the lowest number is out of range)
-      float m = -INFINITY, sum = 0.f;
+      float m = -INFINITY, sum = 0.f;  // in units of log2
       for (int64_t i = threadIdx.x; i < pieces; i += 1024) {
         float f[N];
         load(src, i, f);
         float pm = f[0];
 #pragma unroll
         for (int j = 1; j < N; ++j) pm = fmaxf(pm, f[j]);
+        pm *= kLog2e;
         if (pm > m) {
-          sum *= __builtin_amdgcn_exp2f((m - pm) * kLog2e);  // (m = -inf: sum is still 0, and exp2(-inf) = 0)
+          sum *= __builtin_amdgcn_exp2f(m - pm);  // (m = -inf: sum is still 0, and exp2(-inf) = 0)
           m = pm;
         }
         if (m != -INFINITY) {
 #pragma unroll
-          for (int j = 0; j < N; ++j) sum += __builtin_amdgcn_exp2f((f[j] - m) * kLog2e);
+          for (int j = 0; j < N; ++j) sum += __builtin_amdgcn_exp2f(fmaf(f[j], kLog2e, -m));
         }
       }
       const float rowMax = blockReduce(m, true, red);
-      const float from = (rowMax == -INFINITY) ? 0.f : rowMax;  // all -inf row: the sum is 0 and every output 0 * inf = nan, like the CPU kernel
-      sum = (m == -INFINITY) ? 0.f : sum * __builtin_amdgcn_exp2f((m - from) * kLog2e);
+      if (rowMax == -INFINITY || rowMax == INFINITY) {
+        // no finite maximum in these units: rows of -inf alone or with +inf, which give NaN, and rows of nothing but numbers
+        // around the lowest, or with one around the largest, whose product with log2 e is out of range: differences first
+        float raw = -INFINITY, s = 0.f;
+        for (int64_t i = threadIdx.x; i < cols; i += 1024) raw = fmaxf(raw, static_cast<float>(src[i]));
+        raw = blockReduce(raw, true, red);
+        for (int64_t i = threadIdx.x; i < cols; i += 1024) s += __builtin_amdgcn_exp2f((static_cast<float>(src[i]) - raw) * kLog2e);
+        s = blockReduce(s, false, red);
+        for (int64_t i = threadIdx.x; i < cols; i += 1024)
+          dst[i] = static_cast<T>(__builtin_amdgcn_exp2f((static_cast<float>(src[i]) - raw) * kLog2e) / s);
+        continue;
+      }
+      sum = (m == -INFINITY) ? 0.f : sum * __builtin_amdgcn_exp2f(m - rowMax);
       const float total = blockReduce(sum, false, red);
       const float inv = 1.f / total;
       for (int64_t i = threadIdx.x; i < pieces; i += 1024) {
         float f[N];
         load(src, i, f);
 #pragma unroll
-        for (int j = 0; j < N; ++j) f[j] = __builtin_amdgcn_exp2f((f[j] - from) * kLog2e) * inv;
+        for (int j = 0; j < N; ++j) f[j] = __builtin_amdgcn_exp2f(fmaf(f[j], kLog2e, -rowMax)) * inv;
         store(dst, i, f);
       }
     } else {
