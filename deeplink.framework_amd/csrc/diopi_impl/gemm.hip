@@ -3120,9 +3120,8 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
                          (!p.bias || ptr16(p.bias)) && p.M * p.N * 4 < (int64_t(1) << 31);
       int per = 0;
       const int splits = p.batch == 1 && vecOk ? splitKWays(p.M, p.N, tiles128, p.K / kBK, &per) : 1;
-      if (splits >= 2) {
-        void* ws = nullptr;
-        AMD_TRY(requireWorkspace(ctx, (int64_t)splits * p.M * p.N * 4, &ws));
+      void* ws = nullptr;  // (where there is none, as in a recording that nothing was held for, the tiles go unsplit)
+      if (splits >= 2 && requireWorkspace(ctx, (int64_t)splits * p.M * p.N * 4, &ws) == diopiSuccess) {
         return p.dtype == diopi_dtype_bfloat16 ? launchMfmaPipelined128<bf16_t, kEpiPartial>(stream, p, static_cast<float*>(ws), splits, per, bT)
                                                : launchMfmaPipelined128<half_t, kEpiPartial>(stream, p, static_cast<float*>(ws), splits, per, bT);
       }

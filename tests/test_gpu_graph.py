@@ -142,7 +142,8 @@ def test_products_that_can_do_without_workspace_record_without_it(pkg, ops, dev)
     gen = torch.Generator().manual_seed(7)
     x, w = rnd(1554, 4096), rnd(11008, 4096)
     a, b = rnd(2, 77, 385), rnd(2, 385, 40)
-    calls = [lambda: ops.linear(x, w), lambda: ops.bmm(a, b)]
+    c, d = rnd(600, 11008), rnd(11008, 4096)                                                       # three slices of K
+    calls = [lambda: ops.linear(x, w), lambda: ops.bmm(a, b), lambda: ops.mm(c, d)]
     want = [f() for f in calls]
     torch.cuda.synchronize()
     graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
