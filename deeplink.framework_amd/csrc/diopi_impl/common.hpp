@@ -171,6 +171,20 @@ __device__ __forceinline__ void globalLoadToLds16(const void* lanePtr, unsigned 
       : "memory");
 }
 
+// The same copy marked non-temporal (see loadToLds16Stream).
+__device__ __forceinline__ void globalLoadToLds16Stream(const void* lanePtr, unsigned ldsAddr) {
+  unsigned savedM0;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %2, off nt\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(savedM0)
+      : "s"(ldsAddr), "v"(lanePtr)
+      : "memory");
+}
+
 // The same copy marked non-temporal: for data that is read once (a weight stream), so that it does not push
 // re-used lines (the activations every workgroup reads) out of L2.
 __device__ __forceinline__ void loadToLds16Stream(u32x4 rsrc, int voffset, int soffset, unsigned ldsAddr) {

@@ -26,12 +26,12 @@
 //     when there would otherwise be too few workgroups for the chip, at most 256 per sequence); states are merged by
 //     wave butterflies, then through LDS, then across chunks by a small lane-parallel second kernel.
 //
-// The two halves of the two-call form (scores to memory, then softmax and the sum over V from stored scores) are the same
-// streaming kernel with the other half of the work compiled out: 588 -> 462 us for both at batch 64 with 156 000 cached
-// tokens, and the second half no longer walks a long sequence with one workgroup (1 x 32768 tokens: 1709 -> 60 us).
+// 16-bit rows shared by several query heads, the two-call form (scores to memory, then softmax and the sum over V from
+// stored scores) of 16-bit rows, and the fused form where there are few (sequence, head) pairs run on the matrix pipe
+// instead: decodeGroupedKernel. fp32 rows run on the streaming kernel in every form.
 //
 // Head rows of whole 16-byte pieces up to 512 bytes at 16-byte aligned strides take the kernels above (rows of other
-// lengths than 128, 256 or 512 bytes on the lanes of the next of those, the lanes past the row's end masked); any
+// lengths than 128, 256 or 512 bytes on the layout of the next of those, the places past the row's end masked); any
 // other head size or alignment (up to 1024 elements) takes the generic kernels at the end: one workgroup per (sequence, head), 256 tokens
 // at a time, one token's dot product per thread and P.V with the threads over d. A correctness path.
 #include <algorithm>
@@ -45,7 +45,11 @@ constexpr float kLog2eTA = 1.4426950408889634f;
 constexpr int kTaWaves = 4;
 constexpr int kTaUnroll = 2;
 constexpr int kTaChunk = 512;  // tokens of one sequence handled by one workgroup (grows for very long sequences)
-constexpr int kTaMaxSplit = 256;  // decodeMergeWideKernel holds four splits' weights per lane (decodeMergeKernel: one, up to 64 splits)
+constexpr int kTaMaxSplit = 256;  // decodeMergeWideKernel holds four splits' weights per lane
+// Splits that decodeMergeKernel merges: the eight it requests at once. More take a workgroup per (sequence, head), whose
+// waves request up to 32 at once: 28 splits of 32 heads (1 x 1777 tokens, with the kernel before it) 13.3 -> 12.1 us,
+// 250 splits (1 x 32000) 97.9 -> 91.1; with a workgroup from five splits on 64 x (512 .. 4096) x 8 K/V heads would lose 2 - 4 %.
+constexpr int kTaNarrowSplits = 8;
 constexpr int kTaMinChunk = 128;  // shorter chunks cost more in prologues, partial results and merging than they gain ...
 constexpr int kTaTinyChunk = 64;  // ... unless even those leave CUs without a workgroup
 constexpr int kTaWgsPerCu = 8;    // workgroups per CU the chunk length aims for
@@ -102,41 +106,13 @@ __device__ __forceinline__ float headRowSum(float v) {
   return v;
 }
 
-// c + a[0] b[0] + a[1] b[1] for two packed 16-bit pairs, in one instruction (fp32 accumulation).
-template <typename T>
-__device__ __forceinline__ float dotPair(uint32_t a, uint32_t b, float c) {
-  static_assert(sizeof(T) == 2, "packed pairs of 16-bit elements");
-  if constexpr (std::is_same<T, bf16_t>::value) {
-    typedef __bf16 Pair __attribute__((ext_vector_type(2)));
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(Pair, a), __builtin_bit_cast(Pair, b), c, false);
-  } else {
-    typedef _Float16 Pair __attribute__((ext_vector_type(2)));
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(Pair, a), __builtin_bit_cast(Pair, b), c, false);
-  }
-}
-template <typename T>
-__device__ __forceinline__ uint32_t packPair(float lo, float hi) {
-  const T l = static_cast<T>(lo), h = static_cast<T>(hi);
-  return (uint32_t)__builtin_bit_cast(uint16_t, l) | ((uint32_t)__builtin_bit_cast(uint16_t, h) << 16);
-}
-
 // The three things the streaming kernel below can do with a chunk of a sequence: the whole decode attention (scores,
 // online softmax and the sum over V), only the scores (first half of the two-call form: att[h, start_b + t]), or the
 // softmax and the sum over V from scores computed earlier (second half of the two-call form).
 enum TaMode { kTaFused = 0, kTaLogitsOut = 1, kTaReduceV = 2 };
 
-// The value lane J of every aligned group of four lanes holds, in all four (one DPP move; every lane active).
-template <int J>
-__device__ __forceinline__ uint32_t quadBroadcast(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, J * 0x55, 0xf, 0xf, false);
-}
-template <int J>
-__device__ __forceinline__ float quadBroadcast(float v) {
-  return __builtin_bit_cast(float, quadBroadcast<J>(__builtin_bit_cast(uint32_t, v)));
-}
-
-// T: bf16_t / half_t (8 per 16 B) or float (4 per 16 B). LPT lanes cover one head row. LT: the type of the scores in
-// memory (the two-call modes). QPK: query heads that share this workgroup's K/V head and are all served from one read
+// T: bf16_t / half_t (8 per 16 B; HIW only) or float (4 per 16 B). LPT lanes cover one head row. LT: the type of the scores
+// in memory (the two-call modes). QPK: query heads that share this workgroup's K/V head and are all served from one read
 // of its rows (grouped-query layouts; 1 otherwise). With QPK > 1 the grid is one-dimensional and decoded so that the
 // workgroups that share a K/V head's rows run next to each other on one XCD.
 template <typename T, int LPT, bool HIW, int MODE = kTaFused, typename LT = float, int QPK = 1, bool PART = false>
@@ -224,12 +200,6 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
       __syncthreads();
     }
   }
-  // Several query heads on 16-bit rows: the products are taken two at a time on the packed pairs as they come from
-  // memory (q.k: a pair of q against a pair of k; p.v: the probabilities of the two rows in flight, rounded to 16
-  // bits, against the two rows' values of one element), which halves the arithmetic instructions and needs no
-  // conversions of K and V. 32 query heads on 8 K/V heads, batch 64 x (512..4096), fused: 184 -> 157 us (147 -> 110
-  // registers, three -> four waves per SIMD); batch 256 x (1024..2048): 484 -> 413 us.
-  constexpr bool kPairs = QPK > 1 && sizeof(T) == 2 && UNR == 2;
   // PART: a head row shorter than the LPT pieces the lane group spans (head sizes between the powers of two). The lanes
   // past its end read the row's first piece instead (memory that exists), hold zeros for q, so that they add nothing
   // to a score, and store nothing. (A variant of its own: with these selects in the kernel for whole rows the launch
@@ -238,27 +208,18 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
   const int subIn = PART ? (live ? sub : 0) : sub;
   // scores leave the kernel in natural units, inside it they are in units of log2
   const float qScale = MODE == kTaLogitsOut ? a.scaleLog2e / kLog2eTA : a.scaleLog2e;
-  float qf[kPairs ? 1 : QPK][N];
-  uint32_t qp[kPairs ? QPK : 1][4];
+  float qf[QPK][N];
   if constexpr (kNeedK) {
 #pragma unroll
     for (int j = 0; j < QPK; ++j) {
       V qv = *reinterpret_cast<const V*>(reinterpret_cast<const T*>(a.q) + b * a.qBatchStride + (h + headOf(j)) * a.qHeadStride + subIn * N);
-      if constexpr (kPairs) {
-        const u32x4 raw = __builtin_bit_cast(u32x4, qv);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) qp[j][c] = live ? raw[c] : 0u;
-      } else {
-#pragma unroll
-        for (int e = 0; e < N; ++e) qf[j][e] = live ? static_cast<float>(qv[e]) * qScale : 0.f;
-      }
+      for (int e = 0; e < N; ++e) qf[j][e] = live ? static_cast<float>(qv[e]) * qScale : 0.f;
     }
   }
   const T* kBase = kNeedK ? reinterpret_cast<const T*>(a.k) + kvh * a.kHeadStride + subIn * N : nullptr;
   const T* vBase = kNeedV ? reinterpret_cast<const T*>(a.v) + kvh * a.vHeadStride + subIn * N : nullptr;
 
-  constexpr bool kShared = QPK == 4 && kPairs && MODE == kTaFused;
-  float mOwn = -INFINITY, lOwn = 0.f;  // kShared: the state of head (sub & 3), see the loop
   float m[QPK], l[QPK], acc[QPK][N];
 #pragma unroll
   for (int j = 0; j < QPK; ++j) {
@@ -307,63 +268,13 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
   for (int it = begin; it < end; it += STEP) {
     loadRows(kn, vn, ln, okn);    // rows of the next iteration (all masked past the end)
     loadSlots(it + 2 * STEP);     // indices of the one after
-    float kf[kNeedK && QPK > 1 && !kPairs ? UNR : 1][N];  // several query heads on fp32 rows: the K rows are converted once
-    if constexpr (kNeedK && QPK > 1 && !kPairs) {
+    float kf[kNeedK && QPK > 1 ? UNR : 1][N];  // several query heads on fp32 rows: the K rows are converted once
+    if constexpr (kNeedK && QPK > 1) {
 #pragma unroll
       for (int u = 0; u < UNR; ++u)
 #pragma unroll
         for (int e = 0; e < N; ++e) kf[u][e] = static_cast<float>(kr[u][e]);
     }
-    // kPairs: element 2 c and 2 c + 1 of the two V rows, regrouped as (row 0, row 1) pairs of one element each
-    uint32_t vlo[kPairs && kNeedV ? 4 : 1], vhi[kPairs && kNeedV ? 4 : 1];
-    if constexpr (kPairs && kNeedV) {
-      const u32x4 r0 = __builtin_bit_cast(u32x4, vr[0]), r1 = __builtin_bit_cast(u32x4, vr[1]);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        vlo[c] = __builtin_amdgcn_perm(r1[c], r0[c], 0x05040100u);
-        vhi[c] = __builtin_amdgcn_perm(r1[c], r0[c], 0x07060302u);
-      }
-    }
-    // kShared: four query heads on 16-bit rows in the fused mode. Every lane of a lane group holds the scores of all
-    // four heads after the row sums, so the softmax update of head i is done by lanes i, i + 4, ... alone (their own
-    // running maximum and sum: mOwn, lOwn) and the factors reach the other lanes by one quad broadcast each: three
-    // exponentials per lane and pair of rows instead of twelve. The same arithmetic per head as the loop below.
-    if constexpr (kShared) {
-      float scAll[QPK][UNR];
-#pragma unroll
-      for (int j = 0; j < QPK; ++j)
-#pragma unroll
-        for (int u = 0; u < UNR; ++u) {
-          const u32x4 kraw = __builtin_bit_cast(u32x4, kr[u]);
-          float d = 0.f;
-#pragma unroll
-          for (int c = 0; c < 4; ++c) d = dotPair<T>(qp[j][c], kraw[c], d);
-          d = headRowSum<LPT>(d) * qScale;
-          scAll[j][u] = ok[u] ? d : -INFINITY;
-        }
-      const int own = sub & 3;
-      float my[UNR];
-#pragma unroll
-      for (int u = 0; u < UNR; ++u)
-        my[u] = own == 0 ? scAll[0][u] : (own == 1 ? scAll[1][u] : (own == 2 ? scAll[2][u] : scAll[3][u]));
-      const float mn = fmaxf(mOwn, fmaxf(my[0], my[UNR - 1]));
-      const bool any = mn != -INFINITY;
-      const float corr = any ? __builtin_amdgcn_exp2f(mOwn - mn) : 1.f;  // mOwn == -inf gives 0: acc and l are 0 then anyway
-      const float p0 = any ? __builtin_amdgcn_exp2f(my[0] - mn) : 0.f, p1 = any ? __builtin_amdgcn_exp2f(my[UNR - 1] - mn) : 0.f;
-      lOwn = lOwn * corr + (p0 + p1);
-      mOwn = mn;
-      const uint32_t ppOwn = packPair<T>(p0, p1);
-      staticFor<QPK>([&](auto jc) {
-        constexpr int j = decltype(jc)::value;
-        const float cj = quadBroadcast<j>(corr);
-        const uint32_t pp = quadBroadcast<j>(ppOwn);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          acc[j][2 * c] = dotPair<T>(pp, vlo[c], acc[j][2 * c] * cj);
-          acc[j][2 * c + 1] = dotPair<T>(pp, vhi[c], acc[j][2 * c + 1] * cj);
-        }
-      });
-    } else {
 #pragma unroll
     for (int j = 0; j < QPK; ++j) {
       float sc[UNR];
@@ -372,16 +283,9 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
       for (int u = 0; u < UNR; ++u) {
         if constexpr (kNeedK) {
           float d = 0.f;
-          if constexpr (kPairs) {
-            const u32x4 kraw = __builtin_bit_cast(u32x4, kr[u]);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) d = dotPair<T>(qp[j][c], kraw[c], d);
-            d = headRowSum<LPT>(d) * qScale;
-          } else {
-#pragma unroll
-            for (int e = 0; e < N; ++e) d += qf[j][e] * (QPK > 1 ? kf[u][e] : static_cast<float>(kr[u][e]));
-            d = headRowSum<LPT>(d);
-          }
+          for (int e = 0; e < N; ++e) d += qf[j][e] * (QPK > 1 ? kf[u][e] : static_cast<float>(kr[u][e]));
+          d = headRowSum<LPT>(d);
           sc[u] = ok[u] ? d : -INFINITY;
         } else {
           sc[u] = lr[j][u];
@@ -406,14 +310,6 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
           ps += p[u];
         }
         l[j] = l[j] * corr + ps;
-        if constexpr (kPairs) {
-          const uint32_t pp = packPair<T>(p[0], p[UNR - 1]);
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            acc[j][2 * c] = dotPair<T>(pp, vlo[c], acc[j][2 * c] * corr);
-            acc[j][2 * c + 1] = dotPair<T>(pp, vhi[c], acc[j][2 * c + 1] * corr);
-          }
-        } else {
 #pragma unroll
           for (int e = 0; e < N; ++e) {
             float s = acc[j][e] * corr;
@@ -421,10 +317,8 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
             for (int u = 0; u < UNR; ++u) s += p[u] * static_cast<float>(vr[u][e]);
             acc[j][e] = s;
           }
-        }
         m[j] = mn;
       }
-    }
     }
 #pragma unroll
     for (int u = 0; u < UNR; ++u) {
@@ -432,13 +326,6 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
 #pragma unroll
       for (int j = 0; j < QPK; ++j) lr[j][u] = ln[j][u];
     }
-  }
-  if constexpr (kShared) {  // every lane gets the four heads' maxima and sums back for the merges below
-    staticFor<QPK>([&](auto jc) {
-      constexpr int j = decltype(jc)::value;
-      m[j] = quadBroadcast<j>(mOwn);
-      l[j] = quadBroadcast<j>(lOwn);
-    });
   }
   if constexpr (MODE == kTaLogitsOut) {
     if (useLds) {
@@ -502,16 +389,330 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
   }
 }
 
-// out[b,h,:] = merge over the chunks that hold tokens. One wave per (b,h): lane s takes the (max, sum) of
-// split s, a butterfly gives the global max and normaliser, then every lane combines its elements over the
-// splits. Nothing here waits for anything else before it is requested: the sequence length, the (max, sum)
-// pairs and the first eight splits' elements are all loaded up front (splits that hold no tokens were never
-// written; what is read from them is discarded by a select, never multiplied).
+// ------------------------------------------------ grouped-query layouts: the matrix pipe --
+// 16-bit K/V rows shared by 1 to 16 query heads. Cut into lanes (the kernel above), every head costs its own dot
+// products, lane reductions and exponentials per row; here both products of a tile of 16 tokens are matrix products with
+// the heads as columns (unused columns idle: the pipe is busy for 190 of the 1600 cycles a tile's 8 KiB take to arrive).
+// Bound by memory: 128 KiB are in flight on a CU. bf16, 128 per head, sequences of 512 ... 4096 tokens, lanes -> this (us):
+// 48 sequences, 32 query heads on 8 K/V heads: fused 116 -> 91 (5.2 TB/s), scores 59 -> 50, second half 84 -> 57; 64 sequences,
+// 64 heads on 8: 265 -> 130, 131 -> 75, 180 -> 88; fp16, 16 x (64 .. 2048), 32 on 8: 37.5 -> 22.6, 18.7 -> 11.3, 34.8 -> 15.9.
+//   * S^T = K . Q^T (16x16x32): a lane holds four tokens' scores of ONE head, so the softmax runs in the lane, and its
+//     probabilities are, as they lie in the registers, the operand P^T of O^T += V^T . P^T (16x16x32: each probability as
+//     two 16-bit numbers, its rounding and what that leaves, against the same four tokens of V twice; with the rounding
+//     alone the result is 2.3e-3 from 64 bits in bf16, with both 1.66e-3, which is the rounding of the result).
+//   * K and V rows go from the pool straight into LDS (global_load_lds, a lane's own address per 16 bytes, marked
+//     non-temporal: 104 -> 91 us at 48 sequences), in a ring of kGqStages tiles that belongs to one wave: no barriers, only
+//     the wave's own load counter. V stays as it is in memory
+//     and is read through the transposing LDS read.
+//   * the running maximum is replaced only when a score exceeds it by more than 2^8 (harmless in fp32 sums and 16-bit
+//     operands, as in prefill attention), so a tile needs no exchange between lanes at all.
+//   * slots are looked up once per block of tokens and kept in LDS: the ring's loads then wait for nothing.
+constexpr int kGqWaves = 4;
+constexpr int kGqStages = 2;    // tiles of a wave's ring: three leave room for one workgroup per CU instead of two
+constexpr int kGqWgsPerCu = 2;  // what the chunk length aims for
+constexpr int kGqTile = 16;     // tokens per tile
+constexpr int kGqBlock = 128;   // tokens of a wave whose slots (and stored scores) are held in LDS at once
+constexpr int kGqHeads = 16;    // query heads a workgroup serves
+constexpr int kGqScoreRow = kGqBlock + 4;  // floats per head of a wave's stored scores (16 bytes aside per head: no bank conflicts)
+constexpr float kGqRescaleStep = 8.0f;     // log2 domain
+constexpr int gqRingBytes(int d, int matrices) { return kGqWaves * kGqStages * kGqTile * d * 2 * matrices; }
+
+template <typename T>
+struct GqMfma;
+template <>
+struct GqMfma<bf16_t> {
+  typedef bf16x8 Frag;
+  static __device__ __forceinline__ f32x4 run(Frag a, Frag b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+  typedef bf16x4 Quad;
+};
+template <>
+struct GqMfma<half_t> {
+  typedef f16x8 Frag;
+  static __device__ __forceinline__ f32x4 run(Frag a, Frag b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+  typedef f16x4 Quad;
+};
+
+// XOR on the 16-byte piece index of row r in LDS. K: 16 rows' pieces of one index fall on 16 different 16-byte bank groups;
+// V: the 8 rows x 32 bytes that half a wave's transposing read takes fall on 8 different 32-byte ones.
+template <int D>
+__device__ __forceinline__ int gqSwizzleK(int r) { return D >= 128 ? (r & 15) : ((r >> 1) & 7); }
+template <int D>
+__device__ __forceinline__ int gqSwizzleV(int r) { return D >= 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); }
+
+// What the wave's lanes wrote to LDS is read by its other lanes from here on (LDS serves a wave in order).
+__device__ __forceinline__ void exchangeInWave() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+template <int N>
+__device__ __forceinline__ void waitLoadsBut() {  // all but the wave's N youngest vector-memory operations are done
+  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
+}
+
+// D: head size the rows are laid out for (64, 128, 256); a.d is any multiple of 8 up to it: the pieces past the row's end
+// repeat its first one, meet zeros of q, and give output columns that are not stored.
+template <typename T, int D, int MODE, typename LT>
+__global__ __launch_bounds__(kGqWaves * 64) void decodeGroupedKernel(TaArgs a, T* __restrict__ out, float* __restrict__ partial) {
+  using M = GqMfma<T>;
+  using Frag = typename M::Frag;
+  constexpr bool kNeedK = MODE != kTaReduceV, kNeedV = MODE != kTaLogitsOut;
+  constexpr int kMats = MODE == kTaFused ? 2 : 1;
+  constexpr int ROWB = D * 2, CPR = D / 8, RPL = 64 / CPR, NLD = kGqTile / RPL;  // RPL rows per load, NLD loads per matrix and tile
+  constexpr int KS = D / 32, DT = D / 16;
+  constexpr unsigned kMatBytes = kGqTile * ROWB, kStageBytes = kMatBytes * kMats;
+  extern __shared__ __attribute__((aligned(16))) char gqSmem[];
+  __shared__ int slotBuf[kGqWaves][kGqBlock];
+  __shared__ float stateBuf[kGqWaves][2][kGqHeads];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, quad = lane >> 4;  // matrix operands: row / column index, group of k (or of four result rows)
+
+  // One-dimensional grid. A unit is a (K/V head, sequence, chunk); its qGroups workgroups (more than 16 sharers) read the
+  // same rows, so they get consecutive places on one XCD (workgroup ids go round the 8 XCDs). Units go round the XCDs
+  // K/V head fastest, then sequence, chunks from the last to the first.
+  const int f = blockIdx.x, idx = f >> 3;
+  const int g = idx % a.qGroups, u = (idx / a.qGroups) * 8 + (f & 7);
+  if (u >= a.kvHeads * a.batch * a.nsplit) return;  // the grid is rounded up to whole rounds of the XCDs
+  const int kvh = u % a.kvHeads, rest = u / a.kvHeads;
+  const int b = rest % a.batch, split = a.nsplit - 1 - rest / a.batch;
+  const int perKv = a.heads / a.kvHeads, base = perKv / a.qGroups, rem = perKv % a.qGroups;
+  const int h = kvh * perKv + g * base + min(g, rem), nq = base + (g < rem ? 1 : 0);  // the sharers are dealt evenly
+  const int len = min(max((int)ldIndex(a.bLen, b, a.len64), 0), a.maxLen);
+  const int begin = split * a.chunk;
+  if (begin >= len && !(split == 0 && MODE != kTaLogitsOut)) return;  // split 0 still writes zeros for len == 0
+  const int end = min(len, begin + a.chunk);
+  const int64_t locBase = (int64_t)b * a.locRowStride + (a.maxLen - len);
+  LT* scores = nullptr;
+  if constexpr (MODE != kTaFused)
+    scores = static_cast<LT*>(const_cast<void*>(a.logits)) + h * a.logitsHeadStride + ldIndex(a.bStart, b, a.start64);
+
+  const float qScale = MODE == kTaLogitsOut ? a.scaleLog2e / kLog2eTA : a.scaleLog2e;
+  Frag qf[KS];
+  if constexpr (kNeedK) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int e = 32 * s + 8 * quad;
+      const bool have = col < nq && e < a.d;
+      qf[s] = *reinterpret_cast<const Frag*>(reinterpret_cast<const T*>(a.q) + b * a.qBatchStride + (h + (have ? col : 0)) * a.qHeadStride + (have ? e : 0));
+      if (!have) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) qf[s][j] = static_cast<T>(0.f);
+      }
+    }
+  }
+  f32x4 acc[kNeedV ? DT : 1];
+#pragma unroll
+  for (int t = 0; t < (kNeedV ? DT : 1); ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, mRef = 0.f, l = 0.f;  // this lane's head; mRef: what scores are taken against (m, or 0 while there is none)
+
+  // ring: load i of a matrix fills rows i * RPL ... of its tile; lane (row group lane / CPR, piece lane % CPR) fetches the
+  // piece that the swizzle puts in its place
+  const unsigned ring = (unsigned)(uintptr_t)gqSmem + (unsigned)wave * (kGqStages * kStageBytes);
+  int kOff[NLD], vOff[NLD];
+#pragma unroll
+  for (int i = 0; i < NLD; ++i) {
+    const int row = i * RPL + lane / CPR, p = lane % CPR;
+    const int kc = p ^ gqSwizzleK<D>(row), vc = p ^ gqSwizzleV<D>(row);
+    kOff[i] = kc * 8 < a.d ? kc * 8 : 0;
+    vOff[i] = vc * 8 < a.d ? vc * 8 : 0;
+  }
+  const T* kBase = kNeedK ? reinterpret_cast<const T*>(a.k) + kvh * a.kHeadStride : nullptr;
+  const T* vBase = kNeedV ? reinterpret_cast<const T*>(a.v) + kvh * a.vHeadStride : nullptr;
+  int* const slots = slotBuf[wave];
+  float* const stored = reinterpret_cast<float*>(gqSmem + kGqWaves * kGqStages * kStageBytes) + wave * nq * kGqScoreRow;
+  auto issue = [&](int tile, int stage) {
+    const unsigned to = ring + (unsigned)stage * kStageBytes;
+    int slot[NLD];
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) slot[i] = max(slots[tile * kGqTile + i * RPL + lane / CPR], 0);
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      if constexpr (kNeedK) globalLoadToLds16Stream(kBase + (slot[i] * a.kSlotStride + kOff[i]), to + i * 1024u);
+    }
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      if constexpr (kNeedV) globalLoadToLds16Stream(vBase + (slot[i] * a.vSlotStride + vOff[i]), to + (kMats - 1) * kMatBytes + i * 1024u);
+    }
+  };
+
+  const int share = ((end - begin + kGqWaves - 1) / kGqWaves + kGqTile - 1) / kGqTile * kGqTile;  // tokens per wave, whole tiles
+  const int from = begin + wave * share, to = min(end, from + share);
+  for (int b0 = from; b0 < to; b0 += kGqBlock) {
+    const int cnt = min(kGqBlock, to - b0), tiles = (cnt + kGqTile - 1) / kGqTile;
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < kGqBlock / 64; ++i) {
+      const int t = i * 64 + lane;
+      if (t < tiles * kGqTile) {  // past the wave's last token: that token again (its score is masked)
+        const int64_t s = ldIndex(a.bLoc, locBase + b0 + min(t, cnt - 1), a.loc64);
+        const bool in = s >= 0 && s < a.slots;  // slots outside the pool are skipped, never dereferenced
+        slots[t] = in ? (int)s : -1;
+        bad |= !in;
+      }
+    }
+    const bool skips = __builtin_amdgcn_ballot_w64(bad) != 0;
+    if constexpr (MODE == kTaReduceV) {
+      for (int j = 0; j < nq; ++j)
+#pragma unroll
+        for (int i = 0; i < kGqBlock / 64; ++i) {
+          const int t = i * 64 + lane;
+          if (t < cnt) stored[j * kGqScoreRow + t] = static_cast<float>(scores[j * a.logitsHeadStride + b0 + t]) * kLog2eTA;
+        }
+    }
+    exchangeInWave();
+    // (also the reads of the block before: the ring's loads overwrite what they read)
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : : : "memory");
+#pragma unroll
+    for (int s = 0; s < kGqStages - 1; ++s)
+      if (s < tiles) issue(s, s);
+    int stage = 0;
+    for (int t = 0; t < tiles; ++t) {
+      constexpr int kLoads = NLD * kMats;
+      if (t + kGqStages - 1 < tiles) {
+        // the tile read last in that stage has been consumed: its reads are done before the loads that overwrite it go out
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+        issue(t + kGqStages - 1, stage == 0 ? kGqStages - 1 : stage - 1);
+        waitLoadsBut<kLoads * (kGqStages - 1)>();
+      } else {
+        waitLoadsBut<0>();
+      }
+      const unsigned at = ring + (unsigned)stage * kStageBytes;
+      stage = stage + 1 == kGqStages ? 0 : stage + 1;
+      float sc[4];  // tokens 4 quad ... 4 quad + 3 of the tile
+      const int tok = b0 + t * kGqTile + 4 * quad;
+      if constexpr (kNeedK) {
+        typedef __attribute__((address_space(3))) const Frag* LdsFrag;
+        f32x4 s2[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          const Frag kf = *(LdsFrag)(uintptr_t)(at + (unsigned)(col * ROWB + (((4 * s + quad) ^ gqSwizzleK<D>(col)) << 4)));
+          s2[s & 1] = M::run(kf, qf[s], s2[s & 1]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sc[i] = (s2[0][i] + s2[1][i]) * qScale;
+      } else {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(stored + min(col, nq - 1) * kGqScoreRow + t * kGqTile + 4 * quad);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sc[i] = v[i];
+      }
+      if (skips || (t + 1) * kGqTile > cnt) {  // wave-uniform
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (tok + i >= to || slots[t * kGqTile + 4 * quad + i] < 0) sc[i] = -INFINITY;
+      }
+      if constexpr (MODE == kTaLogitsOut) {
+        if (col < nq) *reinterpret_cast<f32x4*>(stored + col * kGqScoreRow + t * kGqTile + 4 * quad) = f32x4{sc[0], sc[1], sc[2], sc[3]};
+      } else {
+        float mt = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
+        if (__builtin_amdgcn_ballot_w64(mt - mRef > kGqRescaleStep || (m == -INFINITY && mt != -INFINITY)) != 0) {
+          auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
+          mt = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+          sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
+          mt = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+          if (mt > m) {
+            const float corr = __builtin_amdgcn_exp2f(m - mt);  // no maximum yet: 0, and the sums are 0
+            m = mRef = mt;
+            l *= corr;
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) acc[d][i] *= corr;
+          }
+        }
+        Frag p;
+        float ps = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float e = __builtin_amdgcn_exp2f(sc[i] - mRef);
+          ps += e;
+          p[i] = static_cast<T>(e);
+          p[4 + i] = static_cast<T>(e - static_cast<float>(p[i]));
+        }
+        l += ps;
+        typedef __attribute__((address_space(3))) s16x4* LdsTr;
+        const int row = 4 * quad + ((lane & 15) >> 2);
+        const unsigned vRow = at + (kMats - 1) * kMatBytes + (unsigned)(row * ROWB + (lane & 1) * 8);
+#pragma unroll
+        for (int d = 0; d < DT; ++d) {
+          const unsigned piece = (unsigned)((2 * d + ((lane & 3) >> 1)) ^ gqSwizzleV<D>(row)) << 4;
+          const typename M::Quad v = __builtin_bit_cast(typename M::Quad, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsTr)(uintptr_t)(vRow + piece)));
+          acc[d] = M::run(__builtin_shufflevector(v, v, 0, 1, 2, 3, 0, 1, 2, 3), p, acc[d]);
+        }
+      }
+    }
+    if constexpr (MODE == kTaLogitsOut) {
+      exchangeInWave();
+      for (int j = 0; j < nq; ++j)
+#pragma unroll
+        for (int i = 0; i < kGqBlock / 64; ++i) {
+          const int t = i * 64 + lane;
+          if (t < cnt) scores[j * a.logitsHeadStride + b0 + t] = static_cast<LT>(stored[j * kGqScoreRow + t]);
+        }
+    }
+  }
+  if constexpr (MODE == kTaLogitsOut) return;
+
+  // merge the waves: every lane group holds its own share of l; O^T lies in the lanes as (head = column, d = row)
+  {
+    auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+    l = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+    sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+    l = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+  }
+  constexpr int kRedRow = D + 4;  // floats per head
+  float* const red = reinterpret_cast<float*>(gqSmem);  // the ring: every load into it has been waited for
+  __syncthreads();
+  if (col < nq) {
+    if (quad == 0) stateBuf[wave][0][col] = m, stateBuf[wave][1][col] = l;
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+      *reinterpret_cast<f32x4*>(red + (wave * nq + col) * kRedRow + 16 * d + 4 * quad) = acc[d];
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < nq * (D / 4); i += kGqWaves * 64) {
+    const int j = i / (D / 4), e = (i % (D / 4)) * 4;
+    if (e >= a.d) continue;
+    float mAll = -INFINITY, lAll = 0.f, w[kGqWaves];
+#pragma unroll
+    for (int k = 0; k < kGqWaves; ++k) mAll = fmaxf(mAll, stateBuf[k][0][j]);
+#pragma unroll
+    for (int k = 0; k < kGqWaves; ++k) {
+      const float mk = stateBuf[k][0][j];
+      w[k] = mk == -INFINITY ? 0.f : exp2f(mk - mAll);
+      lAll += stateBuf[k][1][j] * w[k];
+    }
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < kGqWaves; ++k) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(red + (k * nq + j) * kRedRow + e);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) o[c] += v[c] * w[k];
+    }
+    if (a.nsplit == 1) {
+      const float inv = lAll > 0.f ? 1.f / lAll : 0.f;
+      typename M::Quad r;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) r[c] = static_cast<T>(o[c] * inv);
+      *reinterpret_cast<typename M::Quad*>(out + ((int64_t)b * a.heads + h + j) * a.d + e) = r;
+    } else {
+      float* dst = partial + (((int64_t)b * a.heads + h + j) * a.nsplit + split) * (2 + a.d);
+      if (e == 0) dst[0] = mAll, dst[1] = lAll;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) dst[2 + e + c] = o[c];
+    }
+  }
+}
+
+// out[b,h,:] = merge over the chunks that hold tokens, up to kTaNarrowSplits of them. One wave per (b,h): lane s takes the
+// (max, sum) of split s, a butterfly gives the global max and normaliser, then every lane combines its elements over the
+// splits. Nothing here waits for anything else before it is requested: the sequence length, the (max, sum) pairs and the
+// splits' elements are all loaded up front (splits that hold no tokens were never written; what is read from them is
+// discarded by a select, never multiplied).
 template <typename T>
 __global__ __launch_bounds__(256) void decodeMergeKernel(T* __restrict__ out, const float* __restrict__ partial,
                                                           const void* bLen, bool len64, int64_t pairs, int heads,
                                                           int d, int nsplit, int chunk) {
-  constexpr int kBatch = 8, kMaxPerLane = 4;  // d <= 256
+  constexpr int kMaxPerLane = 4;  // d <= 256
   const int lane = threadIdx.x & 63;
   const int64_t pair = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (pair >= pairs) return;
@@ -524,35 +725,28 @@ __global__ __launch_bounds__(256) void decodeMergeKernel(T* __restrict__ out, co
     ls = src[lane * row + 1];
   }
   const int len = (int)ldIndex(bLen, b, len64);
+  float v[kTaNarrowSplits][kMaxPerLane];
+#pragma unroll
+  for (int u = 0; u < kTaNarrowSplits; ++u) {
+    const float* r = src + (int64_t)min(u, nsplit - 1) * row + 2;
+#pragma unroll
+    for (int k = 0; k < kMaxPerLane; ++k) {
+      const int e = lane + 64 * k;
+      v[u][k] = e < d ? r[e] : 0.f;
+    }
+  }
+  const int used = len <= 0 ? 1 : min(nsplit, (len + chunk - 1) / chunk);
+  if (lane >= used) ms = -INFINITY, ls = 0.f;
+  const float m = waveMax(ms);
+  float wgt = (ms == -INFINITY) ? 0.f : exp2f(ms - m);
+  const float l = waveSum(ls * wgt);
+  wgt *= l > 0.f ? 1.f / l : 0.f;
   float acc[kMaxPerLane] = {0.f, 0.f, 0.f, 0.f};
-  float m = 0.f, wgt = 0.f;
-  int used = 0;
-  for (int sb = 0; sb < nsplit; sb += kBatch) {
-    float v[kBatch][kMaxPerLane];
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const float* r = src + (int64_t)min(sb + u, nsplit - 1) * row + 2;
+  for (int u = 0; u < kTaNarrowSplits; ++u) {
+    const float w = __shfl(wgt, u, 64);
 #pragma unroll
-      for (int k = 0; k < kMaxPerLane; ++k) {
-        const int e = lane + 64 * k;
-        v[u][k] = e < d ? r[e] : 0.f;
-      }
-    }
-    if (sb == 0) {  // the weights of all splits, once, while the loads above are in flight
-      used = len <= 0 ? 1 : min(nsplit, (len + chunk - 1) / chunk);
-      if (lane >= used) ms = -INFINITY, ls = 0.f;
-      m = waveMax(ms);
-      wgt = (ms == -INFINITY) ? 0.f : exp2f(ms - m);
-      const float l = waveSum(ls * wgt);
-      wgt *= l > 0.f ? 1.f / l : 0.f;
-    }
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int sp = sb + u;
-      const float w = __shfl(wgt, sp & 63, 64);
-#pragma unroll
-      for (int k = 0; k < kMaxPerLane; ++k) acc[k] += sp < used ? w * v[u][k] : 0.f;
-    }
+    for (int k = 0; k < kMaxPerLane; ++k) acc[k] += u < used ? w * v[u][k] : 0.f;
   }
 #pragma unroll
   for (int k = 0; k < kMaxPerLane; ++k) {
@@ -561,7 +755,7 @@ __global__ __launch_bounds__(256) void decodeMergeKernel(T* __restrict__ out, co
   }
 }
 
-// The same merge for 65 to 256 splits (few sequences with long contexts, cut fine to fill the chip): one workgroup per
+// The same merge for 9 to 256 splits (few sequences with long contexts, cut fine to fill the chip): one workgroup per
 // (b, h). Every wave works out the weights of all splits (lane s holds splits s, s + 64, s + 128, s + 192), then wave w
 // combines splits w, w + 4, ... and the four sums meet in LDS.
 template <typename T>
@@ -575,15 +769,33 @@ __global__ __launch_bounds__(256) void decodeMergeWideKernel(T* __restrict__ out
   const int b = (int)(pair / heads);
   const int row = 2 + d;
   const float* src = partial + pair * nsplit * row;
+  // the (max, sum) pairs, the first eight splits of this wave and the length are all requested before any is waited for
+  // (rows of splits that hold no tokens were never written: what is read from them is discarded by a select)
+  float ms[kPerLane], ls[kPerLane], wgt[kPerLane], v[kBatch][kMaxPerLane];
+#pragma unroll
+  for (int k = 0; k < kPerLane; ++k) {
+    const int sp = min(lane + 64 * k, nsplit - 1);
+    ms[k] = src[sp * row];
+    ls[k] = src[sp * row + 1];
+  }
+  auto loadBatch = [&](int s0) {
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const float* r = src + (int64_t)min(s0 + 4 * u, nsplit - 1) * row + 2;
+#pragma unroll
+      for (int k = 0; k < kMaxPerLane; ++k) {
+        const int e = lane + 64 * k;
+        v[u][k] = e < d ? r[e] : 0.f;
+      }
+    }
+  };
+  loadBatch(wave);
   const int len = (int)ldIndex(bLen, b, len64);
   const int used = len <= 0 ? 1 : min(nsplit, (len + chunk - 1) / chunk);
-  float ms[kPerLane], ls[kPerLane], wgt[kPerLane];
   float m = -INFINITY;
 #pragma unroll
   for (int k = 0; k < kPerLane; ++k) {
-    const int sp = lane + 64 * k;
-    ms[k] = sp < used ? src[sp * row] : -INFINITY;  // splits that hold no tokens were never written
-    ls[k] = sp < used ? src[sp * row + 1] : 0.f;
+    if (lane + 64 * k >= used) ms[k] = -INFINITY, ls[k] = 0.f;
     m = fmaxf(m, ms[k]);
   }
   m = waveMax(m);
@@ -597,16 +809,7 @@ __global__ __launch_bounds__(256) void decodeMergeWideKernel(T* __restrict__ out
   const float inv = l > 0.f ? 1.f / l : 0.f;
   float acc[kMaxPerLane] = {0.f, 0.f, 0.f, 0.f};
   for (int s0 = wave; s0 < used; s0 += 4 * kBatch) {
-    float v[kBatch][kMaxPerLane];
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const float* r = src + (int64_t)min(s0 + 4 * u, nsplit - 1) * row + 2;
-#pragma unroll
-      for (int k = 0; k < kMaxPerLane; ++k) {
-        const int e = lane + 64 * k;
-        v[u][k] = e < d ? r[e] : 0.f;
-      }
-    }
+    if (s0 != wave) loadBatch(s0);
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       const int sp = s0 + 4 * u, owner = sp >> 6;  // wave-uniform
@@ -831,8 +1034,9 @@ static diopiError_t fillArgs(const TaViews& t, bool needK, bool needV, int maxLe
                 (q.stride[0] * q.itemsize) % 16 == 0 && (q.stride[1] * q.itemsize) % 16 == 0;
   if (needK && needV)
     vector = vector && t.v.aligned16() && (t.v.stride[0] * q.itemsize) % 16 == 0 && (t.v.stride[1] * q.itemsize) % 16 == 0;
-  a->generic = !vector;
-  AMD_CHECK(vector || q.shape[2] <= kTaGenericMaxD, "token attention: head_dim %ld exceeds %d", (long)q.shape[2], kTaGenericMaxD);
+  // (decodeGroupedKernel holds slot numbers in 32 bits)
+  a->generic = !vector || (q.itemsize == 2 && kv.shape[0] > 0x7fffffff);
+  AMD_CHECK(!a->generic || q.shape[2] <= kTaGenericMaxD, "token attention: head_dim %ld exceeds %d", (long)q.shape[2], kTaGenericMaxD);
   a->q = q.data;
   a->k = needK ? t.k.data : nullptr;
   a->v = needV ? t.v.data : nullptr;
@@ -863,18 +1067,20 @@ static diopiError_t fillArgs(const TaViews& t, bool needK, bool needV, int maxLe
   return diopiSuccess;
 }
 
-// Chunk length of the split over a sequence for the streaming kernels (decodeSplitKernel in its three modes).
-static void chooseChunk(TaArgs* a, int64_t groupsPerSeq, int64_t batch, int maxInputLen) {
-  // A workgroup walks its chunk with two loads per wave in flight, so the rate comes from the number of workgroups a
-  // CU holds at once. Few sequences or short ones are cut into smaller chunks until there are about kTaWgsPerCu
-  // workgroups per CU; large batches keep the 512-token chunks, whose partial results are fewer. Measured (us, 32 heads
-  // x 128, bf16, with 512-token chunks -> with these): 1 x 2048 tokens 72 -> 20, 1 x 32768 130 -> 96, 8 x 4096 130 -> 91,
-  // 4 x (100 .. 16384) 123 -> 86, 64 x (256 .. 512) 101 -> 80; 64 x (512 .. 4096) and 256 x (1024 .. 2048) keep their chunks.
+// Chunk length of the split over a sequence (decodeSplitKernel, or decodeGroupedKernel if `grouped`).
+static void chooseChunk(TaArgs* a, int64_t groupsPerSeq, int64_t batch, int maxInputLen, bool grouped) {
+  // A workgroup of the lanes' kernel walks its chunk with two loads per wave in flight, so the rate comes from the number
+  // of workgroups a CU holds at once. Few sequences or short ones are cut into smaller chunks until there are about
+  // kTaWgsPerCu workgroups per CU; large batches keep the 512-token chunks, whose partial results are fewer. Measured (us,
+  // 32 heads x 128, bf16, with 512-token chunks -> with these): 1 x 32768 130 -> 96, 4 x (100 .. 16384) 123 -> 86,
+  // 64 x (256 .. 512) 101 -> 80; 64 x (512 .. 4096) and 256 x (1024 .. 2048) keep their chunks.
+  // The grouped kernel has 128 KiB in flight on a CU with two workgroups and aims for those: against eight, 32 query heads
+  // on 8 K/V heads, 8 x 4096 tokens 37.4 -> 28.8 us, 16 x (64 .. 2048) 27.4 -> 22.8; four: 30.9 and 23.6.
   const int64_t groups = groupsPerSeq * batch, cus = computeUnits(), len = std::max(maxInputLen, 1);
-  const int64_t wantSplits = std::max<int64_t>(1, ceilDiv(kTaWgsPerCu * cus, groups));
+  const int64_t wantSplits = std::max<int64_t>(1, ceilDiv((grouped ? kGqWgsPerCu : kTaWgsPerCu) * cus, groups));
   const int64_t fine = ceilDiv(ceilDiv(len, wantSplits), 64) * 64;
   const int64_t capped = ceilDiv(ceilDiv(len, (int64_t)kTaMaxSplit), 64) * 64;  // at most kTaMaxSplit chunks
-  const int64_t shortest = groups * ceilDiv(len, (int64_t)kTaMinChunk) < cus ? kTaTinyChunk : kTaMinChunk;
+  const int64_t shortest = !grouped && groups * ceilDiv(len, (int64_t)kTaMinChunk) < cus ? kTaTinyChunk : kTaMinChunk;
   a->chunk = (int)std::max(std::max(capped, shortest), std::min<int64_t>(a->chunk, fine));
 }
 
@@ -939,25 +1145,27 @@ static diopiError_t streamChunks(diopiContextHandle_t ctx, hipStream_t stream, T
   // a head row is spanned by 8, 16 or 32 lanes of 16 bytes: the next of 128 / 256 / 512 bytes (the kernel masks the rest)
   const bool partRows = bytes != 128 && bytes != 256 && bytes != 512;
   bytes = bytes <= 128 ? 128 : bytes <= 256 ? 256 : 512;
-  // The lane groups of a wave take consecutive heads of one token when the head count allows it: a wave load is then
-  // one contiguous piece of a slot (1 KiB) instead of head rows of four different slots (431 -> 421 us at batch 64,
-  // 32 heads x 128, 156 043 cached tokens).
-  const int tpw = (int)(64 / std::max<int64_t>(1, bytes / 16));
-  // (the two-call modes keep four tokens of one head per wave load and a workgroup per head: at batch 64, 156 000
-  // tokens, with the chunk's scores staged in LDS either way, four heads per workgroup read 244 against 219 us for the
-  // scores and 238 against 205 us for the second half)
-  // Grouped-query layouts: one read of a K/V row serves four (or two) of the query heads that share it, with their
-  // softmax states side by side in the lane group's registers; more sharers than that are dealt over several
-  // workgroups that run on the same XCD. At batch 64 x (512..4096) tokens, 32 query heads on 8 K/V heads (every query
-  // head used to read the rows for itself): fused 236 -> 157 us, scores 214 -> 74 us, second half 205 -> 106 us; 64
-  // query heads on 8: 405 -> 240 us fused. Sharing factors that are no multiple of four are dealt over the workgroups
-  // as evenly as they go (28 query heads on 4 K/V heads: 4 + 3 per K/V head).
   const int perKv = a.heads / a.kvHeads;
-  const int qpk = perKv >= 3 ? 4 : perKv;  // 1, 2 or 4 query heads per read
+  // Which kernel. 16-bit rows that several query heads share, and the two-call modes, go to the matrix pipe
+  // (decodeGroupedKernel), up to 16 heads per read of a row. A query head that has its K/V head to itself leaves 15 of 16
+  // matrix columns idle; what the lanes of decodeSplitKernel have on it is one contiguous KiB (four heads) per wave load
+  // and token, and that pays once there are many (sequence, head) pairs. Fused, 128 per head, start of this rule -> now (us):
+  // 1 x 1777 tokens x 32 heads 18.8 -> 12.1, 8 x (256 .. 2048) x 40 44.7 -> 40.0, 16 x (1000 .. 4000) x 32 132 -> 117,
+  // 64 x (512 .. 4096) x 8 138 -> 114, 32 x (100 .. 500) x 32 x 64 per head 29.5 -> 20.0; but 24 x (200 .. 1000) x 40
+  // would take 59 against 57, 64 x (512 .. 4096) x 32 426 against 408, and rows of 512 bytes or of other lengths than a
+  // power of two are the lanes' from 128 pairs on (16 x (512 .. 4096) x 16 x 256 per head 114 against 102).
+  const int tpw = (int)(64 / std::max<int64_t>(1, bytes / 16));  // head rows of a wave-wide load
+  const bool lanesPay = MODE == kTaFused && perKv == 1 && a.heads % tpw == 0 &&
+                        (partRows || bytes > 256 || batch * a.heads * bytes > (int64_t)640 * 256);
+  const bool grouped = dtype != diopi_dtype_float32 && !lanesPay;
+  // (fp32: one read of a K/V row serves four, or two, of the query heads that share it, with their softmax states side by
+  // side in the lane group's registers; more sharers are dealt over several workgroups that run on the same XCD, as evenly
+  // as they go)
+  const int qpk = grouped ? kGqHeads : perKv >= 3 ? 4 : perKv;  // query heads per read
   a.qGroups = (perKv + qpk - 1) / qpk;
-  const bool hiw = qpk == 1 && MODE == kTaFused && (bytes == 128 || bytes == 256 || bytes == 512) && a.heads % tpw == 0;
+  const bool hiw = qpk == 1 && MODE == kTaFused && a.heads % tpw == 0;
   const int groupsPerSeq = qpk > 1 ? a.kvHeads * a.qGroups : (hiw ? a.heads / tpw : a.heads);
-  chooseChunk(&a, groupsPerSeq, batch, maxInputLen);
+  chooseChunk(&a, groupsPerSeq, batch, maxInputLen, grouped);
   a.nsplit = (int)std::max<int64_t>(1, ceilDiv(maxInputLen, a.chunk));
   AMD_CHECK(batch <= 65535 && a.nsplit <= 65535, "token attention: batch %ld / splits %d exceed the grid limits", (long)batch,
             a.nsplit);
@@ -984,30 +1192,50 @@ static diopiError_t streamChunks(diopiContextHandle_t ctx, hipStream_t stream, T
     AMD_CHECK(wgs < ((int64_t)1 << 31), "token attention: %ld workgroups exceed the grid limits", (long)wgs);
     grid = dim3((unsigned)wgs, 1, 1);
   }
-#define STREAM_CALL_PART(T, LPT, LT, PART)                                                                                           \
-  if (qpk == 4) hipLaunchKernelGGL((decodeSplitKernel<T, LPT, false, MODE, LT, 4, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial); \
-  else if (qpk == 2) hipLaunchKernelGGL((decodeSplitKernel<T, LPT, false, MODE, LT, 2, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial); \
-  else if (hiw) hipLaunchKernelGGL((decodeSplitKernel<T, LPT, true, MODE, LT, 1, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial); \
-  else hipLaunchKernelGGL((decodeSplitKernel<T, LPT, false, MODE, LT, 1, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial)
-#define STREAM_CALL_AS(T, LPT, LT)            \
-  if (partRows) {                             \
-    STREAM_CALL_PART(T, LPT, LT, true);       \
-  } else {                                    \
-    STREAM_CALL_PART(T, LPT, LT, false);      \
+  if (grouped) {
+    const int mats = MODE == kTaFused ? 2 : 1, d = (int)(bytes / 2);
+    const int lds = gqRingBytes(d, mats) + (MODE == kTaFused ? 0 : kGqWaves * std::min(perKv, kGqHeads) * kGqScoreRow * (int)sizeof(float));
+#define GROUPED_CALL_AS(T, D, LT)                                                                                               \
+  do {                                                                                                                          \
+    AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(decodeGroupedKernel<T, D, MODE, LT>), lds));                           \
+    hipLaunchKernelGGL((decodeGroupedKernel<T, D, MODE, LT>), grid, dim3(kGqWaves * 64), lds, stream, a, static_cast<T*>(outPtr), \
+                       partial);                                                                                                \
+  } while (0)
+#define GROUPED_CALL(T, D)                          \
+  if (MODE == kTaFused || scoresF32) {              \
+    GROUPED_CALL_AS(T, D, float);                   \
+  } else {                                          \
+    GROUPED_CALL_AS(T, D, T);                       \
   }
-#define STREAM_CALL(T, LPT)                                \
-  if (MODE == kTaFused || scoresF32) {                     \
-    STREAM_CALL_AS(T, LPT, float);                         \
-  } else {                                                 \
-    STREAM_CALL_AS(T, LPT, T);                             \
+#define GROUPED_SIZES(T) \
+  if (d == 64) { GROUPED_CALL(T, 64) } else if (d == 128) { GROUPED_CALL(T, 128) } else { GROUPED_CALL(T, 256) }
+    if (dtype == diopi_dtype_bfloat16) { GROUPED_SIZES(bf16_t) } else { GROUPED_SIZES(half_t) }
+#undef GROUPED_SIZES
+#undef GROUPED_CALL
+#undef GROUPED_CALL_AS
+  } else {
+#define STREAM_CALL_AS(T, LPT, PART)                                                                                                           \
+  if constexpr (sizeof(T) == 4) { /* stored scores have the type of q */                                                                       \
+    if (qpk == 4) hipLaunchKernelGGL((decodeSplitKernel<T, LPT, false, MODE, T, 4, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial); \
+    else if (qpk == 2) hipLaunchKernelGGL((decodeSplitKernel<T, LPT, false, MODE, T, 2, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial); \
+    else if (hiw) hipLaunchKernelGGL((decodeSplitKernel<T, LPT, true, kTaFused, T, 1, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial); \
+    else hipLaunchKernelGGL((decodeSplitKernel<T, LPT, false, MODE, T, 1, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial);  \
+  } else {                                                                                                                                     \
+    hipLaunchKernelGGL((decodeSplitKernel<T, LPT, true, kTaFused, float, 1, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial); \
   }
-  TA_DISPATCH(dtype, bytes, STREAM_CALL);
+#define STREAM_CALL(T, LPT)          \
+  if (partRows) {                    \
+    STREAM_CALL_AS(T, LPT, true);    \
+  } else {                           \
+    STREAM_CALL_AS(T, LPT, false);   \
+  }
+    TA_DISPATCH(dtype, bytes, STREAM_CALL);
 #undef STREAM_CALL
 #undef STREAM_CALL_AS
-#undef STREAM_CALL_PART
+  }
   AMD_LAUNCH_CHECK();
   if (MODE == kTaLogitsOut) return diopiSuccess;
-  if (a.nsplit > 64) {
+  if (a.nsplit > kTaNarrowSplits) {
     const int64_t pairs = batch * a.heads;
     AMD_CHECK(a.nsplit <= kTaMaxSplit && a.d <= 256, "token attention: %d splits of head size %d cannot be merged", a.nsplit, a.d);
 #define MERGE_WIDE_CALL(T, LPT)                                                                                                      \

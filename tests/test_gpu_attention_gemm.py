@@ -892,6 +892,51 @@ def test_token_attention_grouped_query_layouts(ops, dev, heads, kvh, dtype, d, i
         assert_half(out3, want, rel=3e-2, abs_=2e-2)   # softmax of scores rounded to 8 (11) bits
 
 
+@pytest.mark.parametrize("heads,kvh,d,dtype", [
+    (5, 5, 128, torch.bfloat16),     # a head count that is no multiple of four heads per wave load: the matrix pipe at any batch
+    (8, 8, 64, torch.float16),       # few pairs of whole rows
+    (16, 1, 128, torch.float16),     # all 16 columns of the products in use
+    (17, 1, 128, torch.bfloat16),    # two workgroups of 9 and 8 heads
+    (6, 2, 8, torch.float16),        # one 16-byte piece per row
+    (4, 2, 200, torch.bfloat16),     # rows laid out for 512 bytes
+    (2, 1, 256, torch.float16),
+])
+def test_token_attention_tiles_of_sixteen_tokens(ops, dev, heads, kvh, d, dtype):
+    """Sequence lengths around the edges of a tile (16 tokens), of a wave's and of a workgroup's share, scores that grow by
+    more than 2^8 along a sequence (the running maximum has to follow), and slots outside the pool, which are skipped."""
+    lens = [1, 15, 16, 17, 63, 64, 65, 127, 129, 511, 513, 0]
+    slots, width, total = 1500, 513, sum(lens)
+    kp = torch.randn(slots, kvh, d, generator=g(60)).to(dtype)
+    vp = torch.randn(slots, kvh, d, generator=g(61)).to(dtype)
+    q = (3 * torch.randn(len(lens), heads, d, generator=g(62))).to(dtype)
+    b_loc = torch.zeros(len(lens), width, dtype=torch.int32)
+    for b, n in enumerate(lens):
+        b_loc[b, width - n:] = torch.randperm(slots, generator=g(63 + b))[:n].to(torch.int32)
+    kp[b_loc[9, width - 100:].long()] *= 6          # the last 100 tokens of the sequence of 511
+    ln = torch.tensor(lens, dtype=torch.int32)
+    st = torch.zeros(len(lens), dtype=torch.int32)
+    st[1:] = torch.cumsum(ln, 0)[:-1]
+    want = oracle.token_attention(q[:-1].float(), kp.float(), vp.float(), b_loc[:-1], ln[:-1], width)
+    args = (b_loc.to(dev), st.to(dev), ln.to(dev), width)
+    got = ops.token_decode_attention(q.to(dev), kp.to(dev), vp.to(dev), *args)
+    assert_half(got[:-1], want)
+    assert_exact(got[-1].cpu(), torch.zeros(heads, d, dtype=dtype))
+    assert_exact(ops.token_decode_attention(q.to(dev), kp.to(dev), vp.to(dev), *args, no_alloc=True), got.cpu())
+    att = torch.full((heads, total), float("nan"), dtype=torch.float32, device=dev)
+    ops.token_attention(q.to(dev), kp.to(dev), att, *args)
+    assert_fp32(att, oracle.token_logits(q, kp, b_loc, st, ln, width, total), rel=1e-5)
+    out2 = torch.empty_like(got)
+    ops.token_softmax_reducev(att, vp.to(dev), out2, *args)
+    assert_half(out2[:-1], want)
+    # the sequence of 65 tokens without every third one: as if it were the shorter sequence
+    bad = b_loc.clone()
+    bad[6, width - 65::3] = torch.tensor([-1, slots] * 11, dtype=torch.int32)
+    kept = b_loc[6, width - 65:][torch.arange(65) % 3 != 0]
+    short = oracle.token_attention(q[6:7].float(), kp.float(), vp.float(), kept[None], torch.tensor([len(kept)]), len(kept))
+    got = ops.token_decode_attention(q.to(dev), kp.to(dev), vp.to(dev), bad.to(dev), *args[1:])
+    assert_half(got[6:7], short)
+
+
 # ------------------------------------------------------------------ int8 weight-only linear
 @pytest.mark.parametrize("m", [1, 4, 16, 33])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
