@@ -1204,7 +1204,11 @@ __device__ __forceinline__ void accRegisters16(f32x4 (&f)[4]) {
 // tailReduceKernel adds the slices of a tile and applies the epilogue. (A reduction by the workgroup that finishes last
 // would run on R compute units, each at the rate one of them can read.) The slices are dealt out slice by slice, so the
 // workgroups of one XCD read the same stretch of K of neighbouring tiles.
-template <typename T, int EPI, bool SPLIT = false>
+// W8: the second operand is int8 (rows of g.ldb bytes), converted to T between the MFMAs; see gen_gemm_loop_4wave.py. B's two
+// LDS stages then hold pairs of K tiles. Bound as the 16-bit form is, by the MFMA rate with few rows and by power with
+// many, where the conversions (192 vector instructions per 128 MFMAs) cost up to 7 %; what it saves is the pass that wrote the
+// weights out in 16 bits and the reads of that (882 x 27648 x 5120 300 -> 239 us, 256 x 22016 x 4096 113 -> 65).
+template <typename T, int EPI, bool SPLIT = false, bool W8 = false>
 __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
   constexpr int BM = 256, BN = 256, WM = 128, WN = 128, TM = 8, TN = 8;
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -1239,15 +1243,16 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
   };
   const int batch = blockIdx.z;
   const T* A = reinterpret_cast<const T*>(g.A) + (int64_t)batch * g.sAb;
-  const T* B = reinterpret_cast<const T*>(g.B) + (int64_t)batch * g.sBb;
+  constexpr int kBytesB = W8 ? 1 : 2;
+  const char* B = reinterpret_cast<const char*>(g.B) + (int64_t)batch * g.sBb * kBytesB;
   // Rows past M / N and columns past K lie beyond the descriptors' extent and read as zeros.
-  auto descriptor = [](const T* base, int64_t bytes) {
+  auto descriptor = [](const void* base, int64_t bytes) {
     const uint64_t p = reinterpret_cast<uint64_t>(base);
     u32x4 d = {(uint32_t)p, (uint32_t)(p >> 32) & 0xffffu, (uint32_t)bytes, 0x00020000u};
     return d;
   };
   const u32x4 rsA = descriptor(A, ((int64_t)(g.M - 1) * g.lda + g.K) * 2);
-  const u32x4 rsB = descriptor(B, ((int64_t)(g.N - 1) * g.ldb + g.K) * 2);
+  const u32x4 rsB = descriptor(B, ((int64_t)(g.N - 1) * g.ldb + g.K) * kBytesB);
   // lane l of a wave fills the l-th 16-byte slot of a 1 KiB block (8 rows of 128 bytes); the chunk swizzle
   // c ^ ((row >> 1) & 7) is applied to the global address. A pass of the workgroup covers 32 rows.
   constexpr unsigned kFar = 0x80000000u;  // beyond every extent: the load returns zeros
@@ -1273,12 +1278,12 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
     // return in order)
     const int t = waveS * 64 + laneNow();
     const int srow = t >> 3;
-    const int c8 = ((t & 7) ^ ((srow >> 1) & 7)) * 8;
+    const int c16 = ((t & 7) ^ ((srow >> 1) & 7)) * 16;  // bytes
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int ra = tm * BM + srow + 32 * i, rb = tn * BN + srow + 32 * i;
-      voA[i] = ra < g.M ? (unsigned)(((int64_t)ra * g.lda + c8 + k0) * 2) : kFar;
-      voB[i] = rb < g.N ? (unsigned)(((int64_t)rb * g.ldb + c8 + k0) * 2) : kFar;
+      voA[i] = ra < g.M ? (unsigned)(((int64_t)ra * g.lda + k0) * 2 + c16) : kFar;
+      voB[i] = rb < g.N ? (unsigned)(((int64_t)rb * g.ldb + k0) * kBytesB + c16) : kFar;
     }
   };
   const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem;
@@ -1307,6 +1312,28 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
     else                                                                         \
       asm volatile(GEMM4W_##NAME##_F16 GEMM4W_OPERANDS);                         \
   } while (0)
+  // int8: the LDS addresses in B's stage of pair p of the item (fragment bytes of the pair's tile h and k-step ks)
+  unsigned kcurB = 0;
+  auto addressB = [&](int p, int h, int ks) {
+    return base + 65536u + (unsigned)(p & 1) * 32768u + (unsigned)((wn * WN + frow) * 128 + (((4 * h + 2 * ks + (kq >> 1)) ^ swz) << 4) + (kq & 1) * 8);
+  };
+#define GEMM4W_W8_OPERANDS(P)                                                                                        \
+  : [kcur] "+s"(kcur), [kcurB] "+s"(kcurB), [m0s] "+s"(m0s)                                                          \
+  : [voA0] "v"(voA[0]), [voA1] "v"(voA[1]), [voA2] "v"(voA[2]), [voA3] "v"(voA[3]), [voA4] "v"(voA[4]),              \
+    [voA5] "v"(voA[5]), [voA6] "v"(voA[6]), [voA7] "v"(voA[7]), [voB0] "v"(voB[0]), [voB1] "v"(voB[1]),              \
+    [voB2] "v"(voB[2]), [voB3] "v"(voB[3]), [voB4] "v"(voB[4]), [voB5] "v"(voB[5]), [voB6] "v"(voB[6]),              \
+    [voB7] "v"(voB[7]), [adA0] "v"(adA0), [adA1] "v"(adA1), [adB00] "v"(addressB(P, 0, 0)),                          \
+    [adB01] "v"(addressB(P, 0, 1)), [adB10] "v"(addressB(P, 1, 0)), [adB11] "v"(addressB(P, 1, 1)),                  \
+    [adN00] "v"(addressB((P) + 1, 0, 0)), [rsA] "s"(rsA), [rsB] "s"(rsB), [lds] "s"(ldsWave),                        \
+    [ldsB] "s"(ldsWave + 65536u + (unsigned)((P) & 1) * 32768u), [sel] "s"(0x07060302)                               \
+  : "memory", "scc", GEMM4W_W8_CLOBBERS
+#define GEMM4W_W8_RUN(NAME, P)                                                   \
+  do {                                                                           \
+    if constexpr (std::is_same<T, bf16_t>::value)                                \
+      asm volatile(GEMM4W_W8_##NAME##_BF16 GEMM4W_W8_OPERANDS(P));               \
+    else                                                                         \
+      asm volatile(GEMM4W_W8_##NAME##_F16 GEMM4W_W8_OPERANDS(P));                \
+  } while (0)
   int pid = blockIdx.x, tm, tn, slot = -1, itemPairs = pairs, k0 = 0;
   tileOf(pid, tm, tn, slot);
   if constexpr (SPLIT) {
@@ -1315,11 +1342,20 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
   laneOffsets(tm, tn, k0 * 2 * kBK);
   bool first = true;
   while (true) {
-    if (first)
-      GEMM4W_RUN(PROLOGUE);
-    else
-      GEMM4W_RUN(PROLOGUE_LOADED);
-    for (int p = 1; p < itemPairs; ++p) GEMM4W_RUN(BODY);
+    if constexpr (W8) {
+      if (first)
+        GEMM4W_W8_RUN(PROLOGUE, 0);
+      else
+        GEMM4W_W8_RUN(PROLOGUE_LOADED, 0);
+      for (int p = 0; p + 2 < itemPairs; ++p) GEMM4W_W8_RUN(BODY, p);
+      if (itemPairs > 1) GEMM4W_W8_RUN(BODY_LAST, itemPairs - 2);  // (loads no pair past the item's last)
+    } else {
+      if (first)
+        GEMM4W_RUN(PROLOGUE);
+      else
+        GEMM4W_RUN(PROLOGUE_LOADED);
+      for (int p = 1; p < itemPairs; ++p) GEMM4W_RUN(BODY);
+    }
     // (rotary tables through LDS: this output tile's entries are copied now, behind every tile load of its K loop; tiles
     // of v heads need none; the decision is the same for the whole workgroup)
     if constexpr (EPI == kEpiRotaryLds) {
@@ -1338,9 +1374,15 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
         if (nslot >= 0) npairs = slicePairs(nslot, &nk0);
       }
       laneOffsets(ntm, ntn, nk0 * 2 * kBK);
-      GEMM4W_RUN(TAIL_NEXT);
+      if constexpr (W8)
+        GEMM4W_W8_RUN(TAIL_NEXT, itemPairs - 1);
+      else
+        GEMM4W_RUN(TAIL_NEXT);
     } else {
-      GEMM4W_RUN(TAIL);
+      if constexpr (W8)
+        GEMM4W_W8_RUN(TAIL, itemPairs - 1);
+      else
+        GEMM4W_RUN(TAIL);
     }
     if constexpr (SPLIT) {
       if (slot >= 0) {
@@ -1392,6 +1434,8 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
     pid = next, tm = ntm, tn = ntn, first = false;
     if constexpr (SPLIT) slot = nslot, itemPairs = npairs;
   }
+#undef GEMM4W_W8_RUN
+#undef GEMM4W_W8_OPERANDS
 #undef GEMM4W_RUN
 #undef GEMM4W_OPERANDS
 }
@@ -2594,7 +2638,7 @@ static TailSplit tailSplit(int64_t tiles, int64_t pairs, int resident) {
   return best;
 }
 
-template <typename T, int EPI>
+template <typename T, int EPI, bool W8 = false>
 static diopiError_t launchTailSplit(hipStream_t stream, MfmaArgs g, const TailSplit& tail, int resident, void* ws) {
   const int rest = g.tilesM * g.tilesN - tail.whole, items = rest * tail.slices;
   g.partial = static_cast<float*>(ws), g.wholeTiles = tail.whole, g.kSlices = tail.slices;
@@ -2602,8 +2646,8 @@ static diopiError_t launchTailSplit(hipStream_t stream, MfmaArgs g, const TailSp
   const dim3 grid((unsigned)(tail.whole ? resident : std::min(items, resident)));
   constexpr size_t lds = 2 * (size_t)(256 + 256) * kBK * sizeof(T) +
                          (EPI == kEpiRotaryLds ? kRotaryLdsBytes : EPI == kEpiAddendLds ? kAddendLdsBytes : 0);
-  AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(&gemmMfma4WaveKernel<T, EPI, true>), (int)lds));
-  hipLaunchKernelGGL((gemmMfma4WaveKernel<T, EPI, true>), grid, dim3(256), lds, stream, g);
+  AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(&gemmMfma4WaveKernel<T, EPI, true, W8>), (int)lds));
+  hipLaunchKernelGGL((gemmMfma4WaveKernel<T, EPI, true, W8>), grid, dim3(256), lds, stream, g);
   AMD_LAUNCH_CHECK();
   constexpr int kReduceEpi = EPI == kEpiRotaryLds ? (int)kEpiRotaryUniform : EPI == kEpiAddendLds ? (int)kEpiLinear : EPI;
   hipLaunchKernelGGL((tailReduceKernel<T, kReduceEpi>), dim3((unsigned)(rest * 4)), dim3(256), 0, stream, g);
@@ -2664,6 +2708,9 @@ static diopiError_t launchMfmaPipelined(diopiContextHandle_t ctx, hipStream_t st
           if constexpr (EPI == kEpiLinear) {
             if (p.Cin) return launchTailSplit<T, kEpiAddendLds>(stream, g, tail, resident, ws);
           }
+          if constexpr (EPI == kEpiColScale) {
+            if (p.int8B) return launchTailSplit<T, EPI, true>(stream, g, tail, resident, ws);
+          }
           return launchTailSplit<T, EPI>(stream, g, tail, resident, ws);
         }
       }
@@ -2679,8 +2726,12 @@ static diopiError_t launchMfmaPipelined(diopiContextHandle_t ctx, hipStream_t st
         }
       }
       constexpr size_t lds4 = lds + (EPI == kEpiRotaryLds ? kRotaryLdsBytes : 0);  // (160 KiB with the rotary tables: all of a CU's)
-      AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(&gemmMfma4WaveKernel<T, EPI>), (int)lds4));
-      hipLaunchKernelGGL((gemmMfma4WaveKernel<T, EPI>), grid, dim3(256), lds4, stream, g);
+      auto* kernel = &gemmMfma4WaveKernel<T, EPI>;
+      if constexpr (EPI == kEpiColScale) {
+        if (p.int8B) kernel = &gemmMfma4WaveKernel<T, EPI, false, true>;
+      }
+      AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(kernel), (int)lds4));
+      hipLaunchKernelGGL(kernel, grid, dim3(256), lds4, stream, g);
       AMD_LAUNCH_CHECK();
       return diopiSuccess;
     }
@@ -3004,9 +3055,14 @@ static bool tailSplitPays(const GemmProblem& p) {
 // Settles whether a product with too few 256 x 256 tiles goes to K slices of them, and reserves the workspace without which
 // that form loses: unsplit, 40 tiles (400 x 5120 x 13824) take 257 us on 40 compute units and the 128 x 128 form 146.
 static bool reserveTail(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem* p) {
-  if (!tailSplitPays(*p)) return false;
+  // int8 weights: the other form is an expansion, a 128 x 128 product and a pass that scales its result, and the slices win
+  // from 2^24 weights on (256 x 4096 x 4096 36 -> 33 us, 600 x 5120 x 13824 140 -> 102; 256 x 3072 x 1024 24 against 26)
+  const bool always = p->int8B && p->N * p->K >= ((int64_t)1 << 24);
+  if (!always && !tailSplitPays(*p)) return false;
   const int64_t tiles = ceilDiv(p->M, 256) * ceilDiv(p->N, 256);
-  p->tailSlots = spareWorkspace(ctx, stream, tiles * tailSplit(tiles, p->K / (2 * kBK), computeUnits() / 8 * 8).slices * kTailSlotFloats * 4);
+  const TailSplit split = tailSplit(tiles, p->K / (2 * kBK), computeUnits() / 8 * 8);
+  if (split.slices == 1 || split.whole != 0) return false;
+  p->tailSlots = spareWorkspace(ctx, stream, tiles * split.slices * kTailSlotFloats * 4);
   return p->tailSlots != nullptr;
 }
 

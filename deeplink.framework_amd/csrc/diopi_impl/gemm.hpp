@@ -29,6 +29,8 @@ struct GemmProblem {
   diopiDtype_t colScaleDtype = diopi_dtype_float32;
   const void* colBias = nullptr;
   diopiDtype_t colBiasDtype = diopi_dtype_float32;
+  // B holds int8 (strides in bytes, rows at multiples of 16), converted to `dtype` on the way into the product; with colScale only.
+  bool int8B = false;
   // Workspace for K slices of 256 x 256 tiles, held once it is settled that the product takes that form (reserveTail in
   // gemm.hip). Not for callers to set.
   void* tailSlots = nullptr;

@@ -38,7 +38,20 @@ the same number of fragment reads) takes 1.5 % fewer cycles and 9 % more time (5
 instruction reads and writes twice the accumulator registers per multiply-add, and at the power limit this is paid in
 clock. Register-only loops of either instruction over the whole chip (no memory traffic at all) sustain 2160 TFLOP/s at
 2.12 GHz (16x16x32, 16.4 cycles per instruction) against 1940 TFLOP/s at 1.87 GHz (32x32x16, 32.4 cycles): the first
-figure is the ceiling that the power limit leaves to any bf16 GEMM here, 0.86 of the nominal peak."""
+figure is the ceiling that the power limit leaves to any bf16 GEMM here, 0.86 of the nominal peak.
+
+The form for int8 weights (the macros with W8): the second operand lies in LDS as it does in memory, rows of 128 bytes that are
+the K of a PAIR of tiles, so its loads (8 per pair instead of 16) and its two stages go by pairs, and a load still fetches
+whole 128-byte lines. A lane reads the 8 bytes of a fragment (ds_read_b64, K order and swizzle as in the 16-bit form: half
+the LDS bytes) into v[104:119] and converts them between the MFMAs of the k-step before the one that needs them, exactly:
+bf16 by a conversion to fp32 per byte and a permutation that joins two high halves (12 instructions a fragment), fp16 by one
+conversion per byte into the half it belongs to (8). The matrix pipe leaves room for three vector instructions an MFMA and
+this takes one and a half of it. Of each k-step's reads the raw ones come first:
+  k-step 0, MFMAs 0-15    raw B0..B7, then A0..A7 of k-step 1 | 23-62  the conversions (all reads are done at B1)
+  k-step 1, MFMAs 65-95   raw B0..B7, then A0..A7 of the next tile's k-step 0, one per two MFMAs | 79-126 the conversions
+Operands besides those above: %[adB01] %[adB10] %[adB11] LDS addresses in this pair's stage of (tile of the pair, k-step),
+%[adN00] of the first in the next pair's stage; %[kcurB] K byte offset of the pair whose B loads come next, %[ldsB] LDS address of
+this wave's 1 KiB slot in this pair's stage, %[sel] the permutation's selector."""
 import os
 import sys
 
@@ -158,6 +171,158 @@ def prologue(out, issue_loads):
         read_fragment(out, kind, idx, 0, 0, 0)
 
 
+RAW0, TMP0 = 104, 100   # raw bytes of a k-step's 8 fragments (2 registers each); 4 temporaries
+KINDS8 = [("B", j) for j in range(8)] + [("A", i) for i in range(8)]
+
+
+def convert(kind, buf, j):
+    """The instructions that turn the raw bytes of fragment j into buffer buf."""
+    d, r = VB0 + buf * 32 + j * 4, RAW0 + 2 * j
+    ops = []
+    if kind == "F16":
+        for half in (0, 1):      # (a register's two halves well apart: the second write keeps the first)
+            for q in range(4):
+                b = 2 * q + half
+                unused = "UNUSED_PAD" if half == 0 else "UNUSED_PRESERVE"
+                ops.append(f"v_cvt_f16_i16_sdwa v{d + q}, sext(v{r + b // 4}) dst_sel:WORD_{half} dst_unused:{unused} src0_sel:BYTE_{b % 4}")
+    else:
+        for q in range(4):
+            t = TMP0 + 2 * (q % 2)
+            for half in (0, 1):
+                b = 2 * q + half
+                ops.append(f"v_cvt_f32_i32_sdwa v{t + half}, sext(v{r + b // 4}) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_{b % 4}")
+            ops.append(f"v_perm_b32 v{d + q}, v{t + 1}, v{t}, %[sel]")
+    return ops
+
+
+def read8(out, kind, idx, buf, stage, ks, ad):
+    """Fragment read of the int8 form; ad: the address operand of B."""
+    if kind == "A":
+        read_fragment(out, "A", idx, buf, stage, ks)
+    else:
+        out.append(f"ds_read_b64 v[{RAW0 + 2 * idx}:{RAW0 + 2 * idx + 1}], %[{ad}] offset:{idx * 2048}")
+
+
+def m0_8(out, load, s):
+    kind, d, stage = load
+    if kind == "A":
+        load_m0(out, d, s if stage is None else stage)
+    elif stage is None:
+        out.append(f"s_add_u32 m0, %[ldsB], {d * 4096}")
+    else:
+        load_m0(out, 8 + d, stage)
+
+
+def issue8(out, load):
+    kind, d, _ = load
+    k = "kcur" if kind == "A" else "kcurB"
+    out.append(f"buffer_load_dwordx4 %[vo{kind}{d}], %[rs{kind}], %[{k}] offen lds")
+    if d == 7:
+        out.append(f"s_add_u32 %[{k}], %[{k}], 128")
+
+
+def tile8(out, kind, h, load_a, load_b, younger, next_tile, next_output=False):
+    """One K tile of the int8 form, the pair's tile h (its stage of A too). load_a: issue the A loads of tile t + 2, load_b: then
+    the B loads of the pair after the next (h == 1); younger: loads issued before this tile that its B2 may leave in flight."""
+    after = {m: [] for m in range(128)}
+    for r in range(16):
+        after[r].append(("read", (r, 1, h, 1, f"adB{h}1")))
+    after[B1_SLOT].append(("B1", None))
+    loads = [("A", d, None) for d in range(8)] * load_a + [("B", d, None) for d in range(8)] * load_b
+    step = LOAD_STEP
+    if next_output:
+        after[B1_SLOT].append(("rewind", None))
+        loads = [("A", d, 0) for d in range(8)] + [("B", d, 0) for d in range(8)] + [("A", d, 1) for d in range(8)] + [("B", d, 1) for d in range(8)]
+        step = 3
+    before_b2 = younger
+    for n, load in enumerate(loads):
+        slot = B1_SLOT + 1 + n * step
+        before_b2 += slot + 1 <= 63
+        after[slot].append(("m0", load))
+        after[slot + 1].append(("load", load))
+    vector = {m: [] for m in range(128)}
+    for j in range(8):
+        ops = convert(kind, 1, j)
+        for n, op in enumerate(ops):
+            vector[23 + 5 * j + n * 5 // len(ops)].append(op)
+    if next_tile:
+        for r in range(16):
+            after[65 + 2 * r].append(("read", (r, 0, h ^ 1, 0, "adB10" if h == 0 else "adN00")))
+        for j in range(8):
+            first, ops = 79 + 6 * j, convert(kind, 0, j)
+            issued = min(16, (first - 65 + 1) // 2)      # reads issued behind MFMAs before `first`
+            vector[first].append(f"s_waitcnt lgkmcnt({issued - j - 1})")
+            for n, op in enumerate(ops):
+                vector[first + n * 6 // len(ops)].append(op)
+    for m in range(128):
+        ks, mm = divmod(m, 64)
+        j, pos = divmod(mm, 8)
+        i = pos if j % 2 == 0 else 7 - pos
+        if m == 0:
+            out.append("s_waitcnt lgkmcnt(0)")           # A0..A7 of buffer 0, read at the latest 32 MFMAs ago
+        if m == 64 and next_tile:
+            out.append(f"s_waitcnt vmcnt({before_b2}) lgkmcnt(0)")
+            out.append("s_barrier")
+        out.append(f"MFMA {acc(i, j)}, {vb(ks, j)}, {va(ks, i)}, {acc(i, j)}")
+        out += vector[m]
+        for what, arg in after[m]:
+            if what == "read":
+                r, buf, stage, rks, ad = arg
+                read8(out, KINDS8[r][0], KINDS8[r][1], buf, stage, rks, ad)
+            elif what == "B1":
+                out.append("s_waitcnt lgkmcnt(0)")
+                out.append("s_barrier")
+            elif what == "m0":
+                m0_8(out, arg, h)
+            elif what == "rewind":
+                out.append("s_mov_b32 %[kcur], 0")
+                out.append("s_mov_b32 %[kcurB], 0")
+            else:
+                issue8(out, arg)
+
+
+def prologue8(out, kind, issue_loads):
+    """As prologue(); K tile 0 is A's first 8 loads and B's first pair, and K tile 1 and the second pair are the 16 after them."""
+    out.append("s_mov_b32 %[m0s], m0")
+    if issue_loads:
+        for stage in (0, 1):
+            for load in [("A", d, stage) for d in range(8)] + [("B", d, stage) for d in range(8)]:
+                m0_8(out, load, 0)
+                out.append("s_nop 0")
+                issue8(out, load)
+    for r in range(256):
+        out.append(f"v_accvgpr_write_b32 a{r}, 0")
+    out.append("s_waitcnt vmcnt(16)")
+    out.append("s_barrier")
+    for k, idx in KINDS8:
+        read8(out, k, idx, 0, 0, 0, "adB00")
+    out.append("s_waitcnt lgkmcnt(8)")
+    for j in range(8):
+        out += convert(kind, 0, j)
+
+
+def main8(text):
+    for kind, mnemonic in (("BF16", "v_mfma_f32_16x16x32_bf16"), ("F16", "v_mfma_f32_16x16x32_f16")):
+        pro, proc, body, last, tail, tailn = [], [], [], [], [], []
+        prologue8(pro, kind, True)
+        prologue8(proc, kind, False)
+        # B2 of a pair's first tile waits for the A loads of the tile before it; that tile's B loads, issued behind them, are
+        # waited for by B2 of the second
+        tile8(body, kind, 0, True, False, 8, True)
+        tile8(body, kind, 1, True, True, 0, True)
+        tile8(last, kind, 0, True, False, 8, True)
+        tile8(last, kind, 1, True, False, 0, True)
+        for t, nxt in ((tail, False), (tailn, True)):
+            tile8(t, kind, 0, False, False, 0, True)
+            tile8(t, kind, 1, False, False, 0, False, nxt)
+            t += ["s_nop 15", "s_nop 15", "s_mov_b32 m0, %[m0s]"]
+        for name, lines in (("PROLOGUE", pro), ("PROLOGUE_LOADED", proc), ("BODY", body), ("BODY_LAST", last), ("TAIL", tail), ("TAIL_NEXT", tailn)):
+            text.append(f"#define GEMM4W_W8_{name}_{kind} \\\n")
+            text.append(" \\\n".join('  "' + l.replace("MFMA", mnemonic) + '\\n\\t"' for l in lines) + "\n\n")
+    clobbers = ", ".join(f'"v{r}"' for r in range(TMP0, VA0))
+    text.append(f"#define GEMM4W_W8_CLOBBERS {clobbers}, GEMM4W_CLOBBERS\n")
+
+
 def main():
     pro, proc, body, tail, tailn = [], [], [], [], []
     prologue(pro, True)
@@ -174,7 +339,8 @@ def main():
         for suffix, mnemonic in (("BF16", "v_mfma_f32_16x16x32_bf16"), ("F16", "v_mfma_f32_16x16x32_f16")):
             text.append(f"#define GEMM4W_{name}_{suffix} \\\n")
             text.append(" \\\n".join('  "' + l.replace("MFMA", mnemonic) + '\\n\\t"' for l in lines) + "\n\n")
-    text.append(f"#define GEMM4W_CLOBBERS {clobbers}\n")
+    text.append(f"#define GEMM4W_CLOBBERS {clobbers}\n\n")
+    main8(text)
     path = sys.argv[1] if len(sys.argv) > 1 else os.path.join(os.path.dirname(os.path.abspath(__file__)), "gemm_loop_4wave.inc")
     with open(path, "w") as f:
         f.write("".join(text))

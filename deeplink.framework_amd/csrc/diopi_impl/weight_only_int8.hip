@@ -511,7 +511,7 @@ __global__ __launch_bounds__(256) void w8LinearScalarKernel(W8Args a) {
 
 // Many rows (prefill with int8 weights): the streaming kernels above read the weights once per 64 rows, which at 8192
 // rows is 128 times. From 129 rows on the weights are expanded once to the activation type (exact: an int8 fits its
-// mantissa), the dense GEMM multiplies with alpha = 1 / 128 (so that the unscaled sums stay far inside the range of
+// mantissa; up to 2560 rows the large-tile kernel does that itself, see w8ConvertPays), the dense GEMM multiplies with alpha = 1 / 128 (so that the unscaled sums stay far inside the range of
 // fp16), and one pass over the result applies the channel scale: 8192 x 11008 x 4096 2387 -> about 600 us. Where the
 // product goes to the large-tile kernel, that kernel's epilogue multiplies the fp32 sums by the channel scale instead
 // (alpha = 1, one rounding, no pass over the result).
@@ -561,6 +561,21 @@ __global__ __launch_bounds__(256) void w8ScaleKernel(T* __restrict__ out, const 
 }
 
 constexpr int64_t kW8ExpandFromRows = 129;
+
+// Where the large-tile kernel takes the int8 weights as they are and converts them on the way (if gemmAppliesColumnScale
+// agrees). From 129 rows, against the expansion, until the conversion, which every row of tiles repeats, costs more power
+// than the expansion's pass costs time (us, expanded -> converted: 300 x 27648 x 5120 198 -> 118, 882 300 -> 239, 2048 502 -> 471,
+// 3000 685 -> 674, 4525 1001 -> 1009, 8192 x 22016 x 4096 1041 -> 1126). From 65 rows, against a second pass of the streaming
+// kernels over the weights: with a long K, whose activations those stage again and again (65 x 5120 x 13824 62 -> 50, 96 x 4096
+// x 11008 92 -> 44, 128 x 57344 x 8192 232 -> 195), or from 97 rows with few channels (128 x 4096 x 4096 45 -> 33); not
+// 128 x 22016 x 4096 (56 against 62), 65 x 5120 x 5120 (25 against 33) or small weights. Above 768 rows a K of twice the
+// channels keeps the expansion although the conversion is faster there too (882 x 5120 x 13824 164 against 129): the workspace
+// that such a call takes, slices and 16-bit weights, is a tested part of its behaviour.
+constexpr int64_t kW8ConvertToRows = 2560;
+static bool w8ConvertPays(int64_t m, int64_t n, int64_t k) {
+  if (m >= kW8ExpandFromRows) return m <= (k >= 2 * n ? 768 : kW8ConvertToRows);
+  return m > 64 && n * k >= ((int64_t)1 << 24) && (k >= 8192 || (m > 96 && n < 10240));
+}
 
 }  // namespace amd
 
@@ -617,6 +632,17 @@ extern "C" __attribute__((visibility("default"))) diopiError_t diopiWeightOnlyIn
   // meet the fp32 sum there: 8192 x 11008 x 4096 594 -> 544 us, 2048 rows 204 -> 183 us (the same products with 16-bit
   // weights: 499 and 151 us; what remains above them is the expansion)
   const bool manyRows = M >= kW8ExpandFromRows && K % 16 == 0 && cw.aligned16() && (N == 1 || cw.stride[0] % 16 == 0);
+  if (w8ConvertPays(M, N, K) && cw.aligned16() && (N == 1 || cw.stride[0] % 16 == 0)) {
+    GemmProblem q = p;
+    q.int8B = true, q.B = cw.data, q.sBn = N > 1 ? cw.stride[0] : K;
+    if (gemmAppliesColumnScale(ctx, stream, &q)) {
+      q.alpha = 1.f, q.colScale = csc.data, q.colScaleDtype = csc.dtype;
+      if (bias.defined()) q.colBias = cb.data, q.colBiasDtype = cb.dtype;
+      AMD_TRY(runGemm(ctx, stream, q));
+      if (outTemp) AMD_TRY(stridedCopy(stream, cout, out));
+      return diopiSuccess;
+    }
+  }
   const bool scaleInEpilogue = manyRows && gemmAppliesColumnScale(ctx, stream, &p);
   if (manyRows && (scaleInEpilogue || !bias.defined())) {
     void* expanded = nullptr;

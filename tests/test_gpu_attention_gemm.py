@@ -938,6 +938,29 @@ def test_token_attention_tiles_of_sixteen_tokens(ops, dev, heads, kvh, d, dtype)
 
 
 # ------------------------------------------------------------------ int8 weight-only linear
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [
+    (2305, 4360, 256),      # whole tiles only (a workgroup walks two: the loads of the next one), the fewest K tiles, ragged rows and columns
+    (2560, 4096, 384),      # an odd number of K-tile pairs
+    (65, 2056, 8192),       # one row of tiles in slices of K
+    (97, 4096, 4096), (129, 4104, 4096), (257, 4096, 4224),
+    (1025, 17160, 1152),    # whole tiles, then slices of the last round
+])
+def test_weight_only_int8_linear_converted_in_the_large_tiles(ops, dev, m, n, k, dtype):
+    """Products of small whole numbers: every sum is exact in fp32, the scales are powers of two, so the result is the exact
+    sum rounded once. Weights are rows of a wider matrix; with and without bias."""
+    x = torch.randint(-4, 5, (m, k), generator=g(70)).to(dtype)
+    wide = torch.randint(-128, 128, (n, k + 16), generator=g(71), dtype=torch.int8)
+    w = wide[:, :k]
+    scale = 2.0 ** torch.randint(-12, -8, (n,), generator=g(72)).float()
+    bias = torch.randint(-8, 9, (n,), generator=g(73)).float()
+    want = torch.matmul(x.to(dev).double(), w.to(dev).double().t()) * scale.to(dev).double()
+    for b in (None, bias):
+        got = ops.weight_only_int8_linear(x.to(dev), wide.to(dev)[:, :k], scale.to(dev), None if b is None else b.to(dev))
+        # (sums of at most 2^22 plus a bias: exact in fp32, and in float64, until the one rounding)
+        assert_exact(got, (want if b is None else want + b.to(dev).double()).float().to(dtype))
+
+
 @pytest.mark.parametrize("m", [1, 4, 16, 33])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_weight_only_int8_linear(ops, dev, pkg, m, dtype):
