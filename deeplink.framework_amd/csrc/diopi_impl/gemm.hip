@@ -101,6 +101,7 @@ struct MfmaArgs {
   // 4-wave kernel, K-split tail: the first wholeTiles tiles of the order are multiplied whole, each of the others in
   // kSlices slices of K whose accumulators go to partial (see gemmMfma4WaveKernel)
   int wholeTiles = 0, kSlices = 1;
+  int tileRows = 256;  // of the 4-wave kernel's output tile
 };
 
 constexpr int kBK = 64;  // K elements per LDS tile (128-byte rows)
@@ -376,7 +377,7 @@ constexpr int kRotaryLdsBytes = 32768;  // behind the two K-tile stages of the 4
 // bytes for the cosines and four for the sines. The caller waits for its own copies and meets the other waves at a
 // barrier before the epilogue reads.
 template <typename T>
-__device__ __forceinline__ void rotaryTablesToLds(const MfmaArgs& g, int tileRow0, int wave, int lane, unsigned ldsTab) {
+__device__ __forceinline__ void rotaryTablesToLds(const MfmaArgs& g, int tileRow0, int halfRows, int wave, int lane, unsigned ldsTab) {
   int tableRows = g.rotTableRows;
   asm volatile("" : "+s"(tableRows));  // (a division by a run-time value: its set-up is not to be kept across the K loop)
   const int64_t bytes = (int64_t)tableRows * 64 * (int64_t)sizeof(T);
@@ -390,7 +391,7 @@ __device__ __forceinline__ void rotaryTablesToLds(const MfmaArgs& g, int tileRow
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int r = wave * 32 + q * 8 + (lane >> 3);
-    const int row = tileRow0 + (r >> 6) * 128 + ((r >> 4) & 3) * 16 + (r & 15);
+    const int row = tileRow0 + (r >> 6) * halfRows + ((r >> 4) & 3) * 16 + (r & 15);
     const int voff = row < g.M ? ((row % tableRows) * 64 + (lane & 7) * 8) * (int)sizeof(T) : (int)0x80000000u;
     const unsigned to = ldsTab + (unsigned)(wave * 32 + q * 8) * 128u;
     loadToLds16(rsCos, voff, 0, to);
@@ -551,7 +552,7 @@ __device__ __forceinline__ void vectorEpilogue(const MfmaArgs& g, T* out, const 
         }
       }
       typedef __attribute__((address_space(3))) const u32x2* LdsPair;
-      const unsigned tabRow = ldsTab + (unsigned)((((row0 >> 7) & 1) * 64 + frow) * 128);
+      const unsigned tabRow = ldsTab + (unsigned)(frow * 128);  // (of this row half: the caller's ldsTab)
       staticFor<TM>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         f32x4 a[TN];
@@ -1208,9 +1209,10 @@ __device__ __forceinline__ void accRegisters16(f32x4 (&f)[4]) {
 // LDS stages then hold pairs of K tiles. Bound as the 16-bit form is, by the MFMA rate with few rows and by power with
 // many, where the conversions (192 vector instructions per 128 MFMAs) cost up to 7 %; what it saves is the pass that wrote the
 // weights out in 16 bits and the reads of that (882 x 27648 x 5120 300 -> 239 us, 256 x 22016 x 4096 113 -> 65).
-template <typename T, int EPI, bool SPLIT = false, bool W8 = false>
+// TM: fragment rows of a wave, 8 or, for tiles of 224 rows, 7 (see tileRowsOf). The epilogue and the slots keep room for 8.
+template <typename T, int EPI, bool SPLIT = false, bool W8 = false, int TM = 8>
 __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
-  constexpr int BM = 256, BN = 256, WM = 128, WN = 128, TM = 8, TN = 8;
+  constexpr int BM = 32 * TM, BN = 256, WM = 16 * TM, WN = 128, TN = 8, kTileLoads = TM + 8;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -1307,10 +1309,14 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
   : "memory", "scc", GEMM4W_CLOBBERS
 #define GEMM4W_RUN(NAME)                                                         \
   do {                                                                           \
-    if constexpr (std::is_same<T, bf16_t>::value)                                \
+    if constexpr (std::is_same<T, bf16_t>::value && TM == 8)                     \
       asm volatile(GEMM4W_##NAME##_BF16 GEMM4W_OPERANDS);                        \
-    else                                                                         \
+    else if constexpr (TM == 8)                                                  \
       asm volatile(GEMM4W_##NAME##_F16 GEMM4W_OPERANDS);                         \
+    else if constexpr (std::is_same<T, bf16_t>::value)                           \
+      asm volatile(GEMM4W_T7_##NAME##_BF16 GEMM4W_OPERANDS);                     \
+    else                                                                         \
+      asm volatile(GEMM4W_T7_##NAME##_F16 GEMM4W_OPERANDS);                      \
   } while (0)
   // int8: the LDS addresses in B's stage of pair p of the item (fragment bytes of the pair's tile h and k-step ks)
   unsigned kcurB = 0;
@@ -1329,11 +1335,16 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
   : "memory", "scc", GEMM4W_W8_CLOBBERS
 #define GEMM4W_W8_RUN(NAME, P)                                                   \
   do {                                                                           \
-    if constexpr (std::is_same<T, bf16_t>::value)                                \
+    if constexpr (std::is_same<T, bf16_t>::value && TM == 8)                     \
       asm volatile(GEMM4W_W8_##NAME##_BF16 GEMM4W_W8_OPERANDS(P));               \
-    else                                                                         \
+    else if constexpr (TM == 8)                                                  \
       asm volatile(GEMM4W_W8_##NAME##_F16 GEMM4W_W8_OPERANDS(P));                \
+    else if constexpr (std::is_same<T, bf16_t>::value)                           \
+      asm volatile(GEMM4W_W8_T7_##NAME##_BF16 GEMM4W_W8_OPERANDS(P));            \
+    else                                                                         \
+      asm volatile(GEMM4W_W8_T7_##NAME##_F16 GEMM4W_W8_OPERANDS(P));             \
   } while (0)
+  constexpr int kTwoTiles = 0x0f70 | (2 * kTileLoads & 15) | ((2 * kTileLoads >> 4) << 14);  // all but the loads of two K tiles are back
   int pid = blockIdx.x, tm, tn, slot = -1, itemPairs = pairs, k0 = 0;
   tileOf(pid, tm, tn, slot);
   if constexpr (SPLIT) {
@@ -1359,7 +1370,7 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
     // (rotary tables through LDS: this output tile's entries are copied now, behind every tile load of its K loop; tiles
     // of v heads need none; the decision is the same for the whole workgroup)
     if constexpr (EPI == kEpiRotaryLds) {
-      if (tn * BN < g.rotCols && slot < 0) rotaryTablesToLds<T>(g, tm * BM, waveS, laneNow(), base + 131072u);
+      if (tn * BN < g.rotCols && slot < 0) rotaryTablesToLds<T>(g, tm * BM, WM, waveS, laneNow(), base + 131072u);
     }
     // (addend through LDS: every wave copies the addend of its own first two fragment rows, likewise behind the tile loads)
     if constexpr (EPI == kEpiAddendLds)
@@ -1405,15 +1416,15 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
     }
     if constexpr (EPI == kEpiRotaryLds) {
       if (tn * BN < g.rotCols) {
-        // this wave's table copies are older than the 32 tile loads the tail issued for the next output tile (if any)
-        if (next < total) __builtin_amdgcn_s_waitcnt(0x0f70 | (32 & 15) | ((32 >> 4) << 14));
+        // this wave's table copies are older than the tile loads the tail issued for the next output tile (if any)
+        if (next < total) __builtin_amdgcn_s_waitcnt(kTwoTiles);
         else __builtin_amdgcn_s_waitcnt(0x0f70);
         __builtin_amdgcn_s_barrier();
       }
     }
     if constexpr (EPI == kEpiAddendLds) {
       // (a wave reads back only its own copies: no barrier)
-      if (next < total) __builtin_amdgcn_s_waitcnt(0x0f70 | (32 & 15) | ((32 >> 4) << 14));
+      if (next < total) __builtin_amdgcn_s_waitcnt(kTwoTiles);
       else __builtin_amdgcn_s_waitcnt(0x0f70);
     }
     // one fragment row at a time out of the accumulation registers, which the compiler does not know to be live:
@@ -1422,14 +1433,17 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
     // depend on the tile is hoisted out of the persistent loop, has to stay live across the K loop, and is spilled
     // (13 registers in the rotary form, reloaded behind the tile loads already issued for the next output tile).
     const int elane = laneNow(), efrow = elane & 15, ekq = elane >> 4;
-    vectorEpilogue<T, EPI, TM, TN>(g, out, cin, bias, tm * BM + (waveS >> 1) * WM, tn * BN + (waveS & 1) * WN, efrow, ekq, [&](auto ic, f32x4(&row)[TN]) {
+    // (rows past this wave's are the next wave's: as if the matrix ended there)
+    MfmaArgs ge = g;
+    if constexpr (TM < 8) ge.M = min(g.M, tm * BM + (waveS >> 1) * WM + WM);
+    vectorEpilogue<T, EPI, 8, TN>(ge, out, cin, bias, tm * BM + (waveS >> 1) * WM, tn * BN + (waveS & 1) * WN, efrow, ekq, [&](auto ic, f32x4(&row)[TN]) {
       constexpr int i = decltype(ic)::value;
       f32x4 lo[4], hi[4];
       accRegisters16<32 * i>(lo);
       accRegisters16<32 * i + 16>(hi);
 #pragma unroll
       for (int j = 0; j < 4; ++j) row[j] = lo[j], row[4 + j] = hi[j];
-    }, base + 131072u + (EPI == kEpiAddendLds ? (unsigned)waveS * 8192u : 0u));
+    }, base + 131072u + (EPI == kEpiAddendLds ? (unsigned)waveS * 8192u : EPI == kEpiRotaryLds ? (unsigned)(waveS >> 1) * 8192u : 0u));
     if (next >= total) break;
     pid = next, tm = ntm, tn = ntn, first = false;
     if constexpr (SPLIT) slot = nslot, itemPairs = npairs;
@@ -1470,8 +1484,11 @@ __global__ __launch_bounds__(256) void tailReduceKernel(MfmaArgs g) {
   const int logical = g.wholeTiles + tile, width = GROUP * g.tilesN, group = logical / width, firstRow = group * GROUP;
   const int gsize = min(g.tilesM - firstRow, GROUP), in = logical - group * width;
   const int tm = firstRow + in % gsize, tn = in / gsize;
-  vectorEpilogue<T, EPI, 4, 4>(g, reinterpret_cast<T*>(g.out), reinterpret_cast<const T*>(g.Cin), reinterpret_cast<const T*>(g.bias),
-                               tm * 256 + (quadrant >> 1) * 128 + ih * 64, tn * 256 + (quadrant & 1) * 128 + jh * 64, lane & 15, lane >> 4,
+  const int waveRow = tm * g.tileRows + (quadrant >> 1) * (g.tileRows / 2);
+  MfmaArgs ge = g;
+  ge.M = min(g.M, waveRow + g.tileRows / 2);
+  vectorEpilogue<T, EPI, 4, 4>(ge, reinterpret_cast<T*>(g.out), reinterpret_cast<const T*>(g.Cin), reinterpret_cast<const T*>(g.bias),
+                               waveRow + ih * 64, tn * 256 + (quadrant & 1) * 128 + jh * 64, lane & 15, lane >> 4,
                                [&](auto ic, f32x4(&row)[4]) {
 #pragma unroll
                                  for (int j = 0; j < 4; ++j) row[j] = acc[decltype(ic)::value][j];
@@ -2638,6 +2655,24 @@ static TailSplit tailSplit(int64_t tiles, int64_t pairs, int resident) {
   return best;
 }
 
+// Rows of a 4-wave tile: 224 where the rows fit as many tiles of that: an eighth fewer products, all of them with padding.
+// us, 256 -> 224: 400 x 12288 x 4096 60.4 -> 56.6, 882 x 5120 x 13824 114 -> 105, 1554 x 12288 x 4096 137 -> 129, 1340 x 27648 x 5120
+// gated 307 -> 285, int8 weights 882 x 27648 x 5120 234 -> 221; the same where a launch is all prologue and stores (203 x 5120 x 13824
+// 50.4). Tiles of 192 rows would be the next step, for a quarter of the row counts below 600.
+static int tileRowsOf(int64_t m) { return m <= ceilDiv(m, 256) * 224 ? 224 : 256; }
+
+// The 4-wave kernel for an epilogue, by the height of its tiles (the general rotary epilogues exist for 256 rows only).
+template <int EPI>
+constexpr bool hasTiles224() { return EPI != kEpiRotary && EPI != kEpiRotaryUniform; }
+template <typename T, int EPI, bool SPLIT, bool W8>
+static auto fourWaveKernel(int tileRows) {
+  auto* kernel = &gemmMfma4WaveKernel<T, EPI, SPLIT, W8, 8>;
+  if constexpr (hasTiles224<EPI>()) {
+    if (tileRows == 224) kernel = &gemmMfma4WaveKernel<T, EPI, SPLIT, W8, 7>;
+  }
+  return kernel;
+}
+
 template <typename T, int EPI, bool W8 = false>
 static diopiError_t launchTailSplit(hipStream_t stream, MfmaArgs g, const TailSplit& tail, int resident, void* ws) {
   const int rest = g.tilesM * g.tilesN - tail.whole, items = rest * tail.slices;
@@ -2646,8 +2681,9 @@ static diopiError_t launchTailSplit(hipStream_t stream, MfmaArgs g, const TailSp
   const dim3 grid((unsigned)(tail.whole ? resident : std::min(items, resident)));
   constexpr size_t lds = 2 * (size_t)(256 + 256) * kBK * sizeof(T) +
                          (EPI == kEpiRotaryLds ? kRotaryLdsBytes : EPI == kEpiAddendLds ? kAddendLdsBytes : 0);
-  AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(&gemmMfma4WaveKernel<T, EPI, true, W8>), (int)lds));
-  hipLaunchKernelGGL((gemmMfma4WaveKernel<T, EPI, true, W8>), grid, dim3(256), lds, stream, g);
+  auto* kernel = fourWaveKernel<T, EPI, true, W8>(g.tileRows);
+  AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(kernel), (int)lds));
+  hipLaunchKernelGGL(kernel, grid, dim3(256), lds, stream, g);
   AMD_LAUNCH_CHECK();
   constexpr int kReduceEpi = EPI == kEpiRotaryLds ? (int)kEpiRotaryUniform : EPI == kEpiAddendLds ? (int)kEpiLinear : EPI;
   hipLaunchKernelGGL((tailReduceKernel<T, kReduceEpi>), dim3((unsigned)(rest * 4)), dim3(256), 0, stream, g);
@@ -2699,6 +2735,7 @@ static diopiError_t launchMfmaPipelined(diopiContextHandle_t ctx, hipStream_t st
   if constexpr (EPI != kEpiPartial) {
     // the 4-wave kernel: an even number of K tiles, 16-byte epilogue pieces, lane offsets that fit 31 bits
     if (g.vecEpilogue && p.K % (2 * kBK) == 0 && p.M * p.sAm * 2 < (int64_t(1) << 31) && p.N * p.sBn * 2 < (int64_t(1) << 31)) {
+      if constexpr (hasTiles224<EPI>()) g.tileRows = tileRowsOf(p.M);
       // one workgroup per CU (its LDS ring takes most of a CU's), each walking its share of the tiles
       const int resident = computeUnits() / 8 * 8;
       if (p.batch == 1 && resident >= 8) {
@@ -2719,16 +2756,17 @@ static diopiError_t launchMfmaPipelined(diopiContextHandle_t ctx, hipStream_t st
         if (p.Cin) {
           // with an addend: the form that finds a quarter of each tile's addend in LDS (160 KiB: all of a CU's)
           constexpr size_t ldsAddend = lds + kAddendLdsBytes;
-          AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(&gemmMfma4WaveKernel<T, kEpiAddendLds>), (int)ldsAddend));
-          hipLaunchKernelGGL((gemmMfma4WaveKernel<T, kEpiAddendLds>), grid, dim3(256), ldsAddend, stream, g);
+          auto* kernel = fourWaveKernel<T, kEpiAddendLds, false, false>(g.tileRows);
+          AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(kernel), (int)ldsAddend));
+          hipLaunchKernelGGL(kernel, grid, dim3(256), ldsAddend, stream, g);
           AMD_LAUNCH_CHECK();
           return diopiSuccess;
         }
       }
       constexpr size_t lds4 = lds + (EPI == kEpiRotaryLds ? kRotaryLdsBytes : 0);  // (160 KiB with the rotary tables: all of a CU's)
-      auto* kernel = &gemmMfma4WaveKernel<T, EPI>;
+      auto* kernel = fourWaveKernel<T, EPI, false, false>(g.tileRows);
       if constexpr (EPI == kEpiColScale) {
-        if (p.int8B) kernel = &gemmMfma4WaveKernel<T, EPI, false, true>;
+        if (p.int8B) kernel = fourWaveKernel<T, EPI, false, true>(g.tileRows);
       }
       AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(kernel), (int)lds4));
       hipLaunchKernelGGL(kernel, grid, dim3(256), lds4, stream, g);

@@ -40,6 +40,9 @@ clock. Register-only loops of either instruction over the whole chip (no memory 
 2.12 GHz (16x16x32, 16.4 cycles per instruction) against 1940 TFLOP/s at 1.87 GHz (32x32x16, 32.4 cycles): the first
 figure is the ceiling that the power limit leaves to any bf16 GEMM here, 0.86 of the nominal peak.
 
+The forms with 7 instead of 8 A fragments (T7, tiles of 224 x 256; `rows` below) leave out a[4 (56 + j) ..] and their MFMAs, reads and loads: 112
+MFMAs a tile, 15 loads a wave, the same slots otherwise.
+
 The form for int8 weights (the macros with W8): the second operand lies in LDS as it does in memory, rows of 128 bytes that are
 the K of a PAIR of tiles, so its loads (8 per pair instead of 16) and its two stages go by pairs, and a load still fetches
 whole 128-byte lines. A lane reads the 8 bytes of a fragment (ds_read_b64, K order and swizzle as in the 16-bit form: half
@@ -55,7 +58,10 @@ this wave's 1 KiB slot in this pair's stage, %[sel] the permutation's selector."
 import os
 import sys
 
-READ_ORDER = [("B", 0)] + [("A", i) for i in range(8)] + [("B", j) for j in range(1, 8)]
+def read_order(rows):
+    return [("B", 0)] + [("A", i) for i in range(rows)] + [("B", j) for j in range(1, 8)]
+
+
 VA0, VB0 = 120, 184
 
 
@@ -74,14 +80,20 @@ def acc(i, j):
     return f"a[{r}:{r + 3}]"
 
 
-def load_m0(out, d, stage):
-    out.append(f"s_add_u32 m0, %[lds], {stage * 32768 + (65536 if d >= 8 else 0) + (d % 8) * 4096}")
+def tile_loads(rows, stage):
+    """The loads of a K tile into a stage, as (operand, pass of 32 rows, stage)."""
+    return [("A", d, stage) for d in range(rows)] + [("B", d, stage) for d in range(8)]
 
 
-def load_issue(out, d):
-    is_b = d >= 8
-    out.append(f"buffer_load_dwordx4 %[vo{'B' if is_b else 'A'}{d % 8}], %[{'rsB' if is_b else 'rsA'}], %[kcur] offen lds")
-    if d == 15:
+def load_m0(out, load):
+    kind, d, stage = load
+    out.append(f"s_add_u32 m0, %[lds], {stage * 32768 + (65536 if kind == 'B' else 0) + d * 4096}")
+
+
+def load_issue(out, load):
+    kind, d, _ = load
+    out.append(f"buffer_load_dwordx4 %[vo{kind}{d}], %[rs{kind}], %[kcur] offen lds")
+    if kind == "B" and d == 7:
         out.append("s_add_u32 %[kcur], %[kcur], 128")
 
 
@@ -94,85 +106,82 @@ B1_SLOT = 22       # B1 follows this MFMA of k-step 0
 LOAD_STEP = 5      # MFMAs between two tile loads
 
 
-def tile(out, s, loads, next_tile, next_output=False):
-    """128 MFMAs of one K tile in stage s; loads: issue the 16 loads of tile t + 2; next_tile: read tile t + 1's first
+def tile(out, rows, s, loads, next_tile, next_output=False):
+    """16 `rows` MFMAs of one K tile in stage s; loads: issue the loads of tile t + 2; next_tile: read tile t + 1's first
     fragments during k-step 1; next_output (last K tile of an output tile only): once B1 has freed both stages, issue
-    the 32 loads of the first two K tiles of the workgroup's next output tile (the caller passes that tile's lane
+    the loads of the first two K tiles of the workgroup's next output tile (the caller passes that tile's lane
     offsets), so that they land while the epilogue runs."""
-    after = {m: [] for m in range(128)}
-    for r in range(16):                                    # this tile's k-step 1 fragments, right away
+    step, order = 8 * rows, read_order(rows)               # MFMAs of a k-step
+    after = {m: [] for m in range(2 * step)}
+    for r in range(len(order)):                            # this tile's k-step 1 fragments, right away
         after[r].append(("read1", r))
     after[B1_SLOT].append(("B1", None))
     loads_before_b2 = 0
     if loads:
-        for d in range(16):
-            slot = B1_SLOT + 1 + d * LOAD_STEP
-            if slot + 1 <= 63:
+        for n, load in enumerate(tile_loads(rows, s)):
+            slot = B1_SLOT + 1 + n * LOAD_STEP
+            if slot + 1 < step:
                 loads_before_b2 += 1
-            after[slot].append(("m0", d))                  # M0 is written one MFMA before the load that reads it
-            after[slot + 1].append(("load", d))
+            after[slot].append(("m0", load))               # M0 is written one MFMA before the load that reads it
+            after[slot + 1].append(("load", load))
     if next_output:
         after[B1_SLOT].append(("rewind", None))
-        for n in range(32):
+        for n, load in enumerate(tile_loads(rows, 0) + tile_loads(rows, 1)):
             slot = B1_SLOT + 1 + n * 3
-            after[slot].append(("m0n", n))
-            after[slot + 1].append(("load", n % 16))
+            after[slot].append(("m0", load))
+            after[slot + 1].append(("load", load))
     if next_tile:
-        for r in range(16):
-            after[65 + 3 * r].append(("read0", r))
-    for m in range(128):
-        ks, mm = divmod(m, 64)
-        j, pos = divmod(mm, 8)
-        i = pos if j % 2 == 0 else 7 - pos                 # A fragments back and forth: one operand changes per MFMA
+        for r in range(len(order)):
+            after[step + 1 + 3 * r].append(("read0", r))
+    for m in range(2 * step):
+        ks, mm = divmod(m, step)
+        j, pos = divmod(mm, rows)
+        i = pos if j % 2 == 0 else rows - 1 - pos          # A fragments back and forth: one operand changes per MFMA
         if m == 0:
-            out.append("s_waitcnt lgkmcnt(7)")             # B0, A0..A7 of buffer 0 (read during the previous k-step 1)
+            out.append("s_waitcnt lgkmcnt(7)")             # B0 and A of buffer 0 (read during the previous k-step 1)
         elif ks == 0 and pos == 0 and j >= 1 and m <= B1_SLOT:
             # B_j of buffer 0: 7 - j reads of its set are younger, and so are this tile's reads issued so far
-            out.append(f"s_waitcnt lgkmcnt({min(7 - j + min(m, 16), 15)})")
-        if m == 64 and next_tile:                          # B2; the last K tile has no successor to wait for
+            out.append(f"s_waitcnt lgkmcnt({min(7 - j + min(m, len(order)), 15)})")
+        if m == step and next_tile:                        # B2; the last K tile has no successor to wait for
             out.append(f"s_waitcnt vmcnt({loads_before_b2}) lgkmcnt(0)")
             out.append("s_barrier")
         out.append(f"MFMA {acc(i, j)}, {vb(ks, j)}, {va(ks, i)}, {acc(i, j)}")
         for what, arg in after[m]:
             if what == "read1":
-                read_fragment(out, READ_ORDER[arg][0], READ_ORDER[arg][1], 1, s, 1)
+                read_fragment(out, order[arg][0], order[arg][1], 1, s, 1)
             elif what == "read0":
-                read_fragment(out, READ_ORDER[arg][0], READ_ORDER[arg][1], 0, s ^ 1, 0)
+                read_fragment(out, order[arg][0], order[arg][1], 0, s ^ 1, 0)
             elif what == "B1":
                 out.append("s_waitcnt lgkmcnt(0)")
                 out.append("s_barrier")
             elif what == "m0":
-                load_m0(out, arg, s)
-            elif what == "m0n":
-                load_m0(out, arg % 16, arg // 16)
+                load_m0(out, arg)
             elif what == "rewind":
                 out.append("s_mov_b32 %[kcur], 0")
             else:
                 load_issue(out, arg)
 
 
-def prologue(out, issue_loads):
+def prologue(out, rows, issue_loads):
     """issue_loads: issue the loads of K tiles 0 and 1 (otherwise the workgroup's previous output tile did, before its
-    epilogue). The wait that follows allows 16 operations to be outstanding. Loads return in order, so whatever else
-    is still counted (K tile 1's 16 loads, the previous epilogue's stores), K tile 0 has landed: if one of its
-    loads were pending, all 16 younger loads of K tile 1 would be too."""
+    epilogue). The wait that follows allows one K tile's loads to be outstanding. Loads return in order, so whatever else
+    is still counted (K tile 1's loads, the previous epilogue's stores), K tile 0 has landed: if one of its
+    loads were pending, all younger loads of K tile 1 would be too."""
     out.append("s_mov_b32 %[m0s], m0")
     if issue_loads:
-        for stage in (0, 1):
-            for d in range(16):
-                load_m0(out, d, stage)
-                out.append("s_nop 0")
-                load_issue(out, d)
+        for load in tile_loads(rows, 0) + tile_loads(rows, 1):
+            load_m0(out, load)
+            out.append("s_nop 0")
+            load_issue(out, load)
     for r in range(256):                            # while the loads are in flight
         out.append(f"v_accvgpr_write_b32 a{r}, 0")
-    out.append("s_waitcnt vmcnt(16)")
+    out.append(f"s_waitcnt vmcnt({rows + 8})")
     out.append("s_barrier")
-    for kind, idx in READ_ORDER:
+    for kind, idx in read_order(rows):
         read_fragment(out, kind, idx, 0, 0, 0)
 
 
 RAW0, TMP0 = 104, 100   # raw bytes of a k-step's 8 fragments (2 registers each); 4 temporaries
-KINDS8 = [("B", j) for j in range(8)] + [("A", i) for i in range(8)]
 
 
 def convert(kind, buf, j):
@@ -203,64 +212,68 @@ def read8(out, kind, idx, buf, stage, ks, ad):
         out.append(f"ds_read_b64 v[{RAW0 + 2 * idx}:{RAW0 + 2 * idx + 1}], %[{ad}] offset:{idx * 2048}")
 
 
-def m0_8(out, load, s):
+def order8(rows):
+    return [("B", j) for j in range(8)] + [("A", i) for i in range(rows)]
+
+
+def m0_8(out, load):
     kind, d, stage = load
-    if kind == "A":
-        load_m0(out, d, s if stage is None else stage)
-    elif stage is None:
+    if stage is None:
         out.append(f"s_add_u32 m0, %[ldsB], {d * 4096}")
     else:
-        load_m0(out, 8 + d, stage)
+        load_m0(out, load)
 
 
-def issue8(out, load):
+def issue8(out, load, rows):
     kind, d, _ = load
     k = "kcur" if kind == "A" else "kcurB"
     out.append(f"buffer_load_dwordx4 %[vo{kind}{d}], %[rs{kind}], %[{k}] offen lds")
-    if d == 7:
+    if d == (rows if kind == "A" else 8) - 1:
         out.append(f"s_add_u32 %[{k}], %[{k}], 128")
 
 
-def tile8(out, kind, h, load_a, load_b, younger, next_tile, next_output=False):
+def tile8(out, rows, kind, h, load_a, load_b, younger, next_tile, next_output=False):
     """One K tile of the int8 form, the pair's tile h (its stage of A too). load_a: issue the A loads of tile t + 2, load_b: then
     the B loads of the pair after the next (h == 1); younger: loads issued before this tile that its B2 may leave in flight."""
-    after = {m: [] for m in range(128)}
-    for r in range(16):
+    step, order = 8 * rows, order8(rows)
+    after = {m: [] for m in range(2 * step)}
+    for r in range(len(order)):
         after[r].append(("read", (r, 1, h, 1, f"adB{h}1")))
     after[B1_SLOT].append(("B1", None))
-    loads = [("A", d, None) for d in range(8)] * load_a + [("B", d, None) for d in range(8)] * load_b
-    step = LOAD_STEP
+    loads = [("A", d, h) for d in range(rows)] * load_a + [("B", d, None) for d in range(8)] * load_b
+    spacing = LOAD_STEP
     if next_output:
         after[B1_SLOT].append(("rewind", None))
-        loads = [("A", d, 0) for d in range(8)] + [("B", d, 0) for d in range(8)] + [("A", d, 1) for d in range(8)] + [("B", d, 1) for d in range(8)]
-        step = 3
+        loads = tile_loads(rows, 0) + tile_loads(rows, 1)
+        spacing = 3
     before_b2 = younger
     for n, load in enumerate(loads):
-        slot = B1_SLOT + 1 + n * step
-        before_b2 += slot + 1 <= 63
+        slot = B1_SLOT + 1 + n * spacing
+        before_b2 += slot + 1 < step
         after[slot].append(("m0", load))
         after[slot + 1].append(("load", load))
-    vector = {m: [] for m in range(128)}
+    vector = {m: [] for m in range(2 * step)}
     for j in range(8):
         ops = convert(kind, 1, j)
         for n, op in enumerate(ops):
             vector[23 + 5 * j + n * 5 // len(ops)].append(op)
     if next_tile:
-        for r in range(16):
-            after[65 + 2 * r].append(("read", (r, 0, h ^ 1, 0, "adB10" if h == 0 else "adN00")))
+        for r in range(len(order)):
+            after[step + 1 + 2 * r].append(("read", (r, 0, h ^ 1, 0, "adB10" if h == 0 else "adN00")))
+        begin, width = (15, 6) if rows == 8 else (13, 5)
         for j in range(8):
-            first, ops = 79 + 6 * j, convert(kind, 0, j)
-            issued = min(16, (first - 65 + 1) // 2)      # reads issued behind MFMAs before `first`
+            first, ops = step + begin + width * j, convert(kind, 0, j)
+            issued = min(len(order), (first - step) // 2)     # reads issued behind MFMAs before `first`
             vector[first].append(f"s_waitcnt lgkmcnt({issued - j - 1})")
             for n, op in enumerate(ops):
-                vector[first + n * 6 // len(ops)].append(op)
-    for m in range(128):
-        ks, mm = divmod(m, 64)
-        j, pos = divmod(mm, 8)
-        i = pos if j % 2 == 0 else 7 - pos
+                vector[first + n * width // len(ops)].append(op)
+    for m in range(2 * step):
+        ks, mm = divmod(m, step)
+        j, pos = divmod(mm, rows)
+        i = pos if j % 2 == 0 else rows - 1 - pos
         if m == 0:
-            out.append("s_waitcnt lgkmcnt(0)")           # A0..A7 of buffer 0, read at the latest 32 MFMAs ago
-        if m == 64 and next_tile:
+            out.append("s_waitcnt lgkmcnt(0)")           # A of buffer 0, read a good while ago
+        if m == step and next_tile:
             out.append(f"s_waitcnt vmcnt({before_b2}) lgkmcnt(0)")
             out.append("s_barrier")
         out.append(f"MFMA {acc(i, j)}, {vb(ks, j)}, {va(ks, i)}, {acc(i, j)}")
@@ -268,79 +281,80 @@ def tile8(out, kind, h, load_a, load_b, younger, next_tile, next_output=False):
         for what, arg in after[m]:
             if what == "read":
                 r, buf, stage, rks, ad = arg
-                read8(out, KINDS8[r][0], KINDS8[r][1], buf, stage, rks, ad)
+                read8(out, order[r][0], order[r][1], buf, stage, rks, ad)
             elif what == "B1":
                 out.append("s_waitcnt lgkmcnt(0)")
                 out.append("s_barrier")
             elif what == "m0":
-                m0_8(out, arg, h)
+                m0_8(out, arg)
             elif what == "rewind":
                 out.append("s_mov_b32 %[kcur], 0")
                 out.append("s_mov_b32 %[kcurB], 0")
             else:
-                issue8(out, arg)
+                issue8(out, arg, rows)
 
 
-def prologue8(out, kind, issue_loads):
-    """As prologue(); K tile 0 is A's first 8 loads and B's first pair, and K tile 1 and the second pair are the 16 after them."""
+def prologue8(out, rows, kind, issue_loads):
+    """As prologue(); K tile 0 is A's first loads and B's first pair, and K tile 1 and the second pair are those after them."""
     out.append("s_mov_b32 %[m0s], m0")
     if issue_loads:
         for stage in (0, 1):
-            for load in [("A", d, stage) for d in range(8)] + [("B", d, stage) for d in range(8)]:
-                m0_8(out, load, 0)
+            for load in tile_loads(rows, stage):
+                m0_8(out, load)
                 out.append("s_nop 0")
-                issue8(out, load)
+                issue8(out, load, rows)
     for r in range(256):
         out.append(f"v_accvgpr_write_b32 a{r}, 0")
-    out.append("s_waitcnt vmcnt(16)")
+    out.append(f"s_waitcnt vmcnt({rows + 8})")
     out.append("s_barrier")
-    for k, idx in KINDS8:
+    for k, idx in order8(rows):
         read8(out, k, idx, 0, 0, 0, "adB00")
-    out.append("s_waitcnt lgkmcnt(8)")
+    out.append(f"s_waitcnt lgkmcnt({rows})")
     for j in range(8):
         out += convert(kind, 0, j)
 
 
-def main8(text):
-    for kind, mnemonic in (("BF16", "v_mfma_f32_16x16x32_bf16"), ("F16", "v_mfma_f32_16x16x32_f16")):
-        pro, proc, body, last, tail, tailn = [], [], [], [], [], []
-        prologue8(pro, kind, True)
-        prologue8(proc, kind, False)
-        # B2 of a pair's first tile waits for the A loads of the tile before it; that tile's B loads, issued behind them, are
-        # waited for by B2 of the second
-        tile8(body, kind, 0, True, False, 8, True)
-        tile8(body, kind, 1, True, True, 0, True)
-        tile8(last, kind, 0, True, False, 8, True)
-        tile8(last, kind, 1, True, False, 0, True)
-        for t, nxt in ((tail, False), (tailn, True)):
-            tile8(t, kind, 0, False, False, 0, True)
-            tile8(t, kind, 1, False, False, 0, False, nxt)
-            t += ["s_nop 15", "s_nop 15", "s_mov_b32 m0, %[m0s]"]
-        for name, lines in (("PROLOGUE", pro), ("PROLOGUE_LOADED", proc), ("BODY", body), ("BODY_LAST", last), ("TAIL", tail), ("TAIL_NEXT", tailn)):
-            text.append(f"#define GEMM4W_W8_{name}_{kind} \\\n")
-            text.append(" \\\n".join('  "' + l.replace("MFMA", mnemonic) + '\\n\\t"' for l in lines) + "\n\n")
-    clobbers = ", ".join(f'"v{r}"' for r in range(TMP0, VA0))
-    text.append(f"#define GEMM4W_W8_CLOBBERS {clobbers}, GEMM4W_CLOBBERS\n")
+def macros(text, prefix, kind, mnemonic, blocks):
+    for name, lines in blocks:
+        text.append(f"#define GEMM4W_{prefix}{name}_{kind} \\\n")
+        text.append(" \\\n".join('  "' + l.replace("MFMA", mnemonic) + '\\n\\t"' for l in lines) + "\n\n")
+
+
+def finished(block):
+    """The end of an output tile: the last MFMAs have written their accumulators."""
+    return block + ["s_nop 15", "s_nop 15", "s_mov_b32 m0, %[m0s]"]
 
 
 def main():
-    pro, proc, body, tail, tailn = [], [], [], [], []
-    prologue(pro, True)
-    prologue(proc, False)
-    tile(body, 0, True, True)
-    tile(body, 1, True, True)
-    for t, nxt in ((tail, False), (tailn, True)):
-        tile(t, 0, False, True)
-        tile(t, 1, False, False, nxt)
-        t += ["s_nop 15", "s_nop 15", "s_mov_b32 m0, %[m0s]"]   # the last MFMAs have written their accumulators
-    clobbers = ", ".join(f'"v{r}"' for r in range(VA0, VA0 + 128)) + ", " + ", ".join(f'"a{r}"' for r in range(256))
     text = ["// Generated by gen_gemm_loop_4wave.py (see there for the schedule); do not edit.\n"]
-    for name, lines in (("PROLOGUE", pro), ("PROLOGUE_LOADED", proc), ("BODY", body), ("TAIL", tail), ("TAIL_NEXT", tailn)):
-        for suffix, mnemonic in (("BF16", "v_mfma_f32_16x16x32_bf16"), ("F16", "v_mfma_f32_16x16x32_f16")):
-            text.append(f"#define GEMM4W_{name}_{suffix} \\\n")
-            text.append(" \\\n".join('  "' + l.replace("MFMA", mnemonic) + '\\n\\t"' for l in lines) + "\n\n")
-    text.append(f"#define GEMM4W_CLOBBERS {clobbers}\n\n")
-    main8(text)
+
+    def block(fn, *calls):
+        out = []
+        for args in calls:
+            fn(out, *args)
+        return out
+
+    for rows, t7 in ((8, ""), (7, "T7_")):
+        for kind, mnemonic in (("BF16", "v_mfma_f32_16x16x32_bf16"), ("F16", "v_mfma_f32_16x16x32_f16")):
+            macros(text, t7, kind, mnemonic, (
+                ("PROLOGUE", block(prologue, (rows, True))),
+                ("PROLOGUE_LOADED", block(prologue, (rows, False))),
+                ("BODY", block(tile, (rows, 0, True, True), (rows, 1, True, True))),
+                ("TAIL", finished(block(tile, (rows, 0, False, True), (rows, 1, False, False)))),
+                ("TAIL_NEXT", finished(block(tile, (rows, 0, False, True), (rows, 1, False, False, True))))))
+            # int8: B2 of a pair's first tile waits for the A loads of the tile before it; that tile's B loads, issued behind
+            # them, are waited for by B2 of the second
+            macros(text, "W8_" + t7, kind, mnemonic, (
+                ("PROLOGUE", block(prologue8, (rows, kind, True))),
+                ("PROLOGUE_LOADED", block(prologue8, (rows, kind, False))),
+                ("BODY", block(tile8, (rows, kind, 0, True, False, 8, True), (rows, kind, 1, True, True, 0, True))),
+                ("BODY_LAST", block(tile8, (rows, kind, 0, True, False, 8, True), (rows, kind, 1, True, False, 0, True))),
+                ("TAIL", finished(block(tile8, (rows, kind, 0, False, False, 0, True), (rows, kind, 1, False, False, 0, False)))),
+                ("TAIL_NEXT", finished(block(tile8, (rows, kind, 0, False, False, 0, True), (rows, kind, 1, False, False, 0, False, True))))))
+    clobbers = ", ".join(f'"v{r}"' for r in range(VA0, VA0 + 128)) + ", " + ", ".join(f'"a{r}"' for r in range(256))
+    text.append(f"#define GEMM4W_CLOBBERS {clobbers}\n")
+    clobbers = ", ".join(f'"v{r}"' for r in range(TMP0, VA0))
+    text.append(f"#define GEMM4W_W8_CLOBBERS {clobbers}, GEMM4W_CLOBBERS\n")
     path = sys.argv[1] if len(sys.argv) > 1 else os.path.join(os.path.dirname(os.path.abspath(__file__)), "gemm_loop_4wave.inc")
     with open(path, "w") as f:
         f.write("".join(text))

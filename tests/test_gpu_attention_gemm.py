@@ -318,6 +318,20 @@ def test_four_wave_gemm_last_round_split_along_k_exact(ops, dev, pkg, dtype, epi
         ctx.close()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("epilogue,m,n,k", [
+    ("linear", 224, 40960, 256),                      # one row of whole tiles, full
+    ("linear", 225, 40960, 256),                      # one row too many: 256
+    ("bias", 447, 20488, 384), ("silu_mul", 448, 22016, 256), ("addend", 1344, 8192, 256), ("rotary", 1121, 12288, 256),
+    ("rotary", 1120, 12288, 256),                     # 5 rows of tiles each, the first of them just above what 224 rows hold
+    ("linear", 1568, 11008, 1024),                    # a whole round, then slices
+    ("silu_mul", 193, 28672, 4096), ("column_scale", 440, 12288, 4096), ("column_scale", 1100, 10240, 256),
+    ("addend", 400, 12288, 4096), ("rotary", 210, 22016, 4096)])         # slices only
+def test_four_wave_gemm_tiles_of_224_rows_exact(ops, dev, dtype, epilogue, m, n, k):
+    """Row counts at and around those that fill tiles of 224 rows, in every epilogue, whole tiles and slices of K."""
+    check_last_round(ops, dev, dtype, epilogue, m, n, k)
+
+
 def check_last_round(ops, dev, dtype, epilogue, m, n, k):
     g0 = g(78)
     cols = torch.randint(0, k, (m,), generator=g0)
