@@ -200,6 +200,13 @@ __device__ __forceinline__ void loadToLds16Stream(u32x4 rsrc, int voffset, int s
       : "memory");
 }
 
+// What the wave's lanes wrote to LDS is read by its other lanes from here on (LDS serves a wave in order).
+__device__ __forceinline__ void exchangeInWave() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <int... Is, typename F>
 __device__ __forceinline__ void staticForImpl(std::integer_sequence<int, Is...>, F&& f) {
   (f(std::integral_constant<int, Is>{}), ...);

@@ -1103,10 +1103,15 @@ __global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 || ST
     });
     return;
   }
-  // outputs that do not allow 16-byte pieces: a lane's four consecutive columns as one store at element alignment
-  // (bmm [64, 777, 128] x [128, 777]: 75 -> 46 us against one store per element); the addend of a fragment row is
-  // requested before the row's first store, for the reason given above
-  typedef T T4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  // Outputs that do not allow 16-byte pieces: 16 rows at a time through LDS, so that a store writes 16 bytes at element
+  // alignment and 8 lanes 128 consecutive bytes of a row; a lane's own four columns at a time, 32 bytes of a row to an
+  // instruction, bmm [64, 777, 128] x [128, 777] takes 46 us against 38 (and 75 with one element per store). The
+  // addend of a fragment row is requested before the row's first store, for the reason given above.
+  typedef T T4 __attribute__((ext_vector_type(4)));
+  typedef T T8u __attribute__((ext_vector_type(8), aligned(sizeof(T))));
+  constexpr int kPitch = WN + 8;  // elements
+  T* const box = reinterpret_cast<T*>(smem) + wave * 16 * kPitch;
+  __syncthreads();  // the ring is done with
   auto storeScalar = [&](auto withAddend) {
     constexpr bool kAddend = decltype(withAddend)::value;
     float bc[TN][4];  // (once for all rows: for each it is a chain of loads between two stores, 1554 x 7 x 2048 17 -> 21 us)
@@ -1116,8 +1121,7 @@ __global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 || ST
       for (int r = 0; r < 4; ++r) bc[j][r] = bias ? static_cast<float>(bias[min(tn * BN + wn * WN + j * 16 + kq * 4 + r, g.N - 1)]) : 0.f;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      const int row = tm * BM + wm * WM + i * 16 + frow;
-      if (row >= g.M) continue;
+      const int row0 = tm * BM + wm * WM + i * 16, row = min(row0 + frow, g.M - 1);
       float c[TN][4];
       if constexpr (kAddend) {
 #pragma unroll
@@ -1130,7 +1134,6 @@ __global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 || ST
       }
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        const int col0 = tn * BN + wn * WN + j * 16 + kq * 4;
         T4 o;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -1138,15 +1141,26 @@ __global__ __launch_bounds__(TILE == 256 ? kPipeThreads : 256, TILE == 256 || ST
           if constexpr (kAddend) v += g.beta * c[j][r];
           o[r] = static_cast<T>(v);
         }
-        T* dst = out + (int64_t)row * g.ldo + col0;
-        if (col0 + 4 <= g.N) {
-          *reinterpret_cast<T4*>(dst) = o;
-        } else {
+        *reinterpret_cast<T4*>(box + frow * kPitch + j * 16 + kq * 4) = o;
+      }
+      exchangeInWave();
+      constexpr int kPer = WN / 8;  // lanes per row
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (col0 + r < g.N) dst[r] = o[r];
+      for (int h = 0; h < 16 * kPer / 64; ++h) {
+        const int r = (h * 64 + lane) / kPer, col = tn * BN + wn * WN + (lane % kPer) * 8;
+        const Frag v = *reinterpret_cast<const Frag*>(box + r * kPitch + (lane % kPer) * 8);
+        if (row0 + r < g.M) {
+          T* dst = out + (int64_t)(row0 + r) * g.ldo + col;
+          if (col + 8 <= g.N) {
+            *reinterpret_cast<T8u*>(dst) = __builtin_bit_cast(T8u, v);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              if (col + e < g.N) dst[e] = v[e];
+          }
         }
       }
+      exchangeInWave();
     }
   };
   if (cin)
@@ -2009,6 +2023,32 @@ __global__ __launch_bounds__(256) void transposeKernel(U* __restrict__ dst, cons
   for (int i = ty; i < 64; i += 4) {
     int64_t c = c0 + i, r = r0 + tx;
     if (r < rows && c < cols) dst[c * rows + r] = tile[tx][i];
+  }
+}
+
+// The same for 2-byte elements whose source rows are contiguous, in registers: a wave takes 64 x 64 elements, a lane an 8 x 8
+// block of them, read as 8 rows of 16 bytes (8 lanes: 128 consecutive bytes), turned by 32 byte permutations and written as 8
+// columns of 16 bytes, both at element alignment. Bound by the launch and by lines written in part; [64, 777, 128] 11.2 -> 7.4 us
+// against single elements through LDS, [64, 512, 128] 7.2 -> 3.9, [32, 100, 128] 5.4 -> 2.7. At least 8 rows and columns.
+__global__ __launch_bounds__(256) void transposeRows16Kernel(uint16_t* __restrict__ dst, const uint16_t* __restrict__ src, int64_t rows,
+                                                             int64_t cols, int64_t srcRowStride, int64_t srcBatchStride, int64_t dstBatchStride) {
+  typedef uint16_t U8 __attribute__((ext_vector_type(8), aligned(2)));
+  const int lane = threadIdx.x & 63;
+  const int64_t tilesC = (cols + 63) / 64, tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  int64_t r0 = tile / tilesC * 64 + (lane >> 3) * 8, c0 = tile % tilesC * 64 + (lane & 7) * 8;
+  if (r0 >= rows || c0 >= cols) return;
+  r0 = min(r0, rows - 8), c0 = min(c0, cols - 8);  // the last blocks overlap the ones before them and write the same there
+  src += blockIdx.y * srcBatchStride + r0 * srcRowStride + c0;
+  dst += blockIdx.y * dstBatchStride + c0 * rows + r0;
+  u32x4 v[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = __builtin_bit_cast(u32x4, *reinterpret_cast<const U8*>(src + i * srcRowStride));
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    u32x4 o;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) o[q] = __builtin_amdgcn_perm(v[2 * q + 1][c >> 1], v[2 * q][c >> 1], c & 1 ? 0x07060302u : 0x05040100u);
+    *reinterpret_cast<U8*>(dst + c * rows) = __builtin_bit_cast(U8, o);
   }
 }
 
@@ -3046,6 +3086,15 @@ static diopiError_t launchSkinnyForShape(diopiContextHandle_t ctx, hipStream_t s
 template <typename U>
 static diopiError_t launchTranspose(hipStream_t stream, void* dst, const void* src, int64_t batch, int64_t rows,
                                     int64_t cols, int64_t sRow, int64_t sCol, int64_t sBatch) {
+  if constexpr (sizeof(U) == 2) {
+    const int64_t wgs = ceilDiv(ceilDiv(cols, (int64_t)64) * ceilDiv(rows, (int64_t)64), (int64_t)4);
+    if (sCol == 1 && rows >= 8 && cols >= 8 && wgs < ((int64_t)1 << 31)) {
+      hipLaunchKernelGGL(transposeRows16Kernel, dim3((unsigned)wgs, (unsigned)batch), dim3(256), 0, stream, (uint16_t*)dst, (const uint16_t*)src, rows, cols,
+                         sRow, sBatch, rows * cols);
+      AMD_LAUNCH_CHECK();
+      return diopiSuccess;
+    }
+  }
   dim3 grid((unsigned)ceilDiv(cols, 64), (unsigned)ceilDiv(rows, 64), (unsigned)batch);
   hipLaunchKernelGGL(transposeKernel<U>, grid, dim3(256), 0, stream, (U*)dst, (const U*)src, rows, cols, sRow, sCol,
                      sBatch, rows * cols);

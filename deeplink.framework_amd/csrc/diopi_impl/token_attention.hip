@@ -439,12 +439,6 @@ __device__ __forceinline__ int gqSwizzleK(int r) { return D >= 128 ? (r & 15) : 
 template <int D>
 __device__ __forceinline__ int gqSwizzleV(int r) { return D >= 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); }
 
-// What the wave's lanes wrote to LDS is read by its other lanes from here on (LDS serves a wave in order).
-__device__ __forceinline__ void exchangeInWave() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 template <int N>
 __device__ __forceinline__ void waitLoadsBut() {  // all but the wave's N youngest vector-memory operations are done
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");

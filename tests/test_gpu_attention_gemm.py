@@ -318,6 +318,40 @@ def test_four_wave_gemm_last_round_split_along_k_exact(ops, dev, pkg, dtype, epi
         ctx.close()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.int16])
+@pytest.mark.parametrize("shape", [(8, 8), (9, 65), (3, 7, 64), (2, 64, 64), (5, 63, 129), (2, 777, 128), (1, 1000, 9)])
+def test_transposing_copy_of_two_byte_elements(ops, dev, shape, dtype):
+    """Blocks of 8 x 8 in registers, the last ones overlapping those before; fewer than 8 rows take the other kernel. Rows of
+    a wider matrix, from an odd element on; what lies around the destination stays."""
+    wide = torch.randint(-30000, 30000, (*shape[:-1], shape[-1] + 5), generator=g(81)).to(torch.int16)
+    if dtype != torch.int16:
+        wide = torch.randn(wide.shape, generator=g(82)).to(dtype)
+    src = wide.to(dev)[..., 3:3 + shape[-1]]
+    want = src.transpose(-1, -2).contiguous()
+    buf = torch.zeros(want.numel() + 2, dtype=dtype, device=dev)
+    out = buf[1:-1].view(want.shape)
+    ops.copy_(out, src.transpose(-1, -2))
+    assert_exact(out, want)
+    assert buf[0] == 0 and buf[-1] == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(129, 131, 128), (300, 7, 192), (70, 777, 128), (2310, 4101, 256), (128, 255, 320)])
+def test_outputs_without_whole_pieces(ops, dev, dtype, m, n, k):
+    """Rows of an odd number of columns, stored 8 columns at a time at element alignment, the last ones one by one: exact on
+    one-hot activations, with a bias and with an addend whose columns are not contiguous, in both tile sizes."""
+    g0 = g(83)
+    cols = torch.randint(0, k, (m,), generator=g0)
+    x = torch.zeros(m, k, dtype=dtype)
+    x[torch.arange(m), cols] = 1
+    w = torch.randn(n, k, generator=g0).to(dtype)
+    sel = w[:, cols].float().t()
+    b, c = torch.randn(n, generator=g0).to(dtype), torch.randn(n, m, generator=g0).to(dtype)
+    assert_exact(ops.linear(x.to(dev), w.to(dev)), sel.to(dtype))
+    assert_exact(ops.linear(x.to(dev), w.to(dev), b.to(dev)), (sel + b.float()).to(dtype))
+    assert_exact(ops.addmm(c.to(dev).t(), x.to(dev), w.to(dev).t()), (c.t().float() + sel).to(dtype))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("epilogue,m,n,k", [
     ("linear", 224, 40960, 256),                      # one row of whole tiles, full
