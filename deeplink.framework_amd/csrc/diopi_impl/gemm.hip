@@ -1416,6 +1416,7 @@ __global__ __launch_bounds__(256) void gemmMfma4WaveKernel(MfmaArgs g) {
         const int voff = laneNow() * 16;
         staticFor<TM>([&](auto ic) {
           constexpr int i = decltype(ic)::value;
+          if (tm * BM + (waveS >> 1) * WM + 16 * i >= g.M) return;  // (rows past the matrix: nobody reads them)
           f32x4 lo[4], hi[4];
           accRegisters16<32 * i>(lo);
           accRegisters16<32 * i + 16>(hi);
@@ -1476,24 +1477,6 @@ template <typename T, int EPI>
 __global__ __launch_bounds__(256) void tailReduceKernel(MfmaArgs g) {
   const int lane = threadIdx.x & 63, unit = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
   const int tile = unit >> 4, quadrant = (unit >> 2) & 3, ih = (unit >> 1) & 1, jh = unit & 1;
-  const float* src = g.partial + (int64_t)tile * g.kSlices * kTailSlotFloats + quadrant * (kTailSlotFloats / 4) + (ih * 4 * 8 + jh * 4) * 256 + lane * 4;
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = *reinterpret_cast<const f32x4*>(src + (i * 8 + j) * 256);
-  for (int s = 1; s < g.kSlices; ++s) {
-    src += kTailSlotFloats;
-    f32x4 v[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v[i][j] = *reinterpret_cast<const f32x4*>(src + (i * 8 + j) * 256);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] += v[i][j];
-  }
   constexpr int GROUP = 8;
   const int logical = g.wholeTiles + tile, width = GROUP * g.tilesN, group = logical / width, firstRow = group * GROUP;
   const int gsize = min(g.tilesM - firstRow, GROUP), in = logical - group * width;
@@ -1501,6 +1484,26 @@ __global__ __launch_bounds__(256) void tailReduceKernel(MfmaArgs g) {
   const int waveRow = tm * g.tileRows + (quadrant >> 1) * (g.tileRows / 2);
   MfmaArgs ge = g;
   ge.M = min(g.M, waveRow + g.tileRows / 2);
+  const int rows = ge.M - waveRow - ih * 64;  // of this unit's 64; a fragment row that starts past them was never written
+  if (rows <= 0) return;
+  const float* src = g.partial + (int64_t)tile * g.kSlices * kTailSlotFloats + quadrant * (kTailSlotFloats / 4) + (ih * 4 * 8 + jh * 4) * 256 + lane * 4;
+  f32x4 acc[4][4];
+  auto slice = [&](f32x4(&v)[4][4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[i][j] = *reinterpret_cast<const f32x4*>(src + (min(i, (rows - 1) >> 4) * 8 + j) * 256);
+  };
+  slice(acc);
+  for (int s = 1; s < g.kSlices; ++s) {
+    src += kTailSlotFloats;
+    f32x4 v[4][4];
+    slice(v);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] += v[i][j];
+  }
   vectorEpilogue<T, EPI, 4, 4>(ge, reinterpret_cast<T*>(g.out), reinterpret_cast<const T*>(g.Cin), reinterpret_cast<const T*>(g.bias),
                                waveRow + ih * 64, tn * 256 + (quadrant & 1) * 128 + jh * 64, lane & 15, lane >> 4,
                                [&](auto ic, f32x4(&row)[4]) {
