@@ -424,12 +424,14 @@ struct GqMfma<bf16_t> {
   typedef bf16x8 Frag;
   static __device__ __forceinline__ f32x4 run(Frag a, Frag b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
   typedef bf16x4 Quad;
+  static constexpr uint16_t kInfinity = 0x7f80;
 };
 template <>
 struct GqMfma<half_t> {
   typedef f16x8 Frag;
   static __device__ __forceinline__ f32x4 run(Frag a, Frag b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
   typedef f16x4 Quad;
+  static constexpr uint16_t kInfinity = 0x7c00;
 };
 
 // XOR on the 16-byte piece index of row r in LDS. K: 16 rows' pieces of one index fall on 16 different 16-byte bank groups;
@@ -531,6 +533,12 @@ __global__ __launch_bounds__(kGqWaves * 64) void decodeGroupedKernel(TaArgs a, T
 
   const int share = ((end - begin + kGqWaves - 1) / kGqWaves + kGqTile - 1) / kGqTile * kGqTile;  // tokens per wave, whole tiles
   const int from = begin + wave * share, to = min(end, from + share);
+  // The first walk multiplies V by both parts of each probability as V is: an infinity in V against a part that is zero or
+  // negative, or NaN in slot 0, which stands in for a slot outside the pool, then leaves the wave's sums not finite, and the
+  // wave walks its share again with care. (With care in every walk a layer of 16 x (64 .. 2048)
+  // tokens in plain calls takes 153.5 us, so 149.9.)
+  bool careful = false;
+walk:
   for (int b0 = from; b0 < to; b0 += kGqBlock) {
     const int cnt = min(kGqBlock, to - b0), tiles = (cnt + kGqTile - 1) / kGqTile;
     bool bad = false;
@@ -579,7 +587,8 @@ __global__ __launch_bounds__(kGqWaves * 64) void decodeGroupedKernel(TaArgs a, T
         f32x4 s2[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-          const Frag kf = *(LdsFrag)(uintptr_t)(at + (unsigned)(col * ROWB + (((4 * s + quad) ^ gqSwizzleK<D>(col)) << 4)));
+          Frag kf = *(LdsFrag)(uintptr_t)(at + (unsigned)(col * ROWB + (((4 * s + quad) ^ gqSwizzleK<D>(col)) << 4)));
+          if (a.d < D && 32 * s + 8 * quad >= a.d) kf = Frag{};  // (an infinity against q's zeros would be NaN)
           s2[s & 1] = M::run(kf, qf[s], s2[s & 1]);
         }
 #pragma unroll
@@ -589,10 +598,12 @@ __global__ __launch_bounds__(kGqWaves * 64) void decodeGroupedKernel(TaArgs a, T
 #pragma unroll
         for (int i = 0; i < 4; ++i) sc[i] = v[i];
       }
+      // tokens that do not count: no score, and with care rows of V read as zeros
+      u32x2 counts = {~0u, ~0u};
       if (skips || (t + 1) * kGqTile > cnt) {  // wave-uniform
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          if (tok + i >= to || slots[t * kGqTile + 4 * quad + i] < 0) sc[i] = -INFINITY;
+          if (tok + i >= to || slots[t * kGqTile + 4 * quad + i] < 0) sc[i] = -INFINITY, counts[i >> 1] &= i & 1 ? 0xffffu : 0xffff0000u;
       }
       if constexpr (MODE == kTaLogitsOut) {
         if (col < nq) *reinterpret_cast<f32x4*>(stored + col * kGqScoreRow + t * kGqTile + 4 * quad) = f32x4{sc[0], sc[1], sc[2], sc[3]};
@@ -619,18 +630,36 @@ __global__ __launch_bounds__(kGqWaves * 64) void decodeGroupedKernel(TaArgs a, T
         for (int i = 0; i < 4; ++i) {
           const float e = __builtin_amdgcn_exp2f(sc[i] - mRef);
           ps += e;
-          p[i] = static_cast<T>(e);
-          p[4 + i] = static_cast<T>(e - static_cast<float>(p[i]));
+          T hi = static_cast<T>(e);
+          if (careful && e > 0.f && hi == static_cast<T>(0.f)) hi = __builtin_bit_cast(T, (uint16_t)1); 
+          p[i] = hi;
+          p[4 + i] = static_cast<T>(e - static_cast<float>(hi));
         }
         l += ps;
         typedef __attribute__((address_space(3))) s16x4* LdsTr;
         const int row = 4 * quad + ((lane & 15) >> 2);
         const unsigned vRow = at + (kMats - 1) * kMatBytes + (unsigned)(row * ROWB + (lane & 1) * 8);
-#pragma unroll
-        for (int d = 0; d < DT; ++d) {
+        auto quadOfV = [&](int d) {
           const unsigned piece = (unsigned)((2 * d + ((lane & 3) >> 1)) ^ gqSwizzleV<D>(row)) << 4;
-          const typename M::Quad v = __builtin_bit_cast(typename M::Quad, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsTr)(uintptr_t)(vRow + piece)));
-          acc[d] = M::run(__builtin_shufflevector(v, v, 0, 1, 2, 3, 0, 1, 2, 3), p, acc[d]);
+          return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsTr)(uintptr_t)(vRow + piece)));
+        };
+        if (!careful) {
+#pragma unroll
+          for (int d = 0; d < DT; ++d) {
+            const u32x2 v = quadOfV(d);
+            acc[d] = M::run(__builtin_bit_cast(Frag, u32x4{v[0], v[1], v[0], v[1]}), p, acc[d]);
+          }
+        } else {
+#pragma unroll
+          for (int d = 0; d < DT; ++d) {
+            const u32x2 v = quadOfV(d) & counts;
+            // against the low parts infinities and NaN read as zero: the high parts, none of them zero, carry them
+            typedef uint16_t U16x4 __attribute__((ext_vector_type(4)));
+            typedef int16_t S16x4 __attribute__((ext_vector_type(4)));
+            const U16x4 top = (__builtin_bit_cast(U16x4, v) & (uint16_t)0x7fff) + (uint16_t)(0x8000 - M::kInfinity);  // bit 15: not finite
+            const u32x2 low = v & ~__builtin_bit_cast(u32x2, __builtin_bit_cast(S16x4, top) >> (int16_t)15);
+            acc[d] = M::run(__builtin_bit_cast(Frag, u32x4{v[0], v[1], low[0], low[1]}), p, acc[d]);
+          }
         }
       }
     }
@@ -645,6 +674,20 @@ __global__ __launch_bounds__(kGqWaves * 64) void decodeGroupedKernel(TaArgs a, T
     }
   }
   if constexpr (MODE == kTaLogitsOut) return;
+  if (!careful) {
+    uint32_t largest = 0;
+#pragma unroll
+    for (int d = 0; d < (kNeedV ? DT : 0); ++d)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) largest = max(largest, __float_as_uint(acc[d][i]) & 0x7fffffffu);
+    if (__builtin_amdgcn_ballot_w64(col < nq && largest >= 0x7f800000u) != 0) {
+      careful = true;
+      m = -INFINITY, mRef = 0.f, l = 0.f;
+#pragma unroll
+      for (int t = 0; t < (kNeedV ? DT : 1); ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      goto walk;
+    }
+  }
 
   // merge the waves: every lane group holds its own share of l; O^T lies in the lanes as (head = column, d = row)
   {

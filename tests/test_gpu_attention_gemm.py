@@ -985,6 +985,38 @@ def test_token_attention_tiles_of_sixteen_tokens(ops, dev, heads, kvh, d, dtype)
     assert_half(got[6:7], short)
 
 
+@pytest.mark.parametrize("heads,kvh,d", [(8, 2, 128), (8, 2, 200)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_token_attention_values_that_are_not_finite(ops, dev, heads, kvh, d, dtype):
+    """NaN in slot 0, which no sequence holds, changes nothing where slots outside the pool are skipped; an infinity in V
+    stays an infinity in its column, in the last token of a partial tile too; a key whose score is -inf weighs nothing."""
+    slots, width = 100, 37
+    kp = torch.randn(slots, kvh, d, generator=g(75)).to(dtype)
+    vp = torch.randn(slots, kvh, d, generator=g(76)).to(dtype)
+    q = torch.randn(2, heads, d, generator=g(77)).abs().to(dtype)
+    b_loc = torch.randperm(slots - 1, generator=g(78))[:2 * width].view(2, width).to(torch.int32) + 1
+    b_loc[0, 3::5] = torch.tensor([-1, slots, -7, slots + 1, -1, slots, -1], dtype=torch.int32)
+    kept = b_loc[0][(b_loc[0] >= 0) & (b_loc[0] < slots)].long()
+    cut = b_loc[1, 5].long()                        # (every query component is positive: its scores are -inf)
+    kp[0], vp[0] = float("nan"), float("nan")
+    vp[b_loc[0, 36].long(), :, 3], vp[b_loc[0, 20].long(), :, 5], vp[b_loc[1, 0].long(), :, 0] = float("inf"), -float("inf"), float("inf")
+    kp[cut, :, 0] = -float("inf")
+    one = lambda loc, i: oracle.token_attention(q[i:i + 1].float(), kp.float(), vp.float(), loc[None].to(torch.int32), torch.tensor([len(loc)]), len(loc))
+    want = torch.cat([one(kept, 0), one(b_loc[1][b_loc[1] != cut], 1)])
+    ln, st = torch.tensor([width, width], dtype=torch.int32).to(dev), torch.tensor([0, width], dtype=torch.int32).to(dev)
+    args = (b_loc.to(dev), st, ln, width)
+    att = torch.empty(heads, 2 * width, dtype=torch.float32, device=dev)
+    out2 = torch.empty(2, heads, d, dtype=dtype, device=dev)
+    ops.token_attention(q.to(dev), kp.to(dev), att, *args)
+    ops.token_softmax_reducev(att, vp.to(dev), out2, *args)
+    finite = torch.isfinite(want)
+    assert not finite[0, :, 3].any() and not finite[0, :, 5].any() and not finite[1, :, 0].any()
+    for got in (ops.token_decode_attention(q.to(dev), kp.to(dev), vp.to(dev), *args), out2):
+        got = got.cpu()
+        assert torch.equal(got[~finite].float(), want[~finite].float())
+        assert_half(got[finite], want[finite])
+
+
 # ------------------------------------------------------------------ int8 weight-only linear
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k", [
