@@ -588,7 +588,8 @@ walk:
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
           Frag kf = *(LdsFrag)(uintptr_t)(at + (unsigned)(col * ROWB + (((4 * s + quad) ^ gqSwizzleK<D>(col)) << 4)));
-          if (a.d < D && 32 * s + 8 * quad >= a.d) kf = Frag{};  // (an infinity against q's zeros would be NaN)
+          // (an infinity against q's zeros would be NaN: where the sums show that, with care only)
+          if ((MODE == kTaLogitsOut || careful) && a.d < D && 32 * s + 8 * quad >= a.d) kf = Frag{};
           s2[s & 1] = M::run(kf, qf[s], s2[s & 1]);
         }
 #pragma unroll
