@@ -397,9 +397,12 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
 // 48 sequences, 32 query heads on 8 K/V heads: fused 116 -> 91 (5.2 TB/s), scores 59 -> 50, second half 84 -> 57; 64 sequences,
 // 64 heads on 8: 265 -> 130, 131 -> 75, 180 -> 88; fp16, 16 x (64 .. 2048), 32 on 8: 37.5 -> 22.6, 18.7 -> 11.3, 34.8 -> 15.9.
 //   * S^T = K . Q^T (16x16x32): a lane holds four tokens' scores of ONE head, so the softmax runs in the lane, and its
-//     probabilities are, as they lie in the registers, the operand P^T of O^T += V^T . P^T (16x16x32: each probability as
-//     two 16-bit numbers, its rounding and what that leaves, against the same four tokens of V twice; with the rounding
-//     alone the result is 2.3e-3 from 64 bits in bf16, with both 1.66e-3, which is the rounding of the result).
+//     probabilities are, as they lie in the registers, the operand P^T of O^T += V^T . P^T (16x16x32: a probability as
+//     several 16-bit numbers, each the rounding of what the ones before it leave, against the same four tokens of V). In
+//     bf16 three of them hold all 24 bits of it. In fp16 the first two, of the probability times 2^7 (at most 2^15), end at
+//     2^-25; two more, of the remainder times 2^24 in a product of their own, go on to 2^-49: 22 bits of every
+//     probability down to 2^-45 of the largest, so the weight of many keys far below one without values is not lost
+//     (second half, 16 x (64 .. 2048), 32 on 8: 17.3 us with the first two, 18.3 with all; the fused form is the same).
 //   * K and V rows go from the pool straight into LDS (global_load_lds, a lane's own address per 16 bytes, marked
 //     non-temporal: 104 -> 91 us at 48 sequences), in a ring of kGqStages tiles that belongs to one wave: no barriers, only
 //     the wave's own load counter. V stays as it is in memory
@@ -425,6 +428,8 @@ struct GqMfma<bf16_t> {
   static __device__ __forceinline__ f32x4 run(Frag a, Frag b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
   typedef bf16x4 Quad;
   static constexpr uint16_t kInfinity = 0x7f80;
+  static constexpr float kRaise = 0.f;        // log2 of what probabilities are multiplied by before they are cut into parts
+  static constexpr float kRestScale = 1.f;    // what the parts after the second are multiplied by
 };
 template <>
 struct GqMfma<half_t> {
@@ -432,6 +437,8 @@ struct GqMfma<half_t> {
   static __device__ __forceinline__ f32x4 run(Frag a, Frag b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
   typedef f16x4 Quad;
   static constexpr uint16_t kInfinity = 0x7c00;
+  static constexpr float kRaise = 7.f;
+  static constexpr float kRestScale = 16777216.f;
 };
 
 // XOR on the 16-byte piece index of row r in LDS. K: 16 rows' pieces of one index fall on 16 different 16-byte bank groups;
@@ -446,10 +453,12 @@ __device__ __forceinline__ void waitLoadsBut() {  // all but the wave's N younge
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
 }
 
+// (The second launch bound keeps the sums out of the accumulation registers, from and to which the compiler otherwise copies
+// them for the VALU: second half in bf16 2 - 5 % less. Fused rows of 256 need more than half the registers.)
 // D: head size the rows are laid out for (64, 128, 256); a.d is any multiple of 8 up to it: the pieces past the row's end
 // repeat its first one, meet zeros of q, and give output columns that are not stored.
 template <typename T, int D, int MODE, typename LT>
-__global__ __launch_bounds__(kGqWaves * 64) void decodeGroupedKernel(TaArgs a, T* __restrict__ out, float* __restrict__ partial) {
+__global__ __launch_bounds__(kGqWaves * 64, MODE == kTaFused && D == 256 ? 1 : kGqWgsPerCu) void decodeGroupedKernel(TaArgs a, T* __restrict__ out, float* __restrict__ partial) {
   using M = GqMfma<T>;
   using Frag = typename M::Frag;
   constexpr bool kNeedK = MODE != kTaReduceV, kNeedV = MODE != kTaLogitsOut;
@@ -533,7 +542,7 @@ __global__ __launch_bounds__(kGqWaves * 64) void decodeGroupedKernel(TaArgs a, T
 
   const int share = ((end - begin + kGqWaves - 1) / kGqWaves + kGqTile - 1) / kGqTile * kGqTile;  // tokens per wave, whole tiles
   const int from = begin + wave * share, to = min(end, from + share);
-  // The first walk multiplies V by both parts of each probability as V is: an infinity in V against a part that is zero or
+  // The first walk multiplies V by all parts of each probability as V is: an infinity in V against a part that is zero or
   // negative, or NaN in slot 0, which stands in for a slot outside the pool, then leaves the wave's sums not finite, and the
   // wave walks its share again with care. (With care in every walk a layer of 16 x (64 .. 2048)
   // tokens in plain calls takes 153.5 us, so 149.9.)
@@ -625,16 +634,21 @@ walk:
               for (int i = 0; i < 4; ++i) acc[d][i] *= corr;
           }
         }
-        Frag p;
+        Frag p, r;  // a probability's first two parts, and the others
         float ps = 0.f;
+        const float mRaised = mRef - M::kRaise;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float e = __builtin_amdgcn_exp2f(sc[i] - mRef);
+          const float e = __builtin_amdgcn_exp2f(sc[i] - mRaised);
           ps += e;
           T hi = static_cast<T>(e);
-          if (careful && e > 0.f && hi == static_cast<T>(0.f)) hi = __builtin_bit_cast(T, (uint16_t)1); 
-          p[i] = hi;
-          p[4 + i] = static_cast<T>(e - static_cast<float>(hi));
+          if (careful && e > 0.f && hi == static_cast<T>(0.f)) hi = __builtin_bit_cast(T, (uint16_t)1);
+          const float left = e - static_cast<float>(hi);
+          const T lo = static_cast<T>(left);
+          p[i] = hi, p[4 + i] = lo;
+          const float last = (left - static_cast<float>(lo)) * M::kRestScale;
+          r[i] = static_cast<T>(last);
+          r[4 + i] = static_cast<T>(M::kRestScale != 1.f ? last - static_cast<float>(r[i]) : 0.f);
         }
         l += ps;
         typedef __attribute__((address_space(3))) s16x4* LdsTr;
@@ -644,22 +658,32 @@ walk:
           const unsigned piece = (unsigned)((2 * d + ((lane & 3) >> 1)) ^ gqSwizzleV<D>(row)) << 4;
           return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsTr)(uintptr_t)(vRow + piece)));
         };
+        auto multiply = [&](int d, u32x4 first, u32x4 others) {
+          acc[d] = M::run(__builtin_bit_cast(Frag, first), p, acc[d]);
+          if constexpr (M::kRestScale != 1.f) {
+            const f32x4 rest = M::run(__builtin_bit_cast(Frag, others), r, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[d][i] += rest[i] * (1.f / M::kRestScale);
+          } else {
+            acc[d] = M::run(__builtin_bit_cast(Frag, others), r, acc[d]);
+          }
+        };
         if (!careful) {
 #pragma unroll
           for (int d = 0; d < DT; ++d) {
             const u32x2 v = quadOfV(d);
-            acc[d] = M::run(__builtin_bit_cast(Frag, u32x4{v[0], v[1], v[0], v[1]}), p, acc[d]);
+            multiply(d, u32x4{v[0], v[1], v[0], v[1]}, u32x4{v[0], v[1], v[0], v[1]});
           }
         } else {
 #pragma unroll
           for (int d = 0; d < DT; ++d) {
             const u32x2 v = quadOfV(d) & counts;
-            // against the low parts infinities and NaN read as zero: the high parts, none of them zero, carry them
+            // against all parts but the first infinities and NaN read as zero: the first ones, none of them zero, carry them
             typedef uint16_t U16x4 __attribute__((ext_vector_type(4)));
             typedef int16_t S16x4 __attribute__((ext_vector_type(4)));
             const U16x4 top = (__builtin_bit_cast(U16x4, v) & (uint16_t)0x7fff) + (uint16_t)(0x8000 - M::kInfinity);  // bit 15: not finite
             const u32x2 low = v & ~__builtin_bit_cast(u32x2, __builtin_bit_cast(S16x4, top) >> (int16_t)15);
-            acc[d] = M::run(__builtin_bit_cast(Frag, u32x4{v[0], v[1], low[0], low[1]}), p, acc[d]);
+            multiply(d, u32x4{v[0], v[1], low[0], low[1]}, u32x4{low[0], low[1], low[0], low[1]});
           }
         }
       }

@@ -1017,6 +1017,47 @@ def test_token_attention_values_that_are_not_finite(ops, dev, heads, kvh, d, dty
         assert_half(got[finite], want[finite])
 
 
+@pytest.mark.parametrize("heads,kvh", [(4, 4), (8, 2)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_token_attention_weights_are_held_in_full(ops, dev, heads, kvh, dtype):
+    """What a probability holds beyond its rounding to 16 bits, and below the smallest 16-bit number, reaches the result. In
+    twelve sequences three tokens, in different tiles, have values that cancel to about 2^-13 of their terms and the others
+    have none; in the last one every 16th token weighs 4e7 times as much as those between but has no values. K picks the
+    scores: q is 8 in its first element, d = 64."""
+    d, n, batch = 64, 200, 13
+    gen = g(79)
+    score = -torch.randint(0, 64, (batch, n), generator=gen).float() / 64
+    score[-1] = -17.5
+    score[-1, ::16] = 0
+    p = torch.exp(score.double()).view(batch, n, 1, 1)
+    v = torch.zeros(batch, n, kvh, d, dtype=torch.float64)
+    v[:, 20] = torch.randn(batch, kvh, d, generator=gen).to(dtype).double()
+    v[:, 77] = (-v[:, 20] * p[:, 20] / p[:, 77]).to(dtype).double()
+    v[:, 150] = (-(v[:, 20] * p[:, 20] + v[:, 77] * p[:, 77]) * 15 / 16 / p[:, 150]).to(dtype).double()
+    v[-1] = (torch.rand(n, kvh, d, generator=gen) * 20000 + 100).to(dtype).double()
+    v[-1, ::16] = 0
+    q = torch.zeros(batch, heads, d, dtype=dtype)
+    q[:, :, 0] = 8
+    kp = torch.zeros(batch * n, kvh, d, dtype=dtype)
+    kp[:, :, 0] = score.view(-1, 1).to(dtype)
+    vp = v.view(batch * n, kvh, d).to(dtype)
+    want, terms = ((p * t).sum(1).div(p.sum(1)).repeat_interleave(heads // kvh, dim=1) for t in (v, v.abs()))
+    # Bound: the rounding of the result, and fp32 arithmetic on each term: an exponent of at most 1.5 (25.3 in the last
+    # sequence) to 2^-24 of itself twice over, exp2 to 2^-23, the sums to a few 2^-24.
+    half_ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    fp32 = torch.full((batch, 1, 1), 2.0 ** -21)
+    fp32[-1] = 2.0 ** -17
+    bound = 1.01 * half_ulp * want.abs() + fp32 * terms + 2.0 ** -25
+    ln, st = torch.full((batch,), n, dtype=torch.int32), torch.arange(batch, dtype=torch.int32) * n
+    args = (torch.arange(batch * n, dtype=torch.int32).view(batch, n).to(dev), st.to(dev), ln.to(dev), n)
+    out2 = torch.empty(batch, heads, d, dtype=dtype, device=dev)
+    ops.token_softmax_reducev(score.view(1, -1).expand(heads, -1).contiguous().to(dev), vp.to(dev), out2, *args)
+    fused = ops.token_decode_attention(q.to(dev), kp.to(dev), vp.to(dev), *args)
+    for name, got in (("two-call", out2), ("fused", fused)):
+        worst = ((got.cpu().double() - want).abs() / bound).amax(dim=(1, 2))
+        assert worst.max() <= 1, (name, worst)
+
+
 # ------------------------------------------------------------------ int8 weight-only linear
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k", [
