@@ -401,7 +401,7 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
 //     several 16-bit numbers, each the rounding of what the ones before it leave, against the same four tokens of V). In
 //     bf16 three of them hold all 24 bits of it. In fp16 the first two, of the probability times 2^7 (at most 2^15), end at
 //     2^-25; two more, of the remainder times 2^24 in a product of their own, go on to 2^-49: 22 bits of every
-//     probability down to 2^-45 of the largest, so the weight of many keys far below one without values is not lost
+//     probability down to 2^-34 of the largest, so the weight of many keys far below one without values is not lost
 //     (second half, 16 x (64 .. 2048), 32 on 8: 17.3 us with the first two, 18.3 with all; the fused form is the same).
 //   * K and V rows go from the pool straight into LDS (global_load_lds, a lane's own address per 16 bytes, marked
 //     non-temporal: 104 -> 91 us at 48 sequences), in a ring of kGqStages tiles that belongs to one wave: no barriers, only
@@ -544,7 +544,8 @@ __global__ __launch_bounds__(kGqWaves * 64, MODE == kTaFused && D == 256 ? 1 : k
   const int from = begin + wave * share, to = min(end, from + share);
   // The first walk multiplies V by all parts of each probability as V is: an infinity in V against a part that is zero or
   // negative, or NaN in slot 0, which stands in for a slot outside the pool, then leaves the wave's sums not finite, and the
-  // wave walks its share again with care. (With care in every walk a layer of 16 x (64 .. 2048)
+  // wave walks its share again with care, as it does where a probability above one and a value near the type's largest
+  // overflow (with care they are at most one: the running maximum is followed at once). (With care in every walk a layer of 16 x (64 .. 2048)
   // tokens in plain calls takes 153.5 us, so 149.9.)
   bool careful = false;
 walk:
@@ -619,7 +620,7 @@ walk:
         if (col < nq) *reinterpret_cast<f32x4*>(stored + col * kGqScoreRow + t * kGqTile + 4 * quad) = f32x4{sc[0], sc[1], sc[2], sc[3]};
       } else {
         float mt = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
-        if (__builtin_amdgcn_ballot_w64(mt - mRef > kGqRescaleStep || (m == -INFINITY && mt != -INFINITY)) != 0) {
+        if (__builtin_amdgcn_ballot_w64(mt - mRef > (careful ? 0.f : kGqRescaleStep) || (m == -INFINITY && mt != -INFINITY)) != 0) {
           auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
           mt = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
           sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);

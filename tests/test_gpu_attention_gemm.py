@@ -1058,6 +1058,30 @@ def test_token_attention_weights_are_held_in_full(ops, dev, heads, kvh, dtype):
         assert worst.max() <= 1, (name, worst)
 
 
+
+@pytest.mark.parametrize("heads,kvh", [(4, 4), (8, 2)])
+def test_token_attention_values_near_the_largest(ops, dev, heads, kvh):
+    """A later key that weighs 2^7 times what the first tile's do and has values near the type's largest: the weighted sum
+    stays in range as it does with weights of at most one."""
+    d, n, late = 64, 100, 85                         # (a wave takes tokens 64 ... 95, in two tiles)
+    score = torch.zeros(n)
+    score[late] = 4.875                               # log2: 7.03, less than what replaces the running maximum
+    sign = torch.randint(0, 2, (kvh, d), generator=g(84)).double() * 2 - 1
+    v = (torch.randn(n, kvh, d, generator=g(85)) * 1e34).bfloat16()
+    v[late] = (sign * 2e38).bfloat16()
+    kp = torch.zeros(n, kvh, d, dtype=torch.bfloat16)
+    kp[:, :, 0] = score[:, None]
+    q = torch.zeros(1, heads, d, dtype=torch.bfloat16)
+    q[:, :, 0] = 8
+    p = torch.softmax(score.double(), 0).view(n, 1, 1)
+    want = (p * v.double()).sum(0).repeat_interleave(heads // kvh, dim=0)
+    args = (torch.arange(n, dtype=torch.int32).view(1, n).to(dev), torch.zeros(1, dtype=torch.int32, device=dev), torch.full((1,), n, dtype=torch.int32, device=dev), n)
+    out2 = torch.empty(1, heads, d, dtype=torch.bfloat16, device=dev)
+    ops.token_softmax_reducev(score.expand(heads, n).contiguous().to(dev), v.to(dev), out2, *args)
+    for got in (out2, ops.token_decode_attention(q.to(dev), kp.to(dev), v.to(dev), *args)):
+        assert_half(got[0].cpu().double() / 1e38, want / 1e38)
+
+
 # ------------------------------------------------------------------ int8 weight-only linear
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k", [
