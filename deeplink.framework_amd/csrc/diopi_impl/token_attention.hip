@@ -292,6 +292,19 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
         }
         mn = fmaxf(mn, sc[u]);
       }
+      if constexpr (kNeedV) {
+        // Rows that do not count are slot 0's, which may hold anything: their weight is zero, and times NaN that is NaN.
+        // (Not before the scores: the rows of V would be waited for together with those of K, with fp32 rows and four
+        // query heads a fifth of the time.)
+        bool all = true;
+#pragma unroll
+        for (int u = 0; u < UNR; ++u) all &= ok[u];
+        if (j == 0 && __builtin_amdgcn_ballot_w64(!all) != 0) {
+#pragma unroll
+          for (int u = 0; u < UNR; ++u)
+            if (!ok[u]) vr[u] = V{};
+        }
+      }
       if constexpr (MODE == kTaLogitsOut) {
 #pragma unroll
         for (int u = 0; u < UNR; ++u) {

@@ -1082,6 +1082,39 @@ def test_token_attention_values_near_the_largest(ops, dev, heads, kvh):
         assert_half(got[0].cpu().double() / 1e38, want / 1e38)
 
 
+
+@pytest.mark.parametrize("batch,heads,kvh,d,dtype", [
+    (3, 8, 8, 64, torch.float32), (3, 8, 2, 64, torch.float32), (3, 4, 2, 48, torch.float32),
+    (170, 4, 4, 128, torch.bfloat16), (3, 4, 4, 80, torch.float16), (3, 5, 5, 128, torch.bfloat16), (3, 8, 2, 128, torch.float16)])
+def test_token_attention_what_slot_zero_holds(ops, dev, batch, heads, kvh, d, dtype):
+    """NaN in slot 0, which no sequence holds, changes nothing: not where a slot outside the pool is skipped, nor in the places
+    past a sequence's end. Rows on the lanes (fp32, many pairs, rows of other lengths) and on the matrix pipe."""
+    slots, width = 120, 37
+    kp = torch.randn(slots, kvh, d, generator=g(86)).to(dtype)
+    vp = torch.randn(slots, kvh, d, generator=g(87)).to(dtype)
+    q = torch.randn(batch, heads, d, generator=g(88)).to(dtype).to(dev)
+    b_loc = torch.randint(1, slots, (batch, width), generator=g(89)).to(torch.int32)
+    b_loc[0, 3::5] = torch.tensor([-1, slots, -7, slots + 1, -1, slots, -1], dtype=torch.int32)
+    ln = torch.full((batch,), width, dtype=torch.int32)
+    ln[1], ln[2] = 1, 30
+    args = (b_loc.to(dev), torch.arange(batch, dtype=torch.int32).to(dev) * width, ln.to(dev), width)
+
+    def both():
+        k, v = kp.to(dev), vp.to(dev)
+        att = torch.zeros(heads, batch * width, dtype=torch.float32, device=dev)
+        out2 = torch.empty(batch, heads, d, dtype=dtype, device=dev)
+        ops.token_attention(q, k, att, *args)
+        ops.token_softmax_reducev(att, v, out2, *args)
+        return ops.token_decode_attention(q, k, v, *args).cpu(), out2.cpu()
+
+    kp[0], vp[0] = 0, 0
+    want = both()
+    kp[0], vp[0] = float("nan"), float("nan")
+    for got, w in zip(both(), want):
+        assert torch.isfinite(w).all()
+        assert torch.equal(got, w)
+
+
 # ------------------------------------------------------------------ int8 weight-only linear
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k", [
