@@ -2,8 +2,8 @@
 // The impl library only ever learns about a tensor through these callbacks
 // (dipu/torch_dipu/csrc_dipu/diopirt/diopirt_impl.cpp:24-173 is the provider in DIPU).
 #include <cstring>
+#include <map>
 #include <mutex>
-#include <set>
 #include <utility>
 
 #include "common.hpp"
@@ -36,14 +36,15 @@ int computeUnits() {
 
 hipError_t allowDynamicLds(const void* kernel, int bytes) {
   static std::mutex mu;
-  static std::set<std::pair<const void*, int>> done;  // (kernel, device)
+  static std::map<std::pair<const void*, int>, int> allowed;  // (kernel, device): bytes
   int device = 0;
   hipError_t e = hipGetDevice(&device);
   if (e != hipSuccess) return e;
   std::lock_guard<std::mutex> lock(mu);
-  if (done.count({kernel, device})) return hipSuccess;
+  int& most = allowed[{kernel, device}];
+  if (bytes <= most) return hipSuccess;
   e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (e == hipSuccess) done.insert({kernel, device});
+  if (e == hipSuccess) most = bytes;
   return e;
 }
 

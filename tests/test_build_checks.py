@@ -52,3 +52,46 @@ def test_libraries_are_linked_where_the_host_module_does_not_build(monkeypatch):
     with pytest.raises(RuntimeError, match="compilation failed"):
         b.build()
     assert linked == []
+
+
+DYNAMIC_LDS_PROBE = r"""
+#include <cstdio>
+#include <map>
+#include "common.hpp"
+// in place of the runtime's: the largest launch that a kernel was allowed on a device, and whether that can be raised
+static int device = 0, calls = 0;
+static bool refuse = false;
+static std::map<std::pair<const void*, int>, int> allowed;
+extern "C" hipError_t hipGetDevice(int* d) { return *d = device, hipSuccess; }
+extern "C" hipError_t hipFuncSetAttribute(const void* f, hipFuncAttribute, int bytes) {
+  ++calls;
+  if (refuse) return hipErrorInvalidValue;
+  return allowed[{f, device}] = bytes, hipSuccess;
+}
+int main() {
+  static char a, b;  // kernels
+  struct { const void* kernel; int device, bytes; bool refuse; } launches[] = {
+      {&a, 0, 34880, false}, {&a, 0, 66560, false}, {&a, 0, 40000, false}, {&b, 0, 1000, false}, {&a, 1, 66560, true}, {&a, 1, 50000, false}, {&a, 1, 66560, false}};
+  for (auto& l : launches) {
+    device = l.device, refuse = l.refuse;
+    const hipError_t e = amd::allowDynamicLds(l.kernel, l.bytes);
+    if (l.refuse ? e == hipSuccess : e != hipSuccess || allowed[{l.kernel, l.device}] < l.bytes) return printf("%d bytes on device %d\n", l.bytes, l.device), 1;
+  }
+  const int before = calls;
+  for (int i = 0; i < 3; ++i) (void)amd::allowDynamicLds(&a, 66560);
+  return calls == before ? 0 : 2;  // what was allowed is not asked for again
+}
+"""
+
+
+def test_dynamic_lds_limit_follows_the_largest_launch(tmp_path):
+    """A kernel launched with more dynamic LDS than its launches before needs its limit raised, on each device of its own."""
+    b = _build_module()
+    (tmp_path / "probe.cpp").write_text(DYNAMIC_LDS_PROBE)
+    exe = str(tmp_path / "probe")
+    src = b.TARGETS["impl"]["dir"]
+    cmd = [b.hipcc(), "-O0", "-std=c++17", "-w", "--offload-host-only", f"-I{b.INCLUDE}", f"-I{src}", "-x", "hip", str(tmp_path / "probe.cpp"),
+           os.path.join(src, "runtime_glue.cpp"), "-o", exe, "-Wl,--unresolved-symbols=ignore-all"]
+    subprocess.run(cmd, check=True)
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
