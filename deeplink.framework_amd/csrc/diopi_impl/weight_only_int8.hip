@@ -568,12 +568,11 @@ constexpr int64_t kW8ExpandFromRows = 129;
 // 3000 685 -> 674, 4525 1001 -> 1009, 8192 x 22016 x 4096 1041 -> 1126). From 65 rows, against a second pass of the streaming
 // kernels over the weights: with a long K, whose activations those stage again and again (65 x 5120 x 13824 62 -> 50, 96 x 4096
 // x 11008 92 -> 44, 128 x 57344 x 8192 232 -> 195), or from 97 rows with few channels (128 x 4096 x 4096 45 -> 33); not
-// 128 x 22016 x 4096 (56 against 62), 65 x 5120 x 5120 (25 against 33) or small weights. Above 768 rows a K of twice the
-// channels keeps the expansion although the conversion is faster there too (882 x 5120 x 13824 164 against 129): the workspace
-// that such a call takes, slices and 16-bit weights, is a tested part of its behaviour.
+// 128 x 22016 x 4096 (56 against 62), 65 x 5120 x 5120 (25 against 33) or small weights. A long K changes nothing: 882 x 5120 x
+// 13824 157 -> 109, 2048 265 -> 235, 2560 304 -> 280, 769 x 4096 x 14336 120 -> 89, 2560 x 8192 x 28672 900 -> 857, 2700 rows equal.
 constexpr int64_t kW8ConvertToRows = 2560;
 static bool w8ConvertPays(int64_t m, int64_t n, int64_t k) {
-  if (m >= kW8ExpandFromRows) return m <= (k >= 2 * n ? 768 : kW8ConvertToRows);
+  if (m >= kW8ExpandFromRows) return m <= kW8ConvertToRows;
   return m > 64 && n * k >= ((int64_t)1 << 24) && (k >= 8192 || (m > 96 && n < 10240));
 }
 

@@ -302,7 +302,8 @@ def test_four_wave_gemm_every_instantiation_exact(ops, dev, dtype, epilogue):
     ("addend", 5000, 5120, 13824, 144, 3, 0),         # 400 tiles, 144 left: more slices than workgroups
     ("rotary", 1554, 12288, 4096, 80, 3, 0), ("rotary", 203, 22016, 4096, 86, 2, 0),
     ("silu_mul", 1554, 22016, 4096, 90, 2, 0), ("silu_mul", 400, 12288, 4096, 96, 2, 0),
-    ("column_scale", 882, 5120, 13824, 80, 3, 5120 * 13824 * 2)])                # and the weight in 16 bits
+    ("column_scale", 882, 5120, 13824, 80, 3, 0),      # int8 weights as they are
+    ("column_scale", 3000, 6144, 4096, 32, 4, 6144 * 4096 * 2)])                 # and the weight in 16 bits
 def test_four_wave_gemm_last_round_split_along_k_exact(ops, dev, pkg, dtype, epilogue, m, n, k, left, slices, other):
     """The tiles of a partly filled last round in slices of K (the 4-wave kernel's accumulators as fp32 partial sums, added
     and given the epilogue by a second launch): as many as the workspace tells, with whole rounds before them and without.
