@@ -26,9 +26,10 @@
 //     when there would otherwise be too few workgroups for the chip, at most 256 per sequence); states are merged by
 //     wave butterflies, then through LDS, then across chunks by a small lane-parallel second kernel.
 //
-// 16-bit rows shared by several query heads, the two-call form (scores to memory, then softmax and the sum over V from
-// stored scores) of 16-bit rows, and the fused form where there are few (sequence, head) pairs run on the matrix pipe
-// instead: decodeGroupedKernel. fp32 rows run on the streaming kernel in every form.
+// The two halves of the two-call form (scores to memory, then softmax and the sum over V from stored scores) are the same
+// streaming kernel with the other half of the work compiled out. Most 16-bit rows that several query heads share, and the
+// two-call form and the fused one of 16-bit rows where there are few (sequence, head) pairs, run on the matrix pipe
+// instead (decodeGroupedKernel; lanesPay draws the lines). fp32 rows run on the streaming kernel in every form.
 //
 // Head rows of whole 16-byte pieces up to 512 bytes at 16-byte aligned strides take the kernels above (rows of other
 // lengths than 128, 256 or 512 bytes on the layout of the next of those, the places past the row's end masked); any
@@ -106,12 +107,25 @@ __device__ __forceinline__ float headRowSum(float v) {
   return v;
 }
 
+// c + a[0] b[0] + a[1] b[1] for two packed 16-bit pairs, in one instruction (fp32 accumulation).
+template <typename T>
+__device__ __forceinline__ float dotPair(uint32_t a, uint32_t b, float c) {
+  static_assert(sizeof(T) == 2, "packed pairs of 16-bit elements");
+  if constexpr (std::is_same<T, bf16_t>::value) {
+    typedef __bf16 Pair __attribute__((ext_vector_type(2)));
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(Pair, a), __builtin_bit_cast(Pair, b), c, false);
+  } else {
+    typedef _Float16 Pair __attribute__((ext_vector_type(2)));
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(Pair, a), __builtin_bit_cast(Pair, b), c, false);
+  }
+}
+
 // The three things the streaming kernel below can do with a chunk of a sequence: the whole decode attention (scores,
 // online softmax and the sum over V), only the scores (first half of the two-call form: att[h, start_b + t]), or the
 // softmax and the sum over V from scores computed earlier (second half of the two-call form).
 enum TaMode { kTaFused = 0, kTaLogitsOut = 1, kTaReduceV = 2 };
 
-// T: bf16_t / half_t (8 per 16 B; HIW only) or float (4 per 16 B). LPT lanes cover one head row. LT: the type of the scores
+// T: bf16_t / half_t (8 per 16 B) or float (4 per 16 B). LPT lanes cover one head row. LT: the type of the scores
 // in memory (the two-call modes). QPK: query heads that share this workgroup's K/V head and are all served from one read
 // of its rows (grouped-query layouts; 1 otherwise). With QPK > 1 the grid is one-dimensional and decoded so that the
 // workgroups that share a K/V head's rows run next to each other on one XCD.
@@ -208,13 +222,23 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
   const int subIn = PART ? (live ? sub : 0) : sub;
   // scores leave the kernel in natural units, inside it they are in units of log2
   const float qScale = MODE == kTaLogitsOut ? a.scaleLog2e / kLog2eTA : a.scaleLog2e;
-  float qf[QPK][N];
+  // Several query heads on 16-bit rows: the products q.k are taken two at a time on the packed pairs as they come from
+  // memory, with no conversions of K.
+  constexpr bool kPairs = QPK > 1 && sizeof(T) == 2;
+  float qf[kPairs ? 1 : QPK][N];
+  uint32_t qp[kPairs ? QPK : 1][4];
   if constexpr (kNeedK) {
 #pragma unroll
     for (int j = 0; j < QPK; ++j) {
       V qv = *reinterpret_cast<const V*>(reinterpret_cast<const T*>(a.q) + b * a.qBatchStride + (h + headOf(j)) * a.qHeadStride + subIn * N);
+      if constexpr (kPairs) {
+        const u32x4 raw = __builtin_bit_cast(u32x4, qv);
 #pragma unroll
-      for (int e = 0; e < N; ++e) qf[j][e] = live ? static_cast<float>(qv[e]) * qScale : 0.f;
+        for (int c = 0; c < 4; ++c) qp[j][c] = live ? raw[c] : 0u;
+      } else {
+#pragma unroll
+        for (int e = 0; e < N; ++e) qf[j][e] = live ? static_cast<float>(qv[e]) * qScale : 0.f;
+      }
     }
   }
   const T* kBase = kNeedK ? reinterpret_cast<const T*>(a.k) + kvh * a.kHeadStride + subIn * N : nullptr;
@@ -268,13 +292,6 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
   for (int it = begin; it < end; it += STEP) {
     loadRows(kn, vn, ln, okn);    // rows of the next iteration (all masked past the end)
     loadSlots(it + 2 * STEP);     // indices of the one after
-    float kf[kNeedK && QPK > 1 ? UNR : 1][N];  // several query heads on fp32 rows: the K rows are converted once
-    if constexpr (kNeedK && QPK > 1) {
-#pragma unroll
-      for (int u = 0; u < UNR; ++u)
-#pragma unroll
-        for (int e = 0; e < N; ++e) kf[u][e] = static_cast<float>(kr[u][e]);
-    }
 #pragma unroll
     for (int j = 0; j < QPK; ++j) {
       float sc[UNR];
@@ -283,9 +300,16 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
       for (int u = 0; u < UNR; ++u) {
         if constexpr (kNeedK) {
           float d = 0.f;
+          if constexpr (kPairs) {
+            const u32x4 raw = __builtin_bit_cast(u32x4, kr[u]);
 #pragma unroll
-          for (int e = 0; e < N; ++e) d += qf[j][e] * (QPK > 1 ? kf[u][e] : static_cast<float>(kr[u][e]));
-          d = headRowSum<LPT>(d);
+            for (int c = 0; c < 4; ++c) d = dotPair<T>(qp[j][c], raw[c], d);
+            d = headRowSum<LPT>(d) * qScale;
+          } else {
+#pragma unroll
+            for (int e = 0; e < N; ++e) d += qf[j][e] * static_cast<float>(kr[u][e]);
+            d = headRowSum<LPT>(d);
+          }
           sc[u] = ok[u] ? d : -INFINITY;
         } else {
           sc[u] = lr[j][u];
@@ -1211,6 +1235,41 @@ static diopiError_t decodeScratch(float** out) {
 
 using namespace amd;
 
+// Whether 16-bit rows go to the lanes of decodeSplitKernel, and not to the matrix pipe (decodeGroupedKernel, up to 16 heads
+// per read of a row). rows: (sequence, K/V head) pairs, each read by perKv query heads; bytes: of the layout of a head row.
+// The matrix pipe has the shorter way from a row to a result, the more so the more heads share it, and 128 KiB in flight on
+// a CU; but two workgroups fill the CU (one with fused rows of 512 bytes), and each waits for its length, its slots and its
+// first tile in turn. So the lanes, eight workgroups on a CU, win where there are many rows for their length; with rows of
+// 512 bytes from fewer rows on; and with a query head alone on its K/V head, which leaves 15 of 16 matrix columns idle, where
+// a wave's load is a contiguous KiB of a token (wholeLoads: the head count allows it) or where the launch is long. The lines lie
+// where the two are alike in a sweep over 16 to 16384 rows of 64 to 16384 tokens, bf16. In us, matrix pipe -> lanes:
+//   fused: 32 heads of 128 alone: 512 x (16 .. 64) tokens 154 -> 61, 64 x (512 .. 4096) 426 -> 382, 24 x (200 .. 1000), 40 heads,
+//   59 -> 57; not 16 x (1000 .. 4000) (112 -> 130), 1 x 1777 (13.7 -> 19). 30 heads, 256 x (50 .. 300) 141 -> 127. 32 heads on 16:
+//   512 x (16 .. 64) 80 -> 50, 128 x (64 .. 256) 40 -> 44. Heads of 256: 32 on 16, 128 x (512 .. 2048) 554 -> 490, 32 x (16 .. 64) 18 ->
+//   14; 32 on 8, 512 x (16 .. 64) 113 -> 64, 128 x (32 .. 128) 41 -> 37, 128 x (64 .. 256) 58 -> 63; 64 on 8, 512 x (16 .. 64) 128 -> 113
+//   scores: 32 heads of 128, 512 x (16 .. 64) 63 -> 42, x (64 .. 256) 126 -> 133; 32 on 16 35 -> 29
+//   second half: 32 heads of 128, 512 x (16 .. 64) 97 -> 51, 256 x (1024 .. 2048) 590 -> 555, 64 x (512 .. 4096) 224 -> 213, 16 x
+//   (1000 .. 4000) 64 -> 68; 32 x (4096 .. 16384) 444 -> 434; 32 on 16, 512 x (16 .. 64) 54 -> 41, x (64 .. 256) 85 -> 88
+template <int MODE>
+static bool lanesPay(int64_t perKv, bool wholeLoads, bool partRows, int64_t bytes, int64_t rows, int64_t maxLen) {
+  if (perKv == 1) {
+    if (MODE == kTaLogitsOut) return rows >= 1024 && maxLen <= 128 && rows >= 16 * maxLen;
+    if (MODE == kTaReduceV) return rows >= 2048 || (rows >= 512 && rows >= 8 * maxLen) || rows * maxLen >= (int64_t)5 << 19;
+    if (wholeLoads) return partRows || bytes > 256 || rows * bytes > (int64_t)640 * 256;
+    return bytes > 256 || rows * bytes >= (int64_t)2048 * 256 || (rows >= 512 && maxLen <= 128);
+  }
+  if (bytes <= 128 || perKv > 8) return false;
+  const bool wide = bytes > 256;
+  if (MODE == kTaFused) {
+    if (perKv == 2) return wide ? rows >= 256 || rows * maxLen >= 1 << 16 : rows >= 2048 && rows >= (maxLen <= 128 ? 16 : 32) * maxLen;
+    if (perKv <= 4) return wide && rows >= 1024 && rows >= (maxLen <= 128 ? 8 : 16) * maxLen;
+    return wide && rows >= 4096 && maxLen <= 64;
+  }
+  if (perKv == 2) return rows >= 2048 && rows >= 32 * maxLen && (MODE == kTaReduceV || maxLen <= 128);
+  if (MODE == kTaReduceV) return wide && perKv > 4 && rows >= 4096 && maxLen <= 64;
+  return perKv <= 4 ? rows >= 4096 && maxLen <= 64 : wide && rows >= 2048 && maxLen <= 64;
+}
+
 // staticScratch: partial results go to the library's own device array instead of workspace from the context.
 // Launches decodeSplitKernel in one of its modes over (head groups, chunks, sequences) and, for the modes that produce
 // the attention output, merges the chunks. scoresF32: the stored scores of the two-call modes are float32 (else T).
@@ -1222,24 +1281,16 @@ static diopiError_t streamChunks(diopiContextHandle_t ctx, hipStream_t stream, T
   const bool partRows = bytes != 128 && bytes != 256 && bytes != 512;
   bytes = bytes <= 128 ? 128 : bytes <= 256 ? 256 : 512;
   const int perKv = a.heads / a.kvHeads;
-  // Which kernel. 16-bit rows that several query heads share, and the two-call modes, go to the matrix pipe
-  // (decodeGroupedKernel), up to 16 heads per read of a row. A query head that has its K/V head to itself leaves 15 of 16
-  // matrix columns idle; what the lanes of decodeSplitKernel have on it is one contiguous KiB (four heads) per wave load
-  // and token, and that pays once there are many (sequence, head) pairs. Fused, 128 per head, start of this rule -> now (us):
-  // 1 x 1777 tokens x 32 heads 18.8 -> 12.1, 8 x (256 .. 2048) x 40 44.7 -> 40.0, 16 x (1000 .. 4000) x 32 132 -> 117,
-  // 64 x (512 .. 4096) x 8 138 -> 114, 32 x (100 .. 500) x 32 x 64 per head 29.5 -> 20.0; but 24 x (200 .. 1000) x 40
-  // would take 59 against 57, 64 x (512 .. 4096) x 32 426 against 408, and rows of 512 bytes or of other lengths than a
-  // power of two are the lanes' from 128 pairs on (16 x (512 .. 4096) x 16 x 256 per head 114 against 102).
   const int tpw = (int)(64 / std::max<int64_t>(1, bytes / 16));  // head rows of a wave-wide load
-  const bool lanesPay = MODE == kTaFused && perKv == 1 && a.heads % tpw == 0 &&
-                        (partRows || bytes > 256 || batch * a.heads * bytes > (int64_t)640 * 256);
-  const bool grouped = dtype != diopi_dtype_float32 && !lanesPay;
-  // (fp32: one read of a K/V row serves four, or two, of the query heads that share it, with their softmax states side by
-  // side in the lane group's registers; more sharers are dealt over several workgroups that run on the same XCD, as evenly
-  // as they go)
+  const bool wholeLoads = a.heads % tpw == 0;
+  const bool grouped = dtype != diopi_dtype_float32 &&
+                       !lanesPay<MODE>(perKv, wholeLoads, partRows, bytes, batch * a.kvHeads, std::max(maxInputLen, 1));
+  // (on the lanes one read of a K/V row serves four, or two, of the query heads that share it, with their softmax states
+  // side by side in the lane group's registers; more sharers are dealt over several workgroups that run on the same XCD, as
+  // evenly as they go)
   const int qpk = grouped ? kGqHeads : perKv >= 3 ? 4 : perKv;  // query heads per read
   a.qGroups = (perKv + qpk - 1) / qpk;
-  const bool hiw = qpk == 1 && MODE == kTaFused && a.heads % tpw == 0;
+  const bool hiw = qpk == 1 && MODE == kTaFused && wholeLoads;
   const int groupsPerSeq = qpk > 1 ? a.kvHeads * a.qGroups : (hiw ? a.heads / tpw : a.heads);
   chooseChunk(&a, groupsPerSeq, batch, maxInputLen, grouped);
   a.nsplit = (int)std::max<int64_t>(1, ceilDiv(maxInputLen, a.chunk));
@@ -1290,24 +1341,27 @@ static diopiError_t streamChunks(diopiContextHandle_t ctx, hipStream_t stream, T
 #undef GROUPED_CALL
 #undef GROUPED_CALL_AS
   } else {
-#define STREAM_CALL_AS(T, LPT, PART)                                                                                                           \
-  if constexpr (sizeof(T) == 4) { /* stored scores have the type of q */                                                                       \
-    if (qpk == 4) hipLaunchKernelGGL((decodeSplitKernel<T, LPT, false, MODE, T, 4, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial); \
-    else if (qpk == 2) hipLaunchKernelGGL((decodeSplitKernel<T, LPT, false, MODE, T, 2, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial); \
-    else if (hiw) hipLaunchKernelGGL((decodeSplitKernel<T, LPT, true, kTaFused, T, 1, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial); \
-    else hipLaunchKernelGGL((decodeSplitKernel<T, LPT, false, MODE, T, 1, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial);  \
-  } else {                                                                                                                                     \
-    hipLaunchKernelGGL((decodeSplitKernel<T, LPT, true, kTaFused, float, 1, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial); \
+#define STREAM_CALL_PART(T, LPT, LT, PART)                                                                                           \
+  if (qpk == 4) hipLaunchKernelGGL((decodeSplitKernel<T, LPT, false, MODE, LT, 4, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial); \
+  else if (qpk == 2) hipLaunchKernelGGL((decodeSplitKernel<T, LPT, false, MODE, LT, 2, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial); \
+  else if (hiw) hipLaunchKernelGGL((decodeSplitKernel<T, LPT, true, kTaFused, float, 1, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial); \
+  else hipLaunchKernelGGL((decodeSplitKernel<T, LPT, false, MODE, LT, 1, PART>), grid, block, 0, stream, a, static_cast<T*>(outPtr), partial)
+#define STREAM_CALL_AS(T, LPT, LT)            \
+  if (partRows) {                             \
+    STREAM_CALL_PART(T, LPT, LT, true);       \
+  } else {                                    \
+    STREAM_CALL_PART(T, LPT, LT, false);      \
   }
-#define STREAM_CALL(T, LPT)          \
-  if (partRows) {                    \
-    STREAM_CALL_AS(T, LPT, true);    \
-  } else {                           \
-    STREAM_CALL_AS(T, LPT, false);   \
+#define STREAM_CALL(T, LPT)                                                  \
+  if (MODE == kTaFused || scoresF32) {                                       \
+    STREAM_CALL_AS(T, LPT, float);                                           \
+  } else if constexpr (sizeof(T) == 2) { /* (of fp32 rows they are fp32) */  \
+    STREAM_CALL_AS(T, LPT, T);                                               \
   }
     TA_DISPATCH(dtype, bytes, STREAM_CALL);
 #undef STREAM_CALL
 #undef STREAM_CALL_AS
+#undef STREAM_CALL_PART
   }
   AMD_LAUNCH_CHECK();
   if (MODE == kTaLogitsOut) return diopiSuccess;

@@ -1116,6 +1116,52 @@ def test_token_attention_what_slot_zero_holds(ops, dev, batch, heads, kvh, d, dt
         assert torch.equal(got, w)
 
 
+
+@pytest.mark.parametrize("batch,heads,kvh,d,width,dtype", [
+    (128, 8, 8, 128, 24, torch.bfloat16),      # a head to itself: all three forms on the lanes
+    (128, 9, 9, 64, 40, torch.float16),        # a head count that leaves wave loads incomplete
+    (4, 3, 3, 200, 700, torch.bfloat16),       # and rows of other lengths, in splits
+    (128, 32, 16, 128, 30, torch.bfloat16),    # two heads per row
+    (256, 16, 8, 96, 20, torch.float16),
+    (2, 8, 4, 256, 8300, torch.bfloat16),      # long sequences of rows of 512 bytes: the fused form
+    (128, 32, 8, 256, 24, torch.float16),      # four
+    (512, 56, 8, 192, 10, torch.bfloat16),     # seven
+])
+def test_token_attention_many_rows_on_the_lanes(ops, dev, batch, heads, kvh, d, width, dtype):
+    """16-bit rows that are many for their length, and those of 512 bytes: fused, and the two calls with scores in fp32 and in
+    the type of the rows, sequences of one token up to the widest."""
+    gen = g(90)
+    slots = batch * width + 5
+    kp, vp = (torch.randn(slots, kvh, d, generator=gen).to(dtype) for _ in range(2))
+    q = torch.randn(batch, heads, d, generator=gen).to(dtype)
+    ln = torch.randint(1, width + 1, (batch,), generator=gen)
+    ln[0], ln[1] = width, 1
+    b_loc = torch.randperm(slots, generator=gen)[:batch * width].view(batch, width)
+    st = torch.arange(batch) * width
+    rows = b_loc.to(dev)                              # right-aligned: the last ln[b] columns count
+    rep = lambda t: t.to(dev)[rows].float().repeat_interleave(heads // kvh, dim=2)     # [batch, width, heads, d]
+    score = (q.to(dev).float()[:, None] * rep(kp)).sum(-1) / d ** 0.5
+    live = torch.arange(width, device=dev)[None, :] >= width - ln.to(dev)[:, None]
+    p = torch.softmax(score.masked_fill(~live[..., None], float("-inf")), dim=1)
+    want = (p[..., None] * rep(vp)).sum(1)
+    i32 = lambda t: t.to(torch.int32).to(dev)
+    args = (i32(b_loc), i32(st), i32(ln), width)
+    q, kp, vp = q.to(dev), kp.to(dev), vp.to(dev)
+    got = ops.token_decode_attention(q, kp, vp, *args)
+    assert_half(got, want, rel=1e-2, abs_=2e-3)
+    assert_exact(ops.token_decode_attention(q, kp, vp, *args, no_alloc=True), got)
+    for st_type, tight in ((torch.float32, True), (dtype, False)):
+        att = torch.full((heads, batch * width), float("nan"), dtype=st_type, device=dev)
+        ops.token_attention(q, kp, att, *args)
+        for b in (0, 1, batch - 1):
+            n = int(ln[b])
+            col, ref = att[:, b * width:b * width + n], score[b, width - n:].t()
+            assert_fp32(col, ref, rel=1e-5) if tight else assert_half(col, ref)
+        out2 = torch.empty_like(got)
+        ops.token_softmax_reducev(att, vp, out2, *args)
+        assert_half(out2, want, rel=1e-2, abs_=2e-3) if tight else assert_half(out2, want, rel=3e-2, abs_=2e-2)
+
+
 # ------------------------------------------------------------------ int8 weight-only linear
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k", [
