@@ -1134,8 +1134,7 @@ static diopiError_t fillArgs(const TaViews& t, bool needK, bool needV, int maxLe
                 (q.stride[0] * q.itemsize) % 16 == 0 && (q.stride[1] * q.itemsize) % 16 == 0;
   if (needK && needV)
     vector = vector && t.v.aligned16() && (t.v.stride[0] * q.itemsize) % 16 == 0 && (t.v.stride[1] * q.itemsize) % 16 == 0;
-  // (decodeGroupedKernel holds slot numbers in 32 bits)
-  a->generic = !vector || (q.itemsize == 2 && kv.shape[0] > 0x7fffffff);
+  a->generic = !vector;
   AMD_CHECK(!a->generic || q.shape[2] <= kTaGenericMaxD, "token attention: head_dim %ld exceeds %d", (long)q.shape[2], kTaGenericMaxD);
   a->q = q.data;
   a->k = needK ? t.k.data : nullptr;
@@ -1283,7 +1282,8 @@ static diopiError_t streamChunks(diopiContextHandle_t ctx, hipStream_t stream, T
   const int perKv = a.heads / a.kvHeads;
   const int tpw = (int)(64 / std::max<int64_t>(1, bytes / 16));  // head rows of a wave-wide load
   const bool wholeLoads = a.heads % tpw == 0;
-  const bool grouped = dtype != diopi_dtype_float32 &&
+  // (decodeGroupedKernel holds slot numbers in 32 bits)
+  const bool grouped = dtype != diopi_dtype_float32 && a.slots <= 0x7fffffff &&
                        !lanesPay<MODE>(perKv, wholeLoads, partRows, bytes, batch * a.kvHeads, std::max(maxInputLen, 1));
   // (on the lanes one read of a K/V row serves four, or two, of the query heads that share it, with their softmax states
   // side by side in the lane group's registers; more sharers are dealt over several workgroups that run on the same XCD, as

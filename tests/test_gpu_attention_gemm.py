@@ -1162,6 +1162,31 @@ def test_token_attention_many_rows_on_the_lanes(ops, dev, batch, heads, kvh, d, 
         assert_half(out2, want, rel=1e-2, abs_=2e-3) if tight else assert_half(out2, want, rel=3e-2, abs_=2e-2)
 
 
+
+@pytest.mark.parametrize("heads,kvh,dtype", [(4, 4, torch.bfloat16), (8, 2, torch.float16), (2, 1, torch.bfloat16), (4, 1, torch.float32)])
+def test_token_attention_slots_beyond_32_bits(ops, dev, heads, kvh, dtype):
+    """A pool of more slots than 31 bits number (here all of them one row, by a stride of zero) is the lanes' in every form."""
+    d, n, slots = 64, 300, (1 << 31) + 1000
+    row_k, row_v = torch.randn(1, kvh, d, generator=g(91)).to(dtype).to(dev), torch.randn(1, kvh, d, generator=g(92)).to(dtype).to(dev)
+    k, v = row_k.expand(slots, kvh, d), row_v.expand(slots, kvh, d)
+    q = torch.randn(2, heads, d, generator=g(93)).to(dtype).to(dev)
+    b_loc = torch.randint(0, slots, (2, n), generator=g(94))
+    b_loc[0, :3] = torch.tensor([slots - 1, slots, -1])                     # two of them outside the pool
+    args = (b_loc.to(dev), torch.tensor([0, n], device=dev), torch.tensor([n, 7], device=dev), n)
+    want = row_v[0].repeat_interleave(heads // kvh, dim=0).cpu()            # a mean of equal rows
+    score = (q * row_k[0].repeat_interleave(heads // kvh, dim=0)).float().sum(-1) / 8
+    att = torch.zeros(heads, 2 * n, dtype=torch.float32, device=dev)
+    ops.token_attention(q, k, att, *args)
+    assert (att[:, 1:3] == -float("inf")).all()
+    out2 = torch.empty(2, heads, d, dtype=dtype, device=dev)
+    ops.token_softmax_reducev(att, v, out2, *args)
+    for got in (out2, ops.token_decode_attention(q, k, v, *args)):
+        for b in range(2):
+            assert_half(got[b], want, rel=1e-2, abs_=1e-5)
+    assert_half(att[:, 0], score[0])
+    assert_half(att[:, n + 6], score[1])
+
+
 # ------------------------------------------------------------------ int8 weight-only linear
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k", [
