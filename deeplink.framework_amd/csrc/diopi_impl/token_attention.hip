@@ -47,10 +47,11 @@ constexpr int kTaWaves = 4;
 constexpr int kTaUnroll = 2;
 constexpr int kTaChunk = 512;  // tokens of one sequence handled by one workgroup (grows for very long sequences)
 constexpr int kTaMaxSplit = 256;  // decodeMergeWideKernel holds four splits' weights per lane
-// Splits that decodeMergeKernel merges: the eight it requests at once. More take a workgroup per (sequence, head), whose
-// waves request up to 32 at once: 28 splits of 32 heads (1 x 1777 tokens, with the kernel before it) 13.3 -> 12.1 us,
-// 250 splits (1 x 32000) 97.9 -> 91.1; with a workgroup from five splits on 64 x (512 .. 4096) x 8 K/V heads would lose 2 - 4 %.
-constexpr int kTaNarrowSplits = 8;
+// Splits that a wave of decodeMergeKernel requests at once and merges: eight, or sixteen where there are many (sequence,
+// head) pairs. More take a workgroup per pair, whose waves request up to 32 at once: 28 splits of 32 heads (1 x 1777 tokens,
+// with the kernel before it) 13.3 -> 12.1 us, 250 splits (1 x 32000) 97.9 -> 91.1; with a workgroup from five splits on
+// 64 x (512 .. 4096) x 8 K/V heads would lose 2 - 4 %.
+constexpr int kTaNarrowSplits = 8, kTaNarrowSplitsMany = 16, kTaManyPairs = 1024;
 constexpr int kTaMinChunk = 128;  // shorter chunks cost more in prologues, partial results and merging than they gain ...
 constexpr int kTaTinyChunk = 64;  // ... unless even those leave CUs without a workgroup
 constexpr int kTaWgsPerCu = 8;    // workgroups per CU the chunk length aims for
@@ -803,12 +804,12 @@ walk:
   }
 }
 
-// out[b,h,:] = merge over the chunks that hold tokens, up to kTaNarrowSplits of them. One wave per (b,h): lane s takes the
+// out[b,h,:] = merge over the chunks that hold tokens, up to SPLITS of them. One wave per (b,h): lane s takes the
 // (max, sum) of split s, a butterfly gives the global max and normaliser, then every lane combines its elements over the
 // splits. Nothing here waits for anything else before it is requested: the sequence length, the (max, sum) pairs and the
 // splits' elements are all loaded up front (splits that hold no tokens were never written; what is read from them is
 // discarded by a select, never multiplied).
-template <typename T>
+template <typename T, int SPLITS>
 __global__ __launch_bounds__(256) void decodeMergeKernel(T* __restrict__ out, const float* __restrict__ partial,
                                                           const void* bLen, bool len64, int64_t pairs, int heads,
                                                           int d, int nsplit, int chunk) {
@@ -825,9 +826,9 @@ __global__ __launch_bounds__(256) void decodeMergeKernel(T* __restrict__ out, co
     ls = src[lane * row + 1];
   }
   const int len = (int)ldIndex(bLen, b, len64);
-  float v[kTaNarrowSplits][kMaxPerLane];
+  float v[SPLITS][kMaxPerLane];
 #pragma unroll
-  for (int u = 0; u < kTaNarrowSplits; ++u) {
+  for (int u = 0; u < SPLITS; ++u) {
     const float* r = src + (int64_t)min(u, nsplit - 1) * row + 2;
 #pragma unroll
     for (int k = 0; k < kMaxPerLane; ++k) {
@@ -843,7 +844,7 @@ __global__ __launch_bounds__(256) void decodeMergeKernel(T* __restrict__ out, co
   wgt *= l > 0.f ? 1.f / l : 0.f;
   float acc[kMaxPerLane] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int u = 0; u < kTaNarrowSplits; ++u) {
+  for (int u = 0; u < SPLITS; ++u) {
     const float w = __shfl(wgt, u, 64);
 #pragma unroll
     for (int k = 0; k < kMaxPerLane; ++k) acc[k] += u < used ? w * v[u][k] : 0.f;
@@ -1365,8 +1366,8 @@ static diopiError_t streamChunks(diopiContextHandle_t ctx, hipStream_t stream, T
   }
   AMD_LAUNCH_CHECK();
   if (MODE == kTaLogitsOut) return diopiSuccess;
-  if (a.nsplit > kTaNarrowSplits) {
-    const int64_t pairs = batch * a.heads;
+  const int64_t pairs = batch * a.heads;
+  if (a.nsplit > (pairs >= kTaManyPairs ? kTaNarrowSplitsMany : kTaNarrowSplits)) {
     AMD_CHECK(a.nsplit <= kTaMaxSplit && a.d <= 256, "token attention: %d splits of head size %d cannot be merged", a.nsplit, a.d);
 #define MERGE_WIDE_CALL(T, LPT)                                                                                                      \
   hipLaunchKernelGGL((decodeMergeWideKernel<T>), dim3((unsigned)pairs), dim3(256), 0, stream, static_cast<T*>(outPtr), partial, a.bLen, \
@@ -1375,11 +1376,14 @@ static diopiError_t streamChunks(diopiContextHandle_t ctx, hipStream_t stream, T
 #undef MERGE_WIDE_CALL
     AMD_LAUNCH_CHECK();
   } else if (a.nsplit > 1) {
-    int64_t pairs = batch * a.heads;
     dim3 mgrid((unsigned)ceilDiv(pairs, 4)), mblock(256);
-#define MERGE_CALL(T, LPT)                                                                                                     \
-  hipLaunchKernelGGL((decodeMergeKernel<T>), mgrid, mblock, 0, stream, static_cast<T*>(outPtr), partial, a.bLen, a.len64, pairs, \
-                     a.heads, a.d, a.nsplit, a.chunk)
+#define MERGE_CALL(T, LPT)                                                                                                              \
+  if (a.nsplit <= kTaNarrowSplits)                                                                                                      \
+    hipLaunchKernelGGL((decodeMergeKernel<T, kTaNarrowSplits>), mgrid, mblock, 0, stream, static_cast<T*>(outPtr), partial, a.bLen,      \
+                       a.len64, pairs, a.heads, a.d, a.nsplit, a.chunk);                                                                \
+  else                                                                                                                                  \
+    hipLaunchKernelGGL((decodeMergeKernel<T, kTaNarrowSplitsMany>), mgrid, mblock, 0, stream, static_cast<T*>(outPtr), partial, a.bLen,  \
+                       a.len64, pairs, a.heads, a.d, a.nsplit, a.chunk)
     TA_DISPATCH(dtype, bytes, MERGE_CALL);
 #undef MERGE_CALL
     AMD_LAUNCH_CHECK();
