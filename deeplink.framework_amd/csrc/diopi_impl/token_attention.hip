@@ -1244,18 +1244,19 @@ using namespace amd;
 // a wave's load is a contiguous KiB of a token (wholeLoads: the head count allows it) or where the launch is long. The lines lie
 // where the two are alike in a sweep over 16 to 16384 rows of 64 to 16384 tokens, bf16. In us, matrix pipe -> lanes:
 //   fused: 32 heads of 128 alone: 512 x (16 .. 64) tokens 154 -> 61, 64 x (512 .. 4096) 426 -> 382, 24 x (200 .. 1000), 40 heads,
-//   59 -> 57; not 16 x (1000 .. 4000) (112 -> 130), 1 x 1777 (13.7 -> 19). 30 heads, 256 x (50 .. 300) 141 -> 127. 32 heads on 16:
+//   59 -> 57; not 8 x (256 .. 2048), 40 heads (44.5 -> 48.5), 1 x 1777 (13.7 -> 19.6). 30 heads, 256 x (50 .. 300) 141 -> 127. 32 heads of
+//   64, a row of which is 128 bytes here and there: 32 x (1000 .. 4000) 125 -> 111, 24 x (1500 .. 3000) 93 -> 81. 32 heads on 16:
 //   512 x (16 .. 64) 80 -> 50, 128 x (64 .. 256) 40 -> 44. Heads of 256: 32 on 16, 128 x (512 .. 2048) 554 -> 490, 32 x (16 .. 64) 18 ->
 //   14; 32 on 8, 512 x (16 .. 64) 113 -> 64, 128 x (32 .. 128) 41 -> 37, 128 x (64 .. 256) 58 -> 63; 64 on 8, 512 x (16 .. 64) 128 -> 113
 //   scores: 32 heads of 128, 512 x (16 .. 64) 63 -> 42, x (64 .. 256) 126 -> 133; 32 on 16 35 -> 29
 //   second half: 32 heads of 128, 512 x (16 .. 64) 97 -> 51, 256 x (1024 .. 2048) 590 -> 555, 64 x (512 .. 4096) 224 -> 213, 16 x
 //   (1000 .. 4000) 64 -> 68; 32 x (4096 .. 16384) 444 -> 434; 32 on 16, 512 x (16 .. 64) 54 -> 41, x (64 .. 256) 85 -> 88
 template <int MODE>
-static bool lanesPay(int64_t perKv, bool wholeLoads, bool partRows, int64_t bytes, int64_t rows, int64_t maxLen) {
+static bool lanesPay(int64_t perKv, int64_t kvHeads, bool wholeLoads, bool partRows, int64_t bytes, int64_t rows, int64_t maxLen) {
   if (perKv == 1) {
     if (MODE == kTaLogitsOut) return rows >= 1024 && maxLen <= 128 && rows >= 16 * maxLen;
     if (MODE == kTaReduceV) return rows >= 2048 || (rows >= 512 && rows >= 8 * maxLen) || rows * maxLen >= (int64_t)5 << 19;
-    if (wholeLoads) return partRows || bytes > 256 || rows * bytes > (int64_t)640 * 256;
+    if (wholeLoads) return partRows || bytes > 256 || rows * bytes > (int64_t)640 * 256 || (bytes <= 128 && kvHeads >= 32 && rows >= 768 && maxLen >= 1500);
     return bytes > 256 || rows * bytes >= (int64_t)2048 * 256 || (rows >= 512 && maxLen <= 128);
   }
   if (bytes <= 128 || perKv > 8) return false;
@@ -1285,7 +1286,7 @@ static diopiError_t streamChunks(diopiContextHandle_t ctx, hipStream_t stream, T
   const bool wholeLoads = a.heads % tpw == 0;
   // (decodeGroupedKernel holds slot numbers in 32 bits)
   const bool grouped = dtype != diopi_dtype_float32 && a.slots <= 0x7fffffff &&
-                       !lanesPay<MODE>(perKv, wholeLoads, partRows, bytes, batch * a.kvHeads, std::max(maxInputLen, 1));
+                       !lanesPay<MODE>(perKv, a.kvHeads, wholeLoads, partRows, bytes, batch * a.kvHeads, std::max(maxInputLen, 1));
   // (on the lanes one read of a K/V row serves four, or two, of the query heads that share it, with their softmax states
   // side by side in the lane group's registers; more sharers are dealt over several workgroups that run on the same XCD, as
   // evenly as they go)

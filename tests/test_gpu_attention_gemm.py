@@ -1119,6 +1119,7 @@ def test_token_attention_what_slot_zero_holds(ops, dev, batch, heads, kvh, d, dt
 
 @pytest.mark.parametrize("batch,heads,kvh,d,width,dtype", [
     (128, 8, 8, 128, 24, torch.bfloat16),      # a head to itself: all three forms on the lanes
+    (24, 32, 32, 64, 1500, torch.float16),     # (not many, but longer)
     (128, 9, 9, 64, 40, torch.float16),        # a head count that leaves wave loads incomplete
     (4, 3, 3, 200, 700, torch.bfloat16),       # and rows of other lengths, in splits
     (128, 32, 16, 128, 30, torch.bfloat16),    # two heads per row
