@@ -138,8 +138,8 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
   constexpr int N = Vec16<T>::N;
   constexpr int TPW = 64 / LPT;  // tokens per wave-wide load
   constexpr bool kNeedK = MODE != kTaReduceV, kNeedV = MODE != kTaLogitsOut;
-  // rows per wave in flight: 2 K + 2 V in the fused mode, 2 K or 2 V in the halves of the two-call form (at batch 64,
-  // 156 000 tokens: scores 215 us with 2, 219 with 4, 229 with 6; second half 204 with 2, 212 with 3, 221 with 4)
+  // rows per wave in flight: 2 K + 2 V in the fused mode, 2 K or 2 V in the halves of the two-call form (second half at
+  // batch 64, 156 000 tokens: 204 us with 2, 212 with 3, 221 with 4)
   constexpr int UNR = kTaUnroll;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int sub = lane % LPT, grp = lane / LPT;
@@ -185,18 +185,17 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
 
   // Two-call modes: the scores of the chunk pass through LDS, so memory sees them as whole rows of the chunk (one
   // coalesced read before the walk, one coalesced write after it) instead of four floats per wave and row on the way
-  // (at batch 64, 156 000 tokens: scores 225 -> 219 us, second half 234 -> 205 us). Chunks longer than the buffer
+  // (second half at batch 64, 156 000 tokens: 234 -> 205 us). Chunks longer than the buffer
   // (sequences past 131 072 tokens) keep the direct accesses.
   constexpr int kLdsScores = 1024;
   __shared__ float sbuf[MODE != kTaFused ? QPK * kLdsScores : 1];
   const bool useLds = MODE != kTaFused && a.chunk <= kLdsScores;
   // The slot indices of a 512-token chunk take the same way in those modes: one coalesced read of the chunk's piece of
   // b_loc, then the walk finds its slots in LDS instead of asking memory for one index per wave and row (indices
-  // outside the pool are stored as -1): scores 216 -> 209 us, second half 205 -> 199 us at batch 64; 621 -> 595 and
-  // 565 -> 549 us at batch 256 (8 x 4096 tokens, one round of workgroups: 48.5 -> 50.4 us). Not for the shorter chunks
-  // of small batches, where the wait for the whole piece before the first row is requested weighs more, and not for
-  // the fused mode, whose time moves by a few percent either way with anything that shifts the tail of the grid
-  // (batch 64: 371 -> 392 us, batch 256: 1045 -> 1022 us, 8 x 4096: 90.6 -> 96.7 us).
+  // outside the pool are stored as -1): second half 205 -> 199 us at batch 64, 565 -> 549 at batch 256. Not for the
+  // shorter chunks of small batches, where the wait for the whole piece before the first row is requested weighs more,
+  // and not for the fused mode, whose time moves by a few percent either way with anything that shifts the tail of the
+  // grid (batch 64: 371 -> 392 us, batch 256: 1045 -> 1022 us).
   __shared__ int sidx[MODE != kTaFused ? kLdsScores : 1];
   const bool idxInLds = MODE != kTaFused && a.chunk >= kTaChunk && a.chunk <= kLdsScores && a.slots <= 0x7fffffff;
   if (idxInLds) {
@@ -430,10 +429,11 @@ __global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* 
 // ------------------------------------------------ grouped-query layouts: the matrix pipe --
 // 16-bit K/V rows shared by 1 to 16 query heads. Cut into lanes (the kernel above), every head costs its own dot
 // products, lane reductions and exponentials per row; here both products of a tile of 16 tokens are matrix products with
-// the heads as columns (unused columns idle: the pipe is busy for 190 of the 1600 cycles a tile's 8 KiB take to arrive).
+// the heads as columns (unused columns idle: at 64 sequences, 32 query heads on 8, the pipe is busy for 8 % of the cycles and
+// the vector ALUs issue in 28 %, in the lanes' kernel in 64 %; no LDS bank conflicts).
 // Bound by memory: 128 KiB are in flight on a CU. bf16, 128 per head, sequences of 512 ... 4096 tokens, lanes -> this (us):
-// 48 sequences, 32 query heads on 8 K/V heads: fused 116 -> 91 (5.2 TB/s), scores 59 -> 50, second half 84 -> 57; 64 sequences,
-// 64 heads on 8: 265 -> 130, 131 -> 75, 180 -> 88; fp16, 16 x (64 .. 2048), 32 on 8: 37.5 -> 22.6, 18.7 -> 11.3, 34.8 -> 15.9.
+// 48 sequences, 32 query heads on 8 K/V heads: fused 116 -> 88 (5.2 TB/s), scores 59 -> 50, second half 84 -> 57; 64 sequences,
+// 64 heads on 8: 241 -> 119, 118 -> 70, 171 -> 83; fp16, 16 x (64 .. 2048), 32 on 8: 30.5 -> 20.7, 17.0 -> 9.2, 29.4 -> 16.6.
 //   * S^T = K . Q^T (16x16x32): a lane holds four tokens' scores of ONE head, so the softmax runs in the lane, and its
 //     probabilities are, as they lie in the registers, the operand P^T of O^T += V^T . P^T (16x16x32: a probability as
 //     several 16-bit numbers, each the rounding of what the ones before it leave, against the same four tokens of V). In
@@ -1172,8 +1172,9 @@ static void chooseChunk(TaArgs* a, int64_t groupsPerSeq, int64_t batch, int maxI
   // A workgroup of the lanes' kernel walks its chunk with two loads per wave in flight, so the rate comes from the number
   // of workgroups a CU holds at once. Few sequences or short ones are cut into smaller chunks until there are about
   // kTaWgsPerCu workgroups per CU; large batches keep the 512-token chunks, whose partial results are fewer. Measured (us,
-  // 32 heads x 128, bf16, with 512-token chunks -> with these): 1 x 32768 130 -> 96, 4 x (100 .. 16384) 123 -> 86,
-  // 64 x (256 .. 512) 101 -> 80; 64 x (512 .. 4096) and 256 x (1024 .. 2048) keep their chunks.
+  // with 512-token chunks -> with these): 32 heads of 128, fp32, 1 x 2048 71 -> 24, bf16, 64 x (256 .. 512) 95 -> 73; 8 heads of
+  // 256, bf16, 4 x (2048 .. 4096) 79 -> 30. Four workgroups of 512 tokens on a CU are faster than the eight this makes of
+  // them: fp32, 1 x 32768 170 -> 190, 8 x 4096 169 -> 186. 64 x (512 .. 4096) and 256 x (1024 .. 2048) keep their chunks.
   // The grouped kernel has 128 KiB in flight on a CU with two workgroups and aims for those: against eight, 32 query heads
   // on 8 K/V heads, 8 x 4096 tokens 37.4 -> 28.8 us, 16 x (64 .. 2048) 27.4 -> 22.8; four: 30.9 and 23.6.
   const int64_t groups = groupsPerSeq * batch, cus = computeUnits(), len = std::max(maxInputLen, 1);
@@ -1272,7 +1273,7 @@ static bool lanesPay(int64_t perKv, int64_t kvHeads, bool wholeLoads, bool partR
 }
 
 // staticScratch: partial results go to the library's own device array instead of workspace from the context.
-// Launches decodeSplitKernel in one of its modes over (head groups, chunks, sequences) and, for the modes that produce
+// Launches decodeSplitKernel or decodeGroupedKernel in one mode over (head groups, chunks, sequences) and, for the modes that produce
 // the attention output, merges the chunks. scoresF32: the stored scores of the two-call modes are float32 (else T).
 template <int MODE>
 static diopiError_t streamChunks(diopiContextHandle_t ctx, hipStream_t stream, TaArgs a, diopiDtype_t dtype, int64_t bytes,

@@ -897,14 +897,14 @@ def test_token_attention_len_one_and_gqa(ops, dev, heads, kvh):
 
 
 @pytest.mark.parametrize("heads,kvh,dtype,d,idt", [
-    (32, 8, torch.bfloat16, 128, torch.int32),    # four query heads per K/V row read, products on packed pairs
-    (16, 8, torch.float16, 64, torch.int64),      # two per read, 8 lanes per head row
-    (64, 8, torch.bfloat16, 128, torch.int32),    # eight sharers: two workgroups of four per K/V head
-    (8, 1, torch.float32, 64, torch.int32),       # one K/V head for all; fp32 rows take the unpacked arithmetic
-    (8, 2, torch.float16, 256, torch.int32),      # 32 lanes per head row
-    (12, 4, torch.bfloat16, 128, torch.int32),    # three sharers in a group with four places
-    (28, 4, torch.bfloat16, 128, torch.int64),    # seven sharers: a group of four and a group of three per K/V head
-    (10, 2, torch.float16, 128, torch.int32),     # five: three and two
+    (32, 8, torch.bfloat16, 128, torch.int32),    # 16-bit rows so few: the matrix pipe, here four of its 16 columns in use
+    (16, 8, torch.float16, 64, torch.int64),      # two, 128-byte rows
+    (64, 8, torch.bfloat16, 128, torch.int32),    # eight
+    (8, 1, torch.float32, 64, torch.int32),       # fp32 rows: the lanes; one K/V head for all, two workgroups of four heads
+    (8, 2, torch.float16, 256, torch.int32),      # 512-byte rows
+    (12, 4, torch.bfloat16, 128, torch.int32),    # three
+    (28, 4, torch.bfloat16, 128, torch.int64),    # seven
+    (10, 2, torch.float16, 128, torch.int32),     # five
 ])
 def test_token_attention_grouped_query_layouts(ops, dev, heads, kvh, dtype, d, idt):
     """Fused and two-call decode attention with fewer K/V heads than query heads, over sequences of 1 to 1500 tokens
@@ -942,7 +942,7 @@ def test_token_attention_grouped_query_layouts(ops, dev, heads, kvh, dtype, d, i
 
 
 @pytest.mark.parametrize("heads,kvh,d,dtype", [
-    (5, 5, 128, torch.bfloat16),     # a head count that is no multiple of four heads per wave load: the matrix pipe at any batch
+    (5, 5, 128, torch.bfloat16),     # a head count that is no multiple of four heads per wave load: the matrix pipe below 2048 pairs
     (8, 8, 64, torch.float16),       # few pairs of whole rows
     (16, 1, 128, torch.float16),     # all 16 columns of the products in use
     (17, 1, 128, torch.bfloat16),    # two workgroups of 9 and 8 heads
