@@ -126,12 +126,19 @@ __device__ __forceinline__ float dotPair(uint32_t a, uint32_t b, float c) {
 // softmax and the sum over V from scores computed earlier (second half of the two-call form).
 enum TaMode { kTaFused = 0, kTaLogitsOut = 1, kTaReduceV = 2 };
 
+// Waves per SIMD that decodeSplitKernel's registers have to leave room for. What a CU has in flight is its workgroups, and the
+// fused forms of one head just fit: with the two to four registers that the compiler takes more by itself, one workgroup less,
+// 15 x (1925 .. 7700) tokens, 40 heads of 96 in bf16, takes 253 us, so 206; 8 x 4096, 32 heads of 48 in fp32 76, so 68.
+constexpr int splitWavesPerSimd(size_t itemsize, int lpt, bool hiw, int mode, int qpk, bool part) {
+  return mode != kTaFused || qpk > 1 || lpt > 16 || (hiw && !part) ? 1 : itemsize == 2 ? 7 : 8;
+}
+
 // T: bf16_t / half_t (8 per 16 B) or float (4 per 16 B). LPT lanes cover one head row. LT: the type of the scores
 // in memory (the two-call modes). QPK: query heads that share this workgroup's K/V head and are all served from one read
 // of its rows (grouped-query layouts; 1 otherwise). With QPK > 1 the grid is one-dimensional and decoded so that the
 // workgroups that share a K/V head's rows run next to each other on one XCD.
 template <typename T, int LPT, bool HIW, int MODE = kTaFused, typename LT = float, int QPK = 1, bool PART = false>
-__global__ __launch_bounds__(kTaWaves * 64) void decodeSplitKernel(TaArgs a, T* __restrict__ out,
+__global__ __launch_bounds__(kTaWaves * 64, splitWavesPerSimd(sizeof(T), LPT, HIW, MODE, QPK, PART)) void decodeSplitKernel(TaArgs a, T* __restrict__ out,
                                                                      float* __restrict__ partial) {
   static_assert(QPK == 1 || !HIW, "several query heads per lane group: the lane groups of a wave take tokens, not heads");
   using V = typename Vec16<T>::type;
