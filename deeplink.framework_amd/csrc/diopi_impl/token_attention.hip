@@ -1247,36 +1247,48 @@ using namespace amd;
 // per read of a row). rows: (sequence, K/V head) pairs, each read by perKv query heads; bytes: of the layout of a head row.
 // The matrix pipe has the shorter way from a row to a result, the more so the more heads share it, and 128 KiB in flight on
 // a CU; but two workgroups fill the CU (one with fused rows of 512 bytes), and each waits for its length, its slots and its
-// first tile in turn. So the lanes, eight workgroups on a CU, win where there are many rows for their length; with rows of
-// 512 bytes from fewer rows on; and with a query head alone on its K/V head, which leaves 15 of 16 matrix columns idle, where
-// a wave's load is a contiguous KiB of a token (wholeLoads: the head count allows it) or where the launch is long. The lines lie
-// where the two are alike in a sweep over 16 to 16384 rows of 64 to 16384 tokens, bf16. In us, matrix pipe -> lanes:
+// first tile in turn. So the lanes, eight workgroups on a CU, win over short sequences, whose workgroups are nothing but that
+// wait; where there are many rows for their length; with rows of 512 bytes from fewer rows on; and with a query head alone on
+// its K/V head, which leaves 15 of 16 matrix columns idle, where a wave's load is a contiguous KiB of a token (wholeLoads: the
+// head count allows it) or where the launch is long. More than eight sharers are the pipe's. The lines lie where the two are
+// alike in sweeps over 4 to 16384 rows of 8 to 16384 tokens, bf16 and fp16; over 2300 shapes, most of up to 200 tokens, the choice
+// costs 1.4 % (fused), 0.4 % (scores) and 0.2 % (second half) against the faster of the two. In us, matrix pipe -> lanes:
 //   fused: 32 heads of 128 alone: 512 x (16 .. 64) tokens 154 -> 61, 64 x (512 .. 4096) 426 -> 382, 24 x (200 .. 1000), 40 heads,
-//   59 -> 57; not 8 x (256 .. 2048), 40 heads (44.5 -> 48.5), 1 x 1777 (13.7 -> 19.6). 30 heads, 256 x (50 .. 300) 141 -> 127. 32 heads of
-//   64, a row of which is 128 bytes here and there: 32 x (1000 .. 4000) 125 -> 111, 24 x (1500 .. 3000) 93 -> 81. 32 heads on 16:
-//   512 x (16 .. 64) 80 -> 50, 128 x (64 .. 256) 40 -> 44. Heads of 256: 32 on 16, 128 x (512 .. 2048) 554 -> 490, 32 x (16 .. 64) 18 ->
-//   14; 32 on 8, 512 x (16 .. 64) 113 -> 64, 128 x (32 .. 128) 41 -> 37, 128 x (64 .. 256) 58 -> 63; 64 on 8, 512 x (16 .. 64) 128 -> 113
-//   scores: 32 heads of 128, 512 x (16 .. 64) 63 -> 42, x (64 .. 256) 126 -> 133; 32 on 16 35 -> 29
+//   59 -> 57; not 8 x (256 .. 2048), 40 heads (44.5 -> 48.5), 1 x 1777 (13.7 -> 19.6). 8 heads, 74 x (13 .. 26) 8.8 -> 5.3; 30 heads, 256 x
+//   (50 .. 300) 141 -> 127, 9 x 62 6.8 -> 6.2. 32 heads of 64, a row of which is 128 bytes here and there: 32 x (1000 .. 4000) 125 -> 111,
+//   24 x (1500 .. 3000) 93 -> 81. 32 heads on 16: 512 x (16 .. 64) 80 -> 50, 128 x (64 .. 256) 40 -> 44. Heads of 256: 32 on 16, 128 x
+//   (512 .. 2048) 554 -> 490, 32 x (16 .. 64) 18 -> 14; 32 on 8, 512 x (16 .. 64) 113 -> 64; 64 on 8, 140 x 30 38 -> 27, 378 x 21 89 -> 59
+//   scores: 32 heads of 128, 512 x (16 .. 64) 63 -> 42, x (64 .. 256) 126 -> 133; 32 on 16 35 -> 29; 12 on 4, 444 x (16 .. 32) 10.0 -> 8.1
 //   second half: 32 heads of 128, 512 x (16 .. 64) 97 -> 51, 256 x (1024 .. 2048) 590 -> 555, 64 x (512 .. 4096) 224 -> 213, 16 x
-//   (1000 .. 4000) 64 -> 68; 32 x (4096 .. 16384) 444 -> 434; 32 on 16, 512 x (16 .. 64) 54 -> 41, x (64 .. 256) 85 -> 88
+//   (1000 .. 4000) 64 -> 68; 32 x (4096 .. 16384) 444 -> 434; 64 heads, 7 x (9 .. 18) 5.7 -> 4.5; 64 heads of 256, 5 x 12 6.3 -> 4.1
 template <int MODE>
 static bool lanesPay(int64_t perKv, int64_t kvHeads, bool wholeLoads, bool partRows, int64_t bytes, int64_t rows, int64_t maxLen) {
+  constexpr int64_t kAny = INT64_MAX;
+  const bool wide = bytes > 256;
+  // from `least` rows on, `perToken` for each token of the longest sequence, which has up to `tokens`
+  auto many = [&](int64_t least, int64_t perToken, int64_t tokens) { return rows >= least && rows >= perToken * maxLen && maxLen <= tokens; };
   if (perKv == 1) {
-    if (MODE == kTaLogitsOut) return rows >= 1024 && maxLen <= 128 && rows >= 16 * maxLen;
-    if (MODE == kTaReduceV) return rows >= 2048 || (rows >= 512 && rows >= 8 * maxLen) || rows * maxLen >= (int64_t)5 << 19;
-    if (wholeLoads) return partRows || bytes > 256 || rows * bytes > (int64_t)640 * 256 || (bytes <= 128 && kvHeads >= 32 && rows >= 768 && maxLen >= 1500);
-    return bytes > 256 || rows * bytes >= (int64_t)2048 * 256 || (rows >= 512 && maxLen <= 128);
+    if (MODE == kTaLogitsOut) return maxLen <= 32 || (wide ? many(512, 12, 128) : many(1024, 16, 128));
+    if (MODE == kTaReduceV) return maxLen <= (wide ? 48 : 64) || rows >= 2048 || many(512, 8, kAny) || rows * maxLen >= (int64_t)5 << 19;
+    if (wide) return true;
+    if (!wholeLoads) return maxLen <= 64 || rows * bytes >= (int64_t)2048 * 256 || many(512, 0, 128);
+    return partRows || maxLen <= 24 || rows * bytes > (int64_t)640 * 256 || (rows * bytes >= (int64_t)512 * 256 && maxLen <= 64) ||
+           (bytes <= 128 && kvHeads >= 32 && rows >= 768 && maxLen >= 1500);
   }
   if (bytes <= 128 || perKv > 8) return false;
-  const bool wide = bytes > 256;
   if (MODE == kTaFused) {
-    if (perKv == 2) return wide ? rows >= 256 || rows * maxLen >= 1 << 16 : rows >= 2048 && rows >= (maxLen <= 128 ? 16 : 32) * maxLen;
-    if (perKv <= 4) return wide && rows >= 1024 && rows >= (maxLen <= 128 ? 8 : 16) * maxLen;
-    return wide && rows >= 4096 && maxLen <= 64;
+    if (perKv == 2) return wide ? maxLen <= 48 || rows >= 256 || rows * maxLen >= 1 << 16 : many(512, 8, 96) || many(2048, 16, 128) || many(2048, 32, kAny);
+    if (perKv <= 4) return wide ? maxLen <= 16 || many(256, 4, 128) || many(2048, 12, 256) || many(1024, 16, kAny) : many(2048, 0, 32);
+    return wide && (maxLen <= 16 || many(256, 0, 32) || many(512, 16, 64) || many(2048, 0, 80));
   }
-  if (perKv == 2) return rows >= 2048 && rows >= 32 * maxLen && (MODE == kTaReduceV || maxLen <= 128);
-  if (MODE == kTaReduceV) return wide && perKv > 4 && rows >= 4096 && maxLen <= 64;
-  return perKv <= 4 ? rows >= 4096 && maxLen <= 64 : wide && rows >= 2048 && maxLen <= 64;
+  if (MODE == kTaLogitsOut) {
+    if (perKv == 2) return wide ? maxLen <= 16 || many(512, 12, 96) || many(2048, 32, 128) : many(1024, 32, 128);
+    if (perKv <= 4) return wide ? many(512, 24, 96) : many(1024, 24, 64);
+    return wide && (perKv > 6 ? many(256, 0, 32) || many(512, 16, 64) || many(2048, 0, 80) : many(512, 0, 16));
+  }
+  if (perKv == 2) return wide ? maxLen <= 16 || many(512, 12, 128) || many(2048, 32, kAny) : many(1024, 24, 128) || many(2048, 32, kAny);
+  if (perKv <= 4) return wide && many(512, 32, 48);
+  return wide && perKv > 6 && (many(256, 0, 32) || many(512, 16, 64));
 }
 
 // staticScratch: partial results go to the library's own device array instead of workspace from the context.

@@ -1127,9 +1127,15 @@ def test_token_attention_what_slot_zero_holds(ops, dev, batch, heads, kvh, d, dt
     (2, 8, 4, 256, 8300, torch.bfloat16),      # long sequences of rows of 512 bytes: the fused form
     (128, 32, 8, 256, 24, torch.float16),      # four
     (512, 56, 8, 192, 10, torch.bfloat16),     # seven
+    (520, 12, 4, 128, 32, torch.bfloat16),     # three
+    (9, 30, 30, 128, 62, torch.bfloat16),      # short sequences: a head to itself, from few rows on
+    (3, 8, 8, 128, 24, torch.float16),
+    (5, 64, 64, 256, 12, torch.bfloat16),
+    (3, 16, 8, 256, 16, torch.float16),        # two
+    (140, 64, 8, 256, 30, torch.float16),      # eight
 ])
 def test_token_attention_many_rows_on_the_lanes(ops, dev, batch, heads, kvh, d, width, dtype):
-    """16-bit rows that are many for their length, and those of 512 bytes: fused, and the two calls with scores in fp32 and in
+    """16-bit rows that are many for their length, short ones, and those of 512 bytes: fused, and the two calls with scores in fp32 and in
     the type of the rows, sequences of one token up to the widest."""
     gen = g(90)
     slots = batch * width + 5
