@@ -27,9 +27,9 @@
 //     wave butterflies, then through LDS, then across chunks by a small lane-parallel second kernel.
 //
 // The two halves of the two-call form (scores to memory, then softmax and the sum over V from stored scores) are the same
-// streaming kernel with the other half of the work compiled out. Most 16-bit rows that several query heads share, and the
-// two-call form and the fused one of 16-bit rows where there are few (sequence, head) pairs, run on the matrix pipe
-// instead (decodeGroupedKernel; lanesPay draws the lines). fp32 rows run on the streaming kernel in every form.
+// streaming kernel with the other half of the work compiled out. Most 16-bit rows that several query heads share, and those of
+// a head alone where there are few (sequence, head) pairs, run on the matrix pipe instead, short sequences apart
+// (decodeGroupedKernel; lanesPay draws the lines). fp32 rows run on the streaming kernel in every form.
 //
 // Head rows of whole 16-byte pieces up to 512 bytes at 16-byte aligned strides take the kernels above (rows of other
 // lengths than 128, 256 or 512 bytes on the layout of the next of those, the places past the row's end masked); any
@@ -1250,9 +1250,9 @@ using namespace amd;
 // first tile in turn. So the lanes, eight workgroups on a CU, win over short sequences, whose workgroups are nothing but that
 // wait; where there are many rows for their length; with rows of 512 bytes from fewer rows on; and with a query head alone on
 // its K/V head, which leaves 15 of 16 matrix columns idle, where a wave's load is a contiguous KiB of a token (wholeLoads: the
-// head count allows it) or where the launch is long. More than eight sharers are the pipe's. The lines lie where the two are
-// alike in sweeps over 4 to 16384 rows of 8 to 16384 tokens, bf16 and fp16; over 2300 shapes, most of up to 200 tokens, the choice
-// costs 1.4 % (fused), 0.4 % (scores) and 0.2 % (second half) against the faster of the two. In us, matrix pipe -> lanes:
+// head count allows it) or where the launch is long. More than eight sharers, and rows of 128 bytes with any, are the pipe's.
+// The lines lie where the two are alike in sweeps over 4 to 16384 rows of 8 to 16384 tokens, bf16 and fp16; over 2300 shapes, most
+// of up to 200 tokens, the choice costs 1.4 % (fused), 0.3 % (scores) and 0.2 % (second half) against the faster of the two. In us, matrix pipe -> lanes:
 //   fused: 32 heads of 128 alone: 512 x (16 .. 64) tokens 154 -> 61, 64 x (512 .. 4096) 426 -> 382, 24 x (200 .. 1000), 40 heads,
 //   59 -> 57; not 8 x (256 .. 2048), 40 heads (44.5 -> 48.5), 1 x 1777 (13.7 -> 19.6). 8 heads, 74 x (13 .. 26) 8.8 -> 5.3; 30 heads, 256 x
 //   (50 .. 300) 141 -> 127, 9 x 62 6.8 -> 6.2. 32 heads of 64, a row of which is 128 bytes here and there: 32 x (1000 .. 4000) 125 -> 111,
