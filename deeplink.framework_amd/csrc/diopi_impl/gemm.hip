@@ -312,24 +312,6 @@ __device__ __forceinline__ void ldsBarrier() {
 constexpr int kDeepStages = 4;  // K tiles in the LDS ring of the 128 x 128 form with one workgroup per CU
 constexpr int kPipeWavesM = 2, kPipeWavesN = 4, kPipeThreads = kPipeWavesM * kPipeWavesN * 64;
 
-// v_mfma_f32_16x16x32: lane l feeds row (l & 15), K elements [8 * (l >> 4), +8) of both operands and
-// receives D[4 * (l >> 4) + r][l & 15], r = 0..3. The large-tile kernel passes the weight fragment
-// first, so D is the transposed block and a lane holds four consecutive columns of output row (l & 15).
-template <typename T>
-struct MfmaOp16;
-template <>
-struct MfmaOp16<bf16_t> {
-  static __device__ __forceinline__ f32x4 run(bf16x8 a, bf16x8 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-};
-template <>
-struct MfmaOp16<half_t> {
-  static __device__ __forceinline__ f32x4 run(f16x8 a, f16x8 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-};
-
 // EPI selects the epilogue: kEpiLinear is alpha * acc + beta * C + bias; kEpiSiluMul treats every 64 consecutive
 // output columns as 32 gate columns followed by the 32 up columns of the same channels and stores
 // silu(gate) * up, half as wide (out has N / 2 columns); kEpiPartial is the split-K form: workgroup (tile, s)
@@ -2957,6 +2939,20 @@ static diopiError_t launchSkinnyWide(hipStream_t stream, const SkinnyArgs& a) {
 static bool mult8(int64_t v) { return (v & 7) == 0; }
 static bool ptr16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// The kernel for few columns a compute unit, if it pays for the product (16-bit, one batch, K of both operands contiguous).
+static diopiError_t tryNarrowStream(hipStream_t stream, const GemmProblem& p, const RotaryEpilogue* rot, bool* done) {
+  NarrowStreamArgs a;
+  a.A = p.A, a.B = p.B, a.out = p.out, a.Cin = p.Cin, a.bias = p.bias, a.biasDtype = (int)p.dtype;
+  a.lda = p.sAm, a.ldb = p.sBn, a.ldo = p.sOm, a.sCm = p.sCm, a.sCn = p.sCn;
+  a.M = (int)p.M, a.N = (int)p.N, a.K = (int)p.K, a.alpha = p.alpha, a.beta = p.beta;
+  if (rot != nullptr) {
+    a.rotCos = rot->cosT, a.rotSin = rot->sinT, a.rotCols = rot->cols, a.rotHeadDim = rot->headDim, a.rotTableRows = rot->tableRows;
+    a.rotTableF32 = rot->tableF32, a.rotSinSign = rot->sinSign;
+  }
+  *done = narrowStreamPays(a);
+  return *done ? launchNarrowStream(stream, p.dtype, a) : diopiSuccess;
+}
+
 template <typename T>
 // With `rot` (a rotary epilogue) only the LDS-staged form qualifies: *handled tells the caller whether it ran.
 static diopiError_t launchSkinnyForShape(diopiContextHandle_t ctx, hipStream_t stream, const GemmProblem& p,
@@ -2972,6 +2968,8 @@ static diopiError_t launchSkinnyForShape(diopiContextHandle_t ctx, hipStream_t s
     a.rotCos = rot->cosT, a.rotSin = rot->sinT, a.rotCols = rot->cols, a.rotHeadDim = rot->headDim, a.rotTableRows = rot->tableRows;
     a.rotTableF32 = rot->tableF32, a.rotSinSign = rot->sinSign;
   }
+  if (rot != nullptr) AMD_TRY(tryNarrowStream(stream, p, rot, handled));  // (runGemm has asked for the others)
+  if (rot != nullptr && *handled) return diopiSuccess;
   const int tiles = (a.N + 15) / 16, cus = computeUnits(), perCu = (tiles + cus - 1) / cus;
   // Both operands through LDS, see gemmSkinnyLdsKernel. The columns are dealt evenly over as many workgroups as there
   // are CUs (43 each at N = 11008, where 64-column blocks would leave a third of the CUs idle): a CU takes in about
@@ -3232,6 +3230,11 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
       if (sbb == 0) nb = 1;  // a shared (broadcast) weight is transposed once
       AMD_TRY(launchTranspose<uint16_t>(stream, ws, p.B, nb, p.K, p.N, p.sBk, p.sBn, sbb));
       p.B = ws, p.sBk = 1, p.sBn = p.K, p.sBb = (sbb == 0) ? 0 : p.N * p.K;
+    }
+    if (p.batch == 1 && p.M <= 32 && p.K <= 0x7fffffff) {
+      bool done = false;
+      AMD_TRY(tryNarrowStream(stream, p, nullptr, &done));
+      if (done) return diopiSuccess;
     }
     // up to 32 rows always; up to 64 while N is moderate or K is long enough for the whole-K form (measured at 64
     // rows, K = 4096: K-split form + reduction pass 16 us against 50 us for the split-K tiled kernel at N = 4096, 36

@@ -38,6 +38,71 @@ struct GemmProblem {
 
 diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p);
 
+#ifdef __HIPCC__
+// v_mfma_f32_16x16x32: lane l feeds row (l & 15), K elements [8 * (l >> 4), +8) of both operands and
+// receives D[4 * (l >> 4) + r][l & 15], r = 0..3. The large-tile kernel passes the weight fragment
+// first, so D is the transposed block and a lane holds four consecutive columns of output row (l & 15).
+template <typename T>
+struct MfmaOp16;
+template <>
+struct MfmaOp16<bf16_t> {
+  static __device__ __forceinline__ f32x4 run(bf16x8 a, bf16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct MfmaOp16<half_t> {
+  static __device__ __forceinline__ f32x4 run(f16x8 a, f16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+};
+
+// The four int8 of one dword as floats: one SDWA conversion per byte (left to itself the compiler shifts
+// bytes 1 and 3 into place first, two more VALU instructions per dword in a loop that has no slack).
+__device__ __forceinline__ void cvt4(uint32_t w, float& f0, float& f1, float& f2, float& f3) {
+  asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0" : "=v"(f0) : "v"(w));
+  asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1" : "=v"(f1) : "v"(w));
+  asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2" : "=v"(f2) : "v"(w));
+  asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3" : "=v"(f3) : "v"(w));
+}
+
+// converts 8 consecutive int8 (two dwords) to an MFMA operand fragment
+template <typename T>
+__device__ __forceinline__ typename Vec16<T>::type int8Fragment(uint32_t lo, uint32_t hi) {
+  float f[8];
+  cvt4(lo, f[0], f[1], f[2], f[3]);
+  cvt4(hi, f[4], f[5], f[6], f[7]);
+  typename Vec16<T>::type r;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) r[j] = static_cast<T>(f[j]);
+  return r;
+}
+#endif
+
+// narrow_stream.hip: products of at most 32 rows whose columns are few for each compute unit.
+// out[m, n] = (alpha, or scale[n]) * sum + bias[n] + beta * Cin[m, n], then the interleaved rotary embedding on the leading rotCols columns.
+struct NarrowStreamArgs {
+  const void* A = nullptr;
+  const void* B = nullptr;  // of the type of A, or int8
+  void* out = nullptr;
+  const void* Cin = nullptr;
+  const void* scale = nullptr;
+  const void* bias = nullptr;
+  int64_t lda = 0, ldb = 0, ldo = 0, sCm = 0, sCn = 0;
+  int M = 0, N = 0, K = 0;
+  bool int8B = false;
+  int scaleDtype = 0, biasDtype = 0;
+  float alpha = 1.f, beta = 0.f;
+  const void* rotCos = nullptr;
+  const void* rotSin = nullptr;
+  int rotCols = 0, rotHeadDim = 2, rotTableRows = 1;
+  bool rotTableF32 = false;
+  float rotSinSign = 1.f;
+  int colsPerWg = 0;
+};
+bool narrowStreamPays(const NarrowStreamArgs& a);
+diopiError_t launchNarrowStream(hipStream_t stream, diopiDtype_t dtype, NarrowStreamArgs a);
+
 // Whether runGemm would send p to the kernel whose epilogue can multiply every column by a scale of its own (the
 // 4-wave large-tile kernel): the caller sets colScale only then, and applies the scale in a pass of its own otherwise.
 // What it settles and reserves for that stays in *p, which then goes to runGemm.

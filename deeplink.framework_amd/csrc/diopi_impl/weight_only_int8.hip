@@ -26,23 +26,6 @@
 
 namespace amd {
 
-template <typename T>
-struct W8Mfma;
-template <>
-struct W8Mfma<bf16_t> {
-  typedef bf16x8 Frag;
-  static __device__ __forceinline__ f32x4 run(Frag a, Frag b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-};
-template <>
-struct W8Mfma<half_t> {
-  typedef f16x8 Frag;
-  static __device__ __forceinline__ f32x4 run(Frag a, Frag b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-};
-
 struct W8Args {
   const void* x;
   const int8_t* w;
@@ -60,27 +43,6 @@ struct W8Args {
   int stagesPerSlice = 0;
 };
 
-// The four int8 of one dword as floats: one SDWA conversion per byte (left to itself the compiler shifts
-// bytes 1 and 3 into place first, two more VALU instructions per dword in a loop that has no slack).
-__device__ __forceinline__ void cvt4(uint32_t w, float& f0, float& f1, float& f2, float& f3) {
-  asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0" : "=v"(f0) : "v"(w));
-  asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1" : "=v"(f1) : "v"(w));
-  asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2" : "=v"(f2) : "v"(w));
-  asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3" : "=v"(f3) : "v"(w));
-}
-
-// converts 8 consecutive int8 (two dwords) to an MFMA operand fragment
-template <typename T>
-__device__ __forceinline__ typename W8Mfma<T>::Frag cvt8(uint32_t lo, uint32_t hi) {
-  float f[8];
-  cvt4(lo, f[0], f[1], f[2], f[3]);
-  cvt4(hi, f[4], f[5], f[6], f[7]);
-  typename W8Mfma<T>::Frag r;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) r[j] = static_cast<T>(f[j]);
-  return r;
-}
-
 constexpr int kW8Block = 128;   // K elements one wave consumes per step (4 kgrps x 32)
 // One step (two 16-byte loads per lane) is in flight ahead of the one being multiplied, no more: measured,
 // a deeper queue is slower (9.7 us with four steps ahead, 10.4 with eight, 8.8 with one or two at M = 1).
@@ -93,7 +55,7 @@ constexpr int kW8RowsK = 16 * 4096; // staged rows x columns per pass: 16 G x (4
 // of 4096 / G columns so that the rows fit in LDS); more than 16 G rows go to further workgroups along grid.y.
 template <typename T, int NTW, int G>
 __global__ __launch_bounds__(NTW * kW8KSplit * 64) void w8LinearKernel(W8Args a) {
-  using Frag = typename W8Mfma<T>::Frag;
+  using Frag = typename Vec16<T>::type;
   constexpr int THREADS = NTW * kW8KSplit * 64, kW8ChunkK = kW8RowsK / (16 * G);
   extern __shared__ __attribute__((aligned(16))) char w8smem[];
   T* sx = reinterpret_cast<T*>(w8smem);
@@ -152,14 +114,14 @@ __global__ __launch_bounds__(NTW * kW8KSplit * 64) void w8LinearKernel(W8Args a)
         w0 = *reinterpret_cast<const u32x4*>(wk + (s + 1) * kW8Block);
         w1 = *reinterpret_cast<const u32x4*>(wk + (s + 1) * kW8Block + 16);
       }
-      const Frag f0 = cvt8<T>(c0[0], c0[1]), f1 = cvt8<T>(c0[2], c0[3]), f2 = cvt8<T>(c1[0], c1[1]), f3 = cvt8<T>(c1[2], c1[3]);
+      const Frag f0 = int8Fragment<T>(c0[0], c0[1]), f1 = int8Fragment<T>(c0[2], c0[3]), f2 = int8Fragment<T>(c1[0], c1[1]), f3 = int8Fragment<T>(c1[2], c1[3]);
 #pragma unroll
       for (int gi = 0; gi < G; ++gi) {
         const T* xp = xrow[gi] + s * kW8Block;
-        acc[gi] = W8Mfma<T>::run(*reinterpret_cast<const Frag*>(xp), f0, acc[gi]);
-        acc[gi] = W8Mfma<T>::run(*reinterpret_cast<const Frag*>(xp + 8), f1, acc[gi]);
-        acc[gi] = W8Mfma<T>::run(*reinterpret_cast<const Frag*>(xp + 16), f2, acc[gi]);
-        acc[gi] = W8Mfma<T>::run(*reinterpret_cast<const Frag*>(xp + 24), f3, acc[gi]);
+        acc[gi] = MfmaOp16<T>::run(*reinterpret_cast<const Frag*>(xp), f0, acc[gi]);
+        acc[gi] = MfmaOp16<T>::run(*reinterpret_cast<const Frag*>(xp + 8), f1, acc[gi]);
+        acc[gi] = MfmaOp16<T>::run(*reinterpret_cast<const Frag*>(xp + 16), f2, acc[gi]);
+        acc[gi] = MfmaOp16<T>::run(*reinterpret_cast<const Frag*>(xp + 24), f3, acc[gi]);
       }
     }
   }
@@ -209,7 +171,7 @@ constexpr int kW8LdsStagger = 13;
 
 template <typename T, int G, int NTP, int BK, int WST, int XST>
 __global__ __launch_bounds__(512) void w8LinearLdsKernel(W8Args a) {
-  using Frag = typename W8Mfma<T>::Frag;
+  using Frag = typename Vec16<T>::type;
   constexpr int BN = 32 * NTP;
   constexpr int LW = BK / 16, LX = BK * (int)sizeof(T) / 16;   // 16-byte pieces (= lanes of a copy instruction) per weight / activation row
   constexpr int RW = 64 / LW, RX = 64 / LX;                    // rows one copy instruction covers
@@ -336,11 +298,11 @@ __global__ __launch_bounds__(512) void w8LinearLdsKernel(W8Args a) {
 #pragma unroll
           for (int j = 0; j < NTP; ++j) {
             const u32x4 w = *reinterpret_cast<const u32x4*>(wlane[pp] + (u % WST) * WBUF + j * 16 * BK);
-            const Frag f0 = cvt8<T>(w[0], w[1]), f1 = cvt8<T>(w[2], w[3]);
+            const Frag f0 = int8Fragment<T>(w[0], w[1]), f1 = int8Fragment<T>(w[2], w[3]);
 #pragma unroll
             for (int gi = 0; gi < G; ++gi) {
-              acc[gi][j] = W8Mfma<T>::run(x0[gi], f0, acc[gi][j]);
-              acc[gi][j] = W8Mfma<T>::run(x1[gi], f1, acc[gi][j]);
+              acc[gi][j] = MfmaOp16<T>::run(x0[gi], f0, acc[gi][j]);
+              acc[gi][j] = MfmaOp16<T>::run(x1[gi], f1, acc[gi][j]);
             }
           }
         }
@@ -455,8 +417,6 @@ static diopiError_t launchW8ForTiles(hipStream_t stream, const W8Args& a) {
 // 64 x 8192 x 28672 110 -> 73 us, 16 x 8192 x 8192 23.8 -> 16.9 us).
 static int w8SlicesFor(const W8Args& a) {
   if (a.M > 64 || a.N >= 10240 || a.N < 64 || a.N % 4 != 0 || a.K % 256 != 0 || a.K < (a.M <= 16 ? 8192 : 2048)) return 0;
-  // (a few rows against a large weight of medium width stream well as they are: 1 x 8192 x 28672 35.6 us, 39.4 in slices)
-  if (a.M <= 4 && a.N >= 6144 && (int64_t)a.N * a.K >= ((int64_t)1 << 27)) return 0;
   if ((int64_t)(a.N - 1) * a.ldw + a.K >= ((int64_t)1 << 31) || a.ldo % 4 != 0) return 0;
   const int wgs = (a.N + 63) / 64, stages = a.K / 256;
   const int want = std::max(1, computeUnits() / wgs);
@@ -678,6 +638,15 @@ extern "C" __attribute__((visibility("default"))) diopiError_t diopiWeightOnlyIn
   a.ldx = K, a.ldw = N > 1 ? cw.stride[0] : K, a.ldo = N;
   a.M = (int)M, a.N = (int)N, a.K = (int)K;
   a.scaleDtype = csc.dtype, a.biasDtype = bias.defined() ? cb.dtype : diopi_dtype_float32;
+  NarrowStreamArgs narrow;
+  narrow.A = a.x, narrow.B = a.w, narrow.out = a.out, narrow.scale = a.scale, narrow.bias = a.bias;
+  narrow.lda = a.ldx, narrow.ldb = a.ldw, narrow.ldo = a.ldo, narrow.M = a.M, narrow.N = a.N, narrow.K = a.K;
+  narrow.int8B = true, narrow.scaleDtype = a.scaleDtype, narrow.biasDtype = a.biasDtype;
+  if (narrowStreamPays(narrow)) {
+    AMD_TRY(launchNarrowStream(stream, in.dtype, narrow));
+    if (outTemp) AMD_TRY(stridedCopy(stream, cout, out));
+    return diopiSuccess;
+  }
   if (const int slices = w8SlicesFor(a); slices > 0 && cin.aligned16() && cw.aligned16() && a.ldw % 16 == 0 && cout.aligned16() &&
                                            (std::min<int64_t>(M, 64) * K + K) * 2 < (int64_t(1) << 31)) {
     const int stages = (int)(K / 256);

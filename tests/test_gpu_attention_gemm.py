@@ -555,6 +555,46 @@ def test_skinny_m_linear_and_addmm(ops, dev, dtype, m, n, k):
     assert_exact(ops.linear(onehot, dw), dw[:, cols].t().contiguous().cpu())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(3, 16, 16), (1, 250, 16904), (16, 4096, 520), (5, 4098, 1032), (16, 8192, 512), (4, 8190, 8208), (17, 4096, 1544),
+                                   (32, 250, 8192), (32, 300, 48), (2, 4100, 1528)])
+def test_few_columns_for_a_compute_unit(ops, dev, dtype, m, n, k):
+    # the kernel that streams few columns for each compute unit over the whole of K: ragged column shares, a last stage that
+    # is not whole, fewer stages than ring places, one and two row groups; rows lie in a wider matrix of NaNs
+    wide = torch.full((m, k + 24), float("nan"), dtype=dtype)
+    wide[:, :k] = torch.randn(m, k, generator=g(1)).to(dtype)
+    x, xd = wide[:, :k], wide.to(dev)[:, :k]
+    w = (torch.randn(n, k, generator=g(2)) / k**0.5).to(dtype)
+    c, b = torch.randn(m, n, generator=g(3)).to(dtype), torch.randn(n, generator=g(4)).to(dtype)
+    want = x.double() @ w.double().t()
+    assert_half(ops.linear(xd, w.to(dev)), want)
+    assert_half(ops.linear(xd, w.to(dev), b.to(dev)), want + b.double())
+    assert_half(ops.addmm(c.to(dev), xd, w.to(dev).t(), beta=0.5, alpha=2.0), 0.5 * c.double() + 2 * want)
+    q = torch.randint(-127, 128, (n, k), generator=g(5), dtype=torch.int8)
+    scale = (torch.rand(n, generator=g(6)) + 0.5) / (73 * k**0.5)
+    want = (x.double() @ q.double().t()) * scale.half().double()
+    assert_half(ops.weight_only_int8_linear(xd, q.to(dev), scale.half().to(dev)), want)
+    assert_half(ops.weight_only_int8_linear(xd, q.to(dev), scale.half().to(dev), b.to(dev)), want + b.double())
+
+
+@pytest.mark.parametrize("table_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m,heads,hd,vcols,k", [(3, 10, 128, 2 * 128, 4096), (16, 40, 64, 1000, 1032), (17, 6, 128, 256, 768), (5, 33, 64, 130 * 8, 2048 + 128)])
+def test_rotation_with_few_columns_for_a_compute_unit(ops, dev, table_dtype, m, heads, hd, vcols, k):
+    n, cols = heads * hd + vcols, heads * hd
+    x = torch.randn(m, k, generator=g(1)).bfloat16()
+    w = (torch.randn(n, k, generator=g(2)) / k**0.5).bfloat16()
+    b = torch.randn(n, generator=g(3)).bfloat16()
+    angle = torch.rand(m, hd // 2, generator=g(4)) * 6
+    cos, sin = angle.cos().to(table_dtype), angle.sin().to(table_dtype)
+    for bias in (None, b):
+        want = x.double() @ w.double().t() + (0 if bias is None else b.double())
+        pairs = want[:, :cols].reshape(m, heads, hd // 2, 2)
+        c, s = cos.double()[:, None], sin.double()[:, None]
+        rotated = torch.stack([pairs[..., 0] * c - pairs[..., 1] * s, pairs[..., 0] * s + pairs[..., 1] * c], -1).reshape(m, cols)
+        got = ops.linear_rotary(x.to(dev), w.to(dev), cos.to(dev), sin.to(dev), cols, hd, bias=None if bias is None else b.to(dev))
+        assert_half(got, torch.cat([rotated, want[:, cols:]], 1))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("m,f,k", [(4096, 3584, 256), (3700, 4000 - 32, 192), (96, 64, 80), (1, 32, 8),
                                    (5, 2048, 256), (33, 5536, 384), (48, 16384, 128), (64, 11008, 640), (20, 8224, 256)])
