@@ -3231,7 +3231,7 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
       AMD_TRY(launchTranspose<uint16_t>(stream, ws, p.B, nb, p.K, p.N, p.sBk, p.sBn, sbb));
       p.B = ws, p.sBk = 1, p.sBn = p.K, p.sBb = (sbb == 0) ? 0 : p.N * p.K;
     }
-    if (p.batch == 1 && p.M <= 32 && p.K <= 0x7fffffff) {
+    if (p.batch == 1 && p.M <= kSkinnyMaxM && p.K <= 0x7fffffff) {
       bool done = false;
       AMD_TRY(tryNarrowStream(stream, p, nullptr, &done));
       if (done) return diopiSuccess;

@@ -79,7 +79,7 @@ __device__ __forceinline__ typename Vec16<T>::type int8Fragment(uint32_t lo, uin
 }
 #endif
 
-// narrow_stream.hip: products of at most 32 rows whose columns are few for each compute unit.
+// narrow_stream.hip: products of at most 64 rows whose columns are few for each compute unit.
 // out[m, n] = (alpha, or scale[n]) * sum + bias[n] + beta * Cin[m, n], then the interleaved rotary embedding on the leading rotCols columns.
 struct NarrowStreamArgs {
   const void* A = nullptr;

@@ -1,4 +1,4 @@
-// Decode-sized products (at most 32 rows) with few output columns for each compute unit: the o and down projections, stacked
+// Decode-sized products (at most 64 rows) with few output columns for each compute unit: the o and down projections, stacked
 // QKV projections with grouped K/V heads, in 16-bit and int8 weights.
 #include <algorithm>
 #include <type_traits>
@@ -10,10 +10,11 @@ namespace amd {
 // A workgroup owns at most 16 NT columns for the whole of K, so that there are no partial products and no reduction launch.
 //   * What bounds it is the bytes a unit has under way: HBM answers after about a microsecond, so 256 units need some 30 KB each
 //     to reach its rate. With 16 to 32 weight rows per workgroup that takes long pieces of a row: a stage is 512 columns (1 KiB
-//     of a 16-bit row, one copy instruction), and 3 to 5 of them are in the LDS ring.
+//     of a 16-bit row, one copy instruction), and 3 or 4 of them are in the LDS ring. From 33 rows on (and from 17 with two
+//     column tiles of 16 bits) it is 256 columns, as the activations' ring has to fit too.
 //   * Waves 0 - 3 copy weights, waves 4 - 7 activations: loads return to a wave in the order it issued them, so one that
 //     copied both could not keep weights out of HBM further ahead than activations out of L2. One barrier a stage publishes both.
-//   * Wave w multiplies columns 64 w .. 64 w + 63 of every stage; the eight shares meet in LDS at the end.
+//   * Wave w multiplies the w-th eighth of every stage's columns; the eight shares meet in LDS at the end.
 //   * 16-byte pieces are XOR-swizzled by row on the global side, so that the fragment reads are free of bank conflicts.
 //   * Workgroup b starts its walk over K at stage b / 8 + 4 (b % 8): the workgroups of an XCD (every eighth) read the activations,
 //     and rows of a power of two bytes, at different columns, so that the requests of a moment fall on all channels of its
@@ -26,19 +27,19 @@ constexpr int kNarrowBK = 512;
 // out of HBM under way: copies past that hold up the waves that issue them). us at one row, places 5 + 4 -> 4 + 3 (16-bit, one
 // column tile) 4096 x 4096 8.73 -> 8.35; int8, 8 + 4 -> 4 + 4, 4096 x 11008 11.60 -> 10.85; int8, two tiles, 6 + 4 -> 3 + 3, 8192 x 8192
 // 13.9 -> 12.65. Fewer lose: 16-bit 3 + 3 4096 x 11008 16.75 -> 22.7, two tiles 3 + 2 5120 x 13824 24.2 -> 27.6.
-constexpr int narrowStagesW(bool int8, int tiles) { return tiles == 1 ? 4 : 3; }
-constexpr int narrowStagesX(bool int8, int tiles) { return int8 && tiles == 1 ? 4 : 3; }
+constexpr int narrowStagesW(int tiles, int bk) { return tiles == 1 ? 4 : 3; }
+constexpr int narrowStagesX(bool int8, int tiles, int bk) { return int8 && tiles == 1 && bk == kNarrowBK ? 4 : 3; }
 
-template <typename T, bool W8, int G, int NT>
+template <typename T, bool W8, int G, int NT, int BK>
 __global__ __launch_bounds__(512) void narrowStreamKernel(NarrowStreamArgs a) {
   typedef typename Vec16<T>::type Frag;
-  constexpr int BK = kNarrowBK, kSize = W8 ? 1 : 2;                  // bytes of a weight
-  constexpr int WST = narrowStagesW(W8, NT), XST = narrowStagesX(W8, NT);    // ring places
+  constexpr int kSize = W8 ? 1 : 2, KS = BK / 256;                   // bytes of a weight; 32-wide k-steps of a wave and stage
+  constexpr int WST = narrowStagesW(NT, BK), XST = narrowStagesX(W8, NT, BK);    // ring places
   constexpr int kRowBytes = BK * kSize, kLanes = kRowBytes / 16;     // of a weight row's stage, and the lanes that copy it
   constexpr int kRows = 64 / kLanes;                                 // weight rows of a copy instruction (1 KiB)
   static_assert(16 * NT / kRows % 4 == 0, "four waves copy as many pieces each");
-  constexpr int WIPW = 16 * NT / kRows / 4, XIPW = 4 * G, IPW = WIPW > XIPW ? WIPW : XIPW;  // copy instructions of a wave and stage
-  constexpr unsigned WBUF = 16 * NT * kRowBytes, XBUF = 16 * G * 1024;
+  constexpr int WIPW = 16 * NT / kRows / 4, XIPW = 4 * G * BK / 512, IPW = WIPW > XIPW ? WIPW : XIPW;  // copy instructions of a wave and stage
+  constexpr unsigned WBUF = 16 * NT * kRowBytes, XBUF = 32 * G * BK;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   char* const sw = smem;
   char* const sx = smem + WST * WBUF;
@@ -95,9 +96,10 @@ __global__ __launch_bounds__(512) void narrowStreamKernel(NarrowStreamArgs a) {
       pieceCol[i] = piece * (16 / kSize);
       voff[i] = row < nCols ? (unsigned)((int64_t)(n0 + row) * a.ldb * kSize + piece * 16) : 0x80000000u;
     } else {
-      const int piece = lane ^ (q & 15);
+      constexpr int kXLanes = BK / 8;
+      const int row = 64 / kXLanes * q + lane / kXLanes, piece = (lane % kXLanes) ^ (row & 15);
       pieceCol[i] = piece * 8;
-      voff[i] = q < a.M ? (unsigned)((int64_t)q * a.lda * 2 + piece * 16) : 0x80000000u;
+      voff[i] = row < a.M ? (unsigned)((int64_t)row * a.lda * 2 + piece * 16) : 0x80000000u;
     }
   }
   const unsigned ldsBase = (unsigned)(size_t)(__attribute__((address_space(3))) char*)(copiesW ? sw : sx) + (unsigned)ci * 1024u;
@@ -125,37 +127,41 @@ __global__ __launch_bounds__(512) void narrowStreamKernel(NarrowStreamArgs a) {
   for (int gi = 0; gi < G; ++gi)
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[gi][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // This wave's fragments. 16-bit weights: k-step s = 2 w + t, logical piece 4 s + kgrp of both operands; int8: piece 4 w + kgrp
-  // holds 16 weights, which meet activation pieces 8 w + 2 kgrp + t.
-  unsigned xAt[2], wAt[2];
+  // This wave's fragments, columns 32 KS w of a stage on: of k-step s = KS w + t piece 4 s + kgrp of both operands; int8: 8 KS
+  // weights at 8 KS (4 w + kgrp), which meet the activations of the same columns.
+  unsigned xAt[KS], wAt[KS];
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int px = W8 ? 8 * wave + 2 * kgrp + t : 4 * (2 * wave + t) + kgrp;
-    xAt[t] = WST * WBUF + (unsigned)(r16 * 1024 + ((px ^ r16) << 4));
-    wAt[t] = (unsigned)(r16 * kRowBytes + (((W8 ? 4 * wave + kgrp : px) ^ r16) << 4));
+  for (int t = 0; t < KS; ++t) {
+    const int px = W8 ? KS * (4 * wave + kgrp) + t : 4 * (KS * wave + t) + kgrp, w8 = 8 * KS * (4 * wave + kgrp);
+    xAt[t] = WST * WBUF + (unsigned)(r16 * BK * 2 + ((px ^ r16) << 4));
+    wAt[t] = W8 ? (unsigned)(r16 * kRowBytes + (((w8 >> 4) ^ r16) << 4) + (w8 & 8)) : (unsigned)(r16 * kRowBytes + ((px ^ r16) << 4));
   }
-  Frag x[G][2];
-  u32x4 q[NT][W8 ? 1 : 2];
+  typedef typename std::conditional<W8 && KS == 1, u32x2, u32x4>::type Weights;
+  Frag x[G][KS];
+  Weights q[NT][W8 ? 1 : KS];
   auto fetch = [&](unsigned placeW, unsigned placeX) {
 #pragma unroll
     for (int gi = 0; gi < G; ++gi)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) x[gi][t] = *reinterpret_cast<const Frag*>(smem + xAt[t] + placeX * XBUF + gi * 16 * 1024);
+      for (int t = 0; t < KS; ++t) x[gi][t] = *reinterpret_cast<const Frag*>(smem + xAt[t] + placeX * XBUF + gi * 32 * BK);
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int t = 0; t < (W8 ? 1 : 2); ++t) q[j][t] = *reinterpret_cast<const u32x4*>(smem + wAt[t] + placeW * WBUF + j * 16 * kRowBytes);
+      for (int t = 0; t < (W8 ? 1 : KS); ++t) q[j][t] = *reinterpret_cast<const Weights*>(smem + wAt[t] + placeW * WBUF + j * 16 * kRowBytes);
   };
   auto multiply = [&] {
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-      Frag w[2];
-      if constexpr (W8) w[0] = int8Fragment<T>(q[j][0][0], q[j][0][1]), w[1] = int8Fragment<T>(q[j][0][2], q[j][0][3]);
-      else w[0] = __builtin_bit_cast(Frag, q[j][0]), w[1] = __builtin_bit_cast(Frag, q[j][1]);
+      Frag w[KS];
+#pragma unroll
+      for (int t = 0; t < KS; ++t) {
+        if constexpr (W8) w[t] = int8Fragment<T>(q[j][0][2 * t], q[j][0][2 * t + 1]);
+        else w[t] = __builtin_bit_cast(Frag, q[j][t]);
+      }
 #pragma unroll
       for (int gi = 0; gi < G; ++gi)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) acc[gi][j] = MfmaOp16<T>::run(x[gi][t], w[t], acc[gi][j]);
+        for (int t = 0; t < KS; ++t) acc[gi][j] = MfmaOp16<T>::run(x[gi][t], w[t], acc[gi][j]);
     }
   };
   auto walk = [&](auto weights) {
@@ -207,55 +213,66 @@ __global__ __launch_bounds__(512) void narrowStreamKernel(NarrowStreamArgs a) {
   }
 }
 
-template <typename T, bool W8, int G, int NT>
+template <typename T, bool W8, int G, int NT, int BK = kNarrowBK>
 static diopiError_t launchTiles(hipStream_t stream, const NarrowStreamArgs& a) {
-  constexpr int lds = std::max(narrowStagesW(W8, NT) * 16 * NT * kNarrowBK * (W8 ? 1 : 2) + narrowStagesX(W8, NT) * 16 * G * 1024, 8 * G * NT * 1024);
+  constexpr int lds = std::max(narrowStagesW(NT, BK) * 16 * NT * BK * (W8 ? 1 : 2) + narrowStagesX(W8, NT, BK) * 32 * G * BK, 8 * G * NT * 1024);
   static_assert(lds <= 160 * 1024, "LDS of a compute unit");
-  AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(&narrowStreamKernel<T, W8, G, NT>), lds));
-  hipLaunchKernelGGL((narrowStreamKernel<T, W8, G, NT>), dim3((unsigned)ceilDiv(a.N, a.colsPerWg)), dim3(512), lds, stream, a);
+  AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(&narrowStreamKernel<T, W8, G, NT, BK>), lds));
+  hipLaunchKernelGGL((narrowStreamKernel<T, W8, G, NT, BK>), dim3((unsigned)ceilDiv(a.N, a.colsPerWg)), dim3(512), lds, stream, a);
   AMD_LAUNCH_CHECK();
   return diopiSuccess;
+}
+
+template <typename T, bool W8, int G>
+static diopiError_t launchManyRows(hipStream_t stream, const NarrowStreamArgs& a) {
+  return a.colsPerWg <= 16 ? launchTiles<T, W8, G, 1, 256>(stream, a) : launchTiles<T, W8, G, 2, 256>(stream, a);
 }
 
 template <typename T>
 static diopiError_t launchType(hipStream_t stream, const NarrowStreamArgs& a) {
   const int tiles = (a.colsPerWg + 15) / 16;
+  if (a.M > 48) return a.int8B ? launchManyRows<T, true, 4>(stream, a) : launchManyRows<T, false, 4>(stream, a);
+  if (a.M > 32) return a.int8B ? launchManyRows<T, true, 3>(stream, a) : launchManyRows<T, false, 3>(stream, a);
   if (a.int8B) {
     if (a.M > 16) return tiles == 1 ? launchTiles<T, true, 2, 1>(stream, a) : launchTiles<T, true, 2, 2>(stream, a);
     return tiles == 1 ? launchTiles<T, true, 1, 1>(stream, a) : tiles == 2 ? launchTiles<T, true, 1, 2>(stream, a) : launchTiles<T, true, 1, 3>(stream, a);
   }
-  if (a.M > 16) return launchTiles<T, false, 2, 1>(stream, a);
+  if (a.M > 16) return tiles == 1 ? launchTiles<T, false, 2, 1>(stream, a) : launchTiles<T, false, 2, 2, 256>(stream, a);
   return tiles == 1 ? launchTiles<T, false, 1, 1>(stream, a) : launchTiles<T, false, 1, 2>(stream, a);
 }
 
-// Where this kernel is the faster one, from both sides timed over 40 weights of 256 to 16384 rows at 1 to 32 activation rows, with
+// Where this kernel is the faster one, from both sides timed over 40 weights of 256 to 16384 rows at 1 to 64 activation rows, with
 // the weights out of memory (us, kernels of gemm.hip or weight_only_int8.hip -> this one):
 //   16-bit, 1 / 4 / 16 / 32 rows: 4096 x 4096 8.9 -> 8.4, 9.8 -> 8.6, 10.7 -> 8.8, 12.6 -> 9.8; 5120 x 5120 14.2 -> 11.7 at one row; 4096 x 11008
 //     (two K slices and their reduction) 19.4 -> 16.7, 20.2 -> 18.5 at 16 rows; 6144 x 4096 13.0 -> 11.2; 8192 x 28672 73.1 -> 72.4
 //   int8: 4096 x 4096 7.8 -> 6.2, 8.6 -> 6.3, 10.9 -> 7.0, 12.1 -> 8.8; 4096 x 11008 13.9 -> 10.8 at one row; 8192 x 8192 17.3 -> 12.8; 4096 x
 //     6144 15.3 -> 8.7 at 16 rows; 4096 x 4160, which only the one-output-a-lane kernel took, 580 -> 7.1
+//   33 / 64 rows: 16-bit 4096 x 4096 14.3 -> 11.0, 16.5 -> 13.2; 6144 x 4096 15.8 -> 13.6, 18.6 -> 16.2; 8192 x 8192 26.9 -> 24.1, 32.7 -> 27.5; int8
+//     4096 x 4096 13.3 -> 10.1, 14.4 -> 12.3; 6144 x 4096 16.5 -> 11.5, 17.5 -> 14.5; 8192 x 4096 17.7 -> 11.8, 18.9 -> 14.9
 // The others stay where they were:
 //   * more columns for a unit than 32 (16-bit) or 48 (int8): there whole K in shorter stages streams as well (int8 16384 x 4096
-//     13.4 against 14.4, 16-bit 10240 x 8192 the same); from 17 rows on 16 and 32, as far as the rings go;
+//     13.4 against 14.4, 16-bit 10240 x 8192 the same); from 17 rows on 32, as far as the rings go;
 //   * one or two rows of a small weight, all latency (16-bit 2048 x 2048 4.9 against 5.3, int8 2560 x 2560 4.6 against 4.9);
 //   * up to four rows of a 16-bit weight with K no longer than its 7168 and more columns (8192 x 8192 23.0 against 24.0);
 //   * int8 with two or three column tiles and a K of fewer than four stages (8192 x 1024 4.5 against 5.2);
 //   * many rows with a long K, where a unit takes in more of the activations than of its weights and K slices, which divide
 //     them, win: 17 rows, 16-bit 4096 x 11008 20.2 against 20.6, int8 5120 x 13824 19.2 against 21.0; 16 rows, int8 8192 x 28672
-//     41.0 against 42.2 (8192 x 16384 29.3 -> 23.6).
+//     41.0 against 42.2 (8192 x 16384 29.3 -> 23.6); 64 rows, 16-bit 4096 x 8192 20.8 against 21.8, 1024 x 4096 10.1 against 11.8, int8
+//     4096 x 8192 19.0 against 20.6, 2048 x 8192 15.1 against 19.3 (1024 x 4096 11.8 -> 11.3).
 bool narrowStreamPays(const NarrowStreamArgs& a) {
   const int64_t size = a.int8B ? 1 : 2, weights = (int64_t)a.N * a.K;
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  if (a.M < 1 || a.M > 32 || a.N < 1 || a.K < 16 || a.K % (16 / size) != 0 || !al16(a.A) || !al16(a.B) || a.lda % 8 != 0 || a.ldb * size % 16 != 0 ||
+  if (a.M < 1 || a.M > 64 || a.N < 1 || a.K < 16 || a.K % (16 / size) != 0 || !al16(a.A) || !al16(a.B) || a.lda % 8 != 0 || a.ldb * size % 16 != 0 ||
       ((int64_t)(a.N - 1) * a.ldb + a.K) * size >= ((int64_t)1 << 31) || ((int64_t)(a.M - 1) * a.lda + a.K) * 2 >= ((int64_t)1 << 31))
     return false;
   const int64_t cols = ceilDiv(a.N, (int64_t)computeUnits());
+  if (a.M > 32) return cols <= 32 && (2 * (int64_t)a.K <= 3 * (int64_t)a.N || a.K < 4096 || (a.int8B && a.K <= 4096));
   if (a.int8B) {
     if (cols > (a.M > 16 ? 32 : 48) || (cols > 16 && a.K < 4 * kNarrowBK)) return false;
     if (a.M > 16) return a.K <= 8192 || a.K <= 2 * (int64_t)a.N;
     return !(a.M <= 2 && weights <= ((int64_t)1 << 23)) && !(a.M > 12 && weights > ((int64_t)3 << 26));
   }
-  if (a.M > 16) return cols <= 16 && a.K <= 8192;
+  if (a.M > 16) return cols <= 32 && a.K <= 8192;
   return cols <= 32 && !(a.M <= 2 && weights <= ((int64_t)1 << 22)) && !(a.M <= 4 && cols > 28 && a.K <= a.N);
 }
 

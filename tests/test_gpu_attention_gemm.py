@@ -557,7 +557,8 @@ def test_skinny_m_linear_and_addmm(ops, dev, dtype, m, n, k):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k", [(3, 16, 16), (1, 250, 16904), (16, 4096, 520), (5, 4098, 1032), (16, 8192, 512), (4, 8190, 8208), (17, 4096, 1544),
-                                   (32, 250, 8192), (32, 300, 48), (2, 4100, 1528)])
+                                   (32, 250, 8192), (32, 300, 48), (2, 4100, 1528), (33, 4096, 264), (48, 250, 3080), (49, 8192, 1288), (64, 4104, 4096),
+                                   (17, 8190, 1032)])
 def test_few_columns_for_a_compute_unit(ops, dev, dtype, m, n, k):
     # the kernel that streams few columns for each compute unit over the whole of K: ragged column shares, a last stage that
     # is not whole, fewer stages than ring places, one and two row groups; rows lie in a wider matrix of NaNs
@@ -578,7 +579,7 @@ def test_few_columns_for_a_compute_unit(ops, dev, dtype, m, n, k):
 
 
 @pytest.mark.parametrize("table_dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("m,heads,hd,vcols,k", [(3, 10, 128, 2 * 128, 4096), (16, 40, 64, 1000, 1032), (17, 6, 128, 256, 768), (5, 33, 64, 130 * 8, 2048 + 128)])
+@pytest.mark.parametrize("m,heads,hd,vcols,k", [(3, 10, 128, 2 * 128, 4096), (16, 40, 64, 1000, 1032), (17, 6, 128, 256, 768), (5, 33, 64, 130 * 8, 2048 + 128), (40, 10, 128, 2 * 128, 1152), (64, 40, 64, 1000, 1536)])
 def test_rotation_with_few_columns_for_a_compute_unit(ops, dev, table_dtype, m, heads, hd, vcols, k):
     n, cols = heads * hd + vcols, heads * hd
     x = torch.randn(m, k, generator=g(1)).bfloat16()
