@@ -3154,6 +3154,69 @@ static bool reserveTail(diopiContextHandle_t ctx, hipStream_t stream, GemmProble
   return p->tailSlots != nullptr;
 }
 
+// Where one round of rectangles cut to the chip (gemm_weight_stream.hip) is estimated to take at least 7 % less than the other forms: products of
+// 65 to 704 rows whose tiles are a little more than a round of the chip, or leave many of its units without one; small weights, whose slices and
+// reduction cost more than the products; gates and rotations that slices would leave to a pass of their own. us, other forms -> this one:
+//   300 x 12288 x 4096 62.1 -> 42.1, 350 64.1 -> 45.0, 600 69.3 -> 59.4; 300 x 14336 x 4096 63.2 -> 47.1; rotated, 65 x 12288 x 4096 34.4 -> 27.9
+//   300 x 3072 x 1024 15.0 -> 9.7, 128 x 4096 x 1024 9.4 -> 7.7, 512 x 1024 x 1024 12.3 -> 7.6, 256 x 2048 x 2048 17.1 -> 11.2
+//   gated, 100 x 22016 x 4096 44.4 -> 41.7, 160 56.0 -> 48.8, 203 59.1 -> 53.7, 300 70.3 -> 63.9; 65 x 5632 x 1024 14.8 -> 8.0, 256 20.8 -> 11.8
+// and left to the others (they, this one): 203 x 4096 x 4096 19.2, 23.2; 128 x 4096 x 4096 17.5, 19.2; 128 x 4096 x 11008 29.3, 44.3;
+// 300 x 5632 x 1024 10.6, 13.1; 400 x 6144 x 4096 31.2, 35.5.
+// The others' estimates are fitted to what they take with the weights out of memory (540 products of 65 to 700 rows; 5 % on average, slices of
+// K 8 %). A last round in slices of K needs 12 %: its estimate is 7 % off either way, and 7 % is what 400 x 12288 x 4096 would gain.
+// With these lines no choice of the 540 costs more than 3 %, and what is left of the gains is 1 % on average.
+static bool weightStreamPays(const GemmProblem& p, bool separate, float us) {
+  const int resident = computeUnits() / 8 * 8;
+  const int64_t tiles256 = ceilDiv(p.M, 256) * ceilDiv(p.N, 256), pairs = p.K / (2 * kBK);
+  if (tiles256 >= 144) {
+    const float wgs = (float)tiles256 / (float)resident;
+    return us < 0.93f * (2.f + (float)pairs * (wgs <= 1.f ? 2.f + 0.4f * wgs : 2.4f * wgs + 0.7f));
+  }
+  const float megabytes = 2e-6f * (float)(p.N * p.K);
+  if (tailSplitPays(p)) {
+    const float split = tailSplit(tiles256, pairs, resident).us;
+    return us < 0.88f * std::max(0.75f * split, 0.41f * split + 0.048f * (float)p.M + 0.234f * megabytes - 17.3f);
+  }
+  const int64_t tiles = ceilDiv(p.M, 128) * ceilDiv(p.N, 128);
+  const float fill = (float)p.M / (float)(ceilDiv(p.M, 128) * 128);
+  int per = 0;
+  const int ways = splitKWays(p.M, p.N, tiles, p.K / kBK, &per);
+  const float wgs = (float)(tiles * ways) / (float)computeUnits();
+  float other;
+  if (ways > 1)
+    other = 6.5f + (float)per * (0.27f + 0.42f * std::max(0.f, wgs - 1.f) + 0.13f * fill) + 1.7e-6f * (float)(p.M * p.N * ways) + 0.073f * megabytes +
+            0.09f * (float)std::max(0, ways - 3) + (separate ? 5.f : 0.f);
+  else if (wgs > 1.f)
+    other = 1.7f + (float)per * (0.83f + 0.18f * fill);
+  else
+    other = 3.5f + (float)per * (0.14f * wgs + (0.48f - 0.16f * wgs) * fill - 0.03f) + 0.11f * megabytes;
+  return us < 0.93f * other;
+}
+
+static diopiError_t tryWeightStream(hipStream_t stream, const GemmProblem& p, const RotaryEpilogue* rot, bool gate, bool* done) {
+  *done = false;
+  const int64_t outCols = gate ? p.N / 2 : p.N;
+  auto fits = [](int64_t rows, int64_t pitch, int64_t cols) { return ((rows - 1) * pitch + cols) * 2 < (int64_t(1) << 31); };
+  if (p.batch != 1 || p.M <= kSkinnyMaxM || p.M > 704 || p.colScale || p.int8B || p.sAk != 1 || p.sBk != 1 || !mult8(p.sAm) || !ptr16(p.A) ||
+      !mult8(p.sBn) || !ptr16(p.B) || !mult8(p.sOm) || !ptr16(p.out) || (p.bias && !ptr16(p.bias)) ||
+      (p.Cin && (p.sCn != 1 || !mult8(p.sCm) || !ptr16(p.Cin) || !fits(p.M, p.sCm, p.N))) || !fits(p.M, p.sAm, p.K) || !fits(p.N, p.sBn, p.K) ||
+      !fits(p.M, p.sOm, outCols) || p.N % 16 != 0 || p.K % kBK != 0)
+    return diopiSuccess;
+  WeightStreamArgs a;
+  a.siluMul = gate;
+  const float us = weightStreamPlan(p.M, p.N, p.K, &a);
+  if (us == 0.f || !weightStreamPays(p, gate || rot != nullptr, us)) return diopiSuccess;
+  a.A = p.A, a.B = p.B, a.out = p.out, a.Cin = p.Cin, a.bias = p.bias;
+  a.lda = p.sAm, a.ldb = p.sBn, a.ldo = p.sOm, a.sCm = p.sCm;
+  a.M = (int)p.M, a.N = (int)p.N, a.K = (int)p.K, a.alpha = p.alpha, a.beta = p.beta;
+  if (rot != nullptr) {
+    a.rotCos = rot->cosT, a.rotSin = rot->sinT, a.rotCols = rot->cols, a.rotHeadDim = rot->headDim, a.rotTableRows = rot->tableRows;
+    a.rotTableF32 = rot->tableF32, a.rotSinSign = rot->sinSign;
+  }
+  *done = true;
+  return launchWeightStream(stream, p.dtype, a);
+}
+
 // Which kernel applies the gate or the rotation to its fp32 sums: the 256 x 256 one, or the 128 x 128 one where the plain
 // product would take that without a K split (whose slices meet in the reduction pass of the plain product). The pass over
 // the result that this saves took 4.5 us (rotary) and 6.4 us (gate) at 203 rows.
@@ -3243,6 +3306,11 @@ diopiError_t runGemm(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem p
         ((p.M - 1) * p.sAm + p.K) * item < (int64_t(1) << 31))
       return p.dtype == diopi_dtype_bfloat16 ? launchSkinnyForShape<bf16_t>(ctx, stream, p)
                                              : launchSkinnyForShape<half_t>(ctx, stream, p);
+    if (!bT) {
+      bool done = false;
+      AMD_TRY(tryWeightStream(stream, p, nullptr, false, &done));
+      if (done) return diopiSuccess;
+    }
     // from 144 tiles (56 % of the CUs in one round) the large-tile kernel beats the 128 x 128 one even unsplit
     // (a matrix at most 128 columns wide would leave half of every 256-wide tile empty: it takes the 128 x 128 form)
     // and so does a product of only two K tiles, which is all tile turnover: two workgroups per CU overlap one tile's
@@ -3407,6 +3475,11 @@ static diopiError_t runGatedSiluGemm(diopiContextHandle_t ctx, hipStream_t strea
                       p.K % kBK == 0 && p.K >= 2 * kBK &&
                       ((p.M - 1) * p.sAm + p.K) * 2 < (int64_t(1) << 31) && ((p.N - 1) * p.sBn + p.K) * 2 < (int64_t(1) << 31) &&
                       mult8(p.sOm) && ptr16(p.out) && p.M < (int64_t(1) << 31) && p.N < (int64_t(1) << 31);
+  if (direct && p.Cin == nullptr && p.bias == nullptr && p.alpha == 1.f) {
+    bool done = false;
+    AMD_TRY(tryWeightStream(stream, p, nullptr, true, &done));
+    if (done) return diopiSuccess;
+  }
   const FusedTile fused = direct ? fusedTile(ctx, stream, &p) : kFusedNone;
   if (fused == kFused256)
     return p.dtype == diopi_dtype_bfloat16 ? launchMfmaPipelined<bf16_t, kEpiSiluMul>(ctx, stream, p)
@@ -3826,11 +3899,14 @@ GEMM_EXPORT diopiError_t diopiLinearRotary(diopiContextHandle_t ctx, diopiTensor
                       k % kBK == 0 && k >= 2 * kBK && n % 8 == 0 && ptr16(p.out) &&
                       (!p.bias || ptr16(p.bias)) && p.M * k * 2 < (int64_t(1) << 31) && n * k * 2 < (int64_t(1) << 31) &&
                       p.M * n * 2 < (int64_t(1) << 31);
-  const FusedTile tile = direct ? fusedTile(ctx, stream, &p) : kFusedNone;
-  if (tile != kFusedNone) {
-    RotaryEpilogue r;
-    r.cosT = cc.data, r.sinT = cs.data, r.cols = (int)rotaryCols, r.headDim = (int)headDim, r.tableRows = (int)tableRows;
-    r.tableF32 = cc.dtype == diopi_dtype_float32, r.sinSign = conj ? -1.f : 1.f;
+  RotaryEpilogue r;
+  r.cosT = cc.data, r.sinT = cs.data, r.cols = (int)rotaryCols, r.headDim = (int)headDim, r.tableRows = (int)tableRows;
+  r.tableF32 = cc.dtype == diopi_dtype_float32, r.sinSign = conj ? -1.f : 1.f;
+  bool streamed = false;
+  if (direct) AMD_TRY(tryWeightStream(stream, p, &r, false, &streamed));
+  const FusedTile tile = direct && !streamed ? fusedTile(ctx, stream, &p) : kFusedNone;
+  if (streamed) {
+  } else if (tile != kFusedNone) {
     // (what launchMfmaPipelined asks of a problem before it takes the 4-wave kernel, whose LDS has room for the tables)
     const bool fourWave = k % (2 * kBK) == 0 && n % 8 == 0 && ptr16(p.out) && p.M * k * 2 < (int64_t(1) << 31) && n * k * 2 < (int64_t(1) << 31) &&
                           (p.M - 1) * n * 2 + n * 2 < (int64_t(1) << 31);
@@ -3854,9 +3930,6 @@ GEMM_EXPORT diopiError_t diopiLinearRotary(diopiContextHandle_t ctx, diopiTensor
     bool fused = false;
     if (interleaved && rotaryCols > 0 && halfT && tableOk && p.M <= kSkinnyMaxM && k % kSkinnyLdsBK == 0 && ptr16(p.A) && ptr16(p.B) &&
         (p.M - 1) * k * 2 + k * 2 < (int64_t(1) << 31)) {
-      RotaryEpilogue r;
-      r.cosT = cc.data, r.sinT = cs.data, r.cols = (int)rotaryCols, r.headDim = (int)headDim, r.tableRows = (int)tableRows;
-      r.tableF32 = cc.dtype == diopi_dtype_float32, r.sinSign = conj ? -1.f : 1.f;
       AMD_TRY(p.dtype == diopi_dtype_bfloat16 ? launchSkinnyForShape<bf16_t>(ctx, stream, p, &r, &fused)
                                               : launchSkinnyForShape<half_t>(ctx, stream, p, &r, &fused));
     }

@@ -108,6 +108,31 @@ diopiError_t launchNarrowStream(hipStream_t stream, diopiDtype_t dtype, NarrowSt
 // What it settles and reserves for that stays in *p, which then goes to runGemm.
 bool gemmAppliesColumnScale(diopiContextHandle_t ctx, hipStream_t stream, GemmProblem* p);
 
+// gemm_weight_stream.hip: 16-bit products in one round of workgroups, each a rectangle of the output over the whole of K.
+// A and B K-contiguous with 16-byte rows and less than 2 GiB each; out, Cin (n-contiguous) and bias in 8-byte pieces.
+struct WeightStreamArgs {
+  const void* A = nullptr;
+  const void* B = nullptr;
+  void* out = nullptr;
+  const void* Cin = nullptr;
+  const void* bias = nullptr;
+  int64_t lda = 0, ldb = 0, ldo = 0, sCm = 0;
+  int M = 0, N = 0, K = 0;
+  float alpha = 1.f, beta = 0.f;
+  int tilesM = 1, rowsPerWg = 0;   // workgroups along the rows, and the rows of one
+  int tilesN = 0, tilesPerWg = 0;  // column tiles of 16, in all and of a workgroup
+  bool siluMul = false;  // every 64 columns are 32 gate and 32 up columns; out (N / 2 wide) = silu(gate) * up
+  // the interleaved rotary embedding on the leading rotCols columns
+  const void* rotCos = nullptr;
+  const void* rotSin = nullptr;
+  int rotCols = 0, rotHeadDim = 2, rotTableRows = 1;
+  bool rotTableF32 = false;
+  float rotSinSign = 1.f;
+};
+// The estimated time (us) of the best cut, which is left in *g; 0 where there is none.
+float weightStreamPlan(int64_t m, int64_t n, int64_t k, WeightStreamArgs* g);
+diopiError_t launchWeightStream(hipStream_t stream, diopiDtype_t dtype, const WeightStreamArgs& g);
+
 // diopiRotaryEmbedding on views (rotary_kv.hip): out and x of shape [..., heads, head_dim], strided views allowed.
 diopiError_t runRotary(diopiContextHandle_t ctx, hipStream_t stream, const TensorView& out, const TensorView& x,
                        const TensorView& cosT, const TensorView& sinT, bool conj, bool interleaved);

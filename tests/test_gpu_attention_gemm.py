@@ -596,6 +596,35 @@ def test_rotation_with_few_columns_for_a_compute_unit(ops, dev, table_dtype, m, 
         assert_half(got, torch.cat([rotated, want[:, cols:]], 1))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(65, 512, 1024), (128, 4096, 1024), (97, 11008, 1088), (704, 1536, 1152), (257, 11008, 1088), (257, 14336, 4096), (257, 22016, 4096),
+                                   (704, 6144, 1088), (704, 8192, 4096), (203, 22016, 4096), (300, 3072, 1088), (451, 1040, 1024), (600, 2560, 1216)])
+def test_rectangles_cut_to_the_chip(ops, dev, dtype, m, n, k):
+    # the kernel of 65 to 704 rows whose rectangles are cut to the chip: ragged last rows and column tiles,
+    # every width, 16 stages of K and more; rows lie in a wider matrix of NaNs
+    wide = torch.full((m, k + 24), float("nan"), dtype=dtype)
+    wide[:, :k] = torch.randn(m, k, generator=g(1)).to(dtype)
+    x, xd = wide[:, :k], wide.to(dev)[:, :k]
+    w = (torch.randn(n, k, generator=g(2)) / k**0.5).to(dtype)
+    c, b = torch.randn(m, n, generator=g(3)).to(dtype), torch.randn(n, generator=g(4)).to(dtype)
+    want = (x.float() @ w.float().t()).double()
+    assert_half(ops.linear(xd, w.to(dev)), want)
+    assert_half(ops.linear(xd, w.to(dev), b.to(dev)), want + b.double())
+    assert_half(ops.addmm(c.to(dev), xd, w.to(dev).t(), beta=0.5, alpha=2.0), 0.5 * c.double() + 2 * want)
+    if n % 64 == 0:
+        blocks = want.view(m, n // 64, 2, 32)
+        assert_half(ops.linear_silu_mul(xd, w.to(dev)), (torch.nn.functional.silu(blocks[:, :, 0]) * blocks[:, :, 1]).reshape(m, n // 2))
+    for table_dtype in (dtype, torch.float32):
+        hd, cols = 64, n * 2 // 3 // 64 * 64
+        angle = torch.rand(m, hd // 2, generator=g(5)) * 6
+        cos, sin = angle.cos().to(table_dtype), angle.sin().to(table_dtype)
+        pairs = (want + b.double())[:, :cols].reshape(m, cols // hd, hd // 2, 2)
+        co, si = cos.double()[:, None], sin.double()[:, None]
+        rotated = torch.stack([pairs[..., 0] * co - pairs[..., 1] * si, pairs[..., 0] * si + pairs[..., 1] * co], -1).reshape(m, cols)
+        got = ops.linear_rotary(xd, w.to(dev), cos.to(dev), sin.to(dev), cols, hd, bias=b.to(dev))
+        assert_half(got, torch.cat([rotated, (want + b.double())[:, cols:]], 1))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("m,f,k", [(4096, 3584, 256), (3700, 4000 - 32, 192), (96, 64, 80), (1, 32, 8),
                                    (5, 2048, 256), (33, 5536, 384), (48, 16384, 128), (64, 11008, 640), (20, 8224, 256)])
