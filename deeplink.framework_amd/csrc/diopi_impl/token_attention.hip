@@ -1174,8 +1174,9 @@ static diopiError_t fillArgs(const TaViews& t, bool needK, bool needV, int maxLe
   return diopiSuccess;
 }
 
-// Chunk length of the split over a sequence (decodeSplitKernel, or decodeGroupedKernel if `grouped`).
-static void chooseChunk(TaArgs* a, int64_t groupsPerSeq, int64_t batch, int maxInputLen, bool grouped) {
+// Chunk length of the split over a sequence (decodeSplitKernel, or decodeGroupedKernel if `grouped`). wide: 256-byte rows of both
+// K and V are read; merges: a launch that merges the chunks follows if there are more than one.
+static void chooseChunk(TaArgs* a, int64_t groupsPerSeq, int64_t batch, int maxInputLen, bool grouped, bool wide, bool merges) {
   // A workgroup of the lanes' kernel walks its chunk with two loads per wave in flight, so the rate comes from the number
   // of workgroups a CU holds at once. Few sequences or short ones are cut into smaller chunks until there are about
   // kTaWgsPerCu workgroups per CU; large batches keep the 512-token chunks, whose partial results are fewer. Measured (us,
@@ -1190,6 +1191,17 @@ static void chooseChunk(TaArgs* a, int64_t groupsPerSeq, int64_t batch, int maxI
   const int64_t capped = ceilDiv(ceilDiv(len, (int64_t)kTaMaxSplit), 64) * 64;  // at most kTaMaxSplit chunks
   const int64_t shortest = !grouped && groups * ceilDiv(len, (int64_t)kTaMinChunk) < cus ? kTaTinyChunk : kTaMinChunk;
   a->chunk = (int)std::max(std::max(capped, shortest), std::min<int64_t>(a->chunk, fine));
+  // Short sequences in one chunk: the partial results, the launch that merges them (3 us) and the prologues of more workgroups cost more
+  // than an even share of the work gives. us, chunks -> one (fused, sequences of 0.2 to 1 times the longest given): 32 heads of
+  // 128 on 8, 4 x 256 9.0 -> 7.6, 24 x 512 13.1 -> 11.4, 60 x 256 17.4 -> 11.5, 60 x 500 23.4 -> 18.8, 60 x 1000 35.3 -> 33.7; 64 on 8, 32 x 700 18.9 -> 16.3,
+  // 64 x 700 30.6 -> 26.8; second half, 64 on 8, 62 x 500 20.5 -> 14.6. The lines (in workgroups, against the chip's units): one chunk was slower for
+  // 512 tokens and a quarter of a workgroup for a unit (9.1, 11.4), 700 and 1.1 (20.6, 22.0), 1000 and 1.1 ... 1.5 (24.9, 27.5), and
+  // where not all of its workgroups run at once (560 x 1024: 55, 60). 7/8 to one workgroup for a unit: 700 tokens only with wide rows (17.9, 15.8;
+  // second half 13.2, 13.9).
+  const int64_t eighths = groups * 8 / cus;
+  const bool one = len <= 256 || (len <= 512 && eighths >= 5) ||
+                   (groups <= 2 * cus && ((len <= 768 && (eighths >= 11 || (wide && eighths >= 7 && groups <= cus))) || (len <= 1024 && eighths >= 13)));
+  if (grouped && merges && a->d <= 128 && one) a->chunk = (int)std::max<int64_t>(a->chunk, ceilDiv(len, (int64_t)64) * 64);
 }
 
 #define TA_DISPATCH(DTYPE, BYTES, CALL)                                                        \
@@ -1314,7 +1326,7 @@ static diopiError_t streamChunks(diopiContextHandle_t ctx, hipStream_t stream, T
   a.qGroups = (perKv + qpk - 1) / qpk;
   const bool hiw = qpk == 1 && MODE == kTaFused && wholeLoads;
   const int groupsPerSeq = qpk > 1 ? a.kvHeads * a.qGroups : (hiw ? a.heads / tpw : a.heads);
-  chooseChunk(&a, groupsPerSeq, batch, maxInputLen, grouped);
+  chooseChunk(&a, groupsPerSeq, batch, maxInputLen, grouped, MODE == kTaFused && bytes == 256, MODE != kTaLogitsOut);
   a.nsplit = (int)std::max<int64_t>(1, ceilDiv(maxInputLen, a.chunk));
   AMD_CHECK(batch <= 65535 && a.nsplit <= 65535, "token attention: batch %ld / splits %d exceed the grid limits", (long)batch,
             a.nsplit);

@@ -1240,6 +1240,19 @@ def test_token_attention_many_rows_on_the_lanes(ops, dev, batch, heads, kvh, d, 
 
 
 
+@pytest.mark.parametrize("batch,heads,kvh,d,width,dtype", [
+    (2, 8, 2, 128, 256, torch.bfloat16), (2, 8, 2, 128, 257, torch.float16),           # any number of workgroups
+    (20, 32, 8, 128, 512, torch.bfloat16), (19, 32, 8, 128, 512, torch.bfloat16), (20, 32, 8, 128, 513, torch.float16),
+    (28, 32, 8, 128, 768, torch.float16), (28, 16, 8, 64, 768, torch.bfloat16),        # (rows of 128 bytes: chunks)
+    (44, 32, 8, 128, 768, torch.bfloat16), (44, 32, 8, 128, 769, torch.bfloat16),
+    (52, 32, 8, 64, 1024, torch.float16), (52, 32, 8, 128, 1025, torch.bfloat16), (65, 16, 8, 128, 600, torch.bfloat16),
+    (20, 18, 1, 96, 512, torch.float16),                                               # two workgroups a row
+])
+def test_token_attention_one_chunk_or_several(ops, dev, batch, heads, kvh, d, width, dtype):
+    """Both sides of the lines up to which sequences are walked whole by the matrix pipe: longest sequence against workgroups."""
+    test_token_attention_many_rows_on_the_lanes(ops, dev, batch, heads, kvh, d, width, dtype)
+
+
 @pytest.mark.parametrize("heads,kvh,dtype", [(4, 4, torch.bfloat16), (8, 2, torch.float16), (2, 1, torch.bfloat16), (4, 1, torch.float32)])
 def test_token_attention_slots_beyond_32_bits(ops, dev, heads, kvh, dtype):
     """A pool of more slots than 31 bits number (here all of them one row, by a stride of zero) is the lanes' in every form."""
