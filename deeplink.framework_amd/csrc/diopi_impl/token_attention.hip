@@ -1270,6 +1270,9 @@ using namespace amd;
 //   (50 .. 300) 141 -> 127, 9 x 62 6.8 -> 6.2. 32 heads of 64, a row of which is 128 bytes here and there: 32 x (1000 .. 4000) 125 -> 111,
 //   24 x (1500 .. 3000) 93 -> 81. 32 heads on 16: 512 x (16 .. 64) 80 -> 50, 128 x (64 .. 256) 40 -> 44. Heads of 256: 32 on 16, 128 x
 //   (512 .. 2048) 554 -> 490, 32 x (16 .. 64) 18 -> 14; 32 on 8, 512 x (16 .. 64) 113 -> 64; 64 on 8, 140 x 30 38 -> 27, 378 x 21 89 -> 59
+//   and of up to 512 tokens, which the pipe walks whole (fused, a query head alone, rows of 256 bytes; lanes against pipe): 32 heads, 24 x
+//   (60 .. 250) 27.0, 18.9, 32 x (20 .. 130) 24.2, 14.8, 64 x (20 .. 130) 29.3, 24.9; 40 heads, 20 x (100 .. 500) 35.1, 29.1, 60 x (100 .. 380)
+//   55.9, 54.8; not 64 x (60 .. 100), 32 heads (22.6, 25.5), nor 64 x (100 .. 500) (58.5, 60.8) or 50 x (200 .. 700) (66.0, 70.6)
 //   scores: 32 heads of 128, 512 x (16 .. 64) 63 -> 42, x (64 .. 256) 126 -> 133; 32 on 16 35 -> 29; 12 on 4, 444 x (16 .. 32) 10.0 -> 8.1
 //   second half: 32 heads of 128, 512 x (16 .. 64) 97 -> 51, 256 x (1024 .. 2048) 590 -> 555, 64 x (512 .. 4096) 224 -> 213, 16 x
 //   (1000 .. 4000) 64 -> 68; 32 x (4096 .. 16384) 444 -> 434; 64 heads, 7 x (9 .. 18) 5.7 -> 4.5; 64 heads of 256, 5 x 12 6.3 -> 4.1
@@ -1284,7 +1287,9 @@ static bool lanesPay(int64_t perKv, int64_t kvHeads, bool wholeLoads, bool partR
     if (MODE == kTaReduceV) return maxLen <= (wide ? 48 : 64) || rows >= 2048 || many(512, 8, kAny) || rows * maxLen >= (int64_t)5 << 19;
     if (wide) return true;
     if (!wholeLoads) return maxLen <= 64 || rows * bytes >= (int64_t)2048 * 256 || many(512, 0, 128);
-    return partRows || maxLen <= 24 || rows * bytes > (int64_t)640 * 256 || (rows * bytes >= (int64_t)512 * 256 && maxLen <= 64) ||
+    // sequences that the pipe walks whole, up to 2400 rows of 256 bytes, unless they are short for their number
+    const bool whole = bytes > 128 && maxLen <= 512 && rows <= std::min<int64_t>(20 * maxLen - 500, maxLen <= 384 ? 2400 : 2047);
+    return partRows || maxLen <= 24 || (!whole && (rows * bytes > (int64_t)640 * 256 || (rows * bytes >= (int64_t)512 * 256 && maxLen <= 64))) ||
            (bytes <= 128 && kvHeads >= 32 && rows >= 768 && maxLen >= 1500);
   }
   if (bytes <= 128 || perKv > 8) return false;

@@ -1247,6 +1247,9 @@ def test_token_attention_many_rows_on_the_lanes(ops, dev, batch, heads, kvh, d, 
     (44, 32, 8, 128, 768, torch.bfloat16), (44, 32, 8, 128, 769, torch.bfloat16),
     (52, 32, 8, 64, 1024, torch.float16), (52, 32, 8, 128, 1025, torch.bfloat16), (65, 16, 8, 128, 600, torch.bfloat16),
     (20, 18, 1, 96, 512, torch.float16),                                               # two workgroups a row
+    # many rows with a query head to itself: on the pipe, and past each line of that on the lanes
+    (24, 32, 32, 128, 64, torch.bfloat16), (25, 32, 32, 128, 64, torch.bfloat16), (20, 40, 40, 128, 250, torch.float16),
+    (64, 32, 32, 128, 130, torch.bfloat16), (21, 32, 32, 128, 512, torch.float16), (21, 32, 32, 128, 513, torch.bfloat16), (64, 32, 32, 128, 385, torch.bfloat16),
 ])
 def test_token_attention_one_chunk_or_several(ops, dev, batch, heads, kvh, d, width, dtype):
     """Both sides of the lines up to which sequences are walked whole by the matrix pipe: longest sequence against workgroups."""
