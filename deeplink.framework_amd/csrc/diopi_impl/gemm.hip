@@ -35,8 +35,9 @@
 //     accumulator layout;
 //   * more than 64 rows but too few 256x256 tiles to fill the chip: the large-tile kernel with K split over
 //     grid.y, fp32 partial products in workspace, and a reduction pass that applies the epilogue;
-//   * at most 32 rows (64 while N is small), the decode shape: a weight-streaming kernel with 16-column tiles
-//     whose waves split K and stage the activation rows in LDS.
+//   * 65 to 704 rows, where that is faster: one round of rectangles cut to the chip (gemm_weight_stream.hip);
+//   * at most 64 rows, the decode shape, weight-streaming kernels: few columns for each compute unit in narrow_stream.hip, wider
+//     weights through LDS here, and what neither takes in 16-column tiles whose waves split K and stage the activation rows in LDS.
 // Operands that are not K-contiguous (mm with a row-major mat2, bmm's second operand) are
 // transposed once into workspace by a tiled LDS transpose, then use the same engine.
 //
@@ -2971,6 +2972,7 @@ static diopiError_t launchSkinnyForShape(diopiContextHandle_t ctx, hipStream_t s
   if (rot != nullptr) AMD_TRY(tryNarrowStream(stream, p, rot, handled));  // (runGemm has asked for the others)
   if (rot != nullptr && *handled) return diopiSuccess;
   const int tiles = (a.N + 15) / 16, cus = computeUnits(), perCu = (tiles + cus - 1) / cus;
+  // (What follows gets what narrowStreamPays declined; the figures for N up to 8192 were measured without that kernel.)
   // Both operands through LDS, see gemmSkinnyLdsKernel. The columns are dealt evenly over as many workgroups as there
   // are CUs (43 each at N = 11008, where 64-column blocks would leave a third of the CUs idle): a CU takes in about
   // 45 GB/s from a cold stream whatever the software pipeline depth, so the count of CUs at work sets the rate.
