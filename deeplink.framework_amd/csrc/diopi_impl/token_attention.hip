@@ -1197,7 +1197,7 @@ static void chooseChunk(TaArgs* a, int64_t groupsPerSeq, int64_t batch, int maxI
   // 64 x 700 30.6 -> 26.8; second half, 64 on 8, 62 x 500 20.5 -> 14.6. The lines (in workgroups, against the chip's units): one chunk was slower for
   // 512 tokens and a quarter of a workgroup for a unit (9.1, 11.4), 700 and 1.1 (20.6, 22.0), 1000 and 1.1 ... 1.5 (24.9, 27.5), and
   // where not all of its workgroups run at once (560 x 1024: 55, 60). 7/8 to one workgroup for a unit: 700 tokens only with wide rows (17.9, 15.8;
-  // second half 13.2, 13.9).
+  // second half 13.2, 13.9). The scores, which nothing merges, keep their chunks (32 heads on 8, 24 x (100 .. 500) 6.2, 7.1 in one).
   const int64_t eighths = groups * 8 / cus;
   const bool one = len <= 256 || (len <= 512 && eighths >= 5) ||
                    (groups <= 2 * cus && ((len <= 768 && (eighths >= 11 || (wide && eighths >= 7 && groups <= cus))) || (len <= 1024 && eighths >= 13)));
