@@ -30,6 +30,13 @@ constexpr int kNarrowBK = 512;
 constexpr int narrowStagesW(int tiles, int bk) { return tiles == 1 ? 4 : 3; }
 constexpr int narrowStagesX(bool int8, int tiles, int bk) { return int8 && tiles == 1 && bk == kNarrowBK ? 4 : 3; }
 
+// The stage of K that a workgroup which starts its walk at stage `start` visits c-th. Past the end, where copies fetch nothing, the last
+// one again: the range check of a buffer load subtracts its scalar offset from the size, so that offset stays inside the rows.
+__host__ __device__ constexpr int narrowStage(int c, int start, int stages) {
+  const int at = (c < stages ? c : stages - 1) + start;
+  return at >= stages ? at - stages : at;
+}
+
 template <typename T, bool W8, int G, int NT, int BK>
 __global__ __launch_bounds__(512) void narrowStreamKernel(NarrowStreamArgs a) {
   typedef typename Vec16<T>::type Frag;
@@ -105,8 +112,7 @@ __global__ __launch_bounds__(512) void narrowStreamKernel(NarrowStreamArgs a) {
   const unsigned ldsBase = (unsigned)(size_t)(__attribute__((address_space(3))) char*)(copiesW ? sw : sx) + (unsigned)ci * 1024u;
   auto copyStage = [&](auto weights, int c, int place) {
     constexpr bool kW = decltype(weights)::value;
-    int cc = c + kStart;
-    if (cc >= nStages) cc -= nStages;
+    const int cc = narrowStage(c, kStart, nStages);
     const int from = cc * BK * (kW ? kSize : 2);
     const unsigned to = ldsBase + (unsigned)place * (kW ? WBUF : XBUF);
     // (of a stage past the end no column is there: the copies count as the others do, and fetch nothing)

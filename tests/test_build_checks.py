@@ -95,3 +95,35 @@ def test_dynamic_lds_limit_follows_the_largest_launch(tmp_path):
     subprocess.run(cmd, check=True)
     r = subprocess.run([exe], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
+
+
+NARROW_STAGES_PROBE = r"""
+#include <cstdio>
+#include "narrow_stream.hip"
+// Every copy that a workgroup issues: those of the walk and, as its loads are counted, those past the last stage.
+int main() {
+  for (int stages = 1; stages <= 40; ++stages)
+    for (int start = 0; start < stages; ++start)
+      for (int places = 3; places <= 4; ++places)
+        for (int c = 0; c < stages + places - 1; ++c) {
+          const int at = amd::narrowStage(c, start, stages);
+          if (at < 0 || at >= stages) return printf("copy %d of %d stages from %d: stage %d\n", c, stages, start, at), 1;
+          if (c < stages && at != (c + start) % stages) return printf("copy %d of %d stages from %d\n", c, stages, start), 2;
+        }
+  return 0;
+}
+"""
+
+
+def test_copies_past_the_last_stage_keep_their_offset_inside_the_buffer(tmp_path):
+    """The scalar offset of a buffer load counts against the size in the descriptor: also a copy that fetches nothing
+    (its lanes lie past the end) stays at a stage that the rows have."""
+    b = _build_module()
+    (tmp_path / "probe.cpp").write_text(NARROW_STAGES_PROBE)
+    exe = str(tmp_path / "probe")
+    src = b.TARGETS["impl"]["dir"]
+    cmd = [b.hipcc(), "-O0", "-std=c++17", "-w", "--offload-host-only", f"-I{b.INCLUDE}", f"-I{src}", "-x", "hip", str(tmp_path / "probe.cpp"),
+           "-o", exe, "-Wl,--unresolved-symbols=ignore-all"]
+    subprocess.run(cmd, check=True)
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
