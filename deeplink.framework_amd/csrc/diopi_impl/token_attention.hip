@@ -445,9 +445,11 @@ __global__ __launch_bounds__(kTaWaves * 64, splitWavesPerSimd(sizeof(T), LPT, HI
 //     probabilities are, as they lie in the registers, the operand P^T of O^T += V^T . P^T (16x16x32: a probability as
 //     several 16-bit numbers, each the rounding of what the ones before it leave, against the same four tokens of V). In
 //     bf16 three of them hold all 24 bits of it. In fp16 the first two, of the probability times 2^7 (at most 2^15), end at
-//     2^-25; two more, of the remainder times 2^24 in a product of their own, go on to 2^-49: 22 bits of every
-//     probability down to 2^-34 of the largest, so the weight of many keys far below one without values is not lost
-//     (second half, 16 x (64 .. 2048), 32 on 8: 17.3 us with the first two, 18.3 with all; the fused form is the same).
+//     2^-25; two more, of the remainder times 2^24 in a product of their own, go on to 2^-49: all bits of every
+//     probability down to 2^-31 of the largest. A tile with a smaller one multiplies what is left of each, times 2^64, too: to
+//     2^-89, so the weight of many keys far below one without values is not lost (second half, 16 x (64 .. 2048), 32 on 8:
+//     17.3 us with the first two, 18.3 with four; the question whether there is such a tile 0.0 % on average, fused 1.2 %,
+//     with rows of 512 bytes 3 - 4 %: 48 x (500 .. 4000), 16 on 4 127.8 -> 133.4).
 //   * K and V rows go from the pool straight into LDS (global_load_lds, a lane's own address per 16 bytes, marked
 //     non-temporal: 104 -> 91 us at 48 sequences), in a ring of kGqStages tiles that belongs to one wave: no barriers, only
 //     the wave's own load counter. V stays as it is in memory
@@ -474,7 +476,7 @@ struct GqMfma<bf16_t> {
   typedef bf16x4 Quad;
   static constexpr uint16_t kInfinity = 0x7f80;
   static constexpr float kRaise = 0.f;        // log2 of what probabilities are multiplied by before they are cut into parts
-  static constexpr float kRestScale = 1.f;    // what the parts after the second are multiplied by
+  static constexpr float kRestScale = 1.f;    // what the third and fourth part are multiplied by
 };
 template <>
 struct GqMfma<half_t> {
@@ -484,6 +486,7 @@ struct GqMfma<half_t> {
   static constexpr uint16_t kInfinity = 0x7c00;
   static constexpr float kRaise = 7.f;
   static constexpr float kRestScale = 16777216.f;
+  static constexpr float kFarScale = 1099511627776.f;  // and once more, what those leave
 };
 
 // XOR on the 16-byte piece index of row r in LDS. K: 16 rows' pieces of one index fall on 16 different 16-byte bank groups;
@@ -654,6 +657,7 @@ walk:
 #pragma unroll
         for (int i = 0; i < 4; ++i) sc[i] = v[i];
       }
+      const float lowest = fminf(fminf(sc[0], sc[1]), fminf(sc[2], sc[3]));
       // tokens that do not count: no score, and with care rows of V read as zeros
       u32x2 counts = {~0u, ~0u};
       if (skips || (t + 1) * kGqTile > cnt) {  // wave-uniform
@@ -680,15 +684,14 @@ walk:
               for (int i = 0; i < 4; ++i) acc[d][i] *= corr;
           }
         }
-        Frag p, r;  // a probability's first two parts, and the others
-        float ps = 0.f;
+        Frag p, r;  // a probability's first two parts, and the next
+        float ps = 0.f, whole[4];
         const float mRaised = mRef - M::kRaise;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float e = __builtin_amdgcn_exp2f(sc[i] - mRaised);
-          ps += e;
-          T hi = static_cast<T>(e);
-          if (careful && e > 0.f && hi == static_cast<T>(0.f)) hi = __builtin_bit_cast(T, (uint16_t)1);
+          ps += whole[i] = e;
+          const T hi = static_cast<T>(e);
           const float left = e - static_cast<float>(hi);
           const T lo = static_cast<T>(left);
           p[i] = hi, p[4 + i] = lo;
@@ -704,32 +707,59 @@ walk:
           const unsigned piece = (unsigned)((2 * d + ((lane & 3) >> 1)) ^ gqSwizzleV<D>(row)) << 4;
           return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsTr)(uintptr_t)(vRow + piece)));
         };
-        auto multiply = [&](int d, u32x4 first, u32x4 others) {
-          acc[d] = M::run(__builtin_bit_cast(Frag, first), p, acc[d]);
+        auto multiply = [&](int d, u32x4 v) {
+          acc[d] = M::run(__builtin_bit_cast(Frag, v), p, acc[d]);
           if constexpr (M::kRestScale != 1.f) {
-            const f32x4 rest = M::run(__builtin_bit_cast(Frag, others), r, f32x4{0.f, 0.f, 0.f, 0.f});
+            const f32x4 rest = M::run(__builtin_bit_cast(Frag, v), r, f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[d][i] += rest[i] * (1.f / M::kRestScale);
           } else {
-            acc[d] = M::run(__builtin_bit_cast(Frag, others), r, acc[d]);
+            acc[d] = M::run(__builtin_bit_cast(Frag, v), r, acc[d]);
           }
+        };
+        // ones where V is not finite
+        auto infinite = [](u32x2 v) {
+          typedef uint16_t U16x4 __attribute__((ext_vector_type(4)));
+          typedef int16_t S16x4 __attribute__((ext_vector_type(4)));
+          const U16x4 top = (__builtin_bit_cast(U16x4, v) & (uint16_t)0x7fff) + (uint16_t)(0x8000 - M::kInfinity);  // bit 15: not finite
+          return __builtin_bit_cast(u32x2, __builtin_bit_cast(S16x4, top) >> (int16_t)15);
         };
         if (!careful) {
 #pragma unroll
           for (int d = 0; d < DT; ++d) {
             const u32x2 v = quadOfV(d);
-            multiply(d, u32x4{v[0], v[1], v[0], v[1]}, u32x4{v[0], v[1], v[0], v[1]});
+            multiply(d, u32x4{v[0], v[1], v[0], v[1]});
           }
         } else {
+          // infinities and NaN meet none of the parts, some of which are zero or negative, but a one for each probability that is not zero
+          Frag some = {};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) some[i] = static_cast<T>(whole[i] > 0.f ? 1.f : 0.f);
 #pragma unroll
           for (int d = 0; d < DT; ++d) {
-            const u32x2 v = quadOfV(d) & counts;
-            // against all parts but the first infinities and NaN read as zero: the first ones, none of them zero, carry them
-            typedef uint16_t U16x4 __attribute__((ext_vector_type(4)));
-            typedef int16_t S16x4 __attribute__((ext_vector_type(4)));
-            const U16x4 top = (__builtin_bit_cast(U16x4, v) & (uint16_t)0x7fff) + (uint16_t)(0x8000 - M::kInfinity);  // bit 15: not finite
-            const u32x2 low = v & ~__builtin_bit_cast(u32x2, __builtin_bit_cast(S16x4, top) >> (int16_t)15);
-            multiply(d, u32x4{v[0], v[1], low[0], low[1]}, u32x4{low[0], low[1], low[0], low[1]});
+            const u32x2 v = quadOfV(d) & counts, odd = v & infinite(v), low = v ^ odd;
+            multiply(d, u32x4{low[0], low[1], low[0], low[1]});
+            acc[d] = M::run(__builtin_bit_cast(Frag, u32x4{odd[0], odd[1], 0u, 0u}), some, acc[d]);
+          }
+        }
+        if constexpr (M::kRestScale != 1.f) {
+          if (__builtin_amdgcn_ballot_w64(lowest - mRaised < -24.f) != 0) {  // (of a smaller number some bits may be left)
+            Frag f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const float left = whole[i] - static_cast<float>(p[i]) - static_cast<float>(p[4 + i]);
+              const float x = (left * M::kRestScale - static_cast<float>(r[i]) - static_cast<float>(r[4 + i])) * M::kFarScale;
+              f[i] = static_cast<T>(x);
+              f[4 + i] = static_cast<T>(x - static_cast<float>(f[i]));
+            }
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+              u32x2 v = quadOfV(d);
+              if (careful) v &= counts & ~infinite(v);
+              const f32x4 rest = M::run(__builtin_bit_cast(Frag, u32x4{v[0], v[1], v[0], v[1]}), f, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+              for (int i = 0; i < 4; ++i) acc[d][i] += rest[i] * (1.f / M::kRestScale / M::kFarScale);
+            }
           }
         }
       }

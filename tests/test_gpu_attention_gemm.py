@@ -1130,6 +1130,48 @@ def test_token_attention_weights_are_held_in_full(ops, dev, heads, kvh, dtype):
 
 
 
+@pytest.mark.parametrize("infinite", [False, True])
+@pytest.mark.parametrize("batch,heads,kvh", [(21, 32, 32), (20, 32, 8)])
+def test_token_attention_fp16_weights_far_below_the_largest(ops, dev, batch, heads, kvh, infinite):
+    """fp16 probabilities of about 2^-45.5 are held as precisely as larger ones: every 128th token weighs nearly all and has no values, and those
+    between, alike in weight and value, bring results next to the middle between two of the type's smallest numbers, which are rounded
+    to the right side wherever they are no closer to it than fp32 arithmetic errs. Infinities in one column of V change nothing in the
+    others. K picks the scores: q is 32 in its first two elements."""
+    d, n, gen = 128, 512, g(81)
+    live = torch.ones(n, dtype=torch.bool)
+    live[::128] = False
+    first = -torch.randint(177, 180, (batch, kvh), generator=gen).half() / 16
+    second = -torch.randint(0, 512, (batch, kvh), generator=gen).half() / 4096
+    score = 32 * (first.double() + second.double())
+    p = torch.exp(score / d ** 0.5)
+    middle = torch.randint(0, 2, (batch, kvh, d), generator=gen) + 0.5      # in units of the smallest number
+    value = (middle * 2.0 ** -24 * (4 / 508) / p[..., None]).half().double()
+    kp, vp = torch.zeros(2, batch, n, kvh, d, dtype=torch.float16)
+    kp[:, live, :, 0], kp[:, live, :, 1] = first[:, None], second[:, None]
+    vp[:, live] = value.half()[:, None]
+    q = torch.zeros(batch, heads, d, dtype=torch.float16)
+    q[:, :, :2] = 32
+    units = (508 * p[..., None] * value / (4 + 508 * p[..., None]) * 2.0 ** 24).repeat_interleave(heads // kvh, dim=1)
+    # fp32: an exponent of 46 to three roundings of 2^-19, exp2 to 2^-22, 512 sums to 2^-24 each: 2^-14.6 of the result
+    off = units - middle.repeat_interleave(heads // kvh, dim=1)
+    clear = off.abs() > units * 2.0 ** -14
+    if infinite:
+        vp[:, 5::128, :, 7], units[:, :, 7], clear[:, :, 7] = math.inf, math.inf, True
+        off[:, :, 7] = 0
+    assert clear.float().mean() > 0.7 and (off.abs() < units * 2.0 ** -10).all()
+    ln, st = torch.full((batch,), n, dtype=torch.int32), torch.arange(batch, dtype=torch.int32) * n
+    args = (torch.arange(batch * n, dtype=torch.int32).view(batch, n).to(dev), st.to(dev), ln.to(dev), n)
+    kd, vd = kp.view(batch * n, kvh, d).to(dev), vp.view(batch * n, kvh, d).to(dev)
+    att = torch.zeros(heads, batch, n)
+    att[:, :, live] = (score / d ** 0.5).float().t().repeat_interleave(heads // kvh, dim=0)[..., None]
+    out2 = torch.empty(batch, heads, d, dtype=torch.float16, device=dev)
+    ops.token_softmax_reducev(att.view(heads, batch * n).to(dev), vd, out2, *args)
+    for name, got in (("fused", ops.token_decode_attention(q.to(dev), kd, vd, *args)), ("two-call", out2)):
+        wrong = (got.cpu().double() * 2.0 ** 24 != units.round()) & clear
+        assert not bool(wrong.any()), (name, int(wrong.sum()), int(clear.sum()))
+
+
+
 @pytest.mark.parametrize("heads,kvh", [(4, 4), (8, 2)])
 def test_token_attention_values_near_the_largest(ops, dev, heads, kvh):
     """A later key that weighs 2^7 times what the first tile's do and has values near the type's largest: the weighted sum
