@@ -264,7 +264,9 @@ static diopiError_t launchType(hipStream_t stream, const NarrowStreamArgs& a) {
 //   * many rows with a long K, where a unit takes in more of the activations than of its weights and K slices, which divide
 //     them, win: 17 rows, 16-bit 4096 x 11008 20.2 against 20.6, int8 5120 x 13824 19.2 against 21.0; 16 rows, int8 8192 x 28672
 //     41.0 against 42.2 (8192 x 16384 29.3 -> 23.6); 64 rows, 16-bit 4096 x 8192 20.8 against 21.8, 1024 x 4096 10.1 against 11.8, int8
-//     4096 x 8192 19.0 against 20.6, 2048 x 8192 15.1 against 19.3 (1024 x 4096 11.8 -> 11.3).
+//     4096 x 8192 19.0 against 20.6, 2048 x 8192 15.1 against 19.3 (1024 x 4096 11.8 -> 11.3). The 16-bit line below K = 4096, from 760
+//     products: 33 to 64 rows x 64 to 1024, whose four slices are one round of the chip, K = 3328 0.97 to 1.03 of the slices' time, 3456 up
+//     to 1.06, 3968 1.03 to 1.16 (64 x 512 x 3968 10.1 against 11.3); 64 x 1280 x 3584 15.2 -> 11.0, 64 x 2048 x 3968 13.7 -> 12.4.
 bool narrowStreamPays(const NarrowStreamArgs& a) {
   const int64_t size = a.int8B ? 1 : 2, weights = (int64_t)a.N * a.K;
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
@@ -272,7 +274,14 @@ bool narrowStreamPays(const NarrowStreamArgs& a) {
       ((int64_t)(a.N - 1) * a.ldb + a.K) * size >= ((int64_t)1 << 31) || ((int64_t)(a.M - 1) * a.lda + a.K) * 2 >= ((int64_t)1 << 31))
     return false;
   const int64_t cols = ceilDiv(a.N, (int64_t)computeUnits());
-  if (a.M > 32) return cols <= 32 && (2 * (int64_t)a.K <= 3 * (int64_t)a.N || a.K < 4096 || (a.int8B && a.K <= 4096));
+  if (a.M > 32) {
+    if (cols > 32) return false;
+    if (2 * (int64_t)a.K <= 3 * (int64_t)a.N) return true;
+    if (a.int8B) return a.K <= 4096;
+    // (the other form: four slices of up to 1024 columns, eight steps of 128, in pieces of 8 results, and a rotation in a pass of its own)
+    const bool slicesFit = a.rotCols == 0 && ceilDiv(a.N, 16) * 4 <= computeUnits() && a.N >= 16 && a.N % 8 == 0 && a.K % 128 == 0;
+    return a.K < 4096 && !(a.K > 3328 && slicesFit);
+  }
   if (a.int8B) {
     if (cols > (a.M > 16 ? 32 : 48) || (cols > 16 && a.K < 4 * kNarrowBK)) return false;
     if (a.M > 16) return a.K <= 8192 || a.K <= 2 * (int64_t)a.N;

@@ -1,5 +1,6 @@
 """GPU parity: dense contractions, prefill / decode attention, int8 weight-only linear and the
 fp32 decoder block vs the CPU oracle."""
+import contextlib
 import math
 
 import pytest
@@ -14,6 +15,18 @@ pytestmark = pytest.mark.gpu
 
 def g(seed):
     return torch.Generator().manual_seed(seed)
+
+
+@contextlib.contextmanager
+def own_context(ops, pkg):
+    """A context for the calls within, outside of every scope: its workspace tells which form a product took."""
+    ops._ctx = ctx = pkg.diopi.Context()
+    try:
+        yield ctx
+        torch.cuda.synchronize()
+    finally:
+        ops._ctx = 0
+        ctx.close()
 
 
 # ------------------------------------------------------------------ contractions
@@ -576,6 +589,19 @@ def test_few_columns_for_a_compute_unit(ops, dev, dtype, m, n, k):
     want = (x.double() @ q.double().t()) * scale.half().double()
     assert_half(ops.weight_only_int8_linear(xd, q.to(dev), scale.half().to(dev)), want)
     assert_half(ops.weight_only_int8_linear(xd, q.to(dev), scale.half().to(dev), b.to(dev)), want + b.double())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k,slices", [(64, 512, 3968, 4), (33, 1024, 3456, 4), (49, 16, 3584, 4), (64, 512, 3328, 0), (64, 1032, 3968, 0),
+                                          (48, 516, 3968, 0), (33, 512, 3936, 0), (32, 512, 3968, 0), (64, 512, 4096, 4)])
+def test_k_slices_or_a_stream_where_k_is_a_little_less_than_4096(ops, dev, pkg, dtype, m, n, k, slices):
+    """33 to 64 rows and at most 64 column tiles: K slices, which the workspace of their sums tells, from 3329 columns on; a row fewer, a
+    column tile more, and sizes that the slices do not take stay with the kernel that streams the whole of K."""
+    x, w = torch.randn(m, k, generator=g(1)).to(dtype), (torch.randn(n, k, generator=g(2)) / k**0.5).to(dtype)
+    with own_context(ops, pkg) as ctx:
+        got = ops.linear(x.to(dev), w.to(dev))
+        assert ctx.workspace()[1] == slices * m * n * 4
+    assert_half(got, x.double() @ w.double().t())
 
 
 @pytest.mark.parametrize("table_dtype", [torch.bfloat16, torch.float32])
