@@ -3166,8 +3166,10 @@ static bool reserveTail(diopiContextHandle_t ctx, hipStream_t stream, GemmProble
 // 300 x 5632 x 1024 10.6, 13.1; 400 x 6144 x 4096 31.2, 35.5.
 // The others' estimates are fitted to what they take with the weights out of memory (540 products of 65 to 700 rows; 5 % on average, slices of
 // K 8 %). A last round in slices of K needs 12 %: its estimate is 7 % off either way, and 7 % is what 400 x 12288 x 4096 would gain.
-// With these lines no choice of the 540 costs more than 3 %, and what is left of the gains is 1 % on average.
-static bool weightStreamPays(const GemmProblem& p, bool separate, float us) {
+// pass: what a gate or a rotation takes that slices of K leave to a launch of its own, see passUs.
+// With these lines no choice of 6200 products (610 weights of 0.3 to 400 MB; plain, gated and rotated) costs more than 9 %, six more than 3 %,
+// and what is left of the gains is 0.4 % on average.
+static bool weightStreamPays(const GemmProblem& p, float pass, float us) {
   const int resident = computeUnits() / 8 * 8;
   const int64_t tiles256 = ceilDiv(p.M, 256) * ceilDiv(p.N, 256), pairs = p.K / (2 * kBK);
   if (tiles256 >= 144) {
@@ -3187,12 +3189,19 @@ static bool weightStreamPays(const GemmProblem& p, bool separate, float us) {
   float other;
   if (ways > 1)
     other = 6.5f + (float)per * (0.27f + 0.42f * std::max(0.f, wgs - 1.f) + 0.13f * fill) + 1.7e-6f * (float)(p.M * p.N * ways) + 0.073f * megabytes +
-            0.09f * (float)std::max(0, ways - 3) + (separate ? 5.f : 0.f);
+            0.09f * (float)std::max(0, ways - 3) + pass;
   else if (wgs > 1.f)
     other = 1.7f + (float)per * (0.83f + 0.18f * fill);
   else
     other = 3.5f + (float)per * (0.14f * wgs + (0.48f - 0.16f * wgs) * fill - 0.03f) + 0.11f * megabytes;
   return us < 0.93f * other;
+}
+
+// The launch behind K slices that gates or rotates their result, in us: 1.8 and 1.1 ns for each 1000 elements before the gate, 2.3 and 1.1 ns
+// for each 1000 that it rotates (1660 products of each kind against the plain one; 0.4 off). One constant of 5, right for 203 x 22016 alone,
+// sent 111 x 448 x 3072 gated (11.7 in slices) to rectangles (15.4), and 104 x 2624 x 4416 (16.7, 20.2).
+static float passUs(const GemmProblem& p, const RotaryEpilogue* rot, bool gate) {
+  return gate ? 1.8f + 1.1e-6f * (float)(p.M * p.N) : rot != nullptr ? 2.3f + 1.1e-6f * (float)(p.M * rot->cols) : 0.f;
 }
 
 static diopiError_t tryWeightStream(hipStream_t stream, const GemmProblem& p, const RotaryEpilogue* rot, bool gate, bool* done) {
@@ -3206,8 +3215,11 @@ static diopiError_t tryWeightStream(hipStream_t stream, const GemmProblem& p, co
     return diopiSuccess;
   WeightStreamArgs a;
   a.siluMul = gate;
-  const float us = weightStreamPlan(p.M, p.N, p.K, &a);
-  if (us == 0.f || !weightStreamPays(p, gate || rot != nullptr, us)) return diopiSuccess;
+  float us = weightStreamPlan(p.M, p.N, p.K, &a);
+  if (us == 0.f) return diopiSuccess;
+  // (rotating the sums of a rectangle takes 0.6 us and 5.6 ns for each row of each pair of column tiles)
+  if (rot != nullptr) us += 0.6f + 0.0056f * (float)(a.rowsPerWg * ceilDiv(a.tilesPerWg, 2));
+  if (!weightStreamPays(p, passUs(p, rot, gate), us)) return diopiSuccess;
   a.A = p.A, a.B = p.B, a.out = p.out, a.Cin = p.Cin, a.bias = p.bias;
   a.lda = p.sAm, a.ldb = p.sBn, a.ldo = p.sOm, a.sCm = p.sCm;
   a.M = (int)p.M, a.N = (int)p.N, a.K = (int)p.K, a.alpha = p.alpha, a.beta = p.beta;

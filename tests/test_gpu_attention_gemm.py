@@ -651,6 +651,37 @@ def test_rectangles_cut_to_the_chip(ops, dev, dtype, m, n, k):
         assert_half(got, torch.cat([rotated, (want + b.double())[:, cols:]], 1))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("form,m,n,k,slices", [("gated", 111, 448, 3072, 12), ("rotated", 111, 448, 3072, 12), ("gated", 362, 832, 4608, 12), ("rotated", 416, 2368, 3840, 3),
+                                               ("gated", 300, 3072, 1088, 0), ("rotated", 300, 3072, 1088, 0), ("gated", 65, 5632, 1024, 0)])
+def test_gate_and_rotation_in_a_rectangle_or_behind_k_slices(ops, dev, pkg, dtype, form, m, n, k, slices):
+    """What a gate or a rotation in a launch of its own costs decides between rectangles, which take no workspace, and K slices, whose
+    sums (and the two halves before the gate) lie in it."""
+    x, w = torch.randn(m, k, generator=g(1)).to(dtype), (torch.randn(n, k, generator=g(2)) / k**0.5).to(dtype)
+    want = x.double() @ w.double().t()
+    with own_context(ops, pkg) as ctx:
+        if form == "gated":
+            got = ops.linear_silu_mul(x.to(dev), w.to(dev))
+            blocks = want.view(m, n // 64, 2, 32)
+            want = (torch.nn.functional.silu(blocks[:, :, 0]) * blocks[:, :, 1]).reshape(m, n // 2)
+        else:
+            cols = n * 2 // 3 // 64 * 64
+            angle = torch.rand(m, 32, generator=g(3)) * 6
+            got = ops.linear_rotary(x.to(dev), w.to(dev), angle.cos().to(dev), angle.sin().to(dev), cols, 64)
+            pairs, co, si = want[:, :cols].reshape(m, cols // 64, 32, 2), angle.double().cos()[:, None], angle.double().sin()[:, None]
+            rotated = torch.stack([pairs[..., 0] * co - pairs[..., 1] * si, pairs[..., 0] * si + pairs[..., 1] * co], -1).reshape(m, cols)
+            terms = torch.stack([(pairs[..., 0] * co).abs() + (pairs[..., 1] * si).abs(), (pairs[..., 0] * si).abs() + (pairs[..., 1] * co).abs()], -1).reshape(m, cols)
+            want = torch.cat([rotated, want[:, cols:]], 1)
+        assert ctx.workspace()[1] == slices * m * n * 4 + (m * n * 2 if slices and form == "gated" else 0)
+    if form == "gated":
+        assert_half(got, want)
+    else:  # each term of a rotation behind slices is rounded to 16 bits before, the result after it: half a last place; fp32 sums
+        half = 1.01 * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11)
+        bound = half * want.abs() + 1e-4
+        bound[:, :cols] += half * terms
+        assert ((got.cpu().double() - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("m,f,k", [(4096, 3584, 256), (3700, 4000 - 32, 192), (96, 64, 80), (1, 32, 8),
                                    (5, 2048, 256), (33, 5536, 384), (48, 16384, 128), (64, 11008, 640), (20, 8224, 256)])
