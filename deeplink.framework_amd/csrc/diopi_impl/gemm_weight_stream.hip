@@ -314,7 +314,9 @@ static diopiError_t launchTile(hipStream_t stream, const WeightStreamArgs& g) {
 
 template <typename T, int TM>
 static diopiError_t launchRows(hipStream_t stream, const WeightStreamArgs& g) {
-  if (g.tilesPerWg <= 2) return launchTile<T, TM, 1>(stream, g);
+  if constexpr (TM < 8) {  // (240 rows by two column tiles never are the best cut for 256 units)
+    if (g.tilesPerWg <= 2) return launchTile<T, TM, 1>(stream, g);
+  }
   if (g.tilesPerWg <= 4) return launchTile<T, TM, 2>(stream, g);
   if (g.tilesPerWg <= 6) return launchTile<T, TM, 3>(stream, g);
   if constexpr (TM <= 5) {
