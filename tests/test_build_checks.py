@@ -127,3 +127,80 @@ def test_copies_past_the_last_stage_keep_their_offset_inside_the_buffer(tmp_path
     subprocess.run(cmd, check=True)
     r = subprocess.run([exe], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
+
+
+RECTANGLES_PROBE = r"""
+#include <cstdio>
+#include "gemm_weight_stream.hip"
+int amd::computeUnits() { return 256; }
+int main() {
+  long m, n, k, gated;
+  while (scanf("%ld %ld %ld %ld", &m, &n, &k, &gated) == 4) {
+    amd::WeightStreamArgs a;
+    a.siluMul = gated != 0;
+    const float us = amd::weightStreamPlan(m, n, k, &a);
+    printf("%d %d %d %d\n", us > 0, a.tilesM, a.rowsPerWg, a.tilesPerWg);
+  }
+}
+"""
+
+
+def test_rectangles_of_the_gpu_tests_reach_every_tile(tmp_path):
+    """The cases that the GPU tests give to the kernel whose rectangles are cut to the chip: which tile each takes on 256
+    compute units, and that no tile is left out."""
+    from tests.test_gpu_attention_gemm import RECTANGLES
+
+    b = _build_module()
+    (tmp_path / "probe.cpp").write_text(RECTANGLES_PROBE)
+    exe = str(tmp_path / "probe")
+    src = b.TARGETS["impl"]["dir"]
+    cmd = [b.hipcc(), "-O0", "-std=c++17", "-w", "--offload-host-only", f"-I{b.INCLUDE}", f"-I{src}", "-x", "hip", str(tmp_path / "probe.cpp"),
+           "-o", exe, "-Wl,--unresolved-symbols=ignore-all"]
+    subprocess.run(cmd, check=True)
+    text = "".join(f"{m} {n} {k} {int(form == 'gated')}\n" for _, _, form, m, n, k, _ in RECTANGLES)
+    lines = subprocess.run([exe], input=text, capture_output=True, text=True, check=True).stdout.splitlines()
+    assert len(lines) == len(RECTANGLES)
+    for case, line in zip(RECTANGLES, lines):
+        found, tiles_m, rows, tiles = map(int, line.split())
+        tm, tn = max(4, -(-rows // 32)), next(w for w in (2, 4, 6, 8, 12) if tiles <= w) // 2
+        assert found and (tm, tn) == case[:2], (case, line)
+        assert tiles_m * rows >= case[3] > (tiles_m - 1) * rows
+    tiles = {case[:2] for case in RECTANGLES}
+    assert tiles == {(tm, tn) for tm in range(4, 9) for tn in (1, 2, 3, 4, 6) if (tm, tn) != (8, 1) and not (tn == 6 and tm > 5)}
+
+
+NARROW_FORMS_PROBE = r"""
+#include <cstdio>
+#include "narrow_stream.hip"
+int amd::computeUnits() { return 256; }
+int main() {
+  amd::NarrowStreamArgs a;
+  int int8;
+  while (scanf("%d %d %d %d", &int8, &a.M, &a.N, &a.K) == 4) {
+    a.int8B = int8 != 0, a.lda = a.ldb = a.K, a.ldo = a.N;
+    printf("%d\n", (int)amd::narrowStreamPays(a));
+  }
+}
+"""
+
+
+def test_narrow_streams_of_the_gpu_tests_reach_every_form(tmp_path):
+    """The cases that the GPU tests give to the kernel for few columns a compute unit: that it takes them on 256 units, and that
+    no row group, number of column tiles or weight type is left out."""
+    from tests.test_gpu_attention_gemm import NARROW_STREAMS
+
+    b = _build_module()
+    (tmp_path / "probe.cpp").write_text(NARROW_FORMS_PROBE)
+    exe = str(tmp_path / "probe")
+    src = b.TARGETS["impl"]["dir"]
+    cmd = [b.hipcc(), "-O0", "-std=c++17", "-w", "--offload-host-only", f"-I{b.INCLUDE}", f"-I{src}", "-x", "hip", str(tmp_path / "probe.cpp"),
+           "-o", exe, "-Wl,--unresolved-symbols=ignore-all"]
+    subprocess.run(cmd, check=True)
+    text = "".join(f"{int(int8)} {m} {n} {k}\n" for int8, _, _, m, n, k in NARROW_STREAMS)
+    lines = subprocess.run([exe], input=text, capture_output=True, text=True, check=True).stdout.split()
+    assert lines == ["1"] * len(NARROW_STREAMS), [c for c, l in zip(NARROW_STREAMS, lines) if l != "1"]
+    for int8, groups, tiles, m, n, k in NARROW_STREAMS:
+        assert groups == -(-m // 16) and tiles == -(-(-(-n // 256)) // 16)
+    every = {(int8, g, t) for int8 in (False, True) for g in (1, 2, 3, 4) for t in (1, 2)} | {(True, 1, 3)}
+    assert {c[:3] for c in NARROW_STREAMS} == every
+    assert {c[:3] for c in NARROW_STREAMS if c[5] % 128 == 0 and not c[0]} == {c for c in every if not c[0]}  # (rotated)

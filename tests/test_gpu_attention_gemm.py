@@ -536,7 +536,9 @@ def test_slices_of_k_for_one_or_two_workgroups_on_a_compute_unit(ops, dev, pkg, 
                                    (64, 4096, 8192), (40, 4104, 11008), (64, 6144, 4096 + 640),
                                    (20, 8200, 640), (1, 12288, 256), (32, 32000, 384), (7, 8192, 128)])
 def test_skinny_m_linear_and_addmm(ops, dev, dtype, m, n, k):
-    """At most 64 rows against a K-contiguous weight with K a multiple of 128 select the weight-streaming kernel:
+    """(Where few columns come on a compute unit the kernel of the test below takes the product by now: 1 x 4096 x 4096, 64 x 4096 x 4096, 64 x
+    6144 x 4736 and others. What follows is of the shapes that it leaves.)
+    At most 64 rows against a K-contiguous weight with K a multiple of 128 select the weight-streaming kernel:
     one, two and four 16-column tiles per workgroup (N = 4096, 11008, 32000), K in one and in two staged chunks
     and down to a single step per wave, row groups of 16 with a ragged last group, ragged N, bias, and the
     alpha / beta epilogue with a full and a broadcast addend. With more than 32 rows K is also split over the grid
@@ -574,7 +576,8 @@ def test_skinny_m_linear_and_addmm(ops, dev, dtype, m, n, k):
                                    (17, 8190, 1032)])
 def test_few_columns_for_a_compute_unit(ops, dev, dtype, m, n, k):
     # the kernel that streams few columns for each compute unit over the whole of K: ragged column shares, a last stage that
-    # is not whole, fewer stages than ring places, one and two row groups; rows lie in a wider matrix of NaNs
+    # is not whole, fewer stages than ring places, one and two row groups; rows lie in a wider matrix of NaNs. (16 x 8192 x 512 in int8 is
+    # declined, and K that is no multiple of 16 goes to the kernel with one output a lane there: int8 forms in the test below)
     wide = torch.full((m, k + 24), float("nan"), dtype=dtype)
     wide[:, :k] = torch.randn(m, k, generator=g(1)).to(dtype)
     x, xd = wide[:, :k], wide.to(dev)[:, :k]
@@ -589,6 +592,65 @@ def test_few_columns_for_a_compute_unit(ops, dev, dtype, m, n, k):
     want = (x.double() @ q.double().t()) * scale.half().double()
     assert_half(ops.weight_only_int8_linear(xd, q.to(dev), scale.half().to(dev)), want)
     assert_half(ops.weight_only_int8_linear(xd, q.to(dev), scale.half().to(dev), b.to(dev)), want + b.double())
+
+
+def check_rotations(ops, gen, x, w, b, want, hd):
+    """The rotated projection of x by w, whose exact value is `want`, in its forms: either way, with a bias, with tables of both types, of a row
+    for each row of x and of half as many. They hold signed powers of two, so that every result is rounded once."""
+    (m, n), dev, dtype = want.shape, want.device, x.dtype
+    cols = n * 3 // 4 // hd * hd
+    fewer = m // 2 if m % 2 == 0 else m
+    for rows, table_dtype, conj, bias in ((m, dtype, False, None), (fewer, torch.float32, True, b), (fewer, dtype, True, b)):
+        e, sign = (torch.randint(low, high, (rows, hd // 2), generator=gen, device=dev) for low, high in ((-3, 1), (0, 2)))
+        cos, sin = 2.0 ** e, (sign * 2.0 - 1) * 2.0 ** (e - 1)
+        got = ops.linear_rotary(x, w, cos.to(table_dtype), sin.to(table_dtype), cols, hd, bias=bias, conj=conj)
+        v = want if bias is None else want + bias.double()
+        pairs, co, si = v[:, :cols].reshape(m // rows, rows, cols // hd, hd // 2, 2), cos.double()[:, None], sin.double()[:, None] * (-1 if conj else 1)
+        rotated = torch.stack([pairs[..., 0] * co - pairs[..., 1] * si, pairs[..., 0] * si + pairs[..., 1] * co], -1).reshape(m, cols)
+        assert_exact(got, torch.cat([rotated, v[:, cols:]], 1).to(dtype))
+
+
+# int8 weights or not, groups of 16 rows, column tiles of 16 of a workgroup
+NARROW_STREAMS = [
+    (False, 1, 1, 5, 4090, 1032), (False, 1, 2, 16, 8186, 1544), (False, 2, 1, 17, 4090, 1544), (False, 2, 2, 32, 8190, 1032), (False, 3, 1, 33, 4090, 1288),
+    (False, 3, 2, 48, 6144, 4096), (False, 3, 2, 47, 8190, 1288), (False, 4, 1, 64, 4090, 1288), (False, 4, 2, 49, 8190, 1288),
+    (True, 1, 1, 3, 4090, 1040), (True, 1, 2, 16, 8190, 2064), (True, 1, 3, 12, 12280, 2064), (True, 2, 1, 17, 4090, 1040), (True, 2, 2, 32, 8190, 2064),
+    (True, 3, 1, 33, 4090, 1040), (True, 3, 2, 48, 6144, 4096), (True, 3, 2, 47, 8190, 2064), (True, 4, 1, 64, 4090, 1040), (True, 4, 2, 49, 8190, 2064),
+    (False, 1, 1, 6, 4030, 1152), (False, 1, 2, 10, 8190, 1152), (False, 2, 1, 20, 4030, 1152), (False, 2, 2, 32, 8190, 1152), (False, 3, 1, 34, 4030, 1152),
+    (False, 3, 2, 48, 6144, 4096), (False, 4, 1, 64, 4030, 1152), (False, 4, 2, 50, 8190, 1152),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("int8,groups,tiles,m,n,k", NARROW_STREAMS)
+def test_every_form_of_the_narrow_streams_exact(ops, dev, pkg, dtype, int8, groups, tiles, m, n, k):
+    """Every form of the kernel that streams few columns for each compute unit, with a last stage of K that is not whole: plain, with
+    a bias, with an addend and written over it; rotated where K is a multiple of 128, either way, with tables of either type, of a row for each
+    and of half as many; int8 weights with scales and biases in fp32 and in 16 bits. Sums of small whole numbers, which fp32 holds
+    exactly in any order, rounded once. That the forms are these is checked without a GPU, in the build's checks."""
+    gen = torch.Generator(dev).manual_seed(83)
+    whole = lambda *s, scale=1.0: torch.randint(-3, 4, s, generator=gen, device=dev).to(dtype) * scale
+    x, b = whole(m, k), whole(n)
+    with own_context(ops, pkg) as ctx:
+        if int8:
+            w = torch.randint(-127, 128, (n, k), generator=gen, device=dev, dtype=torch.int8)
+            scale = 2.0 ** torch.randint(-12, -8, (n,), generator=gen, device=dev)
+            want = x.double() @ w.double().t() * scale.double()
+            assert_exact(ops.weight_only_int8_linear(x, w, scale.half()), want.to(dtype))
+            assert_exact(ops.weight_only_int8_linear(x, w, scale.float(), b), (want + b.double()).to(dtype))
+            assert_exact(ops.weight_only_int8_linear(x, w, scale.float(), b.float()), (want + b.double()).to(dtype))
+        else:
+            w, c = whole(n, k, scale=2.0 ** -6), whole(m, n)
+            want = x.double() @ w.double().t()
+            assert_exact(ops.linear(x, w), want.to(dtype))
+            assert_exact(ops.linear(x, w, b), (want + b.double()).to(dtype))
+            assert_exact(ops.addmm(b, x, w.t(), beta=-1), (want - b.double()).to(dtype))
+            total = (0.5 * c.double() + 2 * want).to(dtype)
+            assert_exact(ops.addmm(c, x, w.t(), beta=0.5, alpha=2), total)
+            assert_exact(ops.addmm(c, x, w.t(), beta=0.5, alpha=2, out=c), total)
+            if k % 128 == 0:
+                check_rotations(ops, gen, x, w, b, want, 64)
+        assert ctx.workspace()[1] == 0
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -607,6 +669,7 @@ def test_k_slices_or_a_stream_where_k_is_a_little_less_than_4096(ops, dev, pkg, 
 @pytest.mark.parametrize("table_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("m,heads,hd,vcols,k", [(3, 10, 128, 2 * 128, 4096), (16, 40, 64, 1000, 1032), (17, 6, 128, 256, 768), (5, 33, 64, 130 * 8, 2048 + 128), (40, 10, 128, 2 * 128, 1152), (64, 40, 64, 1000, 1536)])
 def test_rotation_with_few_columns_for_a_compute_unit(ops, dev, table_dtype, m, heads, hd, vcols, k):
+    # (K = 1032, no multiple of 128: the product and the rotation in launches of their own)
     n, cols = heads * hd + vcols, heads * hd
     x = torch.randn(m, k, generator=g(1)).bfloat16()
     w = (torch.randn(n, k, generator=g(2)) / k**0.5).bfloat16()
@@ -626,8 +689,8 @@ def test_rotation_with_few_columns_for_a_compute_unit(ops, dev, table_dtype, m, 
 @pytest.mark.parametrize("m,n,k", [(65, 512, 1024), (128, 4096, 1024), (97, 11008, 1088), (704, 1536, 1152), (257, 11008, 1088), (257, 14336, 4096), (257, 22016, 4096),
                                    (704, 6144, 1088), (704, 8192, 4096), (203, 22016, 4096), (300, 3072, 1088), (451, 1040, 1024), (600, 2560, 1216)])
 def test_rectangles_cut_to_the_chip(ops, dev, dtype, m, n, k):
-    # the kernel of 65 to 704 rows whose rectangles are cut to the chip: ragged last rows and column tiles,
-    # every width, 16 stages of K and more; rows lie in a wider matrix of NaNs
+    # the kernel of 65 to 704 rows whose rectangles are cut to the chip, on drawn numbers: ragged last rows and column tiles,
+    # 16 stages of K and more; rows lie in a wider matrix of NaNs (every tile of it: the test below)
     wide = torch.full((m, k + 24), float("nan"), dtype=dtype)
     wide[:, :k] = torch.randn(m, k, generator=g(1)).to(dtype)
     x, xd = wide[:, :k], wide.to(dev)[:, :k]
@@ -649,6 +712,58 @@ def test_rectangles_cut_to_the_chip(ops, dev, dtype, m, n, k):
         rotated = torch.stack([pairs[..., 0] * co - pairs[..., 1] * si, pairs[..., 0] * si + pairs[..., 1] * co], -1).reshape(m, cols)
         got = ops.linear_rotary(xd, w.to(dev), cos.to(dev), sin.to(dev), cols, hd, bias=b.to(dev))
         assert_half(got, torch.cat([rotated, (want + b.double())[:, cols:]], 1))
+
+
+# (TM, TN): an output tile is 32 TM rows by 32 TN columns. The last entry: the other form would take workspace.
+RECTANGLES = [
+    (4, 1, "gated", 70, 2944, 1280, True), (4, 1, "plain", 67, 144, 1088, True), (4, 1, "rotated", 66, 144, 1024, True),
+    (4, 2, "gated", 114, 4160, 1024, True), (4, 2, "plain", 118, 4192, 1024, True), (4, 2, "rotated", 116, 4304, 1024, True),
+    (4, 3, "gated", 103, 8576, 1024, True), (4, 3, "plain", 97, 8576, 1024, True), (4, 3, "rotated", 102, 8352, 1024, True),
+    (4, 4, "gated", 110, 32576, 3904, False), (4, 4, "plain", 79, 32736, 6592, False), (4, 4, "rotated", 80, 31296, 10240, False),
+    (4, 6, "gated", 147, 16640, 1024, False), (4, 6, "plain", 146, 17024, 1152, False), (4, 6, "rotated", 152, 16592, 1856, False),
+    (5, 1, "gated", 257, 3328, 2624, True), (5, 1, "plain", 529, 1648, 1024, True), (5, 1, "rotated", 514, 1680, 1024, True),
+    (5, 2, "gated", 640, 3520, 3520, False), (5, 2, "plain", 130, 16352, 9216, True), (5, 2, "rotated", 284, 6928, 5632, True),
+    (5, 3, "gated", 131, 16512, 1024, False), (5, 3, "plain", 133, 16544, 1088, False), (5, 3, "rotated", 134, 22688, 3712, True),
+    (5, 4, "gated", 129, 24960, 3840, True), (5, 4, "plain", 131, 25888, 3584, True), (5, 4, "rotated", 130, 30240, 3840, True),
+    (5, 6, "gated", 257, 18304, 1024, False), (5, 6, "plain", 264, 18576, 1408, False), (5, 6, "rotated", 258, 17776, 10752, True),
+    (6, 1, "plain", 481, 2704, 1024, True), (6, 1, "rotated", 482, 2704, 1024, True), (6, 2, "gated", 340, 6720, 5952, True),
+    (6, 2, "plain", 383, 8080, 8704, False), (6, 3, "gated", 641, 5632, 3712, True), (6, 3, "plain", 168, 22624, 3584, True),
+    (6, 3, "rotated", 168, 23968, 4480, True), (6, 4, "gated", 163, 26240, 3584, True), (6, 4, "plain", 162, 26944, 3840, True),
+    (6, 4, "rotated", 166, 31888, 4096, True), (7, 1, "plain", 577, 2704, 1024, True), (7, 1, "rotated", 578, 2704, 1024, True),
+    (7, 2, "gated", 650, 5440, 1088, False), (7, 2, "plain", 641, 5392, 3840, True), (7, 2, "rotated", 642, 5392, 1408, False),
+    (7, 3, "gated", 583, 6592, 1024, False), (7, 3, "plain", 660, 7088, 3328, True), (7, 3, "rotated", 204, 24400, 6400, True),
+    (7, 4, "gated", 199, 28160, 3840, True), (7, 4, "plain", 199, 29472, 3968, True), (7, 4, "rotated", 200, 31440, 4736, True),
+    (8, 2, "gated", 697, 5440, 1216, False), (8, 2, "plain", 673, 5408, 3840, True), (8, 2, "rotated", 674, 5392, 1536, False),
+    (8, 3, "gated", 701, 7616, 3328, True), (8, 3, "plain", 673, 7568, 3328, True), (8, 3, "rotated", 686, 6592, 2944, False),
+    (8, 4, "gated", 230, 28992, 3968, True), (8, 4, "plain", 226, 31328, 4096, True), (8, 4, "rotated", 236, 31936, 8064, True),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tm,tn,form,m,n,k,told", RECTANGLES)
+def test_every_form_of_the_rectangles_exact(ops, dev, pkg, dtype, tm, tn, form, m, n, k, told):
+    """Every tile of the kernel whose rectangles are cut to the chip: plain, with a bias, with an addend and written over it; gated; rotated either
+    way, with tables of either type, of a row for each and of half as many. Sums of small whole numbers, which fp32 holds exactly in
+    any order, rounded once (but for the gate). That the cuts are these is checked without a GPU, in the build's checks."""
+    gen = torch.Generator(dev).manual_seed(82)
+    whole = lambda *s, scale=1.0: torch.randint(-3, 4, s, generator=gen, device=dev).to(dtype) * scale
+    x, w = whole(m, k), whole(n, k, scale=2.0 ** -6)
+    want = torch.cat([x.double() @ part.double().t() for part in w.split(4096)], 1)
+    with own_context(ops, pkg) as ctx:
+        if form == "plain":
+            b, c = whole(n), whole(m, n)
+            assert_exact(ops.linear(x, w), want.to(dtype))
+            assert_exact(ops.linear(x, w, b), (want + b.double()).to(dtype))
+            assert_exact(ops.addmm(b, x, w.t(), beta=-1), (want - b.double()).to(dtype))
+            total = (0.5 * c.double() + 2 * want).to(dtype)
+            assert_exact(ops.addmm(c, x, w.t(), beta=0.5, alpha=2), total)
+            assert_exact(ops.addmm(c, x, w.t(), beta=0.5, alpha=2, out=c), total)
+        elif form == "gated":
+            blocks = want.view(m, n // 64, 2, 32)
+            assert_half(ops.linear_silu_mul(x, w), (torch.nn.functional.silu(blocks[:, :, 0]) * blocks[:, :, 1]).reshape(m, n // 2))
+        else:
+            check_rotations(ops, gen, x, w, whole(n), want, 8 if n < 512 else 64)
+        assert not told or ctx.workspace()[1] == 0
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -1455,9 +1570,9 @@ def test_weight_only_int8_linear_chunked_k_row_groups_and_tile_counts(ops, dev, 
 @pytest.mark.parametrize("m,k,n", [(64, 14336, 4096), (33, 4096, 4096), (17, 2048 + 256, 5120), (48, 11008, 4100), (64, 2048, 200),
                                    (4, 8192, 4096), (16, 8192, 8192)])
 def test_weight_only_int8_linear_narrow_weights_split_over_k(ops, dev, pkg, m, k, n, dtype):
-    """Weights of fewer than 10240 channels at 17 - 64 rows, or at fewer rows with K from 8192 on: K split over workgroups
-    (4, 4, 3, 3, 4, 4 and 2 slices here, one with a shorter last slice, two with a ragged last channel block), unscaled fp32 sums reduced by a second launch that applies scale and
-    bias: against the oracle, with a bias in float32, and exactly on one-hot rows."""
+    """Weights of fewer than 10240 channels with few columns for each compute unit: K split over workgroups for 48 and 64 rows with a long K (4 and
+    3 slices, the latter with a ragged last channel block), unscaled fp32 sums reduced by a second launch that applies scale and bias; the
+    others stream the whole of K. Against the oracle, with a bias in float32, and exactly on one-hot rows."""
     w = pkg.workloads.int8_linear(seed=8, m=m, k=k, n=n, dtype=dtype)
     want = oracle.weight_only_int8_linear(w["x"], w["w"], w["scale"])
     assert_half(ops.weight_only_int8_linear(w["x"].to(dev), w["w"].to(dev), w["scale"].to(dev)), want)
@@ -1468,6 +1583,24 @@ def test_weight_only_int8_linear_narrow_weights_split_over_k(ops, dev, pkg, m, k
     x[torch.arange(m), cols] = 1
     got = ops.weight_only_int8_linear(x.to(dev), w["w"].to(dev), w["scale"].to(dev))
     assert_exact(got, (w["w"][:, cols].float() * w["scale"].float()[:, None]).t().to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,k,n,slices", [(16, 28672, 8192, 2), (17, 13824, 5120, 3), (32, 11008, 4096, 4), (24, 11008, 4100, 3), (31, 8448, 200, 11), (48, 11008, 4100, 3),
+                                          (64, 14336, 4096, 4), (17, 8192, 5120, 0)])
+def test_weight_only_int8_linear_k_slices_for_one_to_four_row_groups(ops, dev, pkg, m, k, n, slices, dtype):
+    """K split over workgroups, as the workspace of the slices' sums tells, at 13 to 64 rows: one, two and four row groups, a shorter last
+    slice, a ragged last channel block (and one shape that is left whole). Sums of whole numbers below 2^24, exact in fp32, scaled by
+    powers of two and rounded once."""
+    gen = torch.Generator(dev).manual_seed(39)
+    x = torch.randint(-3, 4, (m, k), generator=gen, device=dev).to(dtype)
+    w = torch.randint(-127, 128, (n, k), generator=gen, device=dev, dtype=torch.int8)
+    scale, bias = 2.0 ** torch.randint(-12, -8, (n,), generator=gen, device=dev), torch.randint(-4, 5, (n,), generator=gen, device=dev).float()
+    want = x.double() @ w.double().t() * scale.double()
+    with own_context(ops, pkg) as ctx:
+        assert_exact(ops.weight_only_int8_linear(x, w, scale.half()), want.to(dtype))
+        assert ctx.workspace()[1] == slices * m * n * 4
+        assert_exact(ops.weight_only_int8_linear(x, w, scale.float(), bias), (want + bias.double()).to(dtype))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
