@@ -2972,28 +2972,22 @@ static diopiError_t launchSkinnyForShape(diopiContextHandle_t ctx, hipStream_t s
   if (rot != nullptr) AMD_TRY(tryNarrowStream(stream, p, rot, handled));  // (runGemm has asked for the others)
   if (rot != nullptr && *handled) return diopiSuccess;
   const int tiles = (a.N + 15) / 16, cus = computeUnits(), perCu = (tiles + cus - 1) / cus;
-  // (What follows gets what narrowStreamPays declined; the figures for N up to 8192 were measured without that kernel.)
+  // What narrowStreamPays declined comes here: weights of more than 32 columns for a unit, 33 to 64 rows against a K of more than one and
+  // a half times the columns, 17 to 32 rows against one above 8192, the smallest weights at one or two rows, 2 GiB and more.
   // Both operands through LDS, see gemmSkinnyLdsKernel. The columns are dealt evenly over as many workgroups as there
   // are CUs (43 each at N = 11008, where 64-column blocks would leave a third of the CUs idle): a CU takes in about
   // 45 GB/s from a cold stream whatever the software pipeline depth, so the count of CUs at work sets the rate.
-  // Measured cold against the forms below on K = 4096 (us, at 1 / 16 / 32 / 64 rows): N = 6144 13.7 -> 12.9,
-  // 15.2 -> 13.4, 24.5 -> 14.9, 25.0 -> 18.2; N = 8192 16.6 -> 13.3, 18.0 -> 14.5, 22.5 -> 16.4, 27.3 -> 19.5;
-  // N = 11008 18.5 -> 16.9, 20.4 -> 17.7, 33 -> 19.3, 30.4 -> 23.2; N = 22016 38.2 -> 30.1, 46.0 -> 31.9,
-  // 52.9 -> 33.6, 55.7 -> 36.0. At N = 4096 (16 columns per workgroup: the activations are four times the weight
-  // bytes on the way into a CU) only 17 to 32 rows gain (14.4 -> 12.7); one row loses (9.1 -> 11.0), and so does
-  // everything narrower.
-  // A 4096-wide weight (the o and down projections of a decode step) takes this form too with K split over grid.y, fp32
-  // slices and the reduction pass: with K of 8192 and more at any row count, two slices up to 16 rows and four beyond
-  // (us cold at K = 11008 against the register-layout kernels below: 1 row 23.9 -> 19.2, 16 rows 28.3 -> 20.3, 32 rows
-  // 27.5 -> 21.6, 64 rows 34.0 -> 24.5 (27.7 with two slices); 64 x 4096 x 14336 34.2 -> 28.5). At K = 4096 two slices are
-  // within the noise of what the other routes do (32 rows 12.4 -> 11.5 .. 12.3, 64 rows 14.5 -> 13.8 .. 14.8) and one row
-  // loses (7.7 -> 10.0). The same split on wider weights loses (N = 11008: 23.0 -> 25.5 us, four ways 33.6).
+  // Measured cold against the forms below on K = 4096 (us, at 1 / 16 / 32 / 64 rows): N = 11008 18.5 -> 16.9, 20.4 -> 17.7,
+  // 33 -> 19.3, 30.4 -> 23.2; N = 22016 38.2 -> 30.1, 46.0 -> 31.9, 52.9 -> 33.6, 55.7 -> 36.0.
+  // A 4096-wide weight with K of 8192 and more (the o and down projections of a decode step) takes this form too with K split over
+  // grid.y, fp32 slices and the reduction pass, in four slices (us cold at K = 11008 against the register-layout kernels below:
+  // 32 rows 27.5 -> 21.6, 64 rows 34.0 -> 24.5 (27.7 with two slices); 64 x 4096 x 14336 34.2 -> 28.5). The same split on
+  // wider weights loses (N = 11008: 23.0 -> 25.5 us, four ways 33.6).
   const bool canSplitLds = a.N % 8 == 0 && mult8(p.sOm) && ptr16(p.out) && (!p.bias || ptr16(p.bias)) &&
                            (!p.Cin || (p.sCn == 1 && mult8(p.sCm) && ptr16(p.Cin))) && rot == nullptr;
-  // Weights of 5120 to 10239 rows take the K slices when K is at least twice their width (the down projections of
-  // larger models; us, 1 / 16 / 32 / 64 rows: 5120 x 13824 30.7 -> 23.7, 31.8 -> 25.4, 36.1 -> 29.1, 46.5 -> 33.4;
-  // 6144 x 16384 at 64 rows 55.7 -> 41.9; 8192 x 28672 at 64 rows 111.6 -> 95.2); a square 8192 x 8192 loses
-  // (one row 21.5 -> 27.8).
+  // Weights of 5120 to 10239 rows take the K slices when K is at least twice their width (the down projections of larger
+  // models; us, 32 / 64 rows: 5120 x 13824 36.1 -> 29.1, 46.5 -> 33.4; 64 rows, 6144 x 16384 55.7 -> 41.9, 8192 x 28672 111.6 -> 95.2).
+  // Up to 16 rows, above 8192 columns only, two slices.
   const bool narrow = a.N >= 4096 && (a.N < 5120 || (a.N < 10240 && a.K >= 2 * a.N)) && a.K % kSkinnyLdsBK == 0 && canSplitLds;
   const int narrowWays = narrow && a.K >= 8192 ? (a.M <= 16 ? 2 : 4) : 1;
   const bool narrowLongK = narrowWays > 1;
@@ -3027,7 +3021,8 @@ static diopiError_t launchSkinnyForShape(diopiContextHandle_t ctx, hipStream_t s
     return diopiSuccess;
   }
   if (a.M <= 16) {
-    // 16-column tiles per workgroup: about one workgroup per CU, the other waves of the 15 or 16 split K
+    // 16-column tiles per workgroup: about one workgroup per CU, the other waves of the 15 or 16 split K (more than two tiles
+    // come on a CU only with weights of 2 GiB and more)
     if (perCu >= 4) return launchSkinny<T, 4, 4, 1>(stream, a);
     if (perCu == 3) return launchSkinny<T, 3, 5, 1>(stream, a);
     if (perCu == 2) return launchSkinny<T, 2, 8, 1>(stream, a);
@@ -3168,7 +3163,8 @@ static bool reserveTail(diopiContextHandle_t ctx, hipStream_t stream, GemmProble
 // K 8 %). A last round in slices of K needs 12 %: its estimate is 7 % off either way, and 7 % is what 400 x 12288 x 4096 would gain.
 // pass: what a gate or a rotation takes that slices of K leave to a launch of its own, see passUs.
 // With these lines no choice of 6200 products (610 weights of 0.3 to 400 MB; plain, gated and rotated) costs more than 9 %, six more than 3 %,
-// and what is left of the gains is 0.4 % on average.
+// and what is left of the gains is 0.4 % on average. (A stream that is recorded, or a context that holds the workspace of many calls, has none to spare
+// for K slices of a last round: where those are the better form here, the product takes 128 x 128 tiles there, and no rectangles either.)
 static bool weightStreamPays(const GemmProblem& p, float pass, float us) {
   const int resident = computeUnits() / 8 * 8;
   const int64_t tiles256 = ceilDiv(p.M, 256) * ceilDiv(p.N, 256), pairs = p.K / (2 * kBK);

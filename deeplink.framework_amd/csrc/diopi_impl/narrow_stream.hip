@@ -27,7 +27,7 @@ constexpr int kNarrowBK = 512;
 // out of HBM under way: copies past that hold up the waves that issue them). us at one row, places 5 + 4 -> 4 + 3 (16-bit, one
 // column tile) 4096 x 4096 8.73 -> 8.35; int8, 8 + 4 -> 4 + 4, 4096 x 11008 11.60 -> 10.85; int8, two tiles, 6 + 4 -> 3 + 3, 8192 x 8192
 // 13.9 -> 12.65. Fewer lose: 16-bit 3 + 3 4096 x 11008 16.75 -> 22.7, two tiles 3 + 2 5120 x 13824 24.2 -> 27.6.
-constexpr int narrowStagesW(int tiles, int bk) { return tiles == 1 ? 4 : 3; }
+constexpr int narrowStagesW(int tiles) { return tiles == 1 ? 4 : 3; }
 constexpr int narrowStagesX(bool int8, int tiles, int bk) { return int8 && tiles == 1 && bk == kNarrowBK ? 4 : 3; }
 
 // The stage of K that a workgroup which starts its walk at stage `start` visits c-th. Past the end, where copies fetch nothing, the last
@@ -41,7 +41,7 @@ template <typename T, bool W8, int G, int NT, int BK>
 __global__ __launch_bounds__(512) void narrowStreamKernel(NarrowStreamArgs a) {
   typedef typename Vec16<T>::type Frag;
   constexpr int kSize = W8 ? 1 : 2, KS = BK / 256;                   // bytes of a weight; 32-wide k-steps of a wave and stage
-  constexpr int WST = narrowStagesW(NT, BK), XST = narrowStagesX(W8, NT, BK);    // ring places
+  constexpr int WST = narrowStagesW(NT), XST = narrowStagesX(W8, NT, BK);    // ring places
   constexpr int kRowBytes = BK * kSize, kLanes = kRowBytes / 16;     // of a weight row's stage, and the lanes that copy it
   constexpr int kRows = 64 / kLanes;                                 // weight rows of a copy instruction (1 KiB)
   static_assert(16 * NT / kRows % 4 == 0, "four waves copy as many pieces each");
@@ -221,7 +221,7 @@ __global__ __launch_bounds__(512) void narrowStreamKernel(NarrowStreamArgs a) {
 
 template <typename T, bool W8, int G, int NT, int BK = kNarrowBK>
 static diopiError_t launchTiles(hipStream_t stream, const NarrowStreamArgs& a) {
-  constexpr int lds = std::max(narrowStagesW(NT, BK) * 16 * NT * BK * (W8 ? 1 : 2) + narrowStagesX(W8, NT, BK) * 32 * G * BK, 8 * G * NT * 1024);
+  constexpr int lds = std::max(narrowStagesW(NT) * 16 * NT * BK * (W8 ? 1 : 2) + narrowStagesX(W8, NT, BK) * 32 * G * BK, 8 * G * NT * 1024);
   static_assert(lds <= 160 * 1024, "LDS of a compute unit");
   AMD_HIP(allowDynamicLds(reinterpret_cast<const void*>(&narrowStreamKernel<T, W8, G, NT, BK>), lds));
   hipLaunchKernelGGL((narrowStreamKernel<T, W8, G, NT, BK>), dim3((unsigned)ceilDiv(a.N, a.colsPerWg)), dim3(512), lds, stream, a);

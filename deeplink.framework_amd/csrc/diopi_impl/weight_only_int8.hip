@@ -436,7 +436,7 @@ static diopiError_t launchW8ForShape(hipStream_t stream, const W8Args& a0) {
   // Wide weights go through w8LinearLdsKernel, the channels dealt evenly over the CUs. Measured cold against the form
   // below at K = 4096 (us, 1 / 16 / 32 / 64 rows): N = 11008 11.0 -> 10.8, 12.9 -> 11.7, 17.0 -> 14.2, 23.1 -> 21.1;
   // N = 22016 22.0 -> 19.2, 26.8 -> 20.2. Both forms have about 10 us of floor at these sizes, so narrower weights
-  // gain only with more than 16 rows (N = 6144: 14.7 -> 13.1 at 32 rows, 9.0 -> 10.4 at one).
+  // gain only with more than 16 rows (of 6144 to 10239 channels narrowStreamPays and the K slices leave few).
   if ((a.N >= 10240 || (a.N >= 6144 && a.M > 16)) && a.K % 256 == 0 && (int64_t)(a.N - 1) * a.ldw + a.K < ((int64_t)1 << 31)) {
     const int cus = computeUnits(), rounds = (a.N + 128 * cus - 1) / (128 * cus);
     a.colsPerWg = (a.N + cus * rounds - 1) / (cus * rounds);
