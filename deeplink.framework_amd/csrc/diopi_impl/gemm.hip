@@ -2941,11 +2941,11 @@ static bool mult8(int64_t v) { return (v & 7) == 0; }
 static bool ptr16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // The kernel for few columns a compute unit, if it pays for the product (16-bit, one batch, K of both operands contiguous).
-static diopiError_t tryNarrowStream(hipStream_t stream, const GemmProblem& p, const RotaryEpilogue* rot, bool* done) {
+static diopiError_t tryNarrowStream(hipStream_t stream, const GemmProblem& p, const RotaryEpilogue* rot, bool* done, bool noSlices = false) {
   NarrowStreamArgs a;
   a.A = p.A, a.B = p.B, a.out = p.out, a.Cin = p.Cin, a.bias = p.bias, a.biasDtype = (int)p.dtype;
   a.lda = p.sAm, a.ldb = p.sBn, a.ldo = p.sOm, a.sCm = p.sCm, a.sCn = p.sCn;
-  a.M = (int)p.M, a.N = (int)p.N, a.K = (int)p.K, a.alpha = p.alpha, a.beta = p.beta;
+  a.M = (int)p.M, a.N = (int)p.N, a.K = (int)p.K, a.alpha = p.alpha, a.beta = p.beta, a.noSlices = noSlices;
   if (rot != nullptr) {
     a.rotCos = rot->cosT, a.rotSin = rot->sinT, a.rotCols = rot->cols, a.rotHeadDim = rot->headDim, a.rotTableRows = rot->tableRows;
     a.rotTableF32 = rot->tableF32, a.rotSinSign = rot->sinSign;
@@ -3064,7 +3064,12 @@ static diopiError_t launchSkinnyForShape(diopiContextHandle_t ctx, hipStream_t s
   const int splits = canSplit && groups == 4 ? (a.K + chunk - 1) / chunk : 1;  // two groups: measured no gain
   if (splits > 1) {
     void* ws = nullptr;
-    AMD_TRY(requireWorkspace(ctx, (int64_t)splits * a.M * a.N * 4, &ws));
+    if (requireWorkspace(ctx, (int64_t)splits * a.M * a.N * 4, &ws) != diopiSuccess) {
+      // (as in a recording that nothing was held for: what came here only because slices are the faster form)
+      bool done = false;
+      AMD_TRY(tryNarrowStream(stream, p, nullptr, &done, true));
+      return done ? diopiSuccess : diopiErrorOccurred;
+    }
     a.partial = static_cast<float*>(ws), a.kPerWg = chunk;
   }
   const int want = std::max(1, std::min(4, tiles * splits / cus));  // tiles per workgroup that still fill the chip
@@ -3200,7 +3205,8 @@ static float passUs(const GemmProblem& p, const RotaryEpilogue* rot, bool gate) 
   return gate ? 1.8f + 1.1e-6f * (float)(p.M * p.N) : rot != nullptr ? 2.3f + 1.1e-6f * (float)(p.M * rot->cols) : 0.f;
 }
 
-static diopiError_t tryWeightStream(hipStream_t stream, const GemmProblem& p, const RotaryEpilogue* rot, bool gate, bool* done) {
+// (anyway: the other forms have no workspace)
+static diopiError_t tryWeightStream(hipStream_t stream, const GemmProblem& p, const RotaryEpilogue* rot, bool gate, bool* done, bool anyway = false) {
   *done = false;
   const int64_t outCols = gate ? p.N / 2 : p.N;
   auto fits = [](int64_t rows, int64_t pitch, int64_t cols) { return ((rows - 1) * pitch + cols) * 2 < (int64_t(1) << 31); };
@@ -3215,7 +3221,7 @@ static diopiError_t tryWeightStream(hipStream_t stream, const GemmProblem& p, co
   if (us == 0.f) return diopiSuccess;
   // (rotating the sums of a rectangle takes 0.6 us and 5.6 ns for each row of each pair of column tiles)
   if (rot != nullptr) us += 0.6f + 0.0056f * (float)(a.rowsPerWg * ceilDiv(a.tilesPerWg, 2));
-  if (!weightStreamPays(p, passUs(p, rot, gate), us)) return diopiSuccess;
+  if (!anyway && !weightStreamPays(p, passUs(p, rot, gate), us)) return diopiSuccess;
   a.A = p.A, a.B = p.B, a.out = p.out, a.Cin = p.Cin, a.bias = p.bias;
   a.lda = p.sAm, a.ldb = p.sBn, a.ldo = p.sOm, a.sCm = p.sCm;
   a.M = (int)p.M, a.N = (int)p.N, a.K = (int)p.K, a.alpha = p.alpha, a.beta = p.beta;
@@ -3485,11 +3491,10 @@ static diopiError_t runGatedSiluGemm(diopiContextHandle_t ctx, hipStream_t strea
                       p.K % kBK == 0 && p.K >= 2 * kBK &&
                       ((p.M - 1) * p.sAm + p.K) * 2 < (int64_t(1) << 31) && ((p.N - 1) * p.sBn + p.K) * 2 < (int64_t(1) << 31) &&
                       mult8(p.sOm) && ptr16(p.out) && p.M < (int64_t(1) << 31) && p.N < (int64_t(1) << 31);
-  if (direct && p.Cin == nullptr && p.bias == nullptr && p.alpha == 1.f) {
-    bool done = false;
-    AMD_TRY(tryWeightStream(stream, p, nullptr, true, &done));
-    if (done) return diopiSuccess;
-  }
+  const bool rectangles = direct && p.Cin == nullptr && p.bias == nullptr && p.alpha == 1.f;
+  bool streamed = false;
+  if (rectangles) AMD_TRY(tryWeightStream(stream, p, nullptr, true, &streamed));
+  if (streamed) return diopiSuccess;
   const FusedTile fused = direct ? fusedTile(ctx, stream, &p) : kFusedNone;
   if (fused == kFused256)
     return p.dtype == diopi_dtype_bfloat16 ? launchMfmaPipelined<bf16_t, kEpiSiluMul>(ctx, stream, p)
@@ -3526,7 +3531,11 @@ static diopiError_t runGatedSiluGemm(diopiContextHandle_t ctx, hipStream_t strea
   // two passes: the full-width projection into workspace, then the gate
   void* ws = nullptr;
   const int64_t item = dtypeSize(p.dtype);
-  AMD_TRY(requireWorkspace(ctx, p.M * p.N * item, &ws));
+  if (requireWorkspace(ctx, p.M * p.N * item, &ws) != diopiSuccess) {
+    // (as in a recording that nothing was held for)
+    if (rectangles) AMD_TRY(tryWeightStream(stream, p, nullptr, true, &streamed, true));
+    return streamed ? diopiSuccess : diopiErrorOccurred;
+  }
   GemmProblem q = p;
   void* finalOut = p.out;
   const int64_t ldo = p.sOm;

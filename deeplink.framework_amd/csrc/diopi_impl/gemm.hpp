@@ -99,6 +99,7 @@ struct NarrowStreamArgs {
   bool rotTableF32 = false;
   float rotSinSign = 1.f;
   int colsPerWg = 0;
+  bool noSlices = false;  // K slices, the faster form of some, have no workspace
 };
 bool narrowStreamPays(const NarrowStreamArgs& a);
 diopiError_t launchNarrowStream(hipStream_t stream, diopiDtype_t dtype, NarrowStreamArgs a);

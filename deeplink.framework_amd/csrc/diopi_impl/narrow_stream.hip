@@ -279,7 +279,7 @@ bool narrowStreamPays(const NarrowStreamArgs& a) {
     if (2 * (int64_t)a.K <= 3 * (int64_t)a.N) return true;
     if (a.int8B) return a.K <= 4096;
     // (the other form: four slices of up to 1024 columns, eight steps of 128, in pieces of 8 results, and a rotation in a pass of its own)
-    const bool slicesFit = a.rotCols == 0 && ceilDiv(a.N, 16) * 4 <= computeUnits() && a.N >= 16 && a.N % 8 == 0 && a.K % 128 == 0;
+    const bool slicesFit = a.rotCols == 0 && !a.noSlices && ceilDiv(a.N, 16) * 4 <= computeUnits() && a.N >= 16 && a.N % 8 == 0 && a.K % 128 == 0;
     return a.K < 4096 && !(a.K > 3328 && slicesFit);
   }
   if (a.int8B) {

@@ -159,6 +159,41 @@ def test_products_that_can_do_without_workspace_record_without_it(pkg, ops, dev)
             assert torch.equal(t, u) and torch.equal(u, v)
 
 
+
+def test_products_whose_faster_form_takes_workspace_record_in_the_other_one(pkg, ops, dev):
+    """Products that take K slices only because those are faster than a kernel without workspace: recorded with nothing held for them they
+    go to that kernel. A few whole numbers in each row, so that the sums are exact and 16 bits hold the gate's two halves."""
+    gen = torch.Generator().manual_seed(10)
+    rnd = lambda *shape: torch.randint(-2, 3, shape, generator=gen).to(torch.bfloat16).to(dev)
+    few = lambda m, k: torch.zeros(m, k).scatter_(1, torch.stack([torch.randperm(k, generator=gen)[:16] for _ in range(m)]), 1).to(torch.bfloat16).to(dev)
+    x, w, y, v = rnd(64, 3968), rnd(512, 3968), few(111, 3072), rnd(448, 3072)
+    calls = [lambda: ops.linear(x, w), lambda: ops.linear_silu_mul(y, v)]
+    with pkg.diopi.Context() as ctx:                                                               # eager, both take slices
+        out = torch.empty(64, 512, dtype=x.dtype, device=dev)
+        handles = [pkg.diopi.handle(t) for t in (out, x, w, None)]
+        pkg.diopi.call("diopiLinear", ctx, *[p for _, p in handles])
+        assert ctx.workspace() == (1, 4 * 64 * 512 * 4)
+        torch.cuda.synchronize()
+    want = [f() for f in calls]
+    torch.cuda.synchronize()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=side):
+        scope = ops.WorkspaceScope()
+        with scope:
+            got = [f() for f in calls]
+    assert scope.ctx.workspace() == (0, 0)
+    for _ in range(3):
+        for t in got:
+            t.zero_()
+        graph.replay()
+        again = [f() for f in calls]
+        torch.cuda.synchronize()
+        for t, u, r in zip(got, want, again):
+            assert torch.equal(t, u) and torch.equal(u, r)
+    del graph
+    scope.close()
+
+
 def test_recorded_int8_products_of_a_few_hundred_rows_keep_a_form_that_fills_the_chip(pkg, ops, dev):
     """An int8 linear whose eager form multiplies K slices of 256 x 256 tiles, with the channel scale on the fp32 sums, has no
     workspace for them while it is recorded: it runs the 128 x 128 form and the scale in a pass over the 16-bit result, not
